@@ -16,7 +16,7 @@
 // before i splits into the tiles of i's segment before i's tile (the "carry",
 // kept per d, a range of d for coarser levels) and the rank inside the tile.
 //
-// Tiles are segment-aligned (each covers <= MLD_T keys of one level-s node),
+// Tiles are segment-aligned (each covers <= 2^tl keys of one level-s node),
 // so every key of a tile shares the top s bits and a tile's ranks are those of
 // its own local subtree over the next g levels.  Per group:
 //   k_mld_count   per tile, the key count of each leaf d (wave ballots find
@@ -39,22 +39,22 @@
 #include "wtg_internal.hpp"
 #include <algorithm>
 #include <cstdlib>
-#include <vector>
+#include <type_traits>
 
 namespace {
 
-constexpr uint32_t MLD_T = 2048;            // keys per tile
+constexpr uint32_t MLD_WT = 2048;           // keys per wave of the count pass
 constexpr uint32_t MLD_GMAX = 8;            // levels per group
-constexpr uint32_t MLD_BW = MLD_T / 32 + 2; // staged bit words per level (+2 read-ahead pad)
-constexpr uint32_t MLD_CPW = MLD_T / 64 / 4; // 64-key chunks per wave
-static_assert(MLD_T / 64 <= 64, "the chunk prefix is one wave scan");
+constexpr uint32_t MLD_T4K_N = 21, MLD_T4K_NODE = 15;  // 4096-key tiles: log2 of the least keys, and per node
+constexpr uint32_t MLD_CPW = 8;             // 64-key chunks per wave of the emit pass
 constexpr uint32_t MLD_SR = 64;             // tiles per block of the carry scan
 
 struct MldArgs {
   const void* keys;          // P_s order; group 0: the input symbols (key type K)
   uint64_t n;
   uint32_t L, s, g;
-  uint32_t ntiles0;          // s == 0: ceil(n / MLD_T)
+  uint32_t tl;               // log2 of the keys per tile
+  uint32_t ntiles0;          // s == 0: ceil(n / 2^tl)
   const uint32_t* tstart;    // s > 0: 2^s + 1 entries, first tile of each level-s node
   const uint32_t* tseg;      // s > 0: the level-s node of each tile
   const uint32_t* cum_s;     // s > 0: 2^s + 1 entries, keys before each level-s node
@@ -82,11 +82,11 @@ __device__ __forceinline__ uint32_t mld_ntiles(const MldArgs& a) {
 __device__ __forceinline__ bool mld_tile(const MldArgs& a, uint32_t t, uint32_t& seg, uint64_t& base,
                                          uint32_t& len, uint32_t& first) {
   if (a.s == 0) {
-    const uint64_t off = (uint64_t)t * MLD_T;
+    const uint64_t off = (uint64_t)t << a.tl;
     if (t >= a.ntiles0 || off >= a.n) return false;
     seg = 0;
     base = off;
-    len = (uint32_t)(a.n - off < MLD_T ? a.n - off : MLD_T);
+    len = (uint32_t)(a.n - off < (1u << a.tl) ? a.n - off : 1u << a.tl);
     first = 0;
     return true;
   }
@@ -95,11 +95,11 @@ __device__ __forceinline__ bool mld_tile(const MldArgs& a, uint32_t t, uint32_t&
   const uint32_t lo = a.tseg[t];  // the segment of tile t (k_mld_tseg)
   seg = lo;
   first = a.tstart[lo];
-  const uint64_t off = (uint64_t)(t - first) * MLD_T;
+  const uint64_t off = (uint64_t)(t - first) << a.tl;
   const uint64_t cnt = a.cum_s[lo + 1] - a.cum_s[lo];
   if (off >= cnt) return false;  // (cannot happen for consistent tables)
   base = a.cum_s[lo] + off;
-  len = (uint32_t)(cnt - off < MLD_T ? cnt - off : MLD_T);
+  len = (uint32_t)(cnt - off < (1u << a.tl) ? cnt - off : 1u << a.tl);
   return true;
 }
 
@@ -144,24 +144,17 @@ __device__ __forceinline__ uint32_t word_leaf(const mld_u4& q, uint32_t e, uint3
   }
 }
 
-// leaf counts of the tiles, one wave per MLD_CNT_TPW<K> consecutive tiles (no
-// block barrier; byte and 16-bit keys take several tiles per wave, so each
-// wave reads 8 KiB).  A tile's keys are read as the aligned 16-byte words
-// that cover them, the loads of all of the wave's tiles in flight at once;
-// counting needs no key order, so every element of every word is counted (LDS
-// atomics; a slot whose 64 elements share one leaf adds once) and the
-// elements of the two edge words that lie outside the tile are taken back
-// afterwards.  The aligned words never leave the pages of the tile's own bytes.
+// leaf counts of the tiles, one wave per MLD_WT keys of a tile (the waves of a
+// tile share its counters).  A wave's keys are read as the aligned 16-byte
+// words that cover them, all loads in flight at once; counting needs no key
+// order, so every element of every word is counted (LDS atomics; a slot whose
+// 64 elements share one leaf adds once) and the elements of the two edge words
+// that lie outside the wave's range are taken back afterwards.  The aligned
+// words never leave the pages of the range's own bytes.
 // Trees of at most SG leaves per tile (SG > 0) count by ballots instead: per
 // slot and leaf one ballot of the lanes holding it, the counts in scalar
 // registers (a few leaves would otherwise put every lane's atomic on one of a
 // few LDS words).
-// tiles per wave of the count kernel: one for every key width, so small
-// trees keep enough waves in flight (2^24 byte keys: 23 vs 31 us with four
-// tiles per wave; the batched 16-bit keys: 239 vs 236 Gsym/s with two)
-template <typename K>
-constexpr uint32_t mld_cnt_tpw() { return 1u; }
-
 __device__ __forceinline__ void wave_sync_lds_mld() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -172,51 +165,49 @@ typedef const __attribute__((address_space(1))) mld_u4* mld_gword;
 
 template <typename K, uint32_t SG>
 __global__ __launch_bounds__(256) void k_mld_count(MldArgs a) {
-  constexpr uint32_t KW = sizeof(K), E = 16 / KW, TPW = mld_cnt_tpw<K>();
-  constexpr uint32_t NW = (MLD_T * KW / 16 + 1 + 63) / 64;  // words per lane (a tile covers <= T*KW/16 + 1)
-  __shared__ uint32_t s_cnt_all[4][TPW][1u << MLD_GMAX];
+  constexpr uint32_t KW = sizeof(K), E = 16 / KW;
+  constexpr uint32_t NW = (MLD_WT * KW / 16 + 1 + 63) / 64;  // words per lane (a range covers <= WT*KW/16 + 1)
+  __shared__ uint32_t s_cnt_all[4][1u << MLD_GMAX];
   const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t G = 1u << a.g, lane = (uint32_t)lane_id();
-  uintptr_t b0[TPW], b1[TPW], w0[TPW];
-  uint64_t pbase[TPW];
-  uint32_t nw[TPW], tt[TPW], plen[TPW];
-  bool ok[TPW];
-  mld_u4 v[TPW][NW];
-#pragma unroll
-  for (uint32_t u = 0; u < TPW; u++) {
-    uint32_t seg, len, first;
-    uint64_t base;
-    tt[u] = (blockIdx.x * 4 + w) * TPW + u;
-    ok[u] = mld_tile(a, tt[u], seg, base, len, first);  // wave-uniform
-    b0[u] = b1[u] = w0[u] = 0;
-    nw[u] = 0;
-    pbase[u] = base;
-    plen[u] = len;
-    if (ok[u]) {
-      b0[u] = (uintptr_t)a.keys + mld_src(a, seg, base) * KW;
-      b1[u] = b0[u] + (uintptr_t)len * KW;
-      w0[u] = b0[u] & ~(uintptr_t)15;
-      nw[u] = (uint32_t)((b1[u] - w0[u] + 15) >> 4);
-    }
-    const mld_gword wp = (mld_gword)w0[u];
+  const uint32_t wl = a.tl - __builtin_ctz(MLD_WT);  // log2 of the waves per tile (0..2)
+  const uint32_t t = (blockIdx.x * 4 + w) >> wl, sub = w & ((1u << wl) - 1);
+  uint32_t* s_cnt = s_cnt_all[w >> wl];
+  uint32_t seg, len = 0, first;
+  uint64_t base = 0;
+  const bool ok = mld_tile(a, t, seg, base, len, first);  // wave-uniform
+  // this wave's keys: [base, base + len) from here on
+  const uint32_t at = sub * MLD_WT;
+  uintptr_t b0 = 0, b1 = 0, w0 = 0;
+  uint32_t nw = 0;
+  if (ok && at < len) {
+    b0 = (uintptr_t)a.keys + (mld_src(a, seg, base) + at) * KW;
+    len = len - at < MLD_WT ? len - at : MLD_WT;
+    base += at;
+    b1 = b0 + (uintptr_t)len * KW;
+    w0 = b0 & ~(uintptr_t)15;
+    nw = (uint32_t)((b1 - w0 + 15) >> 4);
+  } else {
+    len = 0;
+  }
+  mld_u4 v[NW];
+  {
+    const mld_gword wp = (mld_gword)w0;
 #pragma unroll
     for (uint32_t m = 0; m < NW; m++) {
       const uint32_t k = m * 64 + lane;
-      v[u][m] = k < nw[u] ? wp[k] : mld_u4{0u, 0u, 0u, 0u};
+      v[m] = k < nw ? wp[k] : mld_u4{0u, 0u, 0u, 0u};
     }
   }
-  if (!ok[0]) return;
-  // clear the group's level words: a tile clears, at each of the group's
+  // clear the group's level words: a range clears, at each of the group's
   // levels, the words whose first bit falls on one of its positions (the
   // positions of a level-s node keep their range at every later level), so
   // every word is cleared once, by the group of its first bit's level, before
   // that group's emit ORs into it
-#pragma unroll
-  for (uint32_t u = 0; u < TPW; u++) {
-    if (!ok[u]) break;
+  if (len) {
     for (uint32_t j = 0; j < a.g; j++) {
       const uint64_t lb = (uint64_t)(a.s + j - a.lvl0) * a.n;
-      const uint64_t wa = (lb + pbase[u] + 63) >> 6, wb = (lb + pbase[u] + plen[u] + 63) >> 6;
+      const uint64_t wa = (lb + base + 63) >> 6, wb = (lb + base + len + 63) >> 6;
       for (uint64_t k = wa + lane; k < wb; k += 64) a.words[k] = 0ull;
     }
   }
@@ -237,78 +228,66 @@ __global__ __launch_bounds__(256) void k_mld_count(MldArgs a) {
       cm_lo = cm_hi = hm * (B == 8 ? 0x01010101u : B == 16 ? 0x00010001u : 1u);
     }
   }
-#pragma unroll
-  for (uint32_t u = 0; u < TPW; u++)
-    for (uint32_t i = lane; i < G; i += 64) s_cnt_all[w][u][i] = 0;
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (sub == 0)
+    for (uint32_t i = lane; i < G; i += 64) s_cnt[i] = 0;
+  if (wl) __syncthreads();
+  else wave_sync_lds_mld();
   uint32_t acc_lo = 0, acc_hi = 0;  // OR of the interior words (edge words are tested per key below)
   bool bad = false;
+  uint32_t sc[SG > 0 ? SG : 1];  // SG > 0: the counts per leaf (wave-uniform)
 #pragma unroll
-  for (uint32_t u = 0; u < TPW; u++) {
-    if (!ok[u]) break;  // wave-uniform (later tiles are past the end too)
-    uint32_t* s_cnt = s_cnt_all[w][u];
-    uint32_t sc[SG > 0 ? SG : 1];  // SG > 0: the counts per leaf (wave-uniform)
+  for (uint32_t d = 0; d < (SG > 0 ? SG : 1); d++) sc[d] = 0;
 #pragma unroll
-    for (uint32_t d = 0; d < (SG > 0 ? SG : 1); d++) sc[d] = 0;
+  for (uint32_t m = 0; m < NW; m++) {
+    if (m * 64 >= nw) break;  // wave-uniform
+    const uint32_t k = m * 64 + lane;
+    const bool act = k < nw;
+    const uint32_t nact = popc64(wave_ballot(act));
+    if (act && k > 0 && k + 1 < nw) {
+      acc_lo |= v[m].x | v[m].z;
+      acc_hi |= v[m].y | v[m].w;
+    }
 #pragma unroll
-    for (uint32_t m = 0; m < NW; m++) {
-      if (m * 64 >= nw[u]) break;  // wave-uniform
-      const uint32_t k = m * 64 + lane;
-      const bool act = k < nw[u];
-      const uint32_t nact = popc64(wave_ballot(act));
-      if (act && k > 0 && k + 1 < nw[u]) {
-        acc_lo |= v[u][m].x | v[u][m].z;
-        acc_hi |= v[u][m].y | v[u][m].w;
-      }
+    for (uint32_t e = 0; e < E; e++) {
+      const uint32_t d = word_leaf<K>(v[m], e, tsh, gw, gmask);
+      if constexpr (SG > 0) {
 #pragma unroll
-      for (uint32_t e = 0; e < E; e++) {
-        const uint32_t d = word_leaf<K>(v[u][m], e, tsh, gw, gmask);
-        if constexpr (SG > 0) {
-#pragma unroll
-          for (uint32_t q = 0; q < SG; q++) sc[q] += popc64(wave_ballot(act && d == q));
-        } else {
-          const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);  // lane 0 is active
-          if (wave_ballot(act && d != d0) == 0) {
-            if (lane == 0) atomicAdd(&s_cnt[d0], nact);
-          } else if (act) {
-            atomicAdd(&s_cnt[d], 1u);
-          }
+        for (uint32_t q = 0; q < SG; q++) sc[q] += popc64(wave_ballot(act && d == q));
+      } else {
+        const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);  // lane 0 is active
+        if (wave_ballot(act && d != d0) == 0) {
+          if (lane == 0) atomicAdd(&s_cnt[d0], nact);
+        } else if (act) {
+          atomicAdd(&s_cnt[d], 1u);
         }
       }
     }
-    if constexpr (SG > 0) {
+  }
+  if constexpr (SG > 0) {
 #pragma unroll
-      for (uint32_t q = 0; q < SG; q++)
-        if (lane == q && q < G) s_cnt[q] = sc[q];
-      wave_sync_lds_mld();
-    }
-    // edge words: elements outside [b0, b1) were counted above; the others
-    // get the per-key bad-key test
-    if (lane < 2 && (lane == 0 || nw[u] > 1)) {
-      const uint32_t k = lane == 0 ? 0u : nw[u] - 1;
-      const mld_u4 q = ((mld_gword)w0[u])[k];
+    for (uint32_t q = 0; q < SG; q++)
+      if (lane == q && q < G && nw) atomicAdd(&s_cnt[q], sc[q]);
+  }
+  // edge words: elements outside [b0, b1) were counted above; the others
+  // get the per-key bad-key test
+  if (nw && lane < 2 && (lane == 0 || nw > 1)) {
+    const uint32_t k = lane == 0 ? 0u : nw - 1;
+    const mld_u4 q = ((mld_gword)w0)[k];
 #pragma unroll
-      for (uint32_t e = 0; e < E; e++) {
-        const uintptr_t ea = w0[u] + 16 * (uintptr_t)k + e * KW;
-        if (ea < b0[u] || ea >= b1[u]) {
-          atomicSub(&s_cnt[word_leaf<K>(q, e, tsh, gw, gmask)], 1u);
-        } else if (a.check && (word_elem<K>(q, e) >> a.chk_shift) != 0) {
-          bad = true;
-        }
+    for (uint32_t e = 0; e < E; e++) {
+      const uintptr_t ea = w0 + 16 * (uintptr_t)k + e * KW;
+      if (ea < b0 || ea >= b1) {
+        atomicSub(&s_cnt[word_leaf<K>(q, e, tsh, gw, gmask)], 1u);
+      } else if (a.check && (word_elem<K>(q, e) >> a.chk_shift) != 0) {
+        bad = true;
       }
     }
   }
   if (bad || ((acc_lo & cm_lo) | (acc_hi & cm_hi)) != 0) atomicOr(a.err, WTG_FLAG_BADSYM);
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-  for (uint32_t u = 0; u < TPW; u++) {
-    if (!ok[u]) break;
-    for (uint32_t i = lane; i < G; i += 64) a.tcnt_w[(uint64_t)tt[u] * G + i] = s_cnt_all[w][u][i];
-  }
+  if (wl) __syncthreads();
+  else wave_sync_lds_mld();
+  if (ok)  // the waves of a tile write its counts in turns of 64 leaves
+    for (uint32_t i = lane + 64 * sub; i < G; i += 64u << wl) a.tcnt_w[(uint64_t)t * G + i] = s_cnt[i];
 }
 
 // column-wise exclusive prefix of the leaf counts over the tiles, blocks of
@@ -398,10 +377,10 @@ __global__ __launch_bounds__(256) void k_mld_hist(MldArgs a, uint32_t* __restric
 
 // tiles of each level-(s+g) node for the next group
 __global__ __launch_bounds__(256) void k_mld_ntiles(const uint32_t* __restrict__ cum, uint64_t nseg,
-                                                    uint32_t* __restrict__ nt) {
+                                                    uint32_t* __restrict__ nt, uint32_t tl) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nseg) return;
-  nt[i] = (cum[i + 1] - cum[i] + MLD_T - 1) / MLD_T;
+  nt[i] = (uint32_t)(((uint64_t)(cum[i + 1] - cum[i]) + (1u << tl) - 1) >> tl);
 }
 
 // tile -> segment map, one thread per tile: the last segment k with
@@ -440,23 +419,48 @@ __device__ __forceinline__ uint64_t lds_bits64(const uint32_t* row, uint32_t p) 
   return o ? (lo >> o) | (hi << (64 - o)) : lo;
 }
 
-template <typename K, bool SCATTER>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_mld_emit(MldArgs a) {
+// exclusive scan of one value per thread over the block's first 256 threads
+// (the others hold 0 and take part in the barriers only)
+template <bool DPP>
+__device__ __forceinline__ uint32_t mld_scan256(uint32_t v, uint32_t* s_wave, uint32_t& total) {
+  const uint32_t w = threadIdx.x >> 6, l = (uint32_t)lane_id();
+  const uint32_t incl = DPP ? wave_incl_sum_dpp(v) : wave_incl_scan_shfl(v);
+  if (l == 63 && w < 4) s_wave[w] = incl;
+  __syncthreads();
+  uint32_t off = 0, tot = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < 4; k++) {
+    const uint32_t t = s_wave[k];
+    if (k < w) off += t;
+    tot += t;
+  }
+  __syncthreads();
+  total = tot;
+  return incl - v + off;
+}
+
+// T keys per tile (mld_tile_log), T / 8 threads (8 chunks of 64 keys per wave).
+// Bound by VALU issue and the barriers between levels, not by memory
+template <typename K, bool SCATTER, uint32_t T>
+__global__ __launch_bounds__(T / 8) __attribute__((amdgpu_waves_per_eu(8))) void k_mld_emit(MldArgs a) {
+  constexpr uint32_t NT = T / 8, NWV = NT / 64;
+  constexpr uint32_t BW = T / 32 + 2;  // staged bit words per level (+2 read-ahead pad)
+  static_assert(T / 64 <= 64 && NT >= 256, "the chunk prefix is one wave scan; 256 threads build the tables");
   // block scans by DPP moves in the bits-only pass, by shuffles in the pass
   // with key output (measured: the DPP form made the key-output pass 9%
   // slower and the bits-only pass faster: C2 5.68 -> 5.59 ms, C4 9.22 -> 8.96 ms)
   constexpr bool MLD_SCAN_DPP = !SCATTER;
   // LDS of the level pipeline: keys (ping-pong), tile prefix and staged bits
-  // (under 20 KiB at 2048-key tiles)
-  __shared__ __align__(16) uint32_t s_k[2][MLD_T];   // the tile's keys in its level order
-  static_assert(MLD_T <= 65535, "tile positions fit 16 bits");
+  // (20 KiB at 2048-key tiles, 39 KiB at 4096)
+  __shared__ __align__(16) uint32_t s_k[2][T];   // the tile's keys in its level order
+  static_assert(T <= 65535, "tile positions fit 16 bits");
   __shared__ uint16_t s_tpre[(1u << MLD_GMAX) + 1];   // exclusive prefix over d of the tile's counts
-  __shared__ __align__(8) uint32_t s_bits[MLD_GMAX][MLD_BW];  // level bits in the tile's level order
-  static_assert(MLD_BW % 2 == 0, "64-bit rows");
+  __shared__ __align__(8) uint32_t s_bits[MLD_GMAX][BW];  // level bits in the tile's level order
+  static_assert(BW % 2 == 0, "64-bit rows");
   __shared__ uint32_t s_nxy[(1u << MLD_GMAX) - 1];    // node tables of the levels (see below)
   __shared__ uint32_t s_lvl0[MLD_GMAX];
   __shared__ uint32_t s_wave[4];
-  __shared__ uint16_t s_ex[4][MLD_T / 64];  // per wave: zeros before each chunk of the level
+  __shared__ uint16_t s_ex[NWV][T / 64];  // per wave: zeros before each chunk of the level
   uint32_t seg, len, first;
   uint64_t base;
   const uint32_t t = blockIdx.x;
@@ -465,38 +469,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
   const uint32_t g = a.g, G = 1u << g, lane = (uint32_t)lane_id();
   const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t sh = a.L - a.s - g;
-  // carry and tile counts per leaf, their exclusive prefixes over d; thread d
-  // keeps its leaf's node start and carry prefix in registers until the
-  // write-out (they then go to the free key buffer)
+  // the tile's leaf counts and their exclusive prefix over d
   uint32_t xk[MLD_CPW];  // the wave's chunks c = w + 4m, one key per lane
-  uint32_t cum_d = 0, cpre_d, ctot;
   {
     const uint32_t d = threadIdx.x;
-    uint32_t cv = 0, tv = 0;
-    if (d < G) {
-      cv = mld_prefix(a, t, d) - mld_prefix(a, first, d);
-      tv = a.tcnt[(uint64_t)t * G + d];
-      cum_d = a.cum[((uint64_t)seg << g) + d];
-    }
+    const uint32_t tv = d < G ? a.tcnt[(uint64_t)t * G + d] : 0u;
     // the tile's keys go straight to registers (level s needs no LDS copy);
     // all loads are in flight together with the tables above (unconditional:
     // positions past the tile load the tile's first key, replaced below)
     K kr[MLD_CPW];
 #pragma unroll
     for (uint32_t m = 0; m < MLD_CPW; m++) {
-      const uint32_t p = (w + 4 * m) * 64 + lane;
+      const uint32_t p = (w + NWV * m) * 64 + lane;
       kr[m] = reinterpret_cast<const K*>(a.keys)[src + (p < len ? p : 0u)];
     }
-    cpre_d = block_excl_scan_u32<MLD_SCAN_DPP>(cv, s_wave, ctot);
     uint32_t tot;
-    const uint32_t te = block_excl_scan_u32<MLD_SCAN_DPP>(tv, s_wave, tot);
+    const uint32_t te = mld_scan256<MLD_SCAN_DPP>(tv, s_wave, tot);
     if (d < G) s_tpre[d] = (uint16_t)te;
     if (d == 0) s_tpre[G] = (uint16_t)tot;
     // positions past the tile hold the pad key ~0: a one at every level, in
     // the last node, so each split leaves it where it is (behind the real keys)
 #pragma unroll
     for (uint32_t m = 0; m < MLD_CPW; m++) {
-      const uint32_t p = (w + 4 * m) * 64 + lane;
+      const uint32_t p = (w + NWV * m) * 64 + lane;
       xk[m] = p < len ? (uint32_t)((uint64_t)kr[m] >> a.kshift) : ~0u;
     }
   }
@@ -517,7 +512,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
       zn = s_tpre[(2 * q + 1) << (sgj - 1)] - S;
     }
     uint32_t tot;
-    const uint32_t zx = block_excl_scan_u32<MLD_SCAN_DPP>(zn, s_wave, tot);  // over all entries; each level rebased below
+    const uint32_t zx = mld_scan256<MLD_SCAN_DPP>(zn, s_wave, tot);  // over all entries; each level rebased below
     if (r < G - 1 && r + 1 == (1u << j)) s_lvl0[j] = zx;
     __syncthreads();
     if (r < G - 1) {
@@ -531,56 +526,75 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
   // contiguous); the ballots of the level bit in that order are the level's
   // bits, and a stable split of every node by that bit gives the next order
   const uint32_t nch = (len + 63) >> 6;
-  for (uint32_t j = 0; j < g; j++) {
-    const uint32_t* A = s_k[j & 1];
-    uint32_t* B = s_k[(j + 1) & 1];
-    const uint32_t bp = sh + g - 1 - j;  // the key bit of level s+j
-    // the wave's chunks, all loads first; the keys stay in registers until
-    // the split below
-    if (j > 0) {
-#pragma unroll
-      for (uint32_t m = 0; m < MLD_CPW; m++) xk[m] = A[(w + 4 * m) * 64 + lane];
+  const auto levels = [&](auto chunks) __attribute__((always_inline)) {
+    constexpr uint32_t M = decltype(chunks)::value;  // chunks per wave
+    for (uint32_t j = 0; j < g; j++) {
+      const uint32_t* A = s_k[j & 1];
+      uint32_t* B = s_k[(j + 1) & 1];
+      const uint32_t bp = sh + g - 1 - j;  // the key bit of level s+j
+      // the wave's chunks, all loads first; the keys stay in registers until
+      // the split below
+      if (j > 0) {
+  #pragma unroll
+        for (uint32_t m = 0; m < M; m++) xk[m] = A[(w + NWV * m) * 64 + lane];
+      }
+  #pragma unroll
+      for (uint32_t m = 0; m < M; m++) {
+        const uint64_t ones = wave_ballot((xk[m] >> bp) & 1u);
+        if (lane == 0) reinterpret_cast<uint64_t*>(s_bits[j])[w + NWV * m] = ones;
+      }
+      if (j + 1 == g && !SCATTER) break;  // the last level's order is not needed
+      __syncthreads();
+      // every wave: exclusive prefix of the chunk zeros (lane = chunk), into the
+      // wave's own row so that each chunk reads its base with one broadcast
+      // load; zeros before tile position p = that prefix + zeros of p's chunk
+      // below p
+      const uint32_t v = lane < nch ? 64u - popc64(reinterpret_cast<const uint64_t*>(s_bits[j])[lane]) : 0u;
+      const uint32_t incl = wave_incl_scan_dpp(v);
+      if (lane < T / 64) s_ex[w][lane] = (uint16_t)(incl - v);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      // stable split of each node: its zeros first, then its ones.  Every
+      // chunk of the tile takes part (chunks past the keys hold pad keys,
+      // which stay in place), so the node lookups of all chunks are issued
+      // before the first is used
+      const uint32_t* nt = s_nxy + (1u << j) - 1;
+      uint32_t xy[M];
+  #pragma unroll
+      for (uint32_t m = 0; m < M; m++) xy[m] = nt[__builtin_amdgcn_ubfe(xk[m], bp + 1, j)];
+  #pragma unroll
+      for (uint32_t m = 0; m < M; m++) {
+        const uint32_t c = w + NWV * m;
+        const uint32_t p = c * 64 + lane;
+        const uint32_t x = xk[m];
+        const bool zero = ((x >> bp) & 1u) == 0;
+        const uint64_t zm = wave_ballot(zero);
+        const uint32_t cz = s_ex[w][c];
+        const uint32_t zc = __builtin_amdgcn_mbcnt_hi((uint32_t)(zm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)zm, cz));
+        const uint32_t d0 = (xy[m] & 0xFFFFu) + zc, d1 = (xy[m] >> 16) + p - zc;
+        B[zero ? d0 : d1] = x;
+      }
+      __syncthreads();
     }
-#pragma unroll
-    for (uint32_t m = 0; m < MLD_CPW; m++) {
-      const uint64_t ones = wave_ballot((xk[m] >> bp) & 1u);
-      if (lane == 0) reinterpret_cast<uint64_t*>(s_bits[j])[w + 4 * m] = ones;
+  };
+  // the last tile of a segment is often short: up to a quarter of a tile takes
+  // a quarter of the chunks
+  if (nch > 2 * NWV) levels(std::integral_constant<uint32_t, MLD_CPW>{});
+  else levels(std::integral_constant<uint32_t, 2>{});
+  // each leaf's node start and carry (keys of the leaf in its segment's earlier
+  // tiles), the carry's exclusive prefix over d: read here, not before the
+  // level pipeline, whose registers they would take
+  uint32_t cum_d = 0, cpre_d, ctot;
+  {
+    const uint32_t d = threadIdx.x;
+    uint32_t cv = 0;
+    if (d < G) {
+      cv = mld_prefix(a, t, d) - mld_prefix(a, first, d);
+      cum_d = a.cum[((uint64_t)seg << g) + d];
     }
-    if (j + 1 == g && !SCATTER) break;  // the last level's order is not needed
-    __syncthreads();
-    // every wave: exclusive prefix of the chunk zeros (lane = chunk), into the
-    // wave's own row so that each chunk reads its base with one broadcast
-    // load; zeros before tile position p = that prefix + zeros of p's chunk
-    // below p
-    const uint32_t v = lane < nch ? 64u - popc64(reinterpret_cast<const uint64_t*>(s_bits[j])[lane]) : 0u;
-    const uint32_t incl = wave_incl_scan_dpp(v);
-    if (lane < MLD_T / 64) s_ex[w][lane] = (uint16_t)(incl - v);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // stable split of each node: its zeros first, then its ones.  Every
-    // chunk of the tile takes part (chunks past the keys hold pad keys,
-    // which stay in place), so the node lookups of all chunks are issued
-    // before the first is used
-    const uint32_t* nt = s_nxy + (1u << j) - 1;
-    uint32_t xy[MLD_CPW];
-#pragma unroll
-    for (uint32_t m = 0; m < MLD_CPW; m++) xy[m] = nt[__builtin_amdgcn_ubfe(xk[m], bp + 1, j)];
-#pragma unroll
-    for (uint32_t m = 0; m < MLD_CPW; m++) {
-      const uint32_t c = w + 4 * m;
-      const uint32_t p = c * 64 + lane;
-      const uint32_t x = xk[m];
-      const bool zero = ((x >> bp) & 1u) == 0;
-      const uint64_t zm = wave_ballot(zero);
-      const uint32_t cz = s_ex[w][c];
-      const uint32_t zc = __builtin_amdgcn_mbcnt_hi((uint32_t)(zm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)zm, cz));
-      const uint32_t d0 = (xy[m] & 0xFFFFu) + zc, d1 = (xy[m] >> 16) + p - zc;
-      B[zero ? d0 : d1] = x;
-    }
-    __syncthreads();
+    cpre_d = mld_scan256<MLD_SCAN_DPP>(cv, s_wave, ctot);  // (its barriers end the pipeline too)
   }
-  __syncthreads();
   // write the level bits: for level s+j the tile's keys of local node q form
   // one run at NodeStart + carry.  Thread r < G-1 describes run r = (j, q);
   // then the destination words of all runs are dealt out over the block.
@@ -595,7 +609,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
   uint32_t* s_rw = reinterpret_cast<uint32_t*>(rt + 4096);         // first destination word item
   uint32_t* s_cpre = reinterpret_cast<uint32_t*>(rt + 5248);       // carry prefix over d (G + 1)
   uint32_t* s_lb = reinterpret_cast<uint32_t*>(rt + 6400);         // leaf d's key at tile position i goes to s_lb[d] + i
-  static_assert(6400 + 4 * (1u << MLD_GMAX) <= 4 * MLD_T, "tables fit one key buffer");
+  static_assert(6400 + 4 * (1u << MLD_GMAX) <= 4 * T, "tables fit one key buffer");
   uint32_t* s_cum = s_lb;  // node starts first, leaf bases after the run tables are built
   if (threadIdx.x < G) {
     s_cpre[threadIdx.x] = cpre_d;
@@ -622,14 +636,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
       s_rcnt[r] = cnt;
     }
     uint32_t tot;
-    const uint32_t ex = block_excl_scan_u32<MLD_SCAN_DPP>(nw, s_wave, tot);  // (its barriers order the s_cum reads above)
+    const uint32_t ex = mld_scan256<MLD_SCAN_DPP>(nw, s_wave, tot);  // (its barriers order the s_cum reads above)
     if (r < nruns) s_rw[r] = ex;
     if (r == 0) s_rw[nruns] = tot;
     if (SCATTER && r < G) s_lb[r] = cum_d + (s_cpre[r + 1] - s_cpre[r]) - s_tpre[r];
     __syncthreads();
   }
   const uint32_t nwords = s_rw[nruns];
-  for (uint32_t it = threadIdx.x; it < nwords; it += 256) {
+  for (uint32_t it = threadIdx.x; it < nwords; it += NT) {
     uint32_t lo = 0, hi = nruns;  // the last run whose first word item is <= it
     while (hi - lo > 1) {
       const uint32_t mid = (lo + hi) >> 1;
@@ -650,7 +664,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     // keys in leaf order to their P_{s+g} positions
 #pragma unroll
     for (uint32_t m = 0; m < MLD_CPW; m++) {
-      const uint32_t i = (w + 4 * m) * 64 + lane;
+      const uint32_t i = (w + NWV * m) * 64 + lane;
       if (i < len) {
         const uint32_t x = s_k[g & 1][i];
         const uint32_t dest = s_lb[(x >> sh) & (G - 1)] + i;
@@ -698,11 +712,24 @@ __global__ void k_mld_nonzero(const uint32_t* __restrict__ h, uint64_t n, unsign
 }
 
 struct MldPlan {
-  uint32_t ngroups, gs[4], gg[4];
+  uint32_t ngroups, gs[4], gg[4], gt[4];
   uint64_t maxtiles, maxblocks, maxbins;
   size_t off_keys[2], off_tcnt, off_ploc, off_bsum, off_bpre, off_hist, off_cum[2], off_tst, off_nt, off_tseg,
       off_scst, off_ctr, total;
 };
+
+// log2 of the keys per tile of a group of g levels over n keys in 2^s nodes.
+// An 8-level group's tables (256 leaves, 255 runs, a partial word at each end
+// of a run) cost a 2048-key tile about what its keys do, so it takes 4096-key
+// tiles (512 threads): n = 2^24 bytes, emit 140 -> 95 us; 2^27 uniform bytes in
+// 339 sequences 725 -> 593 us.  Narrower groups keep 2048 keys, whose blocks
+// wait for half as many waves at each of the level barriers (5 levels 387 us
+// against 416, 2 levels 217 against 249, a last group of 6 levels 956 against
+// 1068), and so do small inputs and small nodes, where 4096-key tiles would
+// leave the chip or the tiles partly empty.
+uint32_t mld_tile_log(uint64_t n, uint32_t s, uint32_t g) {
+  return g == MLD_GMAX && n >= (1ull << MLD_T4K_N) && (n >> s) >= (1ull << MLD_T4K_NODE) ? 12 : 11;
+}
 
 MldPlan mld_plan(uint64_t n, uint32_t L, uint32_t s0) {
   MldPlan P{};
@@ -717,11 +744,12 @@ MldPlan mld_plan(uint64_t n, uint32_t L, uint32_t s0) {
     left--;
     P.gs[P.ngroups] = s;
     P.gg[P.ngroups] = g;
+    P.gt[P.ngroups] = mld_tile_log(n, s, g);
     P.ngroups++;
     s += g;
   }
   // a group over level-s nodes has at most ceil(n/T) + min(n, 2^s) tiles
-  P.maxtiles = wtg_ceil_div(n, MLD_T) + std::min<uint64_t>(n, 1ull << P.gs[P.ngroups - 1]) + 1;
+  P.maxtiles = wtg_ceil_div(n, MLD_WT) + std::min<uint64_t>(n, 1ull << P.gs[P.ngroups - 1]) + 1;
   P.maxblocks = wtg_ceil_div(P.maxtiles + 1, MLD_SR) + 1;
   P.maxbins = 1ull << L;
   size_t o = 0;
@@ -742,6 +770,17 @@ MldPlan mld_plan(uint64_t n, uint32_t L, uint32_t s0) {
   P.off_ctr = o; o = wtg_align256(o + 256);  // right after the scan states: one fill clears both
   P.total = o;
   return P;
+}
+
+template <typename K, uint32_t T>
+void mld_emit_launch(wtg_ctx* ctx, bool first, bool last, unsigned grid, const MldArgs& a) {
+  if (first) {
+    if (last) WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<K, false, T>), dim3(grid), dim3(T / 8), 0, a);
+    else WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<K, true, T>), dim3(grid), dim3(T / 8), 0, a);
+  } else {
+    if (last) WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<uint32_t, false, T>), dim3(grid), dim3(T / 8), 0, a);
+    else WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<uint32_t, true, T>), dim3(grid), dim3(T / 8), 0, a);
+  }
 }
 
 // Levels [s0, L) of the keys d_sym (in P_{s0} order: sorted by their top s0
@@ -770,7 +809,7 @@ int mld_build_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint32_t s
   uint32_t* kbuf[2] = {(uint32_t*)(ws + P.off_keys[0]), (uint32_t*)(ws + P.off_keys[1])};
   // (the level words are cleared by the leaf-count passes)
   if (d_distinct) WTG_TRY(wtg_fill_u64(ctx, d_distinct, 1, 0));
-  const uint32_t ntiles0 = (uint32_t)wtg_ceil_div(n, MLD_T);
+  const uint32_t ntiles0 = (uint32_t)wtg_ceil_div(n, 1u << P.gt[0]);
   const void* src = d_sym;
   const uint32_t* cum_prev = nullptr;
   if (s0 > 0) {
@@ -782,20 +821,20 @@ int mld_build_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint32_t s
                ctr, ctx->d_flag);
     WTG_LAUNCH_CHECK();
     WTG_LAUNCH(ctx, "mld_ntiles", k_mld_ntiles, dim3((unsigned)wtg_ceil_div(nb0, 256)), dim3(256), 0, cum[1], nb0,
-               nt);
+               nt, P.gt[0]);
     WTG_LAUNCH_CHECK();
     WTG_TRY(wtg_fill_bytes_zero(ctx, scst, (char*)ctr + 256 - (char*)scst));
     WTG_LAUNCH(ctx, "mld_tiles", k_scan_u32<uint32_t>, dim3((unsigned)st0), dim3(256), 0, nt, tst, nb0, scst, ctr,
                ctx->d_flag);
     WTG_LAUNCH_CHECK();
-    const uint64_t nt0 = wtg_ceil_div(n, MLD_T) + std::min<uint64_t>(n, nb0);
+    const uint64_t nt0 = wtg_ceil_div(n, 1u << P.gt[0]) + std::min<uint64_t>(n, nb0);
     WTG_LAUNCH(ctx, "mld_tseg", k_mld_tseg, dim3((unsigned)wtg_ceil_div(nt0, 256)), dim3(256), 0, tst, nb0, tseg,
                (uint64_t)P.maxtiles);
     WTG_LAUNCH_CHECK();
     cum_prev = cum[1];
   }
   for (uint32_t gi = 0; gi < P.ngroups; gi++) {
-    const uint32_t s = P.gs[gi], g = P.gg[gi], G = 1u << g;
+    const uint32_t s = P.gs[gi], g = P.gg[gi], G = 1u << g, tl = P.gt[gi];
     const bool last = gi + 1 == P.ngroups;
     MldArgs a{};
     a.keys = src;
@@ -803,6 +842,7 @@ int mld_build_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint32_t s
     a.L = L;
     a.s = s;
     a.g = g;
+    a.tl = tl;
     a.ntiles0 = ntiles0;
     a.tstart = s ? tst : nullptr;
     a.tseg = s ? tseg : nullptr;
@@ -822,16 +862,15 @@ int mld_build_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint32_t s
     a.kout = last ? nullptr : kbuf[gi & 1];
     a.err = ctx->d_flag;
     // grid: an upper bound of the tiles (blocks past the real count exit)
-    const uint64_t grid = s == 0 ? ntiles0 : wtg_ceil_div(n, MLD_T) + std::min<uint64_t>(n, 1ull << s);
+    const uint64_t grid = s == 0 ? ntiles0 : wtg_ceil_div(n, 1u << tl) + std::min<uint64_t>(n, 1ull << s);
     const uint32_t nrows = (uint32_t)grid + 1;
     const uint32_t nblocks = (uint32_t)wtg_ceil_div(nrows, MLD_SR);
+    const dim3 cg((unsigned)wtg_ceil_div(grid, (uint64_t)4 * MLD_WT >> tl));  // 4 waves of MLD_WT keys per block
     if (gi == 0) {
-      const dim3 cg((unsigned)wtg_ceil_div(grid, 4 * mld_cnt_tpw<K>()));
       if (G <= 4) WTG_LAUNCH(ctx, "mld_count", (k_mld_count<K, 4>), cg, dim3(256), 0, a);
       else if (G <= 8) WTG_LAUNCH(ctx, "mld_count", (k_mld_count<K, 8>), cg, dim3(256), 0, a);
       else WTG_LAUNCH(ctx, "mld_count", (k_mld_count<K, 0>), cg, dim3(256), 0, a);
     } else {
-      const dim3 cg((unsigned)wtg_ceil_div(grid, 4));
       if (G <= 4) WTG_LAUNCH(ctx, "mld_count", (k_mld_count<uint32_t, 4>), cg, dim3(256), 0, a);
       else if (G <= 8) WTG_LAUNCH(ctx, "mld_count", (k_mld_count<uint32_t, 8>), cg, dim3(256), 0, a);
       else WTG_LAUNCH(ctx, "mld_count", (k_mld_count<uint32_t, 0>), cg, dim3(256), 0, a);
@@ -856,24 +895,19 @@ int mld_build_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint32_t s
       WTG_LAUNCH_CHECK();
     }
     // the level bits of the group (and the keys in P_{s+g} order)
-    if (gi == 0) {
-      if (last) WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<K, false>), dim3((unsigned)grid), dim3(256), 0, a);
-      else WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<K, true>), dim3((unsigned)grid), dim3(256), 0, a);
-    } else {
-      if (last) WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<uint32_t, false>), dim3((unsigned)grid), dim3(256), 0, a);
-      else WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<uint32_t, true>), dim3((unsigned)grid), dim3(256), 0, a);
-    }
+    if (tl == 12) mld_emit_launch<K, 4096>(ctx, gi == 0, last, (unsigned)grid, a);
+    else mld_emit_launch<K, 2048>(ctx, gi == 0, last, (unsigned)grid, a);
     WTG_LAUNCH_CHECK();
     if (!last) {
       // the next group's tiles per node of level s+g
       WTG_LAUNCH(ctx, "mld_ntiles", k_mld_ntiles, dim3((unsigned)wtg_ceil_div(nbins, 256)), dim3(256), 0,
-                 cum[gi & 1], nbins, nt);
+                 cum[gi & 1], nbins, nt, P.gt[gi + 1]);
       WTG_LAUNCH_CHECK();
       WTG_TRY(wtg_fill_bytes_zero(ctx, scst, (char*)ctr + 256 - (char*)scst));
       WTG_LAUNCH(ctx, "mld_tiles", k_scan_u32<uint32_t>, dim3((unsigned)stiles), dim3(256), 0, nt, tst, nbins, scst,
                  ctr, ctx->d_flag);
       WTG_LAUNCH_CHECK();
-      const uint64_t ntiles_next = wtg_ceil_div(n, MLD_T) + std::min<uint64_t>(n, nbins);
+      const uint64_t ntiles_next = wtg_ceil_div(n, 1u << P.gt[gi + 1]) + std::min<uint64_t>(n, nbins);
       WTG_LAUNCH(ctx, "mld_tseg", k_mld_tseg, dim3((unsigned)wtg_ceil_div(ntiles_next, 256)), dim3(256), 0, tst,
                  nbins, tseg, (uint64_t)P.maxtiles);
       WTG_LAUNCH_CHECK();
