@@ -1234,7 +1234,10 @@ int wtg_levels_build_async(wtg_ctx* ctx, const void* d_sym, int sym_bytes, uint6
       wtg_set_error("levels > 24: WTnode records are limited to 24 levels (pass no node array)");
       return WTG_ERR_UNSUPPORTED;
     }
-    return n ? wtg_deep_build(ctx, d_sym, sym_bytes, n, levels, d_words, d_distinct) : WTG_OK;
+    if (n == 0) return WTG_OK;
+    if (ctx->level_method == 0 && wtg_mld_enabled())
+      return wtg_mld_build_sparse(ctx, d_sym, sym_bytes, n, levels, d_words, d_distinct);
+    return wtg_deep_build(ctx, d_sym, sym_bytes, n, levels, d_words, d_distinct);
   }
   if (n > 0 && ctx->level_method == 0 && wtg_mld_enabled())
     return wtg_mld_build(ctx, d_sym, sym_bytes, n, levels, d_words, d_nodes, node_slots, d_distinct);

@@ -47,6 +47,7 @@ constexpr uint32_t MLD_WT = 2048;           // keys per wave of the count pass
 constexpr uint32_t MLD_GMAX = 8;            // levels per group
 constexpr uint32_t MLD_T4K_N = 21, MLD_T4K_NODE = 15;  // 4096-key tiles: log2 of the least keys, and per node
 constexpr uint32_t MLD_CPW = 8;             // 64-key chunks per wave of the emit pass
+constexpr uint32_t LOC_CAP = 2048;          // keys of a k_mld_local block
 constexpr uint32_t MLD_SR = 64;             // tiles per block of the carry scan
 
 struct MldArgs {
@@ -55,9 +56,13 @@ struct MldArgs {
   uint32_t L, s, g;
   uint32_t tl;               // log2 of the keys per tile
   uint32_t ntiles0;          // s == 0: ceil(n / 2^tl)
-  const uint32_t* tstart;    // s > 0: 2^s + 1 entries, first tile of each level-s node
-  const uint32_t* tseg;      // s > 0: the level-s node of each tile
-  const uint32_t* cum_s;     // s > 0: 2^s + 1 entries, keys before each level-s node
+  uint32_t nseg;             // s > 0: segments (2^s, or the most the list below can hold)
+  const uint32_t* tstart;    // s > 0: nseg + 1 entries, first tile of each segment
+  const uint32_t* tseg;      // s > 0: the segment of each tile
+  const uint32_t* cum_s;     // s > 0: 2^s + 1 entries, keys before each level-s node, or
+  const uint32_t* seg_start; // null, or the segments are a list of level-s nodes: where each
+  const uint32_t* seg_cnt;   // starts in P_s and its keys (cum_s then unused)
+  uint32_t clear;            // 1: the count pass clears the group's level words
   const uint32_t* tcnt;      // [tile][2^g] leaf counts (written by k_mld_count)
   uint32_t* tcnt_w;
   const uint32_t* ploc;      // [tile][2^g] block-local exclusive prefix over tiles
@@ -68,14 +73,12 @@ struct MldArgs {
   uint32_t check;            // 1: flag input keys with bits at or above chk_shift
   uint32_t chk_shift;
   const uint64_t* src_off;   // null, or (first group) where each level-s node's keys start in `keys`
-  uint32_t kshift;           // first group: the keys are the input values >> kshift (the top L
-                             // levels of a deeper tree); 0 otherwise
-  uint32_t* kout;            // P_{s+g} keys as uint32 (emit with SCATTER)
+  void* kout;                // P_{s+g} keys (emit with SCATTER): uint32, or uint64 (WIDE)
   uint32_t* err;
 };
 
 __device__ __forceinline__ uint32_t mld_ntiles(const MldArgs& a) {
-  return a.s == 0 ? a.ntiles0 : a.tstart[1u << a.s];
+  return a.s == 0 ? a.ntiles0 : a.tstart[a.nseg];
 }
 
 // tile t -> (segment, first key in P_s, keys, first tile of the segment)
@@ -90,15 +93,15 @@ __device__ __forceinline__ bool mld_tile(const MldArgs& a, uint32_t t, uint32_t&
     first = 0;
     return true;
   }
-  const uint32_t nseg = 1u << a.s;
-  if (t >= a.tstart[nseg]) return false;
+  if (t >= a.tstart[a.nseg]) return false;
   const uint32_t lo = a.tseg[t];  // the segment of tile t (k_mld_tseg)
   seg = lo;
   first = a.tstart[lo];
   const uint64_t off = (uint64_t)(t - first) << a.tl;
-  const uint64_t cnt = a.cum_s[lo + 1] - a.cum_s[lo];
+  const uint64_t st = a.seg_cnt ? a.seg_start[lo] : a.cum_s[lo];
+  const uint64_t cnt = a.seg_cnt ? a.seg_cnt[lo] : a.cum_s[lo + 1] - (uint32_t)st;
   if (off >= cnt) return false;  // (cannot happen for consistent tables)
-  base = a.cum_s[lo] + off;
+  base = st + off;
   len = (uint32_t)(cnt - off < (1u << a.tl) ? cnt - off : 1u << a.tl);
   return true;
 }
@@ -204,14 +207,14 @@ __global__ __launch_bounds__(256) void k_mld_count(MldArgs a) {
   // positions of a level-s node keep their range at every later level), so
   // every word is cleared once, by the group of its first bit's level, before
   // that group's emit ORs into it
-  if (len) {
+  if (len && a.clear) {
     for (uint32_t j = 0; j < a.g; j++) {
       const uint64_t lb = (uint64_t)(a.s + j - a.lvl0) * a.n;
       const uint64_t wa = (lb + base + 63) >> 6, wb = (lb + base + len + 63) >> 6;
       for (uint64_t k = wa + lane; k < wb; k += 64) a.words[k] = 0ull;
     }
   }
-  const uint32_t tsh = a.L - a.s - a.g + a.kshift;  // the leaf's first bit in the key
+  const uint32_t tsh = a.L - a.s - a.g;  // the leaf's first bit in the key
   constexpr uint32_t B = 8 * KW;
   const uint32_t gw = KW == 8 ? a.g : (tsh >= B ? 0u : (B - tsh < a.g ? B - tsh : a.g));
   const uint32_t gmask = G - 1;
@@ -440,8 +443,11 @@ __device__ __forceinline__ uint32_t mld_scan256(uint32_t v, uint32_t* s_wave, ui
 }
 
 // T keys per tile (mld_tile_log), T / 8 threads (8 chunks of 64 keys per wave).
-// Bound by VALU issue and the barriers between levels, not by memory
-template <typename K, bool SCATTER, uint32_t T>
+// Bound by VALU issue and the barriers between levels, not by memory.
+// WIDE (trees of more than 32 levels): the level loop moves the leaf d above
+// the key's place in the tile instead of the key, and the scatter reads the
+// 64-bit key again by that place
+template <typename K, bool SCATTER, uint32_t T, bool WIDE>
 __global__ __launch_bounds__(T / 8) __attribute__((amdgpu_waves_per_eu(8))) void k_mld_emit(MldArgs a) {
   constexpr uint32_t NT = T / 8, NWV = NT / 64;
   constexpr uint32_t BW = T / 32 + 2;  // staged bit words per level (+2 read-ahead pad)
@@ -468,7 +474,7 @@ __global__ __launch_bounds__(T / 8) __attribute__((amdgpu_waves_per_eu(8))) void
   const uint64_t src = mld_src(a, seg, base);
   const uint32_t g = a.g, G = 1u << g, lane = (uint32_t)lane_id();
   const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const uint32_t sh = a.L - a.s - g;
+  const uint32_t sh = WIDE ? 16u : a.L - a.s - g;  // the leaf's first bit in what the level loop moves
   // the tile's leaf counts and their exclusive prefix over d
   uint32_t xk[MLD_CPW];  // the wave's chunks c = w + 4m, one key per lane
   {
@@ -492,7 +498,8 @@ __global__ __launch_bounds__(T / 8) __attribute__((amdgpu_waves_per_eu(8))) void
 #pragma unroll
     for (uint32_t m = 0; m < MLD_CPW; m++) {
       const uint32_t p = (w + NWV * m) * 64 + lane;
-      xk[m] = p < len ? (uint32_t)((uint64_t)kr[m] >> a.kshift) : ~0u;
+      if constexpr (WIDE) xk[m] = p < len ? ((uint32_t)((uint64_t)kr[m] >> (a.L - a.s - g)) & (G - 1)) << 16 | p : ~0u;
+      else xk[m] = p < len ? (uint32_t)kr[m] : ~0u;
     }
   }
   __syncthreads();
@@ -668,8 +675,10 @@ __global__ __launch_bounds__(T / 8) __attribute__((amdgpu_waves_per_eu(8))) void
       if (i < len) {
         const uint32_t x = s_k[g & 1][i];
         const uint32_t dest = s_lb[(x >> sh) & (G - 1)] + i;
-        if (dest < n) a.kout[dest] = x;
-        else atomicOr(a.err, WTG_FLAG_BADSYM);
+        if (dest >= n) atomicOr(a.err, WTG_FLAG_BADSYM);
+        else if constexpr (WIDE)
+          reinterpret_cast<uint64_t*>(a.kout)[dest] = (uint64_t) reinterpret_cast<const K*>(a.keys)[src + (x & 0xFFFFu)];
+        else reinterpret_cast<uint32_t*>(a.kout)[dest] = x;
       }
     }
   }
@@ -711,6 +720,26 @@ __global__ void k_mld_nonzero(const uint32_t* __restrict__ h, uint64_t n, unsign
   if (lane_id() == 0 && c) atomicAdd(out, (unsigned long long)c);
 }
 
+// where the dense groups of a tree with small nodes end: whole 8-level groups,
+// and an average node of at most 128 keys (LOC_H leaves room for uneven ones;
+// 6000011 keys, 40 levels: 695 us with 128, 699 with 256, 717 with 64)
+uint32_t mld_split_level(uint64_t n) {
+  if (n <= (1ull << 15)) return 8;
+  uint32_t s = 16;
+  while (s < 24 && (n >> (s + 7)) != 0) s++;
+  return s;
+}
+// Up to 24 levels both ways work.  Dense groups alone start the last of three
+// groups at level 2/3 L; from about 512 keys per node there down, their tiles
+// are mostly padding (one node per tile): n = 2^24, 24 levels (256 keys)
+// 1230 us against 577, n = 3000017, 20 levels (183 keys) 264 against 200; at
+// 1024 keys they are the faster way (n = 2^24, 20 levels: 449 against 506).
+bool mld_use_sparse(uint64_t n, uint32_t L) {
+  if (n <= LOC_CAP) return true;
+  const uint32_t last = L - L / 3;  // where the last of three near-equal groups starts
+  return L > 16 && (n >> last) < 512;
+}
+
 struct MldPlan {
   uint32_t ngroups, gs[4], gg[4], gt[4];
   uint64_t maxtiles, maxblocks, maxbins;
@@ -731,7 +760,9 @@ uint32_t mld_tile_log(uint64_t n, uint32_t s, uint32_t g) {
   return g == MLD_GMAX && n >= (1ull << MLD_T4K_N) && (n >> s) >= (1ull << MLD_T4K_NODE) ? 12 : 11;
 }
 
-MldPlan mld_plan(uint64_t n, uint32_t L, uint32_t s0) {
+// (key_bytes: 0, or the caller reads the keys after the last group too, and
+// writes both buffers)
+MldPlan mld_plan(uint64_t n, uint32_t L, uint32_t s0, uint32_t key_bytes = 0) {
   MldPlan P{};
   // as few groups as MLD_GMAX allows, of near-equal widths (wider first): a
   // pass's per-tile work outside the level pipeline (tables, runs, partial
@@ -755,7 +786,7 @@ MldPlan mld_plan(uint64_t n, uint32_t L, uint32_t s0) {
   size_t o = 0;
   for (int b = 0; b < 2; b++) {
     P.off_keys[b] = o;
-    if (P.ngroups > 1) o = wtg_align256(o + n * 4);
+    if (P.ngroups > 1 || key_bytes) o = wtg_align256(o + n * (key_bytes ? key_bytes : 4));
   }
   P.off_tcnt = o; o = wtg_align256(o + (P.maxtiles + 1) * 256 * 4);
   P.off_ploc = o; o = wtg_align256(o + (P.maxtiles + 1) * 256 * 4);
@@ -772,28 +803,37 @@ MldPlan mld_plan(uint64_t n, uint32_t L, uint32_t s0) {
   return P;
 }
 
-template <typename K, uint32_t T>
-void mld_emit_launch(wtg_ctx* ctx, bool first, bool last, unsigned grid, const MldArgs& a) {
-  if (first) {
-    if (last) WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<K, false, T>), dim3(grid), dim3(T / 8), 0, a);
-    else WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<K, true, T>), dim3(grid), dim3(T / 8), 0, a);
+// the count and emit passes of a group over keys of type K (the input's, or
+// KO of the passes before)
+template <typename K>
+void mld_count_launch(wtg_ctx* ctx, unsigned grid, const MldArgs& a) {
+  const dim3 cg((unsigned)wtg_ceil_div(grid, (uint64_t)4 * MLD_WT >> a.tl));  // 4 waves of MLD_WT keys per block
+  if (a.g <= 2) WTG_LAUNCH(ctx, "mld_count", (k_mld_count<K, 4>), cg, dim3(256), 0, a);
+  else if (a.g == 3) WTG_LAUNCH(ctx, "mld_count", (k_mld_count<K, 8>), cg, dim3(256), 0, a);
+  else WTG_LAUNCH(ctx, "mld_count", (k_mld_count<K, 0>), cg, dim3(256), 0, a);
+}
+template <typename K, bool WIDE>
+void mld_emit_launch(wtg_ctx* ctx, bool scatter, unsigned grid, const MldArgs& a) {
+  if (a.tl == 12) {
+    if (scatter) WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<K, true, 4096, WIDE>), dim3(grid), dim3(512), 0, a);
+    else WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<K, false, 4096, WIDE>), dim3(grid), dim3(512), 0, a);
   } else {
-    if (last) WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<uint32_t, false, T>), dim3(grid), dim3(T / 8), 0, a);
-    else WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<uint32_t, true, T>), dim3(grid), dim3(T / 8), 0, a);
+    if (scatter) WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<K, true, 2048, WIDE>), dim3(grid), dim3(256), 0, a);
+    else WTG_LAUNCH(ctx, "mld_emit", (k_mld_emit<K, false, 2048, WIDE>), dim3(grid), dim3(256), 0, a);
   }
 }
 
 // Levels [s0, L) of the keys d_sym (in P_{s0} order: sorted by their top s0
 // bits, d_cnt0 = the 2^s0 node sizes; s0 = 0: any order, d_cnt0 unused);
-// level l's bits go to bit (l - s0) * n of d_words.  kshift > 0 (s0 = 0): the
-// keys are d_sym >> kshift, i.e. these are the top L levels of an
-// (L + kshift)-level tree.
-template <typename K>
-int mld_build_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint32_t s0, const uint32_t* d_cnt0,
-                const uint64_t* d_src_off, uint64_t* d_words, wtg_node* d_nodes, uint64_t node_slots,
-                unsigned long long* d_distinct, uint32_t kshift = 0) {
-  const MldPlan P = mld_plan(n, L, s0);
-  WTG_TRY(wtg_ws_reserve(ctx, P.total));
+// level l's bits go to bit (l - s0) * n of d_words.
+// P: the plan of levels [s0, Lend) (workspace reserved by the caller); where
+// Lend < L the last group scatters its keys too (as KO, to key buffer
+// (ngroups - 1) & 1).
+template <typename K, typename KO>
+int mld_dense_groups(wtg_ctx* ctx, const MldPlan& P, const K* d_sym, uint64_t n, uint32_t L, uint32_t Lend, uint32_t s0,
+                     const uint32_t* d_cnt0, const uint64_t* d_src_off, uint64_t* d_words,
+                     unsigned long long* d_distinct) {
+  constexpr bool WIDE = sizeof(KO) == 8;
   char* ws = (char*)ctx->ws;
   uint32_t* tcnt = (uint32_t*)(ws + P.off_tcnt);
   uint32_t* ploc = (uint32_t*)(ws + P.off_ploc);
@@ -806,7 +846,7 @@ int mld_build_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint32_t s
   uint32_t* tseg = (uint32_t*)(ws + P.off_tseg);
   uint64_t* scst = (uint64_t*)(ws + P.off_scst);
   uint32_t* ctr = (uint32_t*)(ws + P.off_ctr);
-  uint32_t* kbuf[2] = {(uint32_t*)(ws + P.off_keys[0]), (uint32_t*)(ws + P.off_keys[1])};
+  KO* kbuf[2] = {(KO*)(ws + P.off_keys[0]), (KO*)(ws + P.off_keys[1])};
   // (the level words are cleared by the leaf-count passes)
   if (d_distinct) WTG_TRY(wtg_fill_u64(ctx, d_distinct, 1, 0));
   const uint32_t ntiles0 = (uint32_t)wtg_ceil_div(n, 1u << P.gt[0]);
@@ -835,7 +875,7 @@ int mld_build_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint32_t s
   }
   for (uint32_t gi = 0; gi < P.ngroups; gi++) {
     const uint32_t s = P.gs[gi], g = P.gg[gi], G = 1u << g, tl = P.gt[gi];
-    const bool last = gi + 1 == P.ngroups;
+    const bool more = gi + 1 < P.ngroups, last = !more && Lend == L;
     MldArgs a{};
     a.keys = src;
     a.n = n;
@@ -844,6 +884,8 @@ int mld_build_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint32_t s
     a.g = g;
     a.tl = tl;
     a.ntiles0 = ntiles0;
+    a.nseg = 1u << s;
+    a.clear = 1;
     a.tstart = s ? tst : nullptr;
     a.tseg = s ? tseg : nullptr;
     a.cum_s = s ? cum_prev : nullptr;
@@ -855,26 +897,17 @@ int mld_build_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint32_t s
     a.words = d_words;
     a.lvl0 = s0;
     // the input: no bits at or above L - s0 below the top s0 (none above bit 63)
-    a.check = gi == 0 && L + kshift < 64 ? 1u : 0u;
-    a.chk_shift = d_src_off ? L - s0 : L + kshift;
+    a.check = gi == 0 && L < 64 ? 1u : 0u;
+    a.chk_shift = d_src_off ? L - s0 : L;
     a.src_off = gi == 0 ? d_src_off : nullptr;
-    a.kshift = gi == 0 ? kshift : 0u;
     a.kout = last ? nullptr : kbuf[gi & 1];
     a.err = ctx->d_flag;
     // grid: an upper bound of the tiles (blocks past the real count exit)
     const uint64_t grid = s == 0 ? ntiles0 : wtg_ceil_div(n, 1u << tl) + std::min<uint64_t>(n, 1ull << s);
     const uint32_t nrows = (uint32_t)grid + 1;
     const uint32_t nblocks = (uint32_t)wtg_ceil_div(nrows, MLD_SR);
-    const dim3 cg((unsigned)wtg_ceil_div(grid, (uint64_t)4 * MLD_WT >> tl));  // 4 waves of MLD_WT keys per block
-    if (gi == 0) {
-      if (G <= 4) WTG_LAUNCH(ctx, "mld_count", (k_mld_count<K, 4>), cg, dim3(256), 0, a);
-      else if (G <= 8) WTG_LAUNCH(ctx, "mld_count", (k_mld_count<K, 8>), cg, dim3(256), 0, a);
-      else WTG_LAUNCH(ctx, "mld_count", (k_mld_count<K, 0>), cg, dim3(256), 0, a);
-    } else {
-      if (G <= 4) WTG_LAUNCH(ctx, "mld_count", (k_mld_count<uint32_t, 4>), cg, dim3(256), 0, a);
-      else if (G <= 8) WTG_LAUNCH(ctx, "mld_count", (k_mld_count<uint32_t, 8>), cg, dim3(256), 0, a);
-      else WTG_LAUNCH(ctx, "mld_count", (k_mld_count<uint32_t, 0>), cg, dim3(256), 0, a);
-    }
+    if (gi == 0) mld_count_launch<K>(ctx, (unsigned)grid, a);
+    else mld_count_launch<KO>(ctx, (unsigned)grid, a);
     WTG_LAUNCH_CHECK();
     WTG_LAUNCH(ctx, "mld_scan", k_mld_scan1, dim3(nblocks), dim3(256), 0, tcnt, ploc, bsum,
                s ? (const uint32_t*)(tst + (1u << s)) : nullptr, ntiles0, G, nrows);
@@ -895,10 +928,10 @@ int mld_build_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint32_t s
       WTG_LAUNCH_CHECK();
     }
     // the level bits of the group (and the keys in P_{s+g} order)
-    if (tl == 12) mld_emit_launch<K, 4096>(ctx, gi == 0, last, (unsigned)grid, a);
-    else mld_emit_launch<K, 2048>(ctx, gi == 0, last, (unsigned)grid, a);
+    if (gi == 0) mld_emit_launch<K, WIDE>(ctx, !last, (unsigned)grid, a);
+    else mld_emit_launch<KO, WIDE>(ctx, !last, (unsigned)grid, a);
     WTG_LAUNCH_CHECK();
-    if (!last) {
+    if (more) {
       // the next group's tiles per node of level s+g
       WTG_LAUNCH(ctx, "mld_ntiles", k_mld_ntiles, dim3((unsigned)wtg_ceil_div(nbins, 256)), dim3(256), 0,
                  cum[gi & 1], nbins, nt, P.gt[gi + 1]);
@@ -915,9 +948,460 @@ int mld_build_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint32_t s
       cum_prev = cum[gi & 1];
     }
   }
+  return WTG_OK;
+}
+
+template <typename K>
+int mld_build_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint32_t s0, const uint32_t* d_cnt0,
+                const uint64_t* d_src_off, uint64_t* d_words, wtg_node* d_nodes, uint64_t node_slots,
+                unsigned long long* d_distinct) {
+  const MldPlan P = mld_plan(n, L, s0);
+  WTG_TRY(wtg_ws_reserve(ctx, P.total));
+  WTG_TRY((mld_dense_groups<K, uint32_t>(ctx, P, d_sym, n, L, L, s0, d_cnt0, d_src_off, d_words, d_distinct)));
   if (d_nodes && node_slots && s0 == 0) {
     WTG_LAUNCH(ctx, "nodes", k_mld_nodes, dim3((unsigned)wtg_ceil_div(node_slots, 256)), dim3(256), 0,
-               cum[(P.ngroups - 1) & 1], L, n, d_nodes, node_slots);
+               (const uint32_t*)((char*)ctx->ws + P.off_cum[(P.ngroups - 1) & 1]), L, n, d_nodes, node_slots);
+    WTG_LAUNCH_CHECK();
+  }
+  return WTG_OK;
+}
+
+
+// ---------------------------------------------------- small nodes, all levels
+// Small nodes need no tables: whatever the level, their keys stay inside their
+// own range of positions, so a block that holds whole nodes in LDS builds all
+// their remaining levels alone, and its bits are one run per level.  A block
+// takes the nodes that start in a window of LOC_W positions and end within
+// LOC_CAP of the window's start (all but the window's last node do, and that
+// one does if it has at most LOC_H keys); the others are "large".
+constexpr uint32_t LOC_H = 512, LOC_W = LOC_CAP - LOC_H;
+// a node of c keys that starts `off` positions into its window
+__device__ __forceinline__ bool loc_large(uint32_t off, uint32_t c) { return (uint64_t)off + c > LOC_CAP; }
+constexpr uint32_t LOC_TW = (2048 + LOC_W - 1) / LOC_W;  // windows per 2048-key tile of a listed segment
+
+struct LocArgs {
+  const void* kin;            // keys in P_s order (mode 0: the input)
+  uint64_t n;
+  uint32_t L, s;              // levels s .. L-1
+  uint32_t mode;              // 0: one block, the whole input (n <= LOC_CAP, s = 0);
+                              // 1: windows of the nodes st[0..m) (st[m] = n);
+                              // 2: LOC_TW windows per tile t of the list: its segment k's leaves
+                              //    st[k m .. k m + m), which end with the segment
+  const uint32_t* st;         // node starts, non-decreasing
+  uint32_t m;
+  uint32_t nseg;              // mode 2: the list
+  const uint32_t* tstart;
+  const uint32_t* tseg;
+  const uint32_t* seg_start;
+  const uint32_t* seg_cnt;
+  uint64_t* words;            // level l's bits at bit l * n
+  unsigned long long* distinct;  // nullable: += the nodes that level L would have
+  uint32_t* err;
+};
+
+// the first i in [0, m] with st[i] >= v, where st[m] stands for a value >= v
+// (a whole wave; 64 probes a step)
+__device__ __forceinline__ uint32_t wave_lower_bound(const uint32_t* __restrict__ st, uint32_t m, uint32_t v) {
+  uint32_t lo = 0, hi = m;
+  while (lo < hi) {
+    const uint32_t step = (hi - lo + 63) >> 6;
+    const uint32_t i = lo + (uint32_t)lane_id() * step;
+    const uint32_t c = popc64(wave_ballot(i < hi && st[i] < v));
+    if (c == 0) break;
+    const uint32_t up = lo + c * step;
+    lo = lo + (c - 1) * step + 1;
+    if (up < hi) hi = up;
+  }
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)lo);
+}
+
+// All levels s .. L-1 of at most LOC_CAP consecutive keys of P_s that are whole
+// nodes.  Every key carries its node's range (S, E) in the tile; with O(p) the
+// level's ones before p, a zero at p goes to p - (O(p) - O(S)), a one to
+// E - (O(E) - O(p)), and its node's range is cut at mid = E - (O(E) - O(S)).
+// O comes from the level's bits and their prefix per 32-bit word (one LDS read
+// per lookup).  Once every node is a single key the order stands and only bits
+// remain to be read.  Bound by VALU issue (~30 instructions per key and level
+// while nodes have several keys); 6000011 uint64 keys, 40 levels: levels 16..39
+// in 0.25 ms (2.35 ms level by level over the whole array).  R64: more than 32 levels remain (64-bit keys in LDS).
+template <typename KIN, bool R64>
+__global__ __launch_bounds__(256) void k_mld_local(LocArgs a) {
+  using KT = typename std::conditional<R64, uint64_t, uint32_t>::type;
+  constexpr uint32_t M = LOC_CAP / 256;  // 64-key chunks per wave
+  __shared__ KT s_key[LOC_CAP];
+  __shared__ uint32_t s_se[LOC_CAP];
+  __shared__ __align__(8) uint32_t s_bits[8][LOC_CAP / 32 + 2];
+  __shared__ uint2 s_ow[4][LOC_CAP / 32 + 1];  // per wave: the level's bits and the ones before each word
+  __shared__ uint32_t s_flag[2];
+  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t lane = (uint32_t)lane_id();
+  // the block's keys: [a0, a0 + len) of P_s
+  uint32_t a0 = 0, len = 0;
+  if (a.mode == 0) {
+    len = (uint32_t)a.n;
+  } else {
+    uint64_t lo, end = a.n;        // the window's first position, where the last node ends
+    uint32_t m = a.m, width = LOC_W;
+    const uint32_t* st = a.st;
+    if (a.mode == 1) {
+      lo = (uint64_t)blockIdx.x * LOC_W;
+    } else {
+      const uint32_t t = blockIdx.x / LOC_TW, j = blockIdx.x % LOC_TW;
+      if (t >= a.tstart[a.nseg]) return;
+      const uint32_t k = a.tseg[t];
+      lo = (uint64_t)a.seg_start[k] + ((uint64_t)(t - a.tstart[k]) << 11) + j * LOC_W;
+      if (j + 1 == LOC_TW) width = 2048 - j * LOC_W;
+      end = (uint64_t)a.seg_start[k] + a.seg_cnt[k];
+      st += (uint64_t)k * m;
+    }
+    if (lo >= end) return;
+    const uint32_t i0 = wave_lower_bound(st, m, (uint32_t)lo);
+    const uint32_t i1 = lo + width < end ? wave_lower_bound(st, m, (uint32_t)lo + width) : m;
+    a0 = i0 < m ? st[i0] : (uint32_t)end;
+    uint32_t e0 = i1 < m ? st[i1] : (uint32_t)end;
+    if (a0 >= e0) return;
+    const uint32_t last = st[wave_lower_bound(st, m, e0) - 1];  // the last node that starts in the window
+    if (loc_large(last - (uint32_t)lo, e0 - last)) e0 = last;
+    if (a0 >= e0) return;
+    len = e0 - a0;
+    if (len > LOC_CAP) return;  // (cannot happen for consistent tables)
+  }
+  const uint32_t r = a.L - a.s;  // levels to build
+  const KIN* kin = reinterpret_cast<const KIN*>(a.kin) + a0;
+  if (a.mode == 0) {  // one block: its words are cleared here
+    const uint64_t nw = (a.n * a.L + 63) >> 6;
+    for (uint64_t k = threadIdx.x; k < nw; k += 256) a.words[k] = 0ull;
+    __threadfence();
+  }
+  // keys, and each key's node: heads are the keys whose top s bits differ from
+  // the key before (positions past the keys are heads)
+  KT x[M];
+  uint32_t se[M];
+  uint64_t hm[M];
+  bool bad = false;
+#pragma unroll
+  for (uint32_t m = 0; m < M; m++) {
+    const uint32_t p = (w + 4 * m) * 64 + lane;
+    uint64_t k = 0, q = 0;
+    if (p < len) {
+      k = (uint64_t)kin[p];
+      q = p ? (uint64_t)kin[p - 1] : 0;
+    }
+    const bool head = p >= len || p == 0 || (a.s > 0 && (k >> r) != (q >> r));
+    if (a.mode == 0 && a.L < 64 && (k >> a.L) != 0) bad = true;
+    hm[m] = wave_ballot(head);
+    if (lane == 0) reinterpret_cast<uint64_t*>(s_bits[0])[w + 4 * m] = hm[m];
+    x[m] = (KT)k;
+  }
+  if (bad) atomicOr(a.err, WTG_FLAG_BADSYM);
+  if (threadIdx.x < 2) s_flag[threadIdx.x] = 0;
+  __syncthreads();
+  {
+    const uint64_t* hd = reinterpret_cast<const uint64_t*>(s_bits[0]);
+    const uint64_t upto = ~0ull >> (63 - lane);  // lanes 0 .. lane
+#pragma unroll
+    for (uint32_t m = 0; m < M; m++) {
+      const uint32_t c0 = w + 4 * m;
+      uint32_t c = c0;
+      uint64_t f = hm[m] & upto;
+      while (f == 0 && c > 0) f = hd[--c];
+      const uint32_t S = c * 64 + (f ? 63u - (uint32_t)__builtin_clzll(f) : 0u);
+      c = c0;
+      f = hm[m] & ~upto;
+      while (f == 0 && ++c < LOC_CAP / 64) f = hd[c];
+      const uint32_t E = f ? c * 64 + (uint32_t)__builtin_ctzll(f) : LOC_CAP;
+      se[m] = S | E << 16;
+    }
+  }
+  __syncthreads();
+  bool active = true;  // some node has several keys (block-uniform)
+  uint32_t ndist = 0;
+  const uint64_t n = a.n;
+  for (uint32_t i = 0; i < r; i++) {
+    const uint32_t bp = r - 1 - i, lv = i & 7;
+    uint64_t om[M];
+#pragma unroll
+    for (uint32_t m = 0; m < M; m++) {
+      om[m] = wave_ballot((x[m] >> bp) & 1u);
+      if (lane == 0) reinterpret_cast<uint64_t*>(s_bits[lv])[w + 4 * m] = om[m];
+    }
+    const bool last = i + 1 == r;
+    if (active && !(last && !a.distinct)) {
+      __syncthreads();
+      if (threadIdx.x == 0) s_flag[lv & 1 ? 0 : 1] = 0;  // the next level's
+      const uint32_t b = s_bits[lv][lane];
+      const uint32_t cnt = __popc(b), incl = wave_incl_sum_dpp(cnt);
+      s_ow[w][lane] = make_uint2(b, incl - cnt);
+      if (lane == 63) s_ow[w][64] = make_uint2(0u, incl);
+      wave_sync_lds_mld();
+      bool any = false;
+#pragma unroll
+      for (uint32_t m = 0; m < M; m++) {
+        const uint32_t c = w + 4 * m, p = c * 64 + lane;
+        const uint32_t S = se[m] & 0xFFFFu, E = se[m] >> 16;
+        const uint2 ws = s_ow[w][S >> 5], we = s_ow[w][E >> 5];
+        const uint32_t OS = ws.y + __popc(__builtin_amdgcn_ubfe(ws.x, 0u, S & 31));
+        const uint32_t OE = we.y + __popc(__builtin_amdgcn_ubfe(we.x, 0u, E & 31));
+        const uint32_t base = s_ow[w][2 * c].y;
+        const uint32_t OP =
+            __builtin_amdgcn_mbcnt_hi((uint32_t)(om[m] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)om[m], base));
+        const bool one = (x[m] >> bp) & 1u;
+        const uint32_t mid = E - (OE - OS);
+        const uint32_t dest = one ? E - (OE - OP) : p - (OP - OS);
+        const uint32_t s2 = one ? mid : S, e2 = one ? E : mid;
+        if (last) {
+          ndist += popc64(wave_ballot(p < len && dest == s2));
+        } else {
+          any |= e2 - s2 > 1;
+          s_key[dest] = x[m];
+          s_se[dest] = s2 | e2 << 16;
+        }
+      }
+      if (!last) {
+        if (wave_ballot(any) != 0 && lane == 0) s_flag[lv & 1] = 1;
+        __syncthreads();
+        active = s_flag[lv & 1] != 0;
+#pragma unroll
+        for (uint32_t m = 0; m < M; m++) {
+          const uint32_t p = (w + 4 * m) * 64 + lane;
+          x[m] = s_key[p];
+          se[m] = s_se[p];
+        }
+      }
+    } else if (last && a.distinct && w == 0) {
+      ndist = len;  // every key its own node
+    }
+    if (lv == 7 || last) {
+      // the staged levels' bits: one run per level at l * n + a0
+      __syncthreads();
+      constexpr uint32_t RW = LOC_CAP / 64 + 1;  // words a run can touch
+      for (uint32_t it = threadIdx.x; it < (lv + 1) * RW; it += 256) {
+        const uint32_t k = it / RW;
+        const uint64_t gs = (uint64_t)(a.s + i - lv + k) * n + a0, ge = gs + len;
+        const uint64_t wi = (gs >> 6) + it % RW, wb = wi << 6;
+        if (wb >= ge) continue;
+        const uint32_t b0 = gs > wb ? (uint32_t)(gs - wb) : 0u;
+        const uint32_t b1 = ge < wb + 64 ? (uint32_t)(ge - wb) : 64u;
+        uint64_t v = lds_bits64(s_bits[k], (uint32_t)(wb + b0 - gs)) << b0;
+        if (b1 < 64) v &= (1ull << b1) - 1;
+        if (b0 == 0 && b1 == 64) a.words[wi] = v;
+        else if (v) atomicOr((unsigned long long*)&a.words[wi], (unsigned long long)v);
+      }
+      __syncthreads();
+    }
+  }
+  if (a.distinct && lane == 0 && ndist) atomicAdd(a.distinct, (unsigned long long)ndist);
+}
+
+// the large level-S nodes, as a list (in any order: the
+// order of the segments changes no output)
+__global__ __launch_bounds__(256) void k_mld_big(const uint32_t* __restrict__ cum, uint32_t nn, uint32_t* __restrict__ bs,
+                                                 uint32_t* __restrict__ bc, uint32_t* __restrict__ nb, uint32_t cap,
+                                                 uint32_t* __restrict__ err) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= nn) return;
+  const uint32_t st = cum[i], c = cum[i + 1] - st;
+  if (!loc_large(st % LOC_W, c)) return;
+  const uint32_t k = atomicAdd(nb, 1u);
+  if (k >= cap) { atomicOr(err, WTG_FLAG_BADSYM); return; }  // (cannot happen: the sizes sum to n)
+  bs[k] = st;
+  bc[k] = c;
+}
+
+// tiles of each listed segment (0 past the list)
+__global__ __launch_bounds__(256) void k_mld_list_tiles(const uint32_t* __restrict__ bc, const uint32_t* __restrict__ nb,
+                                                        uint32_t cap, uint32_t* __restrict__ nt, uint32_t tl) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= cap) return;
+  nt[i] = i < *nb ? (uint32_t)(((uint64_t)bc[i] + (1u << tl) - 1) >> tl) : 0u;
+}
+
+// per listed segment (a block each): its leaves' starts, the large leaves as
+// the next list, or (last group) its distinct leaves
+__global__ __launch_bounds__(256) void k_mld_leaf(MldArgs a, uint32_t* __restrict__ lst, const uint32_t* __restrict__ nb,
+                                                  uint32_t* __restrict__ bs2, uint32_t* __restrict__ bc2,
+                                                  uint32_t* __restrict__ nb2, uint32_t cap,
+                                                  unsigned long long* distinct) {
+  __shared__ uint32_t s_wave[4];
+  const uint32_t k = blockIdx.x, d = threadIdx.x, G = 1u << a.g;
+  if (k >= *nb) return;
+  uint32_t c = 0;
+  if (d < G) c = mld_prefix(a, a.tstart[k + 1], d) - mld_prefix(a, a.tstart[k], d);
+  uint32_t tot;
+  const uint32_t st = a.seg_start[k] + mld_scan256<true>(c, s_wave, tot);
+  if (d < G) lst[(uint64_t)k * G + d] = st;
+  const uint32_t in_tile = (st - a.seg_start[k]) & 2047;
+  if (nb2 && c && loc_large(in_tile % LOC_W, c)) {
+    const uint32_t q = atomicAdd(nb2, 1u);
+    if (q >= cap) { atomicOr(a.err, WTG_FLAG_BADSYM); return; }
+    bs2[q] = st;
+    bc2[q] = c;
+  }
+  if (distinct) {
+    const uint32_t q = popc64(wave_ballot(c != 0));
+    if (lane_id() == 0 && q) atomicAdd(distinct, (unsigned long long)q);
+  }
+}
+
+template <typename KIN>
+void mld_local_launch(wtg_ctx* ctx, unsigned grid, const LocArgs& a) {
+  if (a.L - a.s > 32) WTG_LAUNCH(ctx, "mld_local", (k_mld_local<KIN, true>), dim3(grid), dim3(256), 0, a);
+  else WTG_LAUNCH(ctx, "mld_local", (k_mld_local<KIN, false>), dim3(grid), dim3(256), 0, a);
+}
+
+// Levels 0 .. L-1 of an input whose nodes get small before the last level:
+// dense groups (tables over all 2^l prefixes) down to level S, where an average
+// node is small, then the small nodes' remaining levels in one pass
+// (k_mld_local).  Nodes that are still large there (skewed inputs) go on as a
+// list of segments, up to 8 levels per round, each round handing its small
+// leaves to the same kernel; a large node has more than LOC_H keys, so at most
+// n / LOC_H of them exist at any level, and tables and work stay linear in n
+// whatever the values.
+template <typename K, typename KO>
+int mld_sparse_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint64_t* d_words,
+                 unsigned long long* d_distinct) {
+  constexpr bool WIDE = sizeof(KO) == 8;
+  if (d_distinct) WTG_TRY(wtg_fill_u64(ctx, d_distinct, 1, 0));
+  LocArgs q{};
+  q.n = n;
+  q.L = L;
+  q.words = d_words;
+  q.distinct = d_distinct;
+  q.err = ctx->d_flag;
+  if (n <= LOC_CAP) {
+    q.kin = d_sym;
+    mld_local_launch<K>(ctx, 1, q);
+    WTG_LAUNCH_CHECK();
+    return WTG_OK;
+  }
+  const uint32_t S = std::min(mld_split_level(n), L - 1);
+  const MldPlan P = mld_plan(n, S, 0, sizeof(KO));
+  const uint32_t cap = (uint32_t)(n / LOC_H) + 1;  // listed segments
+  const uint64_t maxt = wtg_ceil_div(n, MLD_WT) + cap + 1, maxb = wtg_ceil_div(maxt + 1, MLD_SR) + 1;
+  // the list rounds' tables, after the dense ones (whose keys stay in use)
+  size_t o = P.total;
+  const size_t o_tcnt = o; o = wtg_align256(o + (maxt + 1) * 256 * 4);
+  const size_t o_ploc = o; o = wtg_align256(o + (maxt + 1) * 256 * 4);
+  const size_t o_bsum = o; o = wtg_align256(o + maxb * 256 * 4);
+  const size_t o_bpre = o; o = wtg_align256(o + maxb * 256 * 4);
+  const size_t o_lst = o; o = wtg_align256(o + (size_t)cap * 256 * 4);
+  const size_t o_nt = o; o = wtg_align256(o + (size_t)cap * 4);
+  const size_t o_tst = o; o = wtg_align256(o + ((size_t)cap + 1) * 4);
+  const size_t o_tseg = o; o = wtg_align256(o + maxt * 4);
+  size_t o_bs[2], o_bc[2];
+  for (int b = 0; b < 2; b++) {
+    o_bs[b] = o; o = wtg_align256(o + (size_t)cap * 4);
+    o_bc[b] = o; o = wtg_align256(o + (size_t)cap * 4);
+  }
+  const size_t o_scst = o; o = wtg_align256(o + (wtg_ceil_div(cap, 4096) + 2) * 8);
+  const size_t o_ctr = o; o = wtg_align256(o + 256);
+  const size_t o_nb = o; o = wtg_align256(o + 256);
+  WTG_TRY(wtg_ws_reserve(ctx, o));
+  char* ws = (char*)ctx->ws;
+  KO* kbuf[2] = {(KO*)(ws + P.off_keys[0]), (KO*)(ws + P.off_keys[1])};
+  uint32_t* nb = (uint32_t*)(ws + o_nb);  // list lengths, 8 bytes apart
+  // the words of levels S .. L-1 (level S's first word may end level S-1, whose group clears it)
+  const uint64_t wt = (S * n + 63) >> 6;
+  WTG_TRY(wtg_fill_bytes_zero(ctx, d_words + wt, (wtg_levels_words(n, L) - wt) * 8));
+  WTG_TRY((mld_dense_groups<K, KO>(ctx, P, d_sym, n, L, S, 0, nullptr, nullptr, d_words, nullptr)));
+  const uint32_t* cum = (const uint32_t*)(ws + P.off_cum[(P.ngroups - 1) & 1]);
+  uint32_t kb = (P.ngroups - 1) & 1;  // the buffer that holds P_s
+  WTG_TRY(wtg_fill_u64(ctx, nb, 1, 0));
+  WTG_LAUNCH(ctx, "mld_big", k_mld_big, dim3((unsigned)wtg_ceil_div(1ull << S, 256)), dim3(256), 0, cum, 1u << S,
+             (uint32_t*)(ws + o_bs[0]), (uint32_t*)(ws + o_bc[0]), nb, cap, ctx->d_flag);
+  WTG_LAUNCH_CHECK();
+  q.kin = kbuf[kb];
+  q.s = S;
+  q.mode = 1;
+  q.st = cum;
+  q.m = 1u << S;
+  mld_local_launch<KO>(ctx, (unsigned)wtg_ceil_div(n, LOC_W), q);
+  WTG_LAUNCH_CHECK();
+  // how many large nodes are left: read back where that is allowed (not while
+  // the stream is being captured), so that no empty round is launched
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  WTG_CHECK_HIP(hipStreamIsCapturing(ctx->stream, &cs));
+  const bool ask = cs == hipStreamCaptureStatusNone;
+  uint32_t cur = 0;
+  for (uint32_t s = S; s < L;) {
+    uint32_t hb = cap;
+    if (ask) {
+      WTG_TRY(wtg_stage_d2h(ctx, &hb, nb + 2 * cur, 4));
+      if (hb > cap) hb = cap;  // (flagged on the device)
+      if (hb == 0) break;
+    }
+    const uint32_t g = (L - s + (L - s + MLD_GMAX - 1) / MLD_GMAX - 1) / ((L - s + MLD_GMAX - 1) / MLD_GMAX);
+    const bool last = s + g == L;
+    const uint32_t* bs = (const uint32_t*)(ws + o_bs[cur]);
+    const uint32_t* bc = (const uint32_t*)(ws + o_bc[cur]);
+    uint32_t* tst = (uint32_t*)(ws + o_tst);
+    uint32_t* tcnt = (uint32_t*)(ws + o_tcnt);
+    uint32_t* ploc = (uint32_t*)(ws + o_ploc);
+    uint32_t* bsum = (uint32_t*)(ws + o_bsum);
+    uint32_t* bpre = (uint32_t*)(ws + o_bpre);
+    uint32_t* lst = (uint32_t*)(ws + o_lst);
+    uint64_t* scst = (uint64_t*)(ws + o_scst);
+    uint32_t* ctr = (uint32_t*)(ws + o_ctr);
+    const unsigned sgrid = (unsigned)wtg_ceil_div(hb, 256), stiles = (unsigned)wtg_ceil_div(hb, 4096);
+    const uint64_t grid = wtg_ceil_div(n, MLD_WT) + hb;  // at least the tiles of hb segments of n keys at most
+    const uint32_t nrows = (uint32_t)grid + 1, nblocks = (uint32_t)wtg_ceil_div(nrows, MLD_SR);
+    MldArgs a{};
+    a.keys = kbuf[kb];
+    a.n = n;
+    a.L = L;
+    a.s = s;
+    a.g = g;
+    a.tl = 11;
+    a.nseg = hb;
+    a.tstart = tst;
+    a.tseg = (const uint32_t*)(ws + o_tseg);
+    a.seg_start = bs;
+    a.seg_cnt = bc;
+    a.tcnt = a.tcnt_w = tcnt;
+    a.ploc = ploc;
+    a.bpre = bpre;
+    a.cum = lst;
+    a.words = d_words;
+    a.kout = last ? nullptr : kbuf[kb ^ 1];
+    a.err = ctx->d_flag;
+    WTG_LAUNCH(ctx, "mld_ntiles", k_mld_list_tiles, dim3(sgrid), dim3(256), 0, bc, nb + 2 * cur, hb,
+               (uint32_t*)(ws + o_nt), 11u);
+    WTG_LAUNCH_CHECK();
+    WTG_TRY(wtg_fill_bytes_zero(ctx, scst, (char*)ctr + 256 - (char*)scst));
+    WTG_LAUNCH(ctx, "mld_tiles", k_scan_u32<uint32_t>, dim3(stiles), dim3(256), 0, (uint32_t*)(ws + o_nt), tst,
+               (uint64_t)hb, scst, ctr, ctx->d_flag);
+    WTG_LAUNCH_CHECK();
+    WTG_LAUNCH(ctx, "mld_tseg", k_mld_tseg, dim3((unsigned)wtg_ceil_div(grid, 256)), dim3(256), 0, tst, (uint64_t)hb,
+               (uint32_t*)(ws + o_tseg), maxt);
+    WTG_LAUNCH_CHECK();
+    mld_count_launch<KO>(ctx, (unsigned)grid, a);
+    WTG_LAUNCH_CHECK();
+    WTG_LAUNCH(ctx, "mld_scan", k_mld_scan1, dim3(nblocks), dim3(256), 0, tcnt, ploc, bsum,
+               (const uint32_t*)(tst + hb), 0u, 1u << g, nrows);
+    WTG_LAUNCH_CHECK();
+    WTG_LAUNCH(ctx, "mld_scan", k_mld_scan2, dim3(1u << g), dim3(256), 0, bsum, bpre, nblocks, 1u << g);
+    WTG_LAUNCH_CHECK();
+    if (!last) WTG_TRY(wtg_fill_u64(ctx, nb + 2 * (cur ^ 1), 1, 0));
+    WTG_LAUNCH(ctx, "mld_leaf", k_mld_leaf, dim3(hb), dim3(256), 0, a, lst, nb + 2 * cur, (uint32_t*)(ws + o_bs[cur ^ 1]),
+               (uint32_t*)(ws + o_bc[cur ^ 1]), last ? nullptr : nb + 2 * (cur ^ 1), cap, last ? d_distinct : nullptr);
+    WTG_LAUNCH_CHECK();
+    mld_emit_launch<KO, WIDE>(ctx, !last, (unsigned)grid, a);
+    WTG_LAUNCH_CHECK();
+    s += g;
+    kb ^= 1;
+    cur ^= 1;
+    if (last) break;
+    q.kin = kbuf[kb];
+    q.s = s;
+    q.mode = 2;
+    q.st = lst;
+    q.m = 1u << g;
+    q.nseg = hb;
+    q.tstart = tst;
+    q.tseg = a.tseg;
+    q.seg_start = bs;
+    q.seg_cnt = bc;
+    mld_local_launch<KO>(ctx, (unsigned)(grid * LOC_TW), q);
     WTG_LAUNCH_CHECK();
   }
   return WTG_OK;
@@ -937,22 +1421,41 @@ int wtg_mld_enabled() {
 
 static int mld_dispatch(wtg_ctx* ctx, const void* d_sym, int sym_bytes, uint64_t n, uint32_t L, uint32_t s0,
                         const uint32_t* d_cnt0, const uint64_t* d_src_off, uint64_t* d_words, wtg_node* d_nodes,
-                        uint64_t node_slots, unsigned long long* d_distinct, uint32_t kshift = 0) {
+                        uint64_t node_slots, unsigned long long* d_distinct) {
   switch (sym_bytes) {
     case 1: return mld_build_t<uint8_t>(ctx, (const uint8_t*)d_sym, n, L, s0, d_cnt0, d_src_off, d_words, d_nodes,
-                                        node_slots, d_distinct, kshift);
+                                        node_slots, d_distinct);
     case 2: return mld_build_t<uint16_t>(ctx, (const uint16_t*)d_sym, n, L, s0, d_cnt0, d_src_off, d_words, d_nodes,
-                                         node_slots, d_distinct, kshift);
+                                         node_slots, d_distinct);
     case 4: return mld_build_t<uint32_t>(ctx, (const uint32_t*)d_sym, n, L, s0, d_cnt0, d_src_off, d_words, d_nodes,
-                                         node_slots, d_distinct, kshift);
+                                         node_slots, d_distinct);
     default: return mld_build_t<uint64_t>(ctx, (const uint64_t*)d_sym, n, L, s0, d_cnt0, d_src_off, d_words,
-                                          d_nodes, node_slots, d_distinct, kshift);
+                                          d_nodes, node_slots, d_distinct);
+  }
+}
+
+template <typename K>
+static int mld_sparse_dispatch(wtg_ctx* ctx, const void* d_sym, uint64_t n, uint32_t L, uint64_t* d_words,
+                               unsigned long long* d_distinct) {
+  return L > 32 ? mld_sparse_t<K, uint64_t>(ctx, (const K*)d_sym, n, L, d_words, d_distinct)
+                : mld_sparse_t<K, uint32_t>(ctx, (const K*)d_sym, n, L, d_words, d_distinct);
+}
+
+// n >= 1, 1 <= L <= 64, n < 2^32; no node records
+int wtg_mld_build_sparse(wtg_ctx* ctx, const void* d_sym, int sym_bytes, uint64_t n, uint32_t L, uint64_t* d_words,
+                         unsigned long long* d_distinct) {
+  switch (sym_bytes) {
+    case 1: return mld_sparse_dispatch<uint8_t>(ctx, d_sym, n, L, d_words, d_distinct);
+    case 2: return mld_sparse_dispatch<uint16_t>(ctx, d_sym, n, L, d_words, d_distinct);
+    case 4: return mld_sparse_dispatch<uint32_t>(ctx, d_sym, n, L, d_words, d_distinct);
+    default: return mld_sparse_dispatch<uint64_t>(ctx, d_sym, n, L, d_words, d_distinct);
   }
 }
 
 // n >= 1, 1 <= L <= 24, n < 2^32
 int wtg_mld_build(wtg_ctx* ctx, const void* d_sym, int sym_bytes, uint64_t n, uint32_t L, uint64_t* d_words,
                   wtg_node* d_nodes, uint64_t node_slots, unsigned long long* d_distinct) {
+  if (!d_nodes && mld_use_sparse(n, L)) return wtg_mld_build_sparse(ctx, d_sym, sym_bytes, n, L, d_words, d_distinct);
   return mld_dispatch(ctx, d_sym, sym_bytes, n, L, 0, nullptr, nullptr, d_words, d_nodes, node_slots, d_distinct);
 }
 
@@ -967,10 +1470,3 @@ int wtg_mld_build_from(wtg_ctx* ctx, const void* d_keys, int key_bytes, uint64_t
 }
 
 size_t wtg_mld_ws_bytes(uint64_t n, uint32_t L, uint32_t s0) { return mld_plan(n, L, s0).total; }
-
-// the top Lt levels (Lt <= 24) of an L-level tree over d_sym (L > Lt): the
-// multi-level passes over the keys' top Lt bits; level l at bit l * n
-int wtg_mld_build_top(wtg_ctx* ctx, const void* d_sym, int sym_bytes, uint64_t n, uint32_t L, uint32_t Lt,
-                      uint64_t* d_words) {
-  return mld_dispatch(ctx, d_sym, sym_bytes, n, Lt, 0, nullptr, nullptr, d_words, nullptr, 0, nullptr, L - Lt);
-}
