@@ -16,11 +16,13 @@
 //                    global bit position: bv_pos[v] is the sum of the inner
 //                    nodes before v, the prefix within row v the bits of v before
 //                    segment s.
-//   3. k_huff_emit   up to 32 inner nodes (k_huff_emit_lane): each lane gathers
+//   3. k_huff_emit   up to 16 inner nodes (k_huff_emit_lane): each lane gathers
 //                    the branch bits of its 16 bytes node by node in registers
 //                    and a wave scan per node places them in the node's run of a
-//                    per-wave LDS staging area.  Larger trees (k_huff_emit): the
-//                    wave walks its segment in 64-byte chunks, level by level;
+//                    per-wave LDS staging area.  Larger trees: a block sorts its
+//                    segment down the tree level by level in LDS
+//                    (k_huff_emit_tile).  Codes of more than 23 bits
+//                    (k_huff_emit): the wave walks its segment in 64-byte chunks, level by level;
 //                    per (chunk, level) the lanes are sorted stably by node id
 //                    with one ballot per id bit, a ds_permute puts each node's
 //                    bits into one contiguous slice of a ballot word, and one
@@ -49,6 +51,7 @@ struct HuffTab {
   uint8_t len[256];          // code length, 0 = absent
   uint8_t lvl_first[64];     // first inner node id at depth l (ids are BFS, so a level is a range)
   uint8_t lvl_bits[64];      // bits for an id offset within level l plus one "none" value
+  uint8_t depth[256];        // per inner node
   uint32_t n_inner, max_depth, sigma, single;  // single: the symbol when sigma == 1
 };
 }  // namespace
@@ -379,6 +382,25 @@ __global__ __launch_bounds__(HF_THREADS) void k_huff_count_hist(SegArgs a) {
   }
 }
 
+// exclusive scan of one value per thread over a block's first 256 threads (the
+// others hold 0 and take part in the barriers)
+__device__ __forceinline__ uint32_t huff_scan256(uint32_t v, uint32_t* s_wave, uint32_t& total) {
+  const uint32_t w = threadIdx.x >> 6;
+  const uint32_t incl = wave_incl_sum_dpp(v);
+  if (lane_id() == 63 && w < 4) s_wave[w] = incl;
+  __syncthreads();
+  uint32_t off = 0, tot = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < 4; k++) {
+    const uint32_t t = s_wave[k];
+    if (k < w) off += t;
+    tot += t;
+  }
+  __syncthreads();
+  total = tot;
+  return incl - v + off;
+}
+
 // 64 bits of the staging area starting at local bit d (d may be negative: zeros)
 __device__ __forceinline__ uint64_t stage_bits(const uint64_t* stg, int64_t d) {
   if (d < 0) return d <= -64 ? 0ull : stg[0] << (uint32_t)(-d);
@@ -511,7 +533,8 @@ __global__ __launch_bounds__(HF_THREADS) void k_huff_emit(SegArgs a) {
   }
 }
 
-// pass 3 for trees of at most 32 inner nodes and 1024-byte segments: lane i
+// pass 3 for trees of at most 16 inner nodes (with long codes, 32) and
+// 1024-byte segments: lane i
 // takes bytes 16i..16i+15 of the segment and, node by node, gathers the branch
 // bits of its bytes that pass the node into a register (at most 16 bits); a wave
 // scan of the per-node bit counts (two nodes per scan, 16-bit fields) places
@@ -660,6 +683,180 @@ __global__ __launch_bounds__(HF_THREADS) void k_huff_emit_lane(SegArgs a) {
     }
     wave_sync_lds();
     cur = nxt;
+  }
+}
+
+// pass 3 for trees of more than HF_TILE_MIN inner nodes and codes of at most
+// HF_TILE_DEPTH bits: one block per 4096-byte segment, a level pipeline in LDS.
+// At depth l the keys still on their way (those whose code is longer than l)
+// lie in the order of their inner nodes (BFS ids, so a level's nodes are
+// consecutive), text order inside a node; the ballots of their next code bit
+// are the level's bits, and a stable split of every node by that bit gives the
+// order of depth l + 1, a key whose child is a leaf dropping out.  A key is its
+// remaining code, its node, and whether both children of that node are leaves
+// (its keys all drop out, and they count as ones in the split's prefix, so that
+// the zeros of every node follow from the segment's node counts).  A node's
+// table entry gives where its zeros and ones go: with zc the counted zeros
+// before position p of the level, a zero goes to X + zc and a one to
+// Y + p - zc (both modulo the tile).
+// Bound by VALU issue (~17 instructions per key and level, ~600 per wave for the
+// tables and runs of 255 nodes).  2^26 + 11 Zipf bytes over 256 values: 0.50 ms,
+// where walking 64-byte chunks down the tree (k_huff_emit, now for longer codes
+// only) took 2.77 ms; consecutive segments on one XCD: no change.  Up to 16
+// inner nodes k_huff_emit_lane is as fast or faster (2^24 bytes, whole build: 11
+// nodes 544 us against 561, 19 nodes 608 against 510).
+constexpr uint32_t HF_TILE = 4096, HF_TILE_THREADS = 512, HF_TILE_DEPTH = 23;
+constexpr uint32_t HF_TILE_ROW = HF_TILE / 32 + 4;  // staged words of a level (+ read-ahead)
+constexpr uint32_t HF_TILE_MIN = 16;
+__global__ __launch_bounds__(HF_TILE_THREADS) __attribute__((amdgpu_waves_per_eu(8))) void k_huff_emit_tile(SegArgs a) {
+  constexpr uint32_t M = HF_TILE / HF_TILE_THREADS, NWV = HF_TILE_THREADS / 64;
+  constexpr uint32_t BIT = 1u << 9, FLAG = 1u << 8;  // key: code << 9 | both-leaves << 8 | node
+  __shared__ __align__(16) uint32_t s_k[HF_TILE];
+  __shared__ uint2 s_nd[256];            // X | Y << 16, child0 | child1 << 16 (0xFFFF: leaf)
+  __shared__ uint32_t s_code[256];
+  __shared__ uint64_t s_zw[HF_TILE / 64];
+  __shared__ uint16_t s_ex[NWV][HF_TILE / 64];
+  __shared__ uint32_t s_A[HF_TILE_DEPTH + 2];  // keys at each depth
+  __shared__ uint32_t s_wave[4];
+  extern __shared__ uint64_t s_dyn[];    // [max_depth][HF_TILE_ROW] staged bits
+  uint32_t* s_bits = reinterpret_cast<uint32_t*>(s_dyn);
+  const uint32_t tid = threadIdx.x, lane = (uint32_t)lane_id();
+  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+  const uint64_t s = blockIdx.x, base = s * HF_TILE;
+  const uint32_t len = a.n - base < HF_TILE ? (uint32_t)(a.n - base) : HF_TILE;
+  const uint32_t ni = a.n_inner, md = a.tab->max_depth;
+  // text bytes and this segment's node counts and run positions
+  uint8_t tb[M];
+#pragma unroll
+  for (uint32_t m = 0; m < M; m++) {
+    const uint32_t p = (w + NWV * m) * 64 + lane;
+    tb[m] = a.text[base + (p < len ? p : 0u)];
+  }
+  uint32_t cv = 0, dv = 0, c0 = 0xFFFFu, c1 = 0xFFFFu;
+  uint64_t gp = 0;
+  uint32_t* s_c = s_k;           // node counts; their prefix over the nodes
+  uint32_t* s_E = s_k + 256;
+  uint32_t* s_Z = s_k + 513;     // prefix of the counted zeros
+  uint32_t* s_fl = s_k + 770;    // both children are leaves
+  if (tid < 256) {
+    const uint32_t v = tid;
+    if (v < ni) {
+      cv = a.cnt[(uint64_t)v * a.nseg + s];
+      gp = a.pos[(uint64_t)v * a.nseg + s];
+      dv = a.tab->depth[v];
+      c0 = a.tab->child[v][0];
+      c1 = a.tab->child[v][1];
+      if (c0 >= HF_LEAF) c0 = 0xFFFFu;
+      if (c1 >= HF_LEAF) c1 = 0xFFFFu;
+    }
+    s_code[v] = (uint32_t)a.tab->code[v] << 9;
+    s_c[v] = cv;
+    s_fl[v] = c0 == 0xFFFFu && c1 == 0xFFFFu ? FLAG : 0u;
+  }
+  __syncthreads();
+  const uint32_t zn = c0 != 0xFFFFu ? s_c[c0] : c1 != 0xFFFFu ? cv - s_c[c1] : 0u;
+  uint32_t tot;
+  const uint32_t E = huff_scan256(cv, s_wave, tot), Z = huff_scan256(zn, s_wave, tot);
+  if (tid < 256) {
+    s_E[tid] = E;
+    s_Z[tid] = Z;
+    if (tid == 255) s_E[256] = E + cv;
+  }
+  __syncthreads();
+  uint32_t S = 0;  // the node's start in its level
+  if (tid < ni) {
+    S = E - s_E[a.tab->lvl_first[dv]];
+    const uint32_t ZS = Z - s_Z[a.tab->lvl_first[dv]];
+    uint32_t X = 0, Y = 0, f0 = 0xFFFFu, f1 = 0xFFFFu;
+    const uint32_t nx = dv + 1 < 64 ? s_E[a.tab->lvl_first[dv + 1]] : 0u;  // the next level's first prefix
+    if (c0 != 0xFFFFu) { X = (s_E[c0] - nx - ZS) & 0xFFFFu; f0 = c0 | s_fl[c0]; }
+    if (c1 != 0xFFFFu) { Y = (s_E[c1] - nx - S + ZS) & 0xFFFFu; f1 = c1 | s_fl[c1]; }
+    s_nd[tid] = make_uint2(X | Y << 16, f0 | f1 << 16);
+  }
+  if (tid < md) s_A[tid] = s_E[tid + 1 < md ? a.tab->lvl_first[tid + 1] : 256] - s_E[a.tab->lvl_first[tid]];
+  uint32_t x[M];
+  const uint32_t rootf = s_fl[0];
+#pragma unroll
+  for (uint32_t m = 0; m < M; m++) x[m] = s_code[tb[m]] | rootf;
+  __syncthreads();  // s_k is free from here on
+  for (uint32_t l = 0; l < md; l++) {
+    const uint32_t A = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_A[l]);
+    if (A == 0) break;
+    uint64_t* row = reinterpret_cast<uint64_t*>(s_bits + l * HF_TILE_ROW);
+    uint64_t zm[M];
+#pragma unroll
+    for (uint32_t m = 0; m < M; m++) {
+      const uint32_t c = w + NWV * m;
+      zm[m] = 0;
+      if (c * 64 < A) {
+        const uint32_t p = c * 64 + lane;
+        if (l > 0) x[m] = s_k[p];
+        const uint64_t am = A - c * 64 >= 64 ? ~0ull : (1ull << (A - c * 64)) - 1;
+        const uint64_t ones = wave_ballot((x[m] & BIT) != 0) & am;
+        zm[m] = wave_ballot((x[m] & (BIT | FLAG)) == 0) & am;
+        if (lane == 0) {
+          row[c] = ones;
+          s_zw[c] = zm[m];
+        }
+      }
+    }
+    if (l + 1 == md) break;
+    __syncthreads();
+    const uint32_t v = lane * 64 < A ? popc64(s_zw[lane]) : 0u;
+    const uint32_t incl = wave_incl_sum_dpp(v);
+    s_ex[w][lane] = (uint16_t)(incl - v);
+    wave_sync_lds();
+#pragma unroll
+    for (uint32_t m = 0; m < M; m++) {
+      const uint32_t c = w + NWV * m;
+      if (c * 64 < A) {
+        const uint32_t p = c * 64 + lane;
+        const uint2 e = s_nd[x[m] & 0xFFu];
+        const uint32_t zc =
+            __builtin_amdgcn_mbcnt_hi((uint32_t)(zm[m] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)zm[m], s_ex[w][c]));
+        const bool zero = (x[m] & BIT) == 0;
+        const uint32_t child = zero ? e.y & 0xFFFFu : e.y >> 16;
+        const uint32_t dest = zero ? e.x + zc : (e.x >> 16) + p - zc;
+        if (p < A && child != 0xFFFFu) s_k[dest & (HF_TILE - 1)] = ((x[m] >> 1) & 0xFFFFFE00u) | child;
+      }
+    }
+    __syncthreads();
+  }
+  __syncthreads();
+  // write the runs: thread v describes node v's, then the destination words of
+  // all runs are dealt out over the block
+  uint64_t* s_rgs = reinterpret_cast<uint64_t*>(s_k);  // per run: global start,
+  uint32_t* s_rls = s_k + 512;                         // start in the staged bits,
+  uint32_t* s_rcnt = s_k + 768;                        // length,
+  uint32_t* s_rw = s_k + 1024;                         // first destination word item
+  uint32_t nw = 0;
+  if (tid < 256) {
+    if (cv) nw = (uint32_t)(((gp + cv - 1) >> 6) - (gp >> 6) + 1);
+    s_rgs[tid] = gp;
+    s_rls[tid] = dv * (HF_TILE_ROW * 32) + S;
+    s_rcnt[tid] = cv;
+  }
+  const uint32_t ex = huff_scan256(nw, s_wave, tot);
+  if (tid < 256) s_rw[tid] = ex;
+  __syncthreads();
+  const uint32_t nwords = tot;
+  for (uint32_t it = tid; it < nwords; it += HF_TILE_THREADS) {
+    uint32_t lo = 0, hi = ni;  // the last run whose first word item is <= it
+    while (hi - lo > 1) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (s_rw[mid] <= it) lo = mid; else hi = mid;
+    }
+    const uint64_t gs = s_rgs[lo], ge = gs + s_rcnt[lo];
+    const uint64_t wi = (gs >> 6) + (it - s_rw[lo]), wb = wi << 6;
+    const uint32_t b0 = gs > wb ? (uint32_t)(gs - wb) : 0u;
+    const uint32_t b1 = ge < wb + 64 ? (uint32_t)(ge - wb) : 64u;
+    const uint32_t lp = s_rls[lo] + (uint32_t)(wb + b0 - gs), o = lp & 31;
+    const uint32_t* q = s_bits + (lp >> 5);
+    const uint64_t lo64 = (uint64_t)q[0] | ((uint64_t)q[1] << 32);
+    uint64_t val = (o ? (lo64 >> o) | ((uint64_t)q[2] << (64 - o)) : lo64) << b0;
+    if (b1 < 64) val &= (1ull << b1) - 1;
+    if (b0 == 0 && b1 == 64) a.words[wi] = val;
+    else if (val) atomicOr(reinterpret_cast<unsigned long long*>(&a.words[wi]), (unsigned long long)val);
   }
 }
 
@@ -994,6 +1191,7 @@ void build_shape(const uint64_t* cnt, uint64_t n, wtg_huff_shape& S, HuffTab& T)
       int d = 0;
       for (int x = (int)k; S.parent[x] >= 0; x = S.parent[x]) d++;
       dep[inner_of[k]] = d;
+      T.depth[inner_of[k]] = (uint8_t)d;
     }
     bool bfs = true;
     for (uint32_t v = 1; v < ni; v++) bfs = bfs && dep[v] >= dep[v - 1];
@@ -1157,8 +1355,9 @@ extern "C" int wtg_huff_build(wtg_ctx* ctx, const uint8_t* d_text, uint64_t n, w
     if ((rc = wtg_malloc(ctx, (void**)&wt->dir, wtg_rank9_words(S.bv_size) * 8)) != WTG_OK) goto fail;
     if ((rc = wtg_fill_u64(ctx, wt->words, nw, 0)) != WTG_OK) goto fail;
     if (S.n_inner > 0) {
+      const bool tile = S.n_inner > HF_TILE_MIN && S.max_depth <= HF_TILE_DEPTH;
       // segment: 1024..4096 bytes so the count table stays <= n/4 bytes
-      uint32_t S_bytes = HF_PIECE;
+      uint32_t S_bytes = tile ? HF_TILE : HF_PIECE;
       while (S_bytes < 4 * HF_PIECE && (uint64_t)S.n_inner * 16 > S_bytes) S_bytes *= 2;
       const uint64_t nseg = wtg_ceil_div(n, S_bytes);
       const uint64_t entries = (uint64_t)S.n_inner * nseg;
@@ -1206,7 +1405,10 @@ extern "C" int wtg_huff_build(wtg_ctx* ctx, const uint8_t* d_text, uint64_t n, w
         rc = WTG_ERR_UNSUPPORTED;
         goto fail;
       }
-      if (S.n_inner <= 32 && S_bytes == HF_PIECE) {
+      if (tile) {
+        WTG_LAUNCH(ctx, "huff_emit", k_huff_emit_tile, dim3((unsigned)nseg), dim3(HF_TILE_THREADS),
+                   (size_t)S.max_depth * HF_TILE_ROW * 4, a);
+      } else if (S.n_inner <= 32 && S_bytes == HF_PIECE) {
         WTG_LAUNCH(ctx, "huff_emit", k_huff_emit_lane, dim3(grid), dim3(HF_THREADS), (size_t)4 * a.stage_words * 8,
                    a);
       } else {
