@@ -5,13 +5,15 @@
 // suffix that ends sorts before its extensions); round 0 sorts all suffixes by
 // their first q = floor(63 / c) bytes (7 for 256 values, 21 for DNA).  A
 // suffix's rank is the position of its group's first suffix in the sorted
-// order (32 bits).  Each later round h = q, 2q, 4q, ... re-sorts the suffixes
-// still in groups of two or more (every suffix, in text order, while they are
-// more than half) by (group rank, rank h bytes on + 1; 0 past the end) and
-// splits each group in place: new rank = group rank + offset of the subgroup's
-// first suffix in the group.  A suffix alone in its group keeps its final rank
-// (the ranks stay consistent, as in Larsson-Sadakane doubling) and its sa entry
-// is written then; it stops when no group of two or more is left.
+// order (32 bits).  The suffixes still in groups of two or more form a list in
+// that order, (suffix, group rank) each.  A later round h = q, 2q, 4q, ... reads
+// every listed suffix's rank h bytes on (+ 1; 0 past the end) and orders each
+// group by it: groups that fit a block in LDS by counting the smaller and equal
+// ranks (k_sa_refine), larger ones by a radix sort of (group rank, rank h bytes
+// on).  New rank = group rank + the smaller ones.  A suffix alone in its new
+// group keeps its final rank (the ranks stay consistent, as in Larsson-Sadakane
+// doubling), its sa entry is written and it leaves the list; the end is an empty
+// list.
 #include "wtg_internal.hpp"
 #include <rocprim/device/device_radix_sort.hpp>
 
@@ -55,192 +57,355 @@ __global__ __launch_bounds__(256) void k_sa_init(const uint8_t* __restrict__ t, 
   idx[i] = (uint32_t)i;
 }
 
-// after a sort of m keys, per sorted position k: fb[k] = first position of k's
-// run of equal keys and fa[k] = first position of k's run of equal rank parts
-// (key >> sh; not computed when whole_group), both as inclusive max-scans of
-// run starts within 4096-position tiles, tile maxima to tb / ta (completed by
-// the exclusive max-scan of the tile maxima)
-__global__ __launch_bounds__(256) void k_sa_runs_tiles(const uint64_t* __restrict__ key, uint64_t m,
-                                                       int whole_group, uint32_t sh, uint32_t* __restrict__ fa,
-                                                       uint32_t* __restrict__ fb, uint32_t* __restrict__ ta,
-                                                       uint32_t* __restrict__ tb) {
-  // the tile's keys go through LDS (coalesced loads; thread t then takes keys
-  // 16t..16t+15), padded one slot per 16 against bank conflicts; the same
-  // space then holds the two scanned outputs for coalesced stores
-  constexpr uint32_t PAD = 4096 + 4096 / 16;
-  __shared__ uint64_t s_k[PAD];
-  __shared__ uint32_t s_a[4], s_b[4];
-  uint32_t* s_o = (uint32_t*)s_k;  // [0, PAD) fa, [PAD, 2 PAD) fb
-  const uint64_t tile0 = (uint64_t)blockIdx.x * 4096;
+constexpr uint32_t SA_TILE = 4096;  // sorted positions per block (1024 per wave)
+
+// Run starts after a sort: position p starts a run of equal keys (b), of equal
+// group parts key >> sh (a); p is kept unless it is a run of its own.
+struct SaHeads {
+  bool a, b, keep;
+};
+__device__ __forceinline__ SaHeads sa_heads(const uint64_t* __restrict__ key, uint64_t p, uint64_t m, uint64_t k,
+                                            uint32_t sh) {
+  SaHeads r{false, false, false};
+  if (p >= m) return r;
+  const uint64_t before = p ? key[p - 1] : 0;
+  r.b = p == 0 || before != k;
+  r.a = p == 0 || (before >> sh) != (k >> sh);
+  r.keep = !(r.b && (p + 1 == m || key[p + 1] != k));
+  return r;
+}
+
+// per tile of sorted positions: its last run start (tb), last group start (ta,
+// unless whole) and kept positions (tc)
+__global__ __launch_bounds__(256) void k_sa_tiles(const uint64_t* __restrict__ key, uint64_t m, int whole, uint32_t sh,
+                                                  uint32_t* __restrict__ ta, uint32_t* __restrict__ tb,
+                                                  uint32_t* __restrict__ tc) {
+  __shared__ uint32_t s_a[4], s_b[4], s_c[4];
+  const uint32_t w = threadIdx.x >> 6;
+  const uint64_t base = (uint64_t)blockIdx.x * SA_TILE + threadIdx.x;
+  uint32_t a = 0, b = 0, c = 0;
 #pragma unroll
-  for (uint32_t j = 0; j < 16; j++) {
-    const uint32_t p = j * 256 + threadIdx.x;
-    if (tile0 + p < m) s_k[p + (p >> 4)] = key[tile0 + p];
+  for (uint32_t j = 0; j < SA_TILE / 256; j++) {
+    const uint64_t p = base + j * 256;
+    const SaHeads h = sa_heads(key, p, m, p < m ? key[p] : 0, sh);
+    if (h.b) b = (uint32_t)p;
+    if (h.a) a = (uint32_t)p;
+    c += h.keep;
   }
-  __syncthreads();
-  const uint32_t l0 = threadIdx.x * 16;
-  const uint64_t base = tile0 + l0;
-  uint32_t va[16], vb[16], ma = 0, mb = 0;
-  uint64_t prev = 0;
-  if (base < m) {
-    if (l0 > 0) prev = s_k[(l0 - 1) + ((l0 - 1) >> 4)];
-    else if (tile0 > 0) prev = key[tile0 - 1];
-  }
-#pragma unroll
-  for (uint32_t j = 0; j < 16; j++) {
-    const uint64_t p = base + j;
-    uint32_t a = 0, b = 0;
-    if (p < m) {
-      const uint64_t kc = s_k[threadIdx.x * 17 + j];
-      b = (p == 0 || kc != prev) ? (uint32_t)p : 0u;
-      a = (!whole_group && (p == 0 || (kc >> sh) != (prev >> sh))) ? (uint32_t)p : 0u;
-      prev = kc;
-    }
-    ma = a > ma ? a : ma;
-    mb = b > mb ? b : mb;
-    va[j] = ma;
-    vb[j] = mb;
-  }
-  uint32_t xa = ma, xb = mb;
-  const int lane = lane_id(), w = threadIdx.x >> 6;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t ya = (uint32_t)__shfl_up((int)xa, d);
-    const uint32_t yb = (uint32_t)__shfl_up((int)xb, d);
-    if (lane >= d) {
-      xa = ya > xa ? ya : xa;
-      xb = yb > xb ? yb : xb;
-    }
+    const uint32_t x = (uint32_t)__shfl_xor((int)a, d), y = (uint32_t)__shfl_xor((int)b, d);
+    a = x > a ? x : a;
+    b = y > b ? y : b;
   }
-  if (lane == 63) {
-    s_a[w] = xa;
-    s_b[w] = xb;
-  }
-  __syncthreads();  // also: every thread is done reading s_k
-  uint32_t pa = 0, pb = 0;
-  for (int k = 0; k < w; k++) {
-    pa = s_a[k] > pa ? s_a[k] : pa;
-    pb = s_b[k] > pb ? s_b[k] : pb;
-  }
-  uint32_t ea = (uint32_t)__shfl_up((int)xa, 1), eb = (uint32_t)__shfl_up((int)xb, 1);
-  if (lane == 0) ea = eb = 0;
-  ea = ea > pa ? ea : pa;
-  eb = eb > pb ? eb : pb;
-#pragma unroll
-  for (uint32_t j = 0; j < 16; j++) {
-    s_o[threadIdx.x * 17 + j] = va[j] > ea ? va[j] : ea;
-    s_o[PAD + threadIdx.x * 17 + j] = vb[j] > eb ? vb[j] : eb;
-  }
+  c = wave_sum(c);
+  if (lane_id() == 0) { s_a[w] = a; s_b[w] = b; s_c[w] = c; }
   __syncthreads();
-#pragma unroll
-  for (uint32_t j = 0; j < 16; j++) {
-    const uint32_t p = j * 256 + threadIdx.x;
-    if (tile0 + p < m) {
-      if (!whole_group) fa[tile0 + p] = s_o[p + (p >> 4)];
-      fb[tile0 + p] = s_o[PAD + p + (p >> 4)];
-    }
-  }
   if (threadIdx.x == 0) {
-    uint32_t xa2 = 0, xb2 = 0;
-    for (int k = 0; k < 4; k++) {
-      xa2 = s_a[k] > xa2 ? s_a[k] : xa2;
-      xb2 = s_b[k] > xb2 ? s_b[k] : xb2;
+    for (int k = 1; k < 4; k++) {
+      a = s_a[k] > a ? s_a[k] : a;
+      b = s_b[k] > b ? s_b[k] : b;
+      c += s_c[k];
     }
-    if (!whole_group) ta[blockIdx.x] = xa2;
-    tb[blockIdx.x] = xb2;
+    if (!whole) ta[blockIdx.x] = a;
+    tb[blockIdx.x] = b;
+    tc[blockIdx.x] = c;
   }
 }
 
-// exclusive max-scan of the tile maxima in place (one block, 4096 per chunk)
-__global__ __launch_bounds__(256) void k_sa_tile_prefix(uint32_t* __restrict__ tmax, uint64_t ntiles) {
-  __shared__ uint32_t s_w[4];
-  __shared__ uint32_t s_carry;
-  if (threadIdx.x == 0) s_carry = 0;
-  __syncthreads();
+// over the tiles, in place (one block): exclusive maximum of ta (unless whole)
+// and tb, exclusive sum of tc, whose total goes to *kept
+__global__ __launch_bounds__(256) void k_sa_tile_prefix(uint32_t* __restrict__ ta, uint32_t* __restrict__ tb,
+                                                        uint32_t* __restrict__ tc, uint64_t ntiles, int whole,
+                                                        uint32_t* __restrict__ kept) {
+  __shared__ uint32_t s_w[3][4];
+  uint32_t ca = 0, cb = 0, cc = 0;  // carries (every thread keeps them)
   const int lane = lane_id(), w = threadIdx.x >> 6;
-  for (uint64_t c0 = 0; c0 < ntiles; c0 += 4096) {
-    const uint64_t base = c0 + threadIdx.x * 16;
-    uint32_t v[16], m = 0;
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
-      v[j] = base + j < ntiles ? tmax[base + j] : 0u;
-      m = v[j] > m ? v[j] : m;
-    }
-    uint32_t x = m;
+  for (uint64_t c0 = 0; c0 < ntiles; c0 += 256) {
+    const uint64_t i = c0 + threadIdx.x;
+    const bool in = i < ntiles;
+    const uint32_t a = in && !whole ? ta[i] : 0u, b = in ? tb[i] : 0u, c = in ? tc[i] : 0u;
+    uint32_t xa = a, xb = b, xc = c;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-      const uint32_t y = (uint32_t)__shfl_up((int)x, d);
-      if (lane >= d) x = y > x ? y : x;
+      const uint32_t ya = (uint32_t)__shfl_up((int)xa, d), yb = (uint32_t)__shfl_up((int)xb, d),
+                     yc = (uint32_t)__shfl_up((int)xc, d);
+      if (lane >= d) {
+        xa = ya > xa ? ya : xa;
+        xb = yb > xb ? yb : xb;
+        xc += yc;
+      }
     }
-    if (lane == 63) s_w[w] = x;
+    if (lane == 63) { s_w[0][w] = xa; s_w[1][w] = xb; s_w[2][w] = xc; }
     __syncthreads();
-    uint32_t pre = s_carry;
-    for (int k = 0; k < w; k++) pre = s_w[k] > pre ? s_w[k] : pre;
-    uint32_t ex = (uint32_t)__shfl_up((int)x, 1);
-    if (lane == 0) ex = 0;
-    uint32_t run = ex > pre ? ex : pre;
+    uint32_t ea = (uint32_t)__shfl_up((int)xa, 1), eb = (uint32_t)__shfl_up((int)xb, 1), ec = xc - c;
+    if (lane == 0) ea = eb = 0;
+    ea = ea > ca ? ea : ca;
+    eb = eb > cb ? eb : cb;
+    ec += cc;
+    for (int k = 0; k < 4; k++) {
+      const uint32_t qa = s_w[0][k], qb = s_w[1][k], qc = s_w[2][k];
+      if (k < w) {
+        ea = qa > ea ? qa : ea;
+        eb = qb > eb ? qb : eb;
+        ec += qc;
+      }
+      ca = qa > ca ? qa : ca;
+      cb = qb > cb ? qb : cb;
+      cc += qc;
+    }
+    if (in) {
+      if (!whole) ta[i] = ea;
+      tb[i] = eb;
+      tc[i] = ec;
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *kept = cc;
+}
+
+// After a sort of (group rank << sh | key) pairs (whole: one group of rank 0):
+// the rank of sorted position p is its group's plus the distance of its run's
+// start from its group's.  A run of one has its final rank: its sa entry is
+// written.  The others go to the list, in order, from `list0` on.  A wave takes
+// 1024 consecutive positions, a chunk of 64 at a time: run starts and kept
+// positions are ballots, so nothing but the keys is read twice.
+__global__ __launch_bounds__(256) void k_sa_apply(const uint64_t* __restrict__ key, const uint32_t* __restrict__ val,
+                                                  uint64_t m, uint64_t n, int whole, uint32_t sh,
+                                                  const uint32_t* __restrict__ ta, const uint32_t* __restrict__ tb,
+                                                  const uint32_t* __restrict__ tc, uint32_t* __restrict__ rank,
+                                                  int64_t* __restrict__ sa, uint32_t* __restrict__ idx,
+                                                  uint32_t* __restrict__ grp, uint32_t list0,
+                                                  uint32_t* __restrict__ err) {
+  constexpr uint32_t J = SA_TILE / 256;
+  __shared__ uint32_t s_a[4], s_b[4], s_c[4];
+  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (uint32_t)lane_id();
+  const uint64_t p0 = (uint64_t)blockIdx.x * SA_TILE + w * (SA_TILE / 4);
+  uint64_t kv[J], ma[J], mb[J], mk[J];
+  uint32_t la = 0, lb = 0, lc = 0;  // the wave's last starts, kept positions
 #pragma unroll
-    for (int j = 0; j < 16; j++) {
-      if (base + j < ntiles) tmax[base + j] = run;  // exclusive
-      run = v[j] > run ? v[j] : run;
+  for (uint32_t j = 0; j < J; j++) {
+    const uint64_t p = p0 + j * 64 + lane;
+    kv[j] = p < m ? key[p] : 0;
+  }
+#pragma unroll
+  for (uint32_t j = 0; j < J; j++) {
+    const uint64_t p = p0 + j * 64 + lane;
+    const SaHeads h = sa_heads(key, p, m, kv[j], sh);
+    ma[j] = wave_ballot(h.a);
+    mb[j] = wave_ballot(h.b);
+    mk[j] = wave_ballot(h.keep);
+    if (ma[j]) la = (uint32_t)(p0 + j * 64) + 63u - (uint32_t)__builtin_clzll(ma[j]);
+    if (mb[j]) lb = (uint32_t)(p0 + j * 64) + 63u - (uint32_t)__builtin_clzll(mb[j]);
+    lc += popc64(mk[j]);
+  }
+  if (lane == 0) { s_a[w] = la; s_b[w] = lb; s_c[w] = lc; }
+  __syncthreads();
+  uint32_t ca = whole ? 0u : ta[blockIdx.x], cb = tb[blockIdx.x], cc = list0 + tc[blockIdx.x];
+  for (uint32_t k = 0; k < w; k++) {
+    ca = s_a[k] > ca ? s_a[k] : ca;
+    cb = s_b[k] > cb ? s_b[k] : cb;
+    cc += s_c[k];
+  }
+  const uint64_t upto = ~0ull >> (63 - lane);
+#pragma unroll
+  for (uint32_t j = 0; j < J; j++) {
+    const uint32_t c0 = (uint32_t)(p0 + j * 64);
+    const uint64_t p = p0 + j * 64 + lane;
+    const uint64_t fa = ma[j] & upto, fb = mb[j] & upto;
+    const uint32_t first = whole ? 0u : fa ? c0 + 63u - (uint32_t)__builtin_clzll(fa) : ca;
+    const uint32_t head = fb ? c0 + 63u - (uint32_t)__builtin_clzll(fb) : cb;
+    if (p < m) {
+      const uint32_t g = whole ? 0u : (uint32_t)(kv[j] >> sh);
+      const uint32_t r = g + (head - first), i = val[p];
+      if (whole || r != g) rank[i] = r;  // (a group's first run keeps its rank)
+      if (mk[j] >> lane & 1u) {
+        const uint32_t q = cc + mbcnt64(mk[j]);
+        idx[q] = i;
+        grp[q] = r;
+      } else if (r < n) {
+        sa[r] = (int64_t)i;
+      } else {
+        atomicOr(err, WTG_FLAG_SA_RANKS);  // ranks inconsistent: not expected
+      }
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      uint32_t mx = s_carry;
-      for (int k = 0; k < 4; k++) mx = s_w[k] > mx ? s_w[k] : mx;
-      s_carry = mx;
-    }
-    __syncthreads();
+    if (ma[j]) ca = c0 + 63u - (uint32_t)__builtin_clzll(ma[j]);
+    if (mb[j]) cb = c0 + 63u - (uint32_t)__builtin_clzll(mb[j]);
+    cc += popc64(mk[j]);
   }
 }
 
-// keys (rank << sh) | (rank h bytes on + 1; 0 past the end), sh = bits of n:
-// of the unresolved suffixes act[0..m) or, with act null, of every suffix in
-// text order (coalesced rank reads while most suffixes are unresolved; a
-// resolved suffix sorts alone in its group and keeps its rank)
-__global__ void k_sa_keys(const uint32_t* __restrict__ rank, const uint32_t* __restrict__ act, uint64_t m,
-                          uint64_t n, uint64_t h, uint32_t sh, uint64_t* __restrict__ key, uint32_t* __restrict__ val) {
-  const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// the listed suffixes' ranks h bytes on (+ 1; 0 past the end), before any rank
+// of this round changes; also clears the round's two counters
+__global__ __launch_bounds__(256) void k_sa_gather(const uint32_t* __restrict__ idx, uint64_t m, uint64_t n, uint64_t h,
+                                                   const uint32_t* __restrict__ rank, uint32_t* __restrict__ key2,
+                                                   uint32_t* __restrict__ counts) {
+  const uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+  if (k < 2) counts[k] = 0;
   if (k >= m) return;
-  const uint32_t i = act ? act[k] : (uint32_t)k;
-  key[k] = ((uint64_t)rank[i] << sh) | (i + h < n ? (uint64_t)rank[i + h] + 1 : 0ull);
-  val[k] = i;
+  const uint64_t i = (uint64_t)idx[k] + h;
+  key2[k] = i < n ? rank[i] + 1 : 0u;
 }
 
-// new rank of sorted position k: the group's old rank (0 in round 0) plus the
-// offset of k's subgroup head from the group's first position (fa, fb, ta, tb
-// from k_sa_runs_tiles and the tile prefix).  A suffix alone in its subgroup has
-// its final rank r: sa[r] = suffix (r grows with k, so these stores are nearly
-// sequential) and keep[k] = 0; else keep[k] = 1.
-__global__ void k_sa_update(const uint64_t* __restrict__ key, const uint32_t* __restrict__ val, uint64_t m,
-                            uint64_t n, int whole_group, uint32_t sh, const uint32_t* __restrict__ fa,
-                            const uint32_t* __restrict__ ta, const uint32_t* __restrict__ fb,
-                            const uint32_t* __restrict__ tb, uint32_t* __restrict__ rank, uint32_t* __restrict__ keep,
-                            int64_t* __restrict__ sa, uint32_t* __restrict__ err) {
-  const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= m) return;
-  const uint64_t t = k / 4096;
-  const uint32_t first = whole_group ? 0u : (fa[k] > ta[t] ? fa[k] : ta[t]);
-  const uint32_t head = fb[k] > tb[t] ? fb[k] : tb[t];
-  const uint32_t g = whole_group ? 0u : (uint32_t)(key[k] >> sh);
-  const uint32_t r = g + (head - first);
-  const uint32_t i = val[k];
-  // after round 0 the rank changes only past a group's first subgroup
-  if (whole_group || r != g) rank[i] = r;
-  const bool single = head == (uint32_t)k && (k + 1 == m || key[k + 1] != key[k]);
-  keep[k] = single ? 0u : 1u;
-  // a suffix already alone in its group has its sa entry from an earlier round
-  const bool was_single = !whole_group && first == (uint32_t)k && (k + 1 == m || (key[k + 1] >> sh) != g);
-  if (single && !was_single) {
-    if (r < n) sa[r] = (int64_t)i;
-    else atomicOr(err, WTG_FLAG_SA_RANKS);  // ranks inconsistent: not expected
+// One round over the list: a block takes the groups that start in its window of
+// SA_W list positions and end within SA_CAP of the window's start (as long as a
+// group has at most SA_CAP - SA_W suffixes it does).  For each suffix it counts
+// the group's smaller, equal and earlier equal ranks h bytes on, which gives the
+// new rank, the new place in the group, and whether it is alone.  Suffixes of
+// larger groups go to (bkey, bval) for a sort.  The blocks' outputs follow one
+// another in any order: groups stay whole, and nothing else is read from the
+// order of the list.
+// Groups are mostly small, and one pass over a round's list takes the place of a
+// radix sort's seven passes plus run marking, scan and compaction: 2^25 DNA bytes
+// with copied segments, all rounds after the first
+// 7.2 -> 1.0 ms.
+constexpr uint32_t SA_CAP = 2048, SA_W = 1536;
+__global__ __launch_bounds__(256) void k_sa_refine(const uint32_t* __restrict__ idx, const uint32_t* __restrict__ grp,
+                                                   const uint32_t* __restrict__ key2, uint64_t m, uint64_t n,
+                                                   uint32_t sh, uint32_t* __restrict__ rank, int64_t* __restrict__ sa,
+                                                   uint32_t* __restrict__ idx2, uint32_t* __restrict__ grp2,
+                                                   uint32_t* __restrict__ counts, uint64_t* __restrict__ bkey,
+                                                   uint32_t* __restrict__ bval, uint32_t* __restrict__ err) {
+  constexpr uint32_t M = SA_CAP / 256, NONE = 0xFFFFFFFFu;
+  __shared__ uint32_t s_g[SA_CAP], s_k[SA_CAP], s_i[SA_CAP];
+  __shared__ uint64_t s_h[SA_CAP / 64], s_kp[SA_CAP / 64];
+  __shared__ uint32_t s_base, s_bbase;
+  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (uint32_t)lane_id();
+  const uint64_t lo = (uint64_t)blockIdx.x * SA_W;
+  const uint32_t have = m - lo < SA_CAP ? (uint32_t)(m - lo) : SA_CAP;  // list positions in reach
+  const bool more = m - lo > SA_CAP;                                    // the list goes on past them
+  const uint32_t width = have < SA_W ? have : SA_W;
+  uint32_t g[M], kk[M], ii[M];
+#pragma unroll
+  for (uint32_t j = 0; j < M; j++) {
+    const uint32_t p = (w + 4 * j) * 64 + lane;
+    g[j] = kk[j] = ii[j] = 0;
+    bool head = false;
+    if (p < have) {
+      g[j] = grp[lo + p];
+      kk[j] = key2[lo + p];
+      ii[j] = idx[lo + p];
+      head = lo + p == 0 || grp[lo + p - 1] != g[j];
+      s_g[p] = g[j];
+      s_k[p] = kk[j];
+    }
+    const uint64_t hm = wave_ballot(head);
+    if (lane == 0) s_h[w + 4 * j] = hm;
   }
-}
-
-__global__ void k_sa_compact(const uint32_t* __restrict__ val, const uint32_t* __restrict__ keep,
-                             const uint32_t* __restrict__ pos, uint64_t m, uint32_t* __restrict__ act) {
-  const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < m && keep[k]) act[pos[k]] = val[k];
+  __syncthreads();
+  // f: the first group start in the window; e: the end of the last group that
+  // is this block's (both block-uniform)
+  uint32_t f = SA_CAP, last = 0, next = more ? SA_CAP + 1 : have;  // last start in the window, the start after it
+  {
+    const uint64_t hv = lane < SA_CAP / 64 ? s_h[lane] : 0ull;
+    const uint64_t in = lane < SA_W / 64 ? hv : 0ull, out = hv & ~in;
+    const uint64_t bi = wave_ballot(in != 0), bo = wave_ballot(out != 0);
+    if (bi) {
+      const uint32_t c0 = (uint32_t)__builtin_ctzll(bi), c1 = 63u - (uint32_t)__builtin_clzll(bi);
+      f = c0 * 64 + (uint32_t)__builtin_ctzll(s_h[c0]);
+      last = c1 * 64 + 63u - (uint32_t)__builtin_clzll(s_h[c1]);
+    }
+    if (bo) {
+      const uint32_t c0 = (uint32_t)__builtin_ctzll(bo);
+      next = c0 * 64 + (uint32_t)__builtin_ctzll(s_h[c0]);
+    } else if (more && grp[lo + SA_CAP] != s_g[SA_CAP - 1]) {
+      next = SA_CAP;
+    }
+  }
+  const uint32_t e = f == SA_CAP ? 0u : next <= SA_CAP ? next : last;
+  // positions of the window before f belong to a group of an earlier window: a
+  // large one if it started before the previous window, or ends past its reach
+  bool pre = false;
+  if (lo > 0 && f > 0) {
+    const uint32_t end = f < SA_CAP ? f : (next <= SA_CAP ? next : SA_CAP + 1);
+    pre = end > SA_CAP - SA_W || (lo > SA_W && grp[lo - SA_W - 1] == s_g[0]);
+  }
+  uint32_t np[M], ng[M];  // new place and rank (NONE: leaves the list, or not this block's)
+  uint32_t nbig = 0;
+  uint64_t bigm[M];
+  const uint64_t upto = ~0ull >> (63 - lane);
+#pragma unroll
+  for (uint32_t j = 0; j < M; j++) {
+    const uint32_t c = w + 4 * j, p = c * 64 + lane;
+    const bool mine = p >= f && p < e;
+    const bool big = p < width && ((p < f && pre) || (f < SA_CAP && p >= f && p >= e));
+    bigm[j] = wave_ballot(big);
+    nbig += popc64(bigm[j]);
+    np[j] = ng[j] = NONE;
+    if (mine) {
+      uint32_t q = c;
+      uint64_t h = s_h[q] & upto;
+      while (h == 0) h = s_h[--q];  // (f starts a group at or before p)
+      const uint32_t S = q * 64 + 63u - (uint32_t)__builtin_clzll(h);
+      uint32_t E = e;
+      q = c;
+      h = s_h[q] & ~upto;
+      while (h == 0 && ++q < SA_CAP / 64) h = s_h[q];
+      if (h) E = q * 64 + (uint32_t)__builtin_ctzll(h);
+      uint32_t less = 0, eq = 0, eqb = 0;
+      for (uint32_t t = S; t < E; t++) {
+        const uint32_t kt = s_k[t];
+        less += kt < kk[j];
+        const uint32_t same = kt == kk[j];
+        eq += same;
+        eqb += t < p ? same : 0u;
+      }
+      const uint32_t r = g[j] + less;
+      if (less) rank[ii[j]] = r;
+      if (eq == 1) {
+        if (r < n) sa[r] = (int64_t)ii[j];
+        else atomicOr(err, WTG_FLAG_SA_RANKS);  // ranks inconsistent: not expected
+      } else {
+        ng[j] = r;
+      }
+      np[j] = S + less + eqb;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t j = 0; j < M; j++) {  // into the new order
+    if (np[j] != NONE) {
+      s_g[np[j]] = ng[j];
+      s_i[np[j]] = ii[j];
+    }
+  }
+  if (lane == 0) s_k[w] = nbig;
+  __syncthreads();
+  uint64_t km[M];
+#pragma unroll
+  for (uint32_t j = 0; j < M; j++) {
+    const uint32_t c = w + 4 * j, p = c * 64 + lane;
+    km[j] = wave_ballot(p >= f && p < e && s_g[p] != NONE);
+    if (lane == 0) s_kp[c] = km[j];
+  }
+  __syncthreads();
+  const uint32_t kc = lane < SA_CAP / 64 ? popc64(s_kp[lane]) : 0u;
+  const uint32_t incl = wave_incl_sum_dpp(kc);
+  const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+  if (threadIdx.x == 0) {
+    s_base = total ? atomicAdd(&counts[0], total) : 0u;
+    const uint32_t nb = s_k[0] + s_k[1] + s_k[2] + s_k[3];
+    s_bbase = nb ? atomicAdd(&counts[1], nb) : 0u;
+  }
+  __syncthreads();
+  uint32_t bat = s_bbase;
+  for (uint32_t k = 0; k < w; k++) bat += s_k[k];
+#pragma unroll
+  for (uint32_t j = 0; j < M; j++) {
+    const uint32_t c = w + 4 * j, p = c * 64 + lane;
+    const uint32_t ex = (uint32_t)__builtin_amdgcn_readlane((int)(incl - kc), (int)c);
+    if (km[j] >> lane & 1u) {
+      const uint32_t q = s_base + ex + mbcnt64(km[j]);
+      idx2[q] = s_i[p];
+      grp2[q] = s_g[p];
+    }
+    if (bigm[j] >> lane & 1u) {
+      const uint32_t q = bat + mbcnt64(bigm[j]);
+      bkey[q] = (uint64_t)g[j] << sh | kk[j];
+      bval[q] = ii[j];
+    }
+    bat += popc64(bigm[j]);
+  }
 }
 
 // bwt[i] = t[sa[i]-1], or t[n-1] where sa[i] = 0 (fm-index/par/WT.C:38-41)
@@ -286,39 +451,50 @@ extern "C" int wtg_suffix_array_gpu(wtg_ctx* ctx, const uint8_t* d_text, uint64_
   WTG_REQUIRE(n < (1ull << 31), "wtg_suffix_array_gpu: n >= 2^31");
   if (n == 0) return WTG_OK;
   WTG_TRY(wtg_set_device(ctx));
-  // Each round sorts only the suffixes whose group is not yet a singleton
-  // (ranks of resolved suffixes are final and stay consistent with the order).
-  const uint64_t tiles = wtg_ceil_div(n, 4096);
-  uint64_t *k0 = nullptr, *k1 = nullptr, *st = nullptr;
-  uint32_t *v0 = nullptr, *v1 = nullptr, *act = nullptr, *rank = nullptr, *fa = nullptr, *fb = nullptr;
-  uint32_t *ta = nullptr, *tb = nullptr, *keep = nullptr, *pos = nullptr, *ctr = nullptr, *present = nullptr;
-  void* tmp = nullptr;
+  const uint64_t tiles = wtg_ceil_div(n, SA_TILE);
+  uint64_t *k0 = nullptr, *k1 = nullptr;
+  uint32_t *v0 = nullptr, *v1 = nullptr;
   size_t tmp_bytes = 0;
-  int rc = WTG_OK;
-  if ((rc = wtg_malloc(ctx, (void**)&k0, n * 8)) != WTG_OK || (rc = wtg_malloc(ctx, (void**)&k1, n * 8)) != WTG_OK ||
-      (rc = wtg_malloc(ctx, (void**)&v0, n * 4)) != WTG_OK || (rc = wtg_malloc(ctx, (void**)&v1, n * 4)) != WTG_OK ||
-      (rc = wtg_malloc(ctx, (void**)&act, n * 4)) != WTG_OK ||
-      (rc = wtg_malloc(ctx, (void**)&rank, n * 4)) != WTG_OK ||
-      (rc = wtg_malloc(ctx, (void**)&fa, n * 4)) != WTG_OK || (rc = wtg_malloc(ctx, (void**)&fb, n * 4)) != WTG_OK ||
-      (rc = wtg_malloc(ctx, (void**)&ta, tiles * 4)) != WTG_OK ||
-      (rc = wtg_malloc(ctx, (void**)&tb, tiles * 4)) != WTG_OK ||
-      (rc = wtg_malloc(ctx, (void**)&keep, n * 4)) != WTG_OK ||
-      (rc = wtg_malloc(ctx, (void**)&pos, (n + 1) * 4)) != WTG_OK ||
-      (rc = wtg_malloc(ctx, (void**)&st, (tiles + 1) * 8)) != WTG_OK ||
-      (rc = wtg_malloc(ctx, (void**)&ctr, 256)) != WTG_OK ||
-      (rc = wtg_malloc(ctx, (void**)&present, 256 * 4 + 256 * 2)) != WTG_OK)
-    goto out;
   for (unsigned eb : {63u, 64u}) {  // temporary storage for the widest sort
     size_t b = 0;
     if (rocprim::radix_sort_pairs(nullptr, b, k0, k1, v0, v1, (uint32_t)n, 0, eb, ctx->stream) != hipSuccess) {
       wtg_set_error("wtg_suffix_array_gpu: sort size query failed");
-      rc = WTG_ERR_HIP;
-      goto out;
+      return WTG_ERR_HIP;
     }
     tmp_bytes = b > tmp_bytes ? b : tmp_bytes;
   }
-  if ((rc = wtg_malloc(ctx, &tmp, tmp_bytes)) != WTG_OK) goto out;
+  // All buffers in one block: the context's workspace, or for a large text (its
+  // workspace would stay that large) an allocation of this call.  Thirteen
+  // allocations of 4 to 8 n bytes from the pool cost 2.5 to 50 ms a call
+  // (n = 2^25: the pool unmaps and maps what does not fit its free blocks).
+  size_t o = 0;
+  const auto take = [&](size_t bytes) { const size_t at = o; o = wtg_align256(o + bytes); return at; };
+  const size_t o_k0 = take(n * 8), o_k1 = take(n * 8), o_v0 = take(n * 4), o_v1 = take(n * 4), o_rank = take(n * 4);
+  const size_t o_i0 = take(n * 4), o_i1 = take(n * 4), o_g0 = take(n * 4), o_g1 = take(n * 4), o_key2 = take(n * 4);
+  const size_t o_tab = take((3 * tiles + 4) * 4), o_pres = take(256 * 4 + 256 * 2), o_tmp = take(tmp_bytes);
+  constexpr size_t SA_WS_MAX = 8ull << 30;
+  char* mem = nullptr;
+  int rc = WTG_OK;
+  if (o <= SA_WS_MAX) {
+    WTG_TRY(wtg_ws_reserve(ctx, o));
+    mem = (char*)ctx->ws;
+  } else {
+    WTG_TRY(wtg_malloc(ctx, (void**)&mem, o));
+  }
+  k0 = (uint64_t*)(mem + o_k0);
+  k1 = (uint64_t*)(mem + o_k1);
+  v0 = (uint32_t*)(mem + o_v0);
+  v1 = (uint32_t*)(mem + o_v1);
+  uint32_t* const rank = (uint32_t*)(mem + o_rank);
+  uint32_t* const idx[2] = {(uint32_t*)(mem + o_i0), (uint32_t*)(mem + o_i1)};
+  uint32_t* const grp[2] = {(uint32_t*)(mem + o_g0), (uint32_t*)(mem + o_g1)};
+  uint32_t* const key2 = (uint32_t*)(mem + o_key2);
+  uint32_t* const tab = (uint32_t*)(mem + o_tab);
+  uint32_t* const present = (uint32_t*)(mem + o_pres);
+  void* const tmp = mem + o_tmp;
   {
+    // tile tables, then the kept count, then the round's two counters
+    uint32_t *ta = tab, *tb = tab + tiles, *tc = tab + 2 * tiles, *kept = tab + 3 * tiles, *counts = kept + 1;
     uint32_t nbits = 1;
     while (nbits < 32 && (1ull << nbits) <= n) nbits++;
     // round 0 codes the sigma distinct bytes as 1..sigma in c bits (order kept),
@@ -336,73 +512,57 @@ extern "C" int wtg_suffix_array_gpu(wtg_ctx* ctx, const uint8_t* d_text, uint64_
     uint32_t cbits = 1;
     while ((1u << cbits) <= sigma) cbits++;
     const uint32_t q = 63 / cbits;
-    if (hipMemcpyAsync(d_code, h_code, sizeof(h_code), hipMemcpyHostToDevice, ctx->stream) != hipSuccess ||
-        hipStreamSynchronize(ctx->stream) != hipSuccess) {
-      wtg_set_error("wtg_suffix_array_gpu: code table copy failed");
-      rc = WTG_ERR_HIP;
-      goto out;
-    }
-    uint64_t m = n, h = 0;
-    for (int round = 0; round < 40 && m > 0; round++) {
-      if (round == 0) {
-        WTG_LAUNCH(ctx, "sa_init", k_sa_init, dim3((unsigned)wtg_ceil_div(n, 256)), dim3(256), 0, d_text, n, d_code,
-                   cbits, q, k0, v0);
-      } else {
-        const bool all = 2 * m > n;  // every suffix in text order
-        if (all) m = n;
-        WTG_LAUNCH(ctx, "sa_keys", k_sa_keys, dim3((unsigned)wtg_ceil_div(m, 256)), dim3(256), 0, rank,
-                   all ? (const uint32_t*)nullptr : act, m, n, h, nbits, k0, v0);
-      }
-      SA_LAUNCH_CHECK();
-      const unsigned end_bit = round == 0 ? q * cbits : 2u * nbits;
-      const unsigned grid = (unsigned)wtg_ceil_div(m, 256);
-      const uint64_t mt = wtg_ceil_div(m, 4096);
+    if ((rc = wtg_stage_h2d(ctx, d_code, h_code, sizeof(h_code))) != WTG_OK) goto out;
+    // sorts the m pairs (k0, v0) by their low end_bit bits, then ranks, sa entries
+    // and the list from list0 on; *left: the list's length after it
+    const auto sorted_round = [&](uint64_t m, unsigned end_bit, int whole, int b, uint32_t list0, uint64_t* left) -> int {
+      const unsigned grid = (unsigned)wtg_ceil_div(m, SA_TILE);
       if (rocprim::radix_sort_pairs(tmp, tmp_bytes, k0, k1, v0, v1, (uint32_t)m, 0, end_bit, ctx->stream) !=
           hipSuccess) {
         wtg_set_error("wtg_suffix_array_gpu: sort failed");
-        rc = WTG_ERR_HIP;
-        goto out;
+        return WTG_ERR_HIP;
       }
-      const int whole = round == 0 ? 1 : 0;
-      WTG_LAUNCH(ctx, "sa_runs", k_sa_runs_tiles, dim3((unsigned)mt), dim3(256), 0, k1, m, whole, nbits, fa, fb, ta,
-                 tb);
-      SA_LAUNCH_CHECK();
-      WTG_LAUNCH(ctx, "sa_tile_prefix", k_sa_tile_prefix, dim3(1), dim3(256), 0, tb, mt);
-      SA_LAUNCH_CHECK();
-      if (!whole) {
-        WTG_LAUNCH(ctx, "sa_tile_prefix", k_sa_tile_prefix, dim3(1), dim3(256), 0, ta, mt);
-        SA_LAUNCH_CHECK();
-      }
-      WTG_LAUNCH(ctx, "sa_update", k_sa_update, dim3(grid), dim3(256), 0, k1, v1, m, n, whole, nbits, fa, ta, fb, tb,
-                 rank, keep, d_sa, ctx->d_flag);
-      SA_LAUNCH_CHECK();
-      // compact the unresolved suffixes (exclusive scan of keep)
-      const uint64_t sct = wtg_ceil_div(m, 4096);
-      if ((rc = wtg_fill_bytes_zero(ctx, st, (sct + 1) * 8)) != WTG_OK) goto out;
-      if ((rc = wtg_fill_bytes_zero(ctx, ctr, 4)) != WTG_OK) goto out;
-      WTG_LAUNCH(ctx, "sa_keep_scan", k_scan_u32<uint32_t>, dim3((unsigned)sct), dim3(256), 0, keep, pos, m, st, ctr,
-                 ctx->d_flag);
-      SA_LAUNCH_CHECK();
-      WTG_LAUNCH(ctx, "sa_compact", k_sa_compact, dim3(grid), dim3(256), 0, v1, keep, pos, m, act);
-      SA_LAUNCH_CHECK();
-      uint32_t mnext = 0;
-      if ((rc = wtg_stage_d2h(ctx, &mnext, pos + m, 4)) != WTG_OK) goto out;
-      m = mnext;
-      h = h == 0 ? q : 2 * h;
-      if (m > 0 && (round == 39 || h >= 2 * n)) {
+      WTG_LAUNCH(ctx, "sa_tiles", k_sa_tiles, dim3(grid), dim3(256), 0, k1, m, whole, nbits, ta, tb, tc);
+      WTG_LAUNCH_CHECK();
+      WTG_LAUNCH(ctx, "sa_tile_prefix", k_sa_tile_prefix, dim3(1), dim3(256), 0, ta, tb, tc, (uint64_t)grid, whole,
+                 kept);
+      WTG_LAUNCH_CHECK();
+      WTG_LAUNCH(ctx, "sa_apply", k_sa_apply, dim3(grid), dim3(256), 0, k1, v1, m, n, whole, nbits, ta, tb, tc, rank,
+                 d_sa, idx[b], grp[b], list0, ctx->d_flag);
+      WTG_LAUNCH_CHECK();
+      uint32_t k = 0;
+      WTG_TRY(wtg_stage_d2h(ctx, &k, kept, 4));
+      *left = list0 + (uint64_t)k;
+      return WTG_OK;
+    };
+    WTG_LAUNCH(ctx, "sa_init", k_sa_init, dim3((unsigned)wtg_ceil_div(n, 256)), dim3(256), 0, d_text, n, d_code, cbits,
+               q, k0, v0);
+    SA_LAUNCH_CHECK();
+    uint64_t m = 0, h = q;
+    int b = 0;
+    if ((rc = sorted_round(n, q * cbits, 1, b, 0, &m)) != WTG_OK) goto out;
+    for (; m > 0; h *= 2, b ^= 1) {
+      if (m > n || h >= 2 * n) {
         wtg_set_error("wtg_suffix_array_gpu: ranks did not separate");
         rc = WTG_ERR_DEVICE;
         goto out;
       }
+      WTG_LAUNCH(ctx, "sa_gather", k_sa_gather, dim3((unsigned)wtg_ceil_div(m, 256)), dim3(256), 0, idx[b], m, n, h,
+                 rank, key2, counts);
+      SA_LAUNCH_CHECK();
+      WTG_LAUNCH(ctx, "sa_refine", k_sa_refine, dim3((unsigned)wtg_ceil_div(m, SA_W)), dim3(256), 0, idx[b], grp[b],
+                 key2, m, n, nbits, rank, d_sa, idx[b ^ 1], grp[b ^ 1], counts, k0, v0, ctx->d_flag);
+      SA_LAUNCH_CHECK();
+      uint32_t c[2];
+      if ((rc = wtg_stage_d2h(ctx, c, counts, 8)) != WTG_OK) goto out;
+      m = c[0];
+      if (c[1] && (rc = sorted_round(c[1], 2 * nbits, 0, b ^ 1, c[0], &m)) != WTG_OK) goto out;
     }
   }
   rc = wtg_finish(ctx);
 out:
   if (rc != WTG_OK) wtg_abandon(ctx);
-  wtg_free(ctx, k0); wtg_free(ctx, k1); wtg_free(ctx, v0); wtg_free(ctx, v1); wtg_free(ctx, act);
-  wtg_free(ctx, rank); wtg_free(ctx, fa); wtg_free(ctx, fb); wtg_free(ctx, ta); wtg_free(ctx, tb);
-  wtg_free(ctx, keep); wtg_free(ctx, pos); wtg_free(ctx, st); wtg_free(ctx, ctr); wtg_free(ctx, tmp);
-  wtg_free(ctx, present);
+  if (o > SA_WS_MAX) wtg_free(ctx, mem);
   return rc;
 }
 #undef SA_LAUNCH_CHECK
