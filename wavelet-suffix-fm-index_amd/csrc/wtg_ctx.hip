@@ -40,12 +40,13 @@ extern "C" int wtg_ctx_create(int device, wtg_ctx** out) {
   c->device = device;
   WTG_CHECK_HIP(hipSetDevice(device));
   WTG_CHECK_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-  WTG_CHECK_HIP(hipMalloc(&c->d_flag, 256));
-  WTG_CHECK_HIP(hipMemset(c->d_flag, 0, 256));
   WTG_CHECK_HIP(hipEventCreate(&c->t0));
   WTG_CHECK_HIP(hipEventCreate(&c->t1));
   WTG_CHECK_HIP(hipEventCreateWithFlags(&c->h2d_ev, hipEventDisableTiming));
   WTG_CHECK_HIP(hipHostMalloc((void**)&c->h_stage, WTG_STAGE_BYTES, hipHostMallocDefault));
+  std::memset(c->h_stage, 0, 256);
+  WTG_CHECK_HIP(hipMalloc(&c->d_small, 256));
+  WTG_CHECK_HIP(hipHostGetDevicePointer((void**)&c->d_flag, c->h_stage, 0));
   // library allocations come stream-ordered from the device's default pool,
   // which keeps freed memory for reuse (WTG_NO_POOL=1: plain hipMalloc)
   if (!std::getenv("WTG_NO_POOL")) {
@@ -74,7 +75,7 @@ extern "C" int wtg_ctx_destroy(wtg_ctx* ctx) {
   for (auto& p : ctx->kpending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
   for (auto e : ctx->kpool) (void)hipEventDestroy(e);
   if (ctx->ws) (void)hipFree(ctx->ws);
-  if (ctx->d_flag) (void)hipFree(ctx->d_flag);
+  if (ctx->d_small) (void)hipFree(ctx->d_small);
   if (ctx->t0) (void)hipEventDestroy(ctx->t0);
   if (ctx->t1) (void)hipEventDestroy(ctx->t1);
   if (ctx->h2d_ev) (void)hipEventDestroy(ctx->h2d_ev);
@@ -84,16 +85,24 @@ extern "C" int wtg_ctx_destroy(wtg_ctx* ctx) {
   return WTG_OK;
 }
 
+// the raised error flags (WTG_FLAG bits), cleared; the stream has been waited for
+static uint32_t flags_take(wtg_ctx* ctx) {
+  volatile uint32_t* hf = reinterpret_cast<volatile uint32_t*>(ctx->h_stage);
+  uint32_t f = 0;
+  for (uint32_t k = 0; k < WTG_FLAG_WORDS; k++)
+    if (hf[k]) {
+      f |= 1u << k;
+      hf[k] = 0;
+    }
+  return f;
+}
+
 extern "C" int wtg_ctx_sync(wtg_ctx* ctx) {
   WTG_REQUIRE(ctx, "null ctx");
   WTG_TRY(wtg_set_device(ctx));
-  // the flag rides the stream: one async copy into pinned memory, one sync
-  volatile uint32_t* hf = reinterpret_cast<volatile uint32_t*>(ctx->h_stage);
-  WTG_CHECK_HIP(hipMemcpyAsync(ctx->h_stage, ctx->d_flag, 4, hipMemcpyDeviceToHost, ctx->stream));
   WTG_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-  const uint32_t f = *hf;
+  const uint32_t f = flags_take(ctx);
   if (f) {
-    WTG_CHECK_HIP(hipMemset(ctx->d_flag, 0, 4));
     if (f & WTG_FLAG_BADSYM) {
       wtg_set_error("input symbol >= 2^levels (or inconsistent with the tree); results invalid");
       return WTG_ERR_ARG;
@@ -138,7 +147,7 @@ int wtg_stage_h2d(wtg_ctx* ctx, void* d_dst, const void* src, size_t bytes) {
 
 void wtg_abandon(wtg_ctx* ctx) {
   (void)hipGetLastError();
-  if (hipStreamSynchronize(ctx->stream) == hipSuccess) (void)hipMemset(ctx->d_flag, 0, 4);
+  if (hipStreamSynchronize(ctx->stream) == hipSuccess) (void)flags_take(ctx);
 }
 
 int wtg_finish(wtg_ctx* ctx) {

@@ -41,7 +41,7 @@ __global__ __launch_bounds__(256) void k_deep_flags(const K* __restrict__ keys, 
   bool one = false;
   if (act) {
     x = (uint64_t)keys[i];
-    if (l == 0 && L < 64 && (x >> L) != 0) atomicOr(err, WTG_FLAG_BADSYM);
+    if (l == 0 && L < 64 && (x >> L) != 0) wtg_raise(err, WTG_FLAG_BADSYM);
     const bool head = i == 0 || deep_prefix(x, L, l) != deep_prefix((uint64_t)keys[i - 1], L, l);
     one = (x >> (L - 1 - l)) & 1u;
     flags[i] = (uint64_t)(!one) | ((uint64_t)head << 32);

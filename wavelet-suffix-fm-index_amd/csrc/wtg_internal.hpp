@@ -37,10 +37,13 @@ struct wtg_ctx {
   // growable workspace (device); regions carved per call
   void* ws = nullptr;
   size_t ws_bytes = 0;
-  // device error flag (bounded waits set it), host-visible copy on sync
-  uint32_t* d_flag = nullptr;
+  // error flags, one word per WTG_FLAG bit, in the pinned staging area: kernels
+  // store to them (wtg_raise), so a call's last step is the stream's
+  // synchronization alone, with no copy queued for it
+  uint32_t* d_flag = nullptr;  // the area's first words, as the device sees them
+  void* d_small = nullptr;     // 256 device bytes for a call's counters
   // pinned host staging for small transfers (async copies need no bounce
-  // buffer): [0, 256) the error flag, [WTG_STAGE_D2H, +16 KiB) device-to-host
+  // buffer): [0, 256) the error flags, [WTG_STAGE_D2H, +16 KiB) device-to-host
   // reads (each followed by a stream sync before use), [WTG_STAGE_H2D, +32 KiB)
   // host-to-device tables (h2d_ev marks the last such copy)
   uint8_t* h_stage = nullptr;
@@ -67,7 +70,8 @@ int wtg_stage_d2h(wtg_ctx* ctx, void* dst, const void* d_src, size_t bytes);
 // stream-ordered host-to-device copy of a small table through the staging area
 // (waits for the previous such copy before reusing the buffer)
 int wtg_stage_h2d(wtg_ctx* ctx, void* d_dst, const void* src, size_t bytes);
-// bits of the device error flag (ctx->d_flag), decoded by wtg_ctx_sync
+// bits of the device error flags (word k of ctx->d_flag: bit k), decoded by wtg_ctx_sync
+constexpr uint32_t WTG_FLAG_WORDS = 4;
 constexpr uint32_t WTG_FLAG_WAIT = 1u;      // a bounded look-back wait expired
 constexpr uint32_t WTG_FLAG_BADSYM = 2u;    // input symbol >= 2^levels / tables inconsistent with the keys
 constexpr uint32_t WTG_FLAG_SA_RANKS = 4u;  // suffix ranks inconsistent
@@ -183,6 +187,12 @@ static inline int wtg_hi_host(uint64_t x) { int r = 0; if (!x) return 0; while (
 // ------------------------------------------------------------- device side
 #define WTG_WAVE 64
 #define WTG_SPIN_LIMIT (1u << 26)   // bounded waits: iterations before giving up
+
+// raise an error flag (a plain store to pinned host memory: atomic read-modify-
+// write operations do not reach it; storing the same word twice is harmless)
+__device__ __forceinline__ void wtg_raise(uint32_t* err, uint32_t flag) {
+  __hip_atomic_store(err + __builtin_ctz(flag), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 __device__ __forceinline__ int lane_id() { return (int)__lane_id(); }
 __device__ __forceinline__ uint32_t mbcnt64(uint64_t m) {
@@ -315,7 +325,7 @@ __device__ __forceinline__ uint64_t lb_wait(uint64_t* states, uint64_t tile, uin
       bool notready = (s >> 62) == 0;
       if (wave_ballot(notready) == 0) break;
       if (++spins > WTG_SPIN_LIMIT) {
-        if (l == 0) atomicOr(err, WTG_FLAG_WAIT);
+        if (l == 0) wtg_raise(err, WTG_FLAG_WAIT);
         s = (LB_PRE << 62);  // give up: treat as prefix 0 (results invalid, flag raised)
         break;
       }

@@ -381,7 +381,7 @@ __device__ __forceinline__ void split_groups_many(const LevelArgs& a, uint32_t t
       if (z_hi) atomicAdd(&a.zc_next[D0 + 1], z_hi);
     }
   }
-  if (bad) atomicOr(a.err, FLAG_BADSYM);
+  if (bad) wtg_raise(a.err, FLAG_BADSYM);
 }
 
 // Group phase of a split tile: per group of the next level (contiguous slots
@@ -486,11 +486,11 @@ __device__ __forceinline__ void split_groups(const LevelArgs& a, uint32_t tile, 
     } else if (pnode < a.nnodes) {
       ab = a.tab[pnode];
     } else {
-      if (lane == 0) atomicOr(a.err, FLAG_BADSYM);
+      if (lane == 0) wtg_raise(a.err, FLAG_BADSYM);
       continue;
     }
     const uint64_t dG = (sG < zt) ? zprev + sG + ab.x : oprev + (sG - zt) + ab.y;
-    if (dG + len > a.n || len == 0) { if (lane == 0) atomicOr(a.err, FLAG_BADSYM); continue; }
+    if (dG + len > a.n || len == 0) { if (lane == 0) wtg_raise(a.err, FLAG_BADSYM); continue; }
     const uint64_t b0 = (dG / TILE + 1) * TILE;  // first destination-tile boundary
     const uint32_t rel0 = (dG + len > b0) ? (uint32_t)(b0 - dG) : len;
     const uint64_t GB0 = a.next_base + dG;
@@ -613,7 +613,7 @@ __global__ __launch_bounds__(256) void k_level(LevelArgs a) {
       if (lane == 63) s_edge[1][s * 4 + w] = x[s][V - 1];
     }
   }
-  if (bad) atomicOr(a.err, FLAG_BADSYM);
+  if (bad) wtg_raise(a.err, FLAG_BADSYM);
   __syncthreads();
 
   uint32_t woff[StepsOf<T>::S];
@@ -705,7 +705,7 @@ __global__ __launch_bounds__(256) void k_level(LevelArgs a) {
         else ok = false;
         const uint64_t dest = (q < zt) ? zprev + q + ab.x : oprev + (q - zt) + ab.y;
         if (ok && dest < n) __builtin_nontemporal_store(xv, dst + dest);
-        else atomicOr(a.err, FLAG_BADSYM);
+        else wtg_raise(a.err, FLAG_BADSYM);
       }
     }
     split_groups<T, COUNT, TILE>(a, tile, (uint32_t)valid, zt, zprev, oprev, cached, pfirst, s_stage, s_nb,
@@ -898,7 +898,7 @@ __global__ __launch_bounds__(256) void k_split(LevelArgs a) {
       }
     }
   }
-  if (bad) atomicOr(a.err, FLAG_BADSYM);
+  if (bad) wtg_raise(a.err, FLAG_BADSYM);
   split_groups<T, COUNT, TILE>(a, tile, (uint32_t)TILE, zt, zprev, oprev, cached, pfirst, s_stage, s_nb, s_head,
                                s_tab);
 }
@@ -1302,7 +1302,7 @@ template <typename T>
 static int max_t(wtg_ctx* ctx, const T* s, uint64_t n, uint64_t* out) {
   if (n == 0) { *out = 0; return WTG_OK; }
   unsigned grid = (unsigned)std::min<uint64_t>(wtg_ceil_div(n, 256), 4096);
-  unsigned long long* mx = (unsigned long long*)((char*)ctx->d_flag + 64);
+  unsigned long long* mx = (unsigned long long*)((char*)ctx->d_small + 64);
   WTG_TRY(wtg_fill_u64(ctx, mx, 1, 0));
   WTG_LAUNCH(ctx, "max", k_max<T>, dim3(grid), dim3(256), 0, s, n, mx);
   WTG_LAUNCH_CHECK();

@@ -286,7 +286,7 @@ __global__ __launch_bounds__(256) void k_mld_count(MldArgs a) {
       }
     }
   }
-  if (bad || ((acc_lo & cm_lo) | (acc_hi & cm_hi)) != 0) atomicOr(a.err, WTG_FLAG_BADSYM);
+  if (bad || ((acc_lo & cm_lo) | (acc_hi & cm_hi)) != 0) wtg_raise(a.err, WTG_FLAG_BADSYM);
   if (wl) __syncthreads();
   else wave_sync_lds_mld();
   if (ok)  // the waves of a tile write its counts in turns of 64 leaves
@@ -634,7 +634,7 @@ __global__ __launch_bounds__(T / 8) __attribute__((amdgpu_waves_per_eu(8))) void
       const uint64_t lb = (uint64_t)(a.s + j - a.lvl0) * n;  // the level's first bit
       const uint64_t gs = lb + s_cum[lo] + (s_cpre[hi] - s_cpre[lo]);
       if (gs < lb || gs + cnt > lb + n) {
-        atomicOr(a.err, WTG_FLAG_BADSYM);  // tables inconsistent with the keys: write nothing
+        wtg_raise(a.err, WTG_FLAG_BADSYM);  // tables inconsistent with the keys: write nothing
       } else if (cnt) {
         nw = (uint32_t)(((gs + cnt - 1) >> 6) - (gs >> 6) + 1);
       }
@@ -675,7 +675,7 @@ __global__ __launch_bounds__(T / 8) __attribute__((amdgpu_waves_per_eu(8))) void
       if (i < len) {
         const uint32_t x = s_k[g & 1][i];
         const uint32_t dest = s_lb[(x >> sh) & (G - 1)] + i;
-        if (dest >= n) atomicOr(a.err, WTG_FLAG_BADSYM);
+        if (dest >= n) wtg_raise(a.err, WTG_FLAG_BADSYM);
         else if constexpr (WIDE)
           reinterpret_cast<uint64_t*>(a.kout)[dest] = (uint64_t) reinterpret_cast<const K*>(a.keys)[src + (x & 0xFFFFu)];
         else reinterpret_cast<uint32_t*>(a.kout)[dest] = x;
@@ -1093,7 +1093,7 @@ __global__ __launch_bounds__(256) void k_mld_local(LocArgs a) {
     if (lane == 0) reinterpret_cast<uint64_t*>(s_bits[0])[w + 4 * m] = hm[m];
     x[m] = (KT)k;
   }
-  if (bad) atomicOr(a.err, WTG_FLAG_BADSYM);
+  if (bad) wtg_raise(a.err, WTG_FLAG_BADSYM);
   if (threadIdx.x < 2) s_flag[threadIdx.x] = 0;
   __syncthreads();
   {
@@ -1203,7 +1203,7 @@ __global__ __launch_bounds__(256) void k_mld_big(const uint32_t* __restrict__ cu
   const uint32_t st = cum[i], c = cum[i + 1] - st;
   if (!loc_large(st % LOC_W, c)) return;
   const uint32_t k = atomicAdd(nb, 1u);
-  if (k >= cap) { atomicOr(err, WTG_FLAG_BADSYM); return; }  // (cannot happen: the sizes sum to n)
+  if (k >= cap) { wtg_raise(err, WTG_FLAG_BADSYM); return; }  // (cannot happen: the sizes sum to n)
   bs[k] = st;
   bc[k] = c;
 }
@@ -1233,7 +1233,7 @@ __global__ __launch_bounds__(256) void k_mld_leaf(MldArgs a, uint32_t* __restric
   const uint32_t in_tile = (st - a.seg_start[k]) & 2047;
   if (nb2 && c && loc_large(in_tile % LOC_W, c)) {
     const uint32_t q = atomicAdd(nb2, 1u);
-    if (q >= cap) { atomicOr(a.err, WTG_FLAG_BADSYM); return; }
+    if (q >= cap) { wtg_raise(a.err, WTG_FLAG_BADSYM); return; }
     bs2[q] = st;
     bc2[q] = c;
   }

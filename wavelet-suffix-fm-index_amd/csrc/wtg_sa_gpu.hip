@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256) void k_sa_apply(const uint64_t* __restrict__ k
       } else if (r < n) {
         sa[r] = (int64_t)i;
       } else {
-        atomicOr(err, WTG_FLAG_SA_RANKS);  // ranks inconsistent: not expected
+        wtg_raise(err, WTG_FLAG_SA_RANKS);  // ranks inconsistent: not expected
       }
     }
     if (ma[j]) ca = c0 + 63u - (uint32_t)__builtin_clzll(ma[j]);
@@ -354,7 +354,7 @@ __global__ __launch_bounds__(256) void k_sa_refine(const uint32_t* __restrict__ 
       if (less) rank[ii[j]] = r;
       if (eq == 1) {
         if (r < n) sa[r] = (int64_t)ii[j];
-        else atomicOr(err, WTG_FLAG_SA_RANKS);  // ranks inconsistent: not expected
+        else wtg_raise(err, WTG_FLAG_SA_RANKS);  // ranks inconsistent: not expected
       } else {
         ng[j] = r;
       }
@@ -415,7 +415,7 @@ __global__ void k_bwt(const uint8_t* __restrict__ t, const int64_t* __restrict__
   if (i >= n) return;
   const int64_t p = sa[i];
   if (p < 0 || (uint64_t)p >= n) {  // not a suffix array of this text
-    atomicOr(err, WTG_FLAG_BAD_SA);
+    wtg_raise(err, WTG_FLAG_BAD_SA);
     bwt[i] = 0;
     return;
   }

@@ -220,7 +220,7 @@ extern "C" int wtg_wtint_build(wtg_ctx* ctx, const void* d_sym, int sym_bytes, u
   wt->L = L;
   wt->nbits = n * L;
   const uint64_t nw = wtg_levels_words(n, L);
-  unsigned long long* d_distinct = (unsigned long long*)((char*)ctx->d_flag + 128);
+  unsigned long long* d_distinct = (unsigned long long*)((char*)ctx->d_small + 128);
   if ((rc = wtg_malloc(ctx, (void**)&wt->words, nw * 8)) != WTG_OK) goto fail;
   if ((rc = wtg_malloc(ctx, (void**)&wt->dir, wtg_rank9_words(wt->nbits) * 8)) != WTG_OK) goto fail;
   if ((rc = wtg_levels_build_async(ctx, d_sym, sym_bytes, n, L, wt->words, nullptr, 0, d_distinct)) != WTG_OK)
