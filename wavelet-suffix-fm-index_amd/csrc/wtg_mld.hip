@@ -293,6 +293,26 @@ __global__ __launch_bounds__(256) void k_mld_count(MldArgs a) {
     for (uint32_t i = lane + 64 * sub; i < G; i += 64u << wl) a.tcnt_w[(uint64_t)t * G + i] = s_cnt[i];
 }
 
+// exclusive scan of one value per thread over the block's first 256 threads
+// (the others hold 0 and take part in the barriers only)
+template <bool DPP>
+__device__ __forceinline__ uint32_t mld_scan256(uint32_t v, uint32_t* s_wave, uint32_t& total) {
+  const uint32_t w = threadIdx.x >> 6, l = (uint32_t)lane_id();
+  const uint32_t incl = DPP ? wave_incl_sum_dpp(v) : wave_incl_scan_shfl(v);
+  if (l == 63 && w < 4) s_wave[w] = incl;
+  __syncthreads();
+  uint32_t off = 0, tot = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < 4; k++) {
+    const uint32_t t = s_wave[k];
+    if (k < w) off += t;
+    tot += t;
+  }
+  __syncthreads();
+  total = tot;
+  return incl - v + off;
+}
+
 // column-wise exclusive prefix of the leaf counts over the tiles, blocks of
 // MLD_SR tiles: ploc = prefix inside the block, bsum = the block's totals.
 // Thread (q, c) takes column c of MLD_SR/Q consecutive rows (Q = 256/G), all
@@ -333,6 +353,41 @@ __global__ __launch_bounds__(256) void k_mld_scan1(const uint32_t* __restrict__ 
     if (r < per && row < nrows) ploc[row * G + c] = v[r] + pre;
   }
   if (q == 0) bsum[(uint64_t)blockIdx.x * G + c] = tot;
+}
+
+// The first group's tables from the block sums in one launch (one block; few
+// block sums): their exclusive prefix per column as k_mld_scan2 makes it, the
+// histogram (the column totals) and its exclusive prefix cum.  Four launches in
+// one: 2^24 bytes, 8 levels, nodes and rank directory: 172 -> 168 us.
+constexpr uint32_t MLD_ROOT_BLOCKS = 128;
+__global__ __launch_bounds__(1024) void k_mld_root(const uint32_t* __restrict__ bsum, uint32_t* __restrict__ bpre,
+                                                   uint32_t nblocks, uint32_t G, uint32_t* __restrict__ hist,
+                                                   uint32_t* __restrict__ cum) {
+  __shared__ uint32_t s_tot[1024], s_wave[4];
+  const uint32_t c = threadIdx.x % G, q = threadIdx.x / G, Q = 1024 / G < 16 ? 1024 / G : 16;
+  const uint32_t per = (nblocks + Q - 1) / Q, r0 = q * per, r1 = r0 + per < nblocks ? r0 + per : nblocks;  // (none past Q)
+  uint32_t sum = 0;
+  for (uint32_t r = r0; r < r1; r++) sum += bsum[(uint64_t)r * G + c];
+  s_tot[threadIdx.x] = sum;
+  __syncthreads();
+  uint32_t run = 0, tot = 0;
+  for (uint32_t k = 0; k < Q; k++) {
+    const uint32_t t = s_tot[k * G + c];
+    if (k < q) run += t;
+    tot += t;
+  }
+  for (uint32_t r = r0; r < r1; r++) {
+    const uint32_t v = bsum[(uint64_t)r * G + c];
+    bpre[(uint64_t)r * G + c] = run;
+    run += v;
+  }
+  uint32_t all;
+  const uint32_t ex = mld_scan256<true>(threadIdx.x < G ? tot : 0u, s_wave, all);
+  if (threadIdx.x < G) {
+    hist[threadIdx.x] = tot;
+    cum[threadIdx.x] = ex;
+  }
+  if (threadIdx.x == 0) cum[G] = all;
 }
 
 // exclusive prefix of the block sums per column: block c scans column c
@@ -420,26 +475,6 @@ __device__ __forceinline__ uint64_t lds_bits64(const uint32_t* row, uint32_t p) 
   const uint64_t lo = (uint64_t)row[k] | ((uint64_t)row[k + 1] << 32);
   const uint64_t hi = row[k + 2];
   return o ? (lo >> o) | (hi << (64 - o)) : lo;
-}
-
-// exclusive scan of one value per thread over the block's first 256 threads
-// (the others hold 0 and take part in the barriers only)
-template <bool DPP>
-__device__ __forceinline__ uint32_t mld_scan256(uint32_t v, uint32_t* s_wave, uint32_t& total) {
-  const uint32_t w = threadIdx.x >> 6, l = (uint32_t)lane_id();
-  const uint32_t incl = DPP ? wave_incl_sum_dpp(v) : wave_incl_scan_shfl(v);
-  if (l == 63 && w < 4) s_wave[w] = incl;
-  __syncthreads();
-  uint32_t off = 0, tot = 0;
-#pragma unroll
-  for (uint32_t k = 0; k < 4; k++) {
-    const uint32_t t = s_wave[k];
-    if (k < w) off += t;
-    tot += t;
-  }
-  __syncthreads();
-  total = tot;
-  return incl - v + off;
 }
 
 // T keys per tile (mld_tile_log), T / 8 threads (8 chunks of 64 keys per wave).
@@ -684,12 +719,9 @@ __global__ __launch_bounds__(T / 8) __attribute__((amdgpu_waves_per_eu(8))) void
   }
 }
 
-// WTnode records from the histogram prefix of all L bits (node (l, p) holds
+// WTnode record v from the histogram prefix of all L bits (node (l, p) holds
 // the keys with top l bits p: start Cum[p << (L-l)], count up to the next)
-__global__ void k_mld_nodes(const uint32_t* __restrict__ cum, uint32_t L, uint64_t n, wtg_node* __restrict__ nodes,
-                            uint64_t slots) {
-  const uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= slots) return;
+__device__ __forceinline__ wtg_node mld_node(const uint32_t* cum, uint32_t L, uint64_t n, uint64_t v) {
   wtg_node r;
   r.bitmapPtr = 0; r.length = 0; r.parent = WTG_NONE; r.leftChild = WTG_NONE; r.rightChild = WTG_NONE;
   if (v < (1ull << L) - 1) {
@@ -708,7 +740,128 @@ __global__ void k_mld_nodes(const uint32_t* __restrict__ cum, uint32_t L, uint64
       }
     }
   }
-  nodes[v] = r;
+  return r;
+}
+__global__ void k_mld_nodes(const uint32_t* __restrict__ cum, uint32_t L, uint64_t n, wtg_node* __restrict__ nodes,
+                            uint64_t slots) {
+  const uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (v < slots) nodes[v] = mld_node(cum, L, n, v);
+}
+
+// A whole tree of at most 8 levels over at most ONE_CAP keys in one block:
+// counts, node tables, the level pipeline of k_mld_emit, then every output word
+// once (a word may hold several levels' bits) and the node records.  Such a
+// call is launches and waits only: 5003 bytes, 5 levels, with nodes: one launch of
+// 11 us instead of eight and a copy, the call
+// 45-60 -> 22 us.
+constexpr uint32_t ONE_CAP = 8192;
+template <typename K>
+__global__ __launch_bounds__(1024) void k_mld_one(const K* __restrict__ keys, uint32_t n, uint32_t L,
+                                                  uint64_t* __restrict__ words, wtg_node* __restrict__ nodes,
+                                                  uint64_t slots, unsigned long long* __restrict__ distinct,
+                                                  uint32_t* __restrict__ err) {
+  constexpr uint32_t M = ONE_CAP / 1024, NWV = 16;
+  __shared__ uint32_t s_k[ONE_CAP];
+  __shared__ uint32_t s_cnt[256], s_pre[257], s_nxy[255], s_lvl0[MLD_GMAX], s_wave[4];
+  __shared__ __align__(8) uint32_t s_bits[MLD_GMAX][ONE_CAP / 32 + 2];
+  __shared__ uint16_t s_ex[NWV][ONE_CAP / 64];
+  const uint32_t tid = threadIdx.x, lane = (uint32_t)lane_id(), G = 1u << L;
+  const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+  if (tid < 256) s_cnt[tid] = 0;
+  K kr[M];
+#pragma unroll
+  for (uint32_t m = 0; m < M; m++) {
+    const uint32_t p = (w + NWV * m) * 64 + lane;
+    kr[m] = p < n ? keys[p] : (K)0;
+  }
+  __syncthreads();
+  // (positions past the keys hold a one at every level: they stay behind the keys)
+  uint32_t x[M];
+  bool bad = false;
+#pragma unroll
+  for (uint32_t m = 0; m < M; m++) {
+    const uint32_t p = (w + NWV * m) * 64 + lane;
+    const bool in = p < n;
+    x[m] = in ? (uint32_t)kr[m] & (G - 1) : G - 1;
+    bad |= in && ((uint64_t)kr[m] >> L) != 0;
+    if (in) atomicAdd(&s_cnt[x[m]], 1u);
+  }
+  if (bad) wtg_raise(err, WTG_FLAG_BADSYM);
+  __syncthreads();
+  if (distinct) {
+    const uint32_t k = (uint32_t)__syncthreads_count(tid < 256 && s_cnt[tid & 255] != 0);
+    if (tid == 0) *distinct = k;
+  }
+  uint32_t tot;
+  const uint32_t ex = mld_scan256<true>(tid < 256 ? s_cnt[tid] : 0u, s_wave, tot);
+  if (tid < 256) s_pre[tid] = ex;
+  if (tid == 0) s_pre[256] = tot;
+  __syncthreads();
+  {  // node tables as in k_mld_emit
+    const uint32_t r = tid, j = 31 - __clz(r + 1);
+    uint32_t S = 0, zn = 0;
+    if (r < G - 1) {
+      const uint32_t q = r + 1 - (1u << j), sgj = L - j;
+      S = s_pre[q << sgj];
+      zn = s_pre[(2 * q + 1) << (sgj - 1)] - S;
+    }
+    const uint32_t zx = mld_scan256<true>(r < G - 1 ? zn : 0u, s_wave, tot);
+    if (r < G - 1 && r + 1 == (1u << j)) s_lvl0[j] = zx;
+    __syncthreads();
+    if (r < G - 1) {
+      const uint32_t zs = zx - s_lvl0[j];
+      s_nxy[r] = (S - zs) | ((zs + zn) << 16);
+    }
+  }
+  __syncthreads();
+  for (uint32_t j = 0; j < L; j++) {
+    const uint32_t bp = L - 1 - j;
+    uint64_t zm[M];
+    if (j > 0) {
+#pragma unroll
+      for (uint32_t m = 0; m < M; m++) x[m] = s_k[(w + NWV * m) * 64 + lane];
+    }
+#pragma unroll
+    for (uint32_t m = 0; m < M; m++) {
+      const uint64_t ones = wave_ballot((x[m] >> bp) & 1u);
+      zm[m] = ~ones;
+      if (lane == 0) reinterpret_cast<uint64_t*>(s_bits[j])[w + NWV * m] = ones;
+    }
+    __syncthreads();
+    if (j + 1 == L) break;
+    const uint64_t* row = reinterpret_cast<const uint64_t*>(s_bits[j]);
+    const uint32_t v0 = 64u - popc64(row[2 * lane]), v1 = 64u - popc64(row[2 * lane + 1]);
+    const uint32_t incl = wave_incl_sum_dpp(v0 + v1);
+    s_ex[w][2 * lane] = (uint16_t)(incl - v0 - v1);
+    s_ex[w][2 * lane + 1] = (uint16_t)(incl - v1);
+    wave_sync_lds_mld();
+    const uint32_t* nt = s_nxy + (1u << j) - 1;
+#pragma unroll
+    for (uint32_t m = 0; m < M; m++) {
+      const uint32_t c = w + NWV * m, p = c * 64 + lane;
+      const uint32_t xy = nt[__builtin_amdgcn_ubfe(x[m], bp + 1, j)];
+      const uint32_t zc = __builtin_amdgcn_mbcnt_hi((uint32_t)(zm[m] >> 32),
+                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)zm[m], s_ex[w][c]));
+      const bool zero = ((x[m] >> bp) & 1u) == 0;
+      s_k[(zero ? (xy & 0xFFFFu) + zc : (xy >> 16) + p - zc) & (ONE_CAP - 1)] = x[m];
+    }
+    __syncthreads();
+  }
+  const uint32_t nbits = n * L;
+  for (uint32_t b = tid * 64; b < nbits; b += 1024 * 64) {
+    const uint32_t end = b + 64 < nbits ? b + 64 : nbits;
+    uint64_t v = 0;
+    for (uint32_t at = b; at < end;) {
+      const uint32_t l = at / n, o = at - l * n;
+      const uint32_t cnt = end - at < n - o ? end - at : n - o;
+      const uint64_t bits = lds_bits64(s_bits[l], o) & (cnt < 64 ? (1ull << cnt) - 1 : ~0ull);
+      v |= bits << (at - b);
+      at += cnt;
+    }
+    words[b >> 6] = v;
+  }
+  if (nodes)
+    for (uint64_t v = tid; v < slots; v += 1024) nodes[v] = mld_node(s_pre, L, n, v);
 }
 
 __global__ void k_mld_nonzero(const uint32_t* __restrict__ h, uint64_t n, unsigned long long* out) {
@@ -735,7 +888,7 @@ uint32_t mld_split_level(uint64_t n) {
 // 1230 us against 577, n = 3000017, 20 levels (183 keys) 264 against 200; at
 // 1024 keys they are the faster way (n = 2^24, 20 levels: 449 against 506).
 bool mld_use_sparse(uint64_t n, uint32_t L) {
-  if (n <= LOC_CAP) return true;
+  if (n <= LOC_CAP) return L > MLD_GMAX;  // (k_mld_one otherwise)
   const uint32_t last = L - L / 3;  // where the last of three near-equal groups starts
   return L > 16 && (n >> last) < 512;
 }
@@ -912,16 +1065,21 @@ int mld_dense_groups(wtg_ctx* ctx, const MldPlan& P, const K* d_sym, uint64_t n,
     WTG_LAUNCH(ctx, "mld_scan", k_mld_scan1, dim3(nblocks), dim3(256), 0, tcnt, ploc, bsum,
                s ? (const uint32_t*)(tst + (1u << s)) : nullptr, ntiles0, G, nrows);
     WTG_LAUNCH_CHECK();
-    WTG_LAUNCH(ctx, "mld_scan", k_mld_scan2, dim3(G), dim3(256), 0, bsum, bpre, nblocks, G);
-    WTG_LAUNCH_CHECK();
     const uint64_t nbins = 1ull << (s + g);
-    WTG_LAUNCH(ctx, "mld_hist", k_mld_hist, dim3((unsigned)wtg_ceil_div(nbins, 256)), dim3(256), 0, a, hist);
-    WTG_LAUNCH_CHECK();
     const uint64_t stiles = wtg_ceil_div(nbins, 4096);
-    WTG_TRY(wtg_fill_bytes_zero(ctx, scst, (char*)ctr + 256 - (char*)scst));
-    WTG_LAUNCH(ctx, "mld_cum", k_scan_u32<uint32_t>, dim3((unsigned)stiles), dim3(256), 0, hist, cum[gi & 1], nbins,
-               scst, ctr, ctx->d_flag);
-    WTG_LAUNCH_CHECK();
+    if (s == 0 && nblocks <= MLD_ROOT_BLOCKS) {
+      WTG_LAUNCH(ctx, "mld_scan", k_mld_root, dim3(1), dim3(1024), 0, bsum, bpre, nblocks, G, hist, cum[gi & 1]);
+      WTG_LAUNCH_CHECK();
+    } else {
+      WTG_LAUNCH(ctx, "mld_scan", k_mld_scan2, dim3(G), dim3(256), 0, bsum, bpre, nblocks, G);
+      WTG_LAUNCH_CHECK();
+      WTG_LAUNCH(ctx, "mld_hist", k_mld_hist, dim3((unsigned)wtg_ceil_div(nbins, 256)), dim3(256), 0, a, hist);
+      WTG_LAUNCH_CHECK();
+      WTG_TRY(wtg_fill_bytes_zero(ctx, scst, (char*)ctr + 256 - (char*)scst));
+      WTG_LAUNCH(ctx, "mld_cum", k_scan_u32<uint32_t>, dim3((unsigned)stiles), dim3(256), 0, hist, cum[gi & 1], nbins,
+                 scst, ctr, ctx->d_flag);
+      WTG_LAUNCH_CHECK();
+    }
     if (last && d_distinct) {
       WTG_LAUNCH(ctx, "mld_distinct", k_mld_nonzero, dim3((unsigned)std::min<uint64_t>(wtg_ceil_div(nbins, 256), 1024)),
                  dim3(256), 0, hist, nbins, d_distinct);
@@ -955,6 +1113,12 @@ template <typename K>
 int mld_build_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint32_t s0, const uint32_t* d_cnt0,
                 const uint64_t* d_src_off, uint64_t* d_words, wtg_node* d_nodes, uint64_t node_slots,
                 unsigned long long* d_distinct) {
+  if (n <= ONE_CAP && L <= MLD_GMAX && s0 == 0) {
+    WTG_LAUNCH(ctx, "mld_one", k_mld_one<K>, dim3(1), dim3(1024), 0, d_sym, (uint32_t)n, L, d_words, d_nodes,
+               node_slots, d_distinct, ctx->d_flag);
+    WTG_LAUNCH_CHECK();
+    return WTG_OK;
+  }
   const MldPlan P = mld_plan(n, L, s0);
   WTG_TRY(wtg_ws_reserve(ctx, P.total));
   WTG_TRY((mld_dense_groups<K, uint32_t>(ctx, P, d_sym, n, L, L, s0, d_cnt0, d_src_off, d_words, d_distinct)));
