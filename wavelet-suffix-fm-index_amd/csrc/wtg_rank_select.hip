@@ -12,8 +12,8 @@
 // Two passes over the words: ones per 512-word tile (k_rank_tile_sums) and,
 // after their exclusive scan, one lane per directory entry (k_rank_entries):
 // the lane's 8 word counts give the entry's 9-bit fields, a DPP scan of the
-// entry totals its prefix, and for each word the lane emits the sample of the
-// argument rank j%64==0 the word holds (at most one per bit value): the low
+// entry totals its prefix, and the samples of the argument ranks j%64==0 (at
+// most one per word and bit value) are found and written slot by slot: the low
 // 32 bits of pos(j) straight into slot j/64 of the final mini
 // array (mini offsets are < logn^4 < 2^32, so subtracting the low 32 bits of
 // the superblock start later gives the exact offset), and the superblock
@@ -73,21 +73,26 @@ __global__ __launch_bounds__(256) void k_rank_tile_sums(const uint64_t* __restri
   }
 }
 
-// Directory entries and select samples, one lane per word, one wave per tile
-// of 512 words.  Lanes 8i..8i+7 of a round hold directory entry i of the round;
-// a word holds at most one argument rank that is a multiple of 64 (per bit
-// value), so each lane emits at most one sample per select structure.
-__device__ __forceinline__ void word_sample(uint64_t x, uint64_t r, uint32_t c, uint64_t w, const SelOut& o) {
-  if (c == 0) return;
-  const uint64_t j = (r + 63) & ~63ull;
-  if (j < r + c) {
-    const uint64_t pos = (w << 6) + select_in_word(x, (uint32_t)(j - r));
-    o.mini[j >> 6] = (uint32_t)pos;
-    if ((j & 4095) == 0) o.sbstart[j >> 12] = pos;
+__device__ __forceinline__ void rs_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// position (0..63) of the k-th set bit of hi:lo, halving the window: k - c wraps
+// past k where the bit is below the middle
+__device__ __forceinline__ uint32_t select_halves(uint32_t lo, uint32_t hi, uint32_t k) {
+  uint32_t c = (uint32_t)__popc(lo), pos = 0;
+  uint32_t w = lo;
+  if (k >= c) { w = hi; pos = 32; }
+  k = min(k, k - c);
+#pragma unroll
+  for (uint32_t s = 16; s > 0; s >>= 1) {
+    c = (uint32_t)__popc(__builtin_amdgcn_ubfe(w, pos, s));  // (offset taken modulo 32)
+    pos += k >= c ? s : 0u;
+    k = min(k, k - c);
   }
-  uint64_t je = ((r >> 12) << 12) + 4095;
-  if (je < r) je += 4096;
-  if (je < r + c) o.sbend[je >> 12] = (w << 6) + select_in_word(x, (uint32_t)(je - r));
+  return pos;
 }
 
 // inclusive scan over the 64 lanes: DPP shifts inside each row of 16, then the
@@ -107,8 +112,37 @@ __device__ __forceinline__ uint32_t wave_incl_scan_dpp(uint32_t v) {
 // Directory entries and select samples: one lane per directory entry (8
 // words), one wave per tile of 512 words.  The lane's word counts give the
 // entry's 9-bit fields directly; one DPP scan of the entry totals gives each
-// entry's prefix inside the tile.
+// entry's prefix inside the tile.  Select samples (argument ranks that are
+// multiples of 64): a word holds at most one per bit value, and a tile's are
+// consecutive slots, 512 of both values together.  Each word that holds one
+// writes its number to the slot's place in LDS; then the lanes take the slots in
+// order, 64 at a time, every lane with work, and the samples leave as whole
+// lines.  n = 2^28, 20 levels (5.37 Gbit): 461 us with the owner of each word
+// selecting (half of the lanes idle) and storing, 298 us so; the directory
+// alone takes 140.  A lane going through its entry's samples in a loop: 530 us
+// (one chain of dependent steps), 700 us two of each value at a time.
+constexpr uint32_t RS_SLOTS = RS_TILE_WORDS + 1, RS_ENDS = 9;  // a tile's samples, superblock ends of one value, at most
+struct TileSel {       // one bit value's arguments in a tile
+  uint64_t t0;         // the vector's arguments before the tile
+  uint16_t* slot;      // the word of each sample (LDS)
+  uint16_t* end;       // the word of each superblock end (LDS)
+};
+// word number `widx` of the tile holds c arguments, r of the tile's before it
+__device__ __forceinline__ void word_marks(const TileSel& s, uint32_t widx, uint32_t r, uint32_t c) {
+  const uint32_t q = ((uint32_t)s.t0 & 4095u) + r;       // rank, from the superblock of the tile's first argument
+  const uint32_t d = (0u - q) & 63u;
+  if (d < c) s.slot[((q + 63) >> 6) - ((((uint32_t)s.t0 & 4095u) + 63) >> 6)] = (uint16_t)widx;
+  const uint32_t de = 4095u - (q & 4095u);
+  if (de < c) s.end[q >> 12] = (uint16_t)widx;
+}
+__device__ __forceinline__ uint32_t rs_at(uint32_t widx) {  // a word's place in LDS (spread over the banks)
+  return widx ^ ((widx >> 5) & 7);
+}
+
 __global__ __launch_bounds__(256) void k_rank_entries(RankSelArgs a, uint64_t ntiles, bool write_dir, bool aligned) {
+  __shared__ uint64_t s_x[4][RS_TILE_WORDS];
+  __shared__ uint16_t s_f[4][RS_TILE_WORDS];          // ones of the tile before each word
+  __shared__ uint16_t s_slot[4][2][RS_SLOTS + 1], s_end[4][2][RS_ENDS + 1];
   const uint64_t t = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= ntiles) return;
   const int lane = lane_id();
@@ -132,7 +166,9 @@ __global__ __launch_bounds__(256) void k_rank_entries(RankSelArgs a, uint64_t nt
 #pragma unroll
   for (int k = 0; k < 8; k++) f[k + 1] = f[k] + popc64(x[k]);
   const uint32_t incl = wave_incl_scan_dpp(f[8]);
-  const uint64_t pre = a.tpre[t] + (incl - f[8]);  // ones before word w0
+  const uint64_t tp0 = a.tpre[t], tp1 = a.tpre[t + 1], T = a.tpre[ntiles];
+  const uint32_t tin = incl - f[8];   // ones of the tile before word w0
+  const uint64_t pre = tp0 + tin;
   if (write_dir && e <= a.S) {
     const uint64_t m = a.W > w0 ? (a.W - w0 < 8 ? a.W - w0 : 8) : 0;  // words of the entry
     uint64_t F = 0;
@@ -142,35 +178,70 @@ __global__ __launch_bounds__(256) void k_rank_entries(RankSelArgs a, uint64_t nt
     a.D[2 * e] = pre;
     a.D[2 * e + 1] = F;
   }
-  uint64_t last1 = 0, last0 = 0;
+  if (t == 0 && lane == 0) *a.ones_total = T;
+  if (!a.want[0] && !a.want[1]) return;
+  const uint64_t tb = t * RS_TILE_WORDS * 64;  // the tile's first bit
+  const uint64_t v0 = tb < a.nbits ? tb : a.nbits;
+  const uint64_t v1 = tb + RS_TILE_WORDS * 64 < a.nbits ? tb + RS_TILE_WORDS * 64 : a.nbits;
+  const uint32_t wv = threadIdx.x >> 6;
+  const TileSel g1{tp0, s_slot[wv][1], s_end[wv][1]}, g0{v0 - tp0, s_slot[wv][0], s_end[wv][0]};
 #pragma unroll
-  for (int k = 0; k < 8; k++) {
-    const uint64_t w = w0 + k;
-    if (w < a.W) {
-      const uint32_t c = f[k + 1] - f[k];
-      const uint64_t r = pre + f[k];
-      const uint64_t lo = w * 64;
-      if (a.want[1]) {
-        word_sample(x[k], r, c, w, a.sel[1]);
-        if (c) last1 = lo + (63 - __clzll(x[k])) + 1;
-      }
-      if (a.want[0]) {
-        const uint64_t vm = a.nbits - lo >= 64 ? ~0ull : ((1ull << (a.nbits - lo)) - 1);
-        const uint64_t z = ~x[k] & vm;
-        word_sample(z, lo - r, popc64(z), w, a.sel[0]);
-        if (z) last0 = lo + (63 - __clzll(z)) + 1;
-      }
-      if (w + 1 == a.W) *a.ones_total = r + c;
+  for (uint32_t k = 0; k < 8; k++) {
+    const uint32_t widx = (uint32_t)lane * 8 + k, r = tin + f[k], c = f[k + 1] - f[k];
+    s_x[wv][rs_at(widx)] = x[k];
+    s_f[wv][widx] = (uint16_t)r;
+    if (a.want[1]) word_marks(g1, widx, r, c);
+    if (a.want[0]) {
+      const uint64_t lo = (w0 + k) * 64;
+      const uint32_t z = lo + 64 <= a.nbits ? 64 - c
+                         : lo >= a.nbits   ? 0u
+                                           : popc64(~x[k] & ((1ull << (a.nbits - lo)) - 1));
+      word_marks(g0, widx, widx * 64 - r, z);
     }
+  }
+  rs_wave_sync();
+  // position in the tile of argument rank j of the vector, in word widx
+  const auto position = [&](uint32_t b, uint64_t j, uint64_t t0, uint32_t widx) {
+    const uint64_t xw = s_x[wv][rs_at(widx)];
+    const uint32_t fw = s_f[wv][widx], flip = b ? 0u : ~0u;
+    const uint32_t before = b ? fw : widx * 64 - fw;
+    return widx * 64 + select_halves((uint32_t)xw ^ flip, (uint32_t)(xw >> 32) ^ flip, (uint32_t)(j - t0) - before);
+  };
+  // (a tile's argument count wraps only where set bits past the vector's end
+  // outnumber its last zeros)
+#pragma unroll
+  for (uint32_t b = 0; b < 2; b++) {
+    if (!a.want[b]) continue;
+    const uint64_t t0 = b ? tp0 : v0 - tp0, t1 = b ? tp1 : v1 - tp1;
+    const uint64_t first = (t0 + 63) >> 6, end = (t1 + 63) >> 6;
+    const uint32_t n = end <= first ? 0u : end - first < RS_SLOTS ? (uint32_t)(end - first) : RS_SLOTS;
+#pragma unroll 2
+    for (uint32_t i = (uint32_t)lane; i < n; i += 64) {
+      const uint64_t slot = first + i;
+      const uint64_t pos = tb + position(b, slot * 64, t0, s_slot[wv][b][i]);
+      a.sel[b].mini[slot] = (uint32_t)pos;
+      if ((slot & 63) == 0) a.sel[b].sbstart[slot >> 6] = pos;
+    }
+    const uint64_t eb = t0 >> 12, ee = t1 >> 12;  // superblocks that end in the tile
+    const uint32_t ne = ee <= eb ? 0u : ee - eb < RS_ENDS ? (uint32_t)(ee - eb) : RS_ENDS;
+    if ((uint32_t)lane < ne)
+      a.sel[b].sbend[eb + lane] = tb + position(b, (eb + lane) * 4096 + 4095, t0, s_end[wv][b][lane]);
   }
   // last argument position (+1): only the tile holding the last one (the last
   // zero) writes it, a plain store; the scanned tile counts identify that tile
-  const uint64_t T = a.tpre[ntiles], tp0 = a.tpre[t], tp1 = a.tpre[t + 1];
-  const uint64_t v0 = t * RS_TILE_WORDS * 64 < a.nbits ? t * RS_TILE_WORDS * 64 : a.nbits;
-  const uint64_t v1 = (t + 1) * RS_TILE_WORDS * 64 < a.nbits ? (t + 1) * RS_TILE_WORDS * 64 : a.nbits;
   const bool has_last1 = tp0 < T && tp1 == T;
   const bool has_last0 = v0 - tp0 < a.nbits - T && v1 - tp1 == a.nbits - T;
   if (has_last1 || has_last0) {
+    uint64_t last1 = 0, last0 = 0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const uint64_t lo = (w0 + k) * 64;
+      if (lo < a.nbits) {
+        const uint64_t z = ~x[k] & (a.nbits - lo >= 64 ? ~0ull : (1ull << (a.nbits - lo)) - 1);
+        if (x[k]) last1 = lo + (63 - __clzll(x[k])) + 1;
+        if (z) last0 = lo + (63 - __clzll(z)) + 1;
+      }
+    }
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
       const uint64_t o1 = (uint64_t)__shfl_xor((unsigned long long)last1, d);
