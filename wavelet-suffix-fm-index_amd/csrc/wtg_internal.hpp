@@ -287,6 +287,22 @@ __device__ __forceinline__ uint32_t select_in_word(uint64_t x, uint32_t k) {
   return pos;
 }
 
+// position (0..63) of the k-th set bit of hi:lo, halving the window: k - c wraps
+// past k where the bit is below the middle
+__device__ __forceinline__ uint32_t select_halves(uint32_t lo, uint32_t hi, uint32_t k) {
+  uint32_t c = (uint32_t)__popc(lo), pos = 0;
+  uint32_t w = lo;
+  if (k >= c) { w = hi; pos = 32; }
+  k = min(k, k - c);
+#pragma unroll
+  for (uint32_t s = 16; s > 0; s >>= 1) {
+    c = (uint32_t)__popc(__builtin_amdgcn_ubfe(w, pos, s));  // (offset taken modulo 32)
+    pos += k >= c ? s : 0u;
+    k = min(k, k - c);
+  }
+  return pos;
+}
+
 // ---------------------------------------------------- decoupled look-back
 // status word = flag<<62 | value; flag 1 = tile aggregate, 2 = inclusive prefix.
 #define LB_AGG 1ull
@@ -421,6 +437,24 @@ __device__ __forceinline__ uint64_t rank9_dev(const uint64_t* __restrict__ D,
   if (i & 63) r += popc64(words[i >> 6] & ((1ull << (i & 63)) - 1));
   return r;
 }
+// The same in two steps, so that several lookups' loads are in flight together:
+// the directory entry in one 16-byte load and the word, read without a test of
+// i (W: the vector's words, at least one; the last word stands in for the one
+// past it, of which no bit is counted), then the rank.
+typedef uint32_t wtg_u4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+struct RankAt {
+  uint64_t i, base, sub, word;
+};
+__device__ __forceinline__ RankAt rank9_fetch(const uint64_t* __restrict__ D, const uint64_t* __restrict__ words,
+                                              uint64_t W, uint64_t i) {
+  const wtg_u4_a8 d = *reinterpret_cast<const wtg_u4_a8*>(D + 2 * (i >> 9));
+  const uint64_t k = i >> 6;
+  return {i, (uint64_t)d.x | (uint64_t)d.y << 32, (uint64_t)d.z | (uint64_t)d.w << 32, words[k < W ? k : W - 1]};
+}
+__device__ __forceinline__ uint64_t rank9_of(const RankAt& a) {
+  const uint32_t lo = (uint32_t)a.i;
+  return a.base + ((a.sub >> (63 - 9 * ((lo >> 6) & 7))) & 0x1FF) + popc64(a.word & ((1ull << (lo & 63)) - 1));
+}
 __device__ __forceinline__ int bit_dev(const uint64_t* __restrict__ words, uint64_t i) {
   return (int)((words[i >> 6] >> (i & 63)) & 1ull);
 }
@@ -439,29 +473,45 @@ __device__ __forceinline__ uint64_t select_plain(const SelQ& s, uint64_t i) {
   // select/select_support_mcl_par.hpp:564-611
   i -= 1;
   const uint64_t sb = i >> 12, off = i & 0xFFF;
+  // (all three loads at once: the long superblocks are the rare ones)
   const int64_t li = s.long_index[sb];
+  const uint64_t start = s.superblock[sb];
+  const uint32_t mini = s.mini[sb * 64 + (off >> 6)];
   if (li >= 0) return s.long_pool[(uint64_t)li * 4096 + off];
-  const uint64_t base = s.superblock[sb] + s.mini[sb * 64 + (off >> 6)];
+  const uint64_t base = start + mini;
   uint32_t r = (uint32_t)(off & 63);
   if (r == 0) return base;
-  uint64_t pos = base + 1;
-  uint64_t wp = pos >> 6;
-  const uint32_t wo = (uint32_t)(pos & 63);
-  if (wp >= s.W) return WTG_NONE;
-  uint64_t x = s.words[wp];
-  if (!s.bit) x = ~x;
-  x >>= wo;
-  uint32_t c = popc64(x);
-  if (c >= r) return (wp << 6) + wo + select_in_word(x, r - 1);
-  r -= c;
-  for (;;) {
-    ++wp;
-    if (wp >= s.W) return WTG_NONE;
-    x = s.words[wp];
-    if (!s.bit) x = ~x;
-    c = popc64(x);
-    if (c >= r) return (wp << 6) + select_in_word(x, r - 1);
-    r -= c;
+  uint64_t wp = (base + 1) >> 6;
+  const uint64_t flip = s.bit ? 0ull : ~0ull;
+  uint64_t keep = ~0ull << ((base + 1) & 63);
+  // four words a step, all loaded before one is looked at: samples are 64 ones
+  // apart, so at the density of a tree's levels one step has the bit
+  for (; wp < s.W; wp += 4) {
+    uint64_t x[4];
+    if (wp + 4 <= s.W) {
+      const wtg_u4_a8 a = *reinterpret_cast<const wtg_u4_a8*>(s.words + wp);
+      const wtg_u4_a8 b = *reinterpret_cast<const wtg_u4_a8*>(s.words + wp + 2);
+      x[0] = (uint64_t)a.x | (uint64_t)a.y << 32;
+      x[1] = (uint64_t)a.z | (uint64_t)a.w << 32;
+      x[2] = (uint64_t)b.x | (uint64_t)b.y << 32;
+      x[3] = (uint64_t)b.z | (uint64_t)b.w << 32;
+#pragma unroll
+      for (int k = 0; k < 4; k++) x[k] ^= flip;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; k++) x[k] = wp + k < s.W ? s.words[wp + k] ^ flip : 0ull;
+    }
+    x[0] &= keep;
+    keep = ~0ull;
+    const uint32_t c0 = popc64(x[0]), c1 = c0 + popc64(x[1]), c2 = c1 + popc64(x[2]), c3 = c2 + popc64(x[3]);
+    if (c3 >= r) {
+      const int k = (c0 < r) + (c1 < r) + (c2 < r);
+      const uint32_t before = k == 0 ? 0u : k == 1 ? c0 : k == 2 ? c1 : c2;
+      const uint64_t y = k == 0 ? x[0] : k == 1 ? x[1] : k == 2 ? x[2] : x[3];
+      return ((wp + k) << 6) + select_halves((uint32_t)y, (uint32_t)(y >> 32), r - 1 - before);
+    }
+    r -= c3;
   }
+  return WTG_NONE;
 }
 

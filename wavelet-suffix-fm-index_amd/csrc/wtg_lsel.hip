@@ -1239,7 +1239,7 @@ extern "C" int wtg_lsel_build(wtg_ctx* ctx, uint32_t nvec, const uint64_t* const
   for (uint32_t b = 0; b < nvec; b++) {
     LselDesc& d = ls->desc[b];
     const wtg_select& s = ls->sel[b];
-    d.s1 = SelQ{s.superblock, s.mini, s.long_index, s.long_pool, d_words[b], (nbits[b] + 63) / 64 + 1, 1};
+    d.s1 = SelQ{s.superblock, s.mini, s.long_index, s.long_pool, d_words[b], (nbits[b] + 63) / 64, 1};
     ls->info[b].nbits = nbits[b];
     ls->info[b].ones = s.arg_cnt;
   }

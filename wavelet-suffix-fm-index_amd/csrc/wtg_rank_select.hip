@@ -79,22 +79,6 @@ __device__ __forceinline__ void rs_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// position (0..63) of the k-th set bit of hi:lo, halving the window: k - c wraps
-// past k where the bit is below the middle
-__device__ __forceinline__ uint32_t select_halves(uint32_t lo, uint32_t hi, uint32_t k) {
-  uint32_t c = (uint32_t)__popc(lo), pos = 0;
-  uint32_t w = lo;
-  if (k >= c) { w = hi; pos = 32; }
-  k = min(k, k - c);
-#pragma unroll
-  for (uint32_t s = 16; s > 0; s >>= 1) {
-    c = (uint32_t)__popc(__builtin_amdgcn_ubfe(w, pos, s));  // (offset taken modulo 32)
-    pos += k >= c ? s : 0u;
-    k = min(k, k - c);
-  }
-  return pos;
-}
-
 // inclusive scan over the 64 lanes: DPP shifts inside each row of 16, then the
 // row totals read back as scalars
 __device__ __forceinline__ uint32_t wave_incl_scan_dpp(uint32_t v) {
@@ -368,9 +352,8 @@ __global__ void k_rank9_query(const uint64_t* __restrict__ words, const uint64_t
   if (q >= nq) return;
   const uint64_t i = idx[q];
   if (i > nbits) { out[q] = WTG_NONE; return; }
-  const uint64_t b = i >> 9;
-  uint64_t r = D[2 * b] + ((D[2 * b + 1] >> (63 - 9 * ((i & 511) >> 6))) & 0x1FF);
-  if (i & 63) r += popc64(words[i >> 6] & ((1ull << (i & 63)) - 1));
+  if (nbits == 0) { out[q] = 0; return; }
+  const uint64_t r = rank9_of(rank9_fetch(D, words, (nbits + 63) >> 6, i));
   out[q] = BIT ? r : i - r;
 }
 
