@@ -43,3 +43,63 @@ def test_every_position(ctx, n, levels):
     nth = (np.arange(n) - np.searchsorted(v, v) + 1).astype(np.uint64)
     assert np.array_equal(wt.select(nth, v), order)
     wt.free()
+
+
+@pytest.fixture(scope="module")
+def large(ctx):
+    """2^26 level bits: batches of 2^18 queries on it are put in order."""
+    n, levels = (1 << 26) // 9 + 1, 9
+    s = np.random.default_rng(5).integers(0, 1 << levels, n)
+    s[::3] = 77
+    wt = ctx.wtint_build(ctx.to_device(s.astype(np.uint32)), n, levels)
+    yield wt
+    wt.free()
+
+
+@pytest.mark.parametrize("nq", [1 << 18, (1 << 18) + 2049, (1 << 20) + 3])
+@pytest.mark.parametrize("keys", ["any", "one", "few", "refused"])
+def test_ordered_batch(ctx, large, nq, keys):
+    """A batch in order gives what the same queries give in small batches, as they came."""
+    wt, rng = large, np.random.default_rng(nq)
+    n, top = wt.n, 1 << wt.L
+    i, j = (rng.integers(0, n + 3, nq).astype(np.uint64) for _ in range(2))
+    lo, hi = (rng.integers(0, top + 2, nq).astype(np.uint64) for _ in range(2))
+    k = rng.integers(0, 3000, nq).astype(np.uint64)
+    if keys == "one":
+        i[:], lo[:] = n // 2, 77
+    elif keys == "few":
+        i, lo = i % np.uint64(3), lo % np.uint64(3)
+    elif keys == "refused":
+        i[::2], lo[::2], hi[::2] = n + 1, 1 << 62, np.uint64(2**64 - 1)
+    calls = [(wt.rank, (i, lo)), (wt.access, (i,)), (wt.inverse_select, (i,)), (wt.lex_count, (i, j, lo)),
+             (wt.lex_smaller_count, (i, lo)), (wt.range_count, (i, j, lo, hi)), (wt.select, (k, lo))]
+    step = 100000
+    for f, a in calls:
+        got = f(*a)
+        parts = [f(*(x[at:at + step] for x in a)) for at in range(0, nq, step)]
+        if isinstance(got, list):
+            want = [np.concatenate([p[c] for p in parts]) for c in range(len(got))]
+            assert all(np.array_equal(g, w) for g, w in zip(got, want)), f.__name__
+        else:
+            assert np.array_equal(got, np.concatenate(parts)), f.__name__
+
+
+def test_ordered_answers_over_their_queries(ctx, large):
+    """Answers written over a column of the batch itself."""
+    from wavelet_suffix_fm_index_amd import _check, lib
+    wt, rng, nq = large, np.random.default_rng(1), 1 << 18
+    lb, rb = np.sort(rng.integers(0, wt.n, (2, nq)), axis=0).astype(np.uint64)
+    lo, hi = np.sort(rng.integers(0, 1 << wt.L, (2, nq)), axis=0).astype(np.uint64)
+    want = wt.range_count(lb, rb, lo, hi)
+    ranks = wt.rank(lb, lo)
+    for over in range(4):
+        d = [ctx.to_device(x) for x in (lb, rb, lo, hi)]
+        _check(lib().wtg_wtint_range_count_batch(ctx.h, wt.h, *[x.ptr for x in d], nq, d[over].ptr))
+        assert np.array_equal(d[over].get(), want)
+        for x in d:
+            x.free()
+    d = [ctx.to_device(x) for x in (lb, lo)]
+    _check(lib().wtg_wtint_rank_batch(ctx.h, wt.h, d[0].ptr, d[1].ptr, nq, d[1].ptr))
+    assert np.array_equal(d[1].get(), ranks)
+    for x in d:
+        x.free()

@@ -76,6 +76,7 @@ extern "C" int wtg_ctx_destroy(wtg_ctx* ctx) {
   for (auto e : ctx->kpool) (void)hipEventDestroy(e);
   if (ctx->ws) (void)hipFree(ctx->ws);
   if (ctx->d_small) (void)hipFree(ctx->d_small);
+  if (ctx->qscratch) (void)hipFree(ctx->qscratch);
   if (ctx->t0) (void)hipEventDestroy(ctx->t0);
   if (ctx->t1) (void)hipEventDestroy(ctx->t1);
   if (ctx->h2d_ev) (void)hipEventDestroy(ctx->h2d_ev);
@@ -184,6 +185,25 @@ int wtg_ws_reserve(wtg_ctx* ctx, size_t bytes) {
   }
   ctx->ws_bytes = want;
   return WTG_OK;
+}
+
+void* wtg_query_scratch(wtg_ctx* ctx, size_t bytes) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (!ctx->qscratch) {
+    // (relaxed: another stream of this thread may be capturing)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+    if (hipMalloc(&ctx->qscratch, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      ctx->qscratch = nullptr;
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+  return ctx->qscratch;
 }
 
 extern "C" int wtg_malloc(wtg_ctx* ctx, void** dptr, uint64_t bytes) {

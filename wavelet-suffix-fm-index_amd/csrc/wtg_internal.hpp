@@ -48,6 +48,8 @@ struct wtg_ctx {
   // host-to-device tables (h2d_ev marks the last such copy)
   uint8_t* h_stage = nullptr;
   hipEvent_t h2d_ev = nullptr;
+  // where large query batches are put in order (wtg_query_scratch)
+  void* qscratch = nullptr;
   // stream timer
   hipEvent_t t0 = nullptr, t1 = nullptr;
   // per-kernel timing
@@ -61,6 +63,11 @@ struct wtg_ctx {
 
 // workspace of at least `bytes`, 256-byte aligned regions carved by the caller
 int wtg_ws_reserve(wtg_ctx* ctx, size_t bytes);
+// A block of `bytes` (the same in every call) for a batch of queries, allocated at
+// the first use, never moved, and freed with the context.  Null while the stream
+// is being captured (a graph may be replayed beside the context's other work) or
+// when there is no memory: the caller then answers the batch as it came.
+void* wtg_query_scratch(wtg_ctx* ctx, size_t bytes);
 constexpr size_t WTG_STAGE_AUX = 256;  // [256, 4096): reads collected by a later sync of the call
 constexpr size_t WTG_STAGE_D2H = 4096, WTG_STAGE_D2H_MAX = 16384;
 constexpr size_t WTG_STAGE_H2D = 32768, WTG_STAGE_H2D_MAX = 32768;

@@ -29,15 +29,180 @@ struct WtQ {
 // lookups).  10^6 queries each on a 20-level tree of 2^24 symbols: rank 593 ->
 // 540 us, access 850 -> 554, select 953 -> 897, lex_count 1030 -> 843,
 // range_count 2157 -> 1540: 128-byte lines from behind the L2 at 7.4 TB/s, the same in
-// every one of them.
+// every one of them.  Ordered batches below.
 __device__ __forceinline__ RankAt wt_fetch(const WtQ& w, uint64_t i) { return rank9_fetch(w.D, w.words, w.W, i); }
 
+// --------------------------------------------- order of a large batch
+// The walks of a large batch are bound by 128-byte lines from behind the L2s:
+// 10^6 random queries touch most of a level that is several times an XCD's 4 MiB.
+// Such a batch is first split into 256 parts by symbol (by position where the
+// symbol is not known), at 255 of a sample of its own keys, so the parts are
+// even whatever the keys are; the walk then takes the parts in order, each XCD
+// an eighth of them, and an XCD's queries in flight share a small part of every
+// level.  Answers are written where the query stood.  What it measured is at
+// order_pays.
+constexpr uint32_t QO_BINS = 256, QO_SAMPLE = 1024, QO_XCDS = 8;
+constexpr uint32_t QO_THREADS = 512, QO_PER = 8, QO_TILE = QO_THREADS * QO_PER;
+constexpr uint64_t QO_CHUNK = 1ull << 20;  // queries ordered at a time: the scratch is 36 bytes for each
+constexpr uint32_t QO_COLS = 4;
+struct QCols {
+  const uint64_t* c[QO_COLS];
+};
+struct QOrder {
+  uint64_t* col[QO_COLS];  // the columns, in order
+  uint32_t* q;             // where the query stood
+  uint64_t* split;         // [QO_BINS - 1] first key of bins 1..
+  uint32_t* tot;           // [QO_BINS] queries of each bin
+  uint32_t* cur;           // [QO_BINS] of which placed
+};
+constexpr size_t QO_BYTES = QO_CHUNK * (QO_COLS * 8 + 4) + QO_BINS * 16;
+
+__device__ __forceinline__ uint32_t qo_bin(const uint64_t* s_split, uint64_t key) {
+  uint32_t b = 0;  // splitters <= key
+#pragma unroll
+  for (uint32_t h = QO_BINS / 2; h > 0; h >>= 1)
+    if (s_split[b + h - 1] <= key) b += h;
+  return b;
+}
+
+// The splitters: every fourth of 1024 keys of the batch.  A block places 16 of
+// them, 16 threads to a key, each counting the smaller ones among 64 (44 -> 5 us
+// with one block and a thread for each key).
+__global__ __launch_bounds__(256) void k_order_split(const uint64_t* __restrict__ key, uint64_t nq, QOrder o) {
+  __shared__ uint64_t s_key[QO_SAMPLE + 16];
+  const uint32_t t = threadIdx.x;
+#pragma unroll
+  for (uint32_t k = t; k < QO_SAMPLE; k += 256) s_key[k + (k >> 6)] = key[(k * nq) / QO_SAMPLE];
+  if (blockIdx.x == 0) o.tot[t] = o.cur[t] = 0;
+  __syncthreads();
+  const uint32_t mine = blockIdx.x * 16 + (t >> 4), part = (t & 15) * 64;
+  const uint64_t v = s_key[mine + (mine >> 6)];
+  uint32_t r = 0;
+#pragma unroll 8
+  for (uint32_t k = part; k < part + 64; k++) {
+    const uint64_t x = s_key[k + (part >> 6)];
+    r += x < v || (x == v && k < mine);
+  }
+#pragma unroll
+  for (uint32_t d = 1; d < 16; d <<= 1) r += __shfl_xor(r, d, 64);
+  constexpr uint32_t E = QO_SAMPLE / QO_BINS;
+  if ((t & 15) == 0 && r % E == 0 && r) o.split[r / E - 1] = v;
+}
+
+__device__ __forceinline__ void qo_bins(const uint64_t* s_split, const uint64_t* __restrict__ key, uint64_t base,
+                                        uint64_t nq, uint32_t (&bin)[QO_PER]) {
+  uint64_t v[QO_PER];
+#pragma unroll
+  for (uint32_t k = 0; k < QO_PER; k++) v[k] = base + k * QO_THREADS < nq ? key[base + k * QO_THREADS] : 0ull;
+#pragma unroll
+  for (uint32_t k = 0; k < QO_PER; k++) bin[k] = qo_bin(s_split, v[k]);
+}
+
+__global__ __launch_bounds__(QO_THREADS) void k_order_count(const uint64_t* __restrict__ key, uint64_t nq, QOrder o) {
+  __shared__ uint64_t s_split[QO_BINS];
+  __shared__ uint32_t s_cnt[QO_BINS];
+  const uint32_t t = threadIdx.x;
+  if (t < QO_BINS) {
+    s_split[t] = t < QO_BINS - 1 ? o.split[t] : ~0ull;
+    s_cnt[t] = 0;
+  }
+  __syncthreads();
+  const uint64_t base = (uint64_t)blockIdx.x * QO_TILE + t;
+  uint32_t bin[QO_PER];
+  qo_bins(s_split, key, base, nq, bin);
+#pragma unroll
+  for (uint32_t k = 0; k < QO_PER; k++)
+    if (base + k * QO_THREADS < nq) atomicAdd(&s_cnt[bin[k]], 1u);
+  __syncthreads();
+  if (t < QO_BINS && s_cnt[t]) atomicAdd(&o.tot[t], s_cnt[t]);
+}
+
+// A tile's queries by bin in LDS, a column at a time, so that neighbouring threads
+// store to one run of a bin (16 queries, one line, in an even tile; stored where
+// they were found 25-87 us, so 14-25 for one to four columns of 10^6).
+// (the order inside a bin is the one the blocks arrive in: no answer depends on it)
+template <uint32_t NC>
+__global__ __launch_bounds__(QO_THREADS) void k_order_put(QCols in, uint32_t key, uint64_t nq, QOrder o) {
+  __shared__ uint64_t s_split[QO_BINS];
+  __shared__ uint32_t s_cnt[QO_BINS], s_first[QO_BINS], s_tot[2][QO_BINS / 64];
+  __shared__ uint32_t s_to[QO_TILE];
+  __shared__ uint64_t s_buf[QO_TILE];
+  const uint32_t t = threadIdx.x;
+  uint32_t tot = 0, incl = 0;
+  if (t < QO_BINS) {
+    s_split[t] = t < QO_BINS - 1 ? o.split[t] : ~0ull;
+    s_cnt[t] = 0;
+    tot = o.tot[t];
+    incl = wave_incl_sum_dpp(tot);
+    if ((t & 63) == 63) s_tot[0][t >> 6] = incl;
+  }
+  __syncthreads();
+  const uint64_t tile = (uint64_t)blockIdx.x * QO_TILE, base = tile + t;
+  uint32_t bin[QO_PER], at[QO_PER];
+  qo_bins(s_split, in.c[key], base, nq, bin);
+#pragma unroll
+  for (uint32_t k = 0; k < QO_PER; k++) at[k] = base + k * QO_THREADS < nq ? atomicAdd(&s_cnt[bin[k]], 1u) : 0u;
+  __syncthreads();
+  uint32_t cnt = 0, here = 0;
+  if (t < QO_BINS) {
+    cnt = s_cnt[t];
+    here = wave_incl_sum_dpp(cnt);
+    if ((t & 63) == 63) s_tot[1][t >> 6] = here;
+  }
+  __syncthreads();
+  if (t < QO_BINS) {
+    uint32_t to = incl - tot;
+    here -= cnt;
+    for (uint32_t w = 0; w < (t >> 6); w++) {
+      to += s_tot[0][w];
+      here += s_tot[1][w];
+    }
+    s_first[t] = here;                                            // in the tile
+    s_cnt[t] = cnt ? to + atomicAdd(&o.cur[t], cnt) - here : 0u;  // from there to the ordered batch
+  }
+  __syncthreads();
+  const uint32_t m = (uint32_t)(nq - tile < QO_TILE ? nq - tile : QO_TILE);
+  uint32_t* s_q = reinterpret_cast<uint32_t*>(s_buf);
+#pragma unroll
+  for (uint32_t k = 0; k < QO_PER; k++)
+    if (t + k * QO_THREADS < m) {
+      at[k] += s_first[bin[k]];
+      s_to[at[k]] = at[k] + s_cnt[bin[k]];
+      s_q[at[k]] = (uint32_t)tile + t + k * QO_THREADS;
+    }
+  __syncthreads();
+  for (uint32_t k = t; k < m; k += QO_THREADS) o.q[s_to[k]] = s_q[k];
+#pragma unroll
+  for (uint32_t c = 0; c < NC; c++) {
+    uint64_t v[QO_PER];
+#pragma unroll
+    for (uint32_t k = 0; k < QO_PER; k++) v[k] = t + k * QO_THREADS < m ? in.c[c][base + k * QO_THREADS] : 0ull;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < QO_PER; k++)
+      if (t + k * QO_THREADS < m) s_buf[at[k]] = v[k];
+    __syncthreads();
+    for (uint32_t k = t; k < m; k += QO_THREADS) o.col[c][s_to[k]] = s_buf[k];
+  }
+}
+
+// the query of this thread: where its columns are (p) and its answer goes (q);
+// false past the end.  An ordered batch's grid is a multiple of the XCDs.
+__device__ __forceinline__ bool q_slot(const uint32_t* __restrict__ order, uint64_t nq, uint64_t& p, uint64_t& q) {
+  const uint32_t b = order ? (blockIdx.x % QO_XCDS) * (gridDim.x / QO_XCDS) + blockIdx.x / QO_XCDS : blockIdx.x;
+  p = (uint64_t)b * blockDim.x + threadIdx.x;
+  if (p >= nq) return false;
+  q = order ? order[p] : p;
+  return true;
+}
+
 __global__ void k_wtint_rank(WtQ w, const uint64_t* __restrict__ qi, const uint64_t* __restrict__ qc,
-                             uint64_t nq, uint64_t* __restrict__ out) {
-  const uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nq) return;
-  uint64_t i = qi[q];
-  const uint64_t c = qc[q];
+                             uint64_t nq, uint64_t* __restrict__ out,
+                             const uint32_t* __restrict__ order) {
+  uint64_t p, q;
+  if (!q_slot(order, nq, p, q)) return;
+  uint64_t i = qi[p];
+  const uint64_t c = qc[p];
   if (i > w.n) { out[q] = WTG_NONE; return; }
   if (w.L < 64 && (1ull << w.L) <= c) { out[q] = 0; return; }
   uint64_t offset = 0, mask = 1ull << (w.L - 1), node_size = w.n;
@@ -100,12 +265,13 @@ __device__ __forceinline__ void wtint_lex(const WtQ& w, uint64_t i, uint64_t j, 
 
 __global__ void k_wtint_lex_count(WtQ w, const uint64_t* __restrict__ qi, const uint64_t* __restrict__ qj,
                                   const uint64_t* __restrict__ qc, uint64_t nq, uint64_t* __restrict__ out_rank,
-                                  uint64_t* __restrict__ out_smaller, uint64_t* __restrict__ out_greater) {
-  const uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nq) return;
-  const uint64_t i = qi[q], j = qj[q];
+                                  uint64_t* __restrict__ out_smaller, uint64_t* __restrict__ out_greater,
+                                  const uint32_t* __restrict__ order) {
+  uint64_t p, q;
+  if (!q_slot(order, nq, p, q)) return;
+  const uint64_t i = qi[p], j = qj[p];
   uint64_t rk = WTG_NONE, sm = WTG_NONE, gr = WTG_NONE;
-  if (i <= j && j <= w.n) wtint_lex(w, i, j, qc[q], rk, sm, gr);
+  if (i <= j && j <= w.n) wtint_lex(w, i, j, qc[p], rk, sm, gr);
   out_rank[q] = rk;
   out_smaller[q] = sm;
   out_greater[q] = gr;
@@ -114,11 +280,12 @@ __global__ void k_wtint_lex_count(WtQ w, const uint64_t* __restrict__ qi, const 
 // lex_smaller_count (wt_int/wt_int_par.hpp:753-780): rank(i,c) and the number of
 // values below c in [0, i)
 __global__ void k_wtint_lex_smaller(WtQ w, const uint64_t* __restrict__ qi, const uint64_t* __restrict__ qc,
-                                    uint64_t nq, uint64_t* __restrict__ out_rank, uint64_t* __restrict__ out_smaller) {
-  const uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nq) return;
-  uint64_t i = qi[q];
-  const uint64_t c = qc[q];
+                                    uint64_t nq, uint64_t* __restrict__ out_rank, uint64_t* __restrict__ out_smaller,
+                                    const uint32_t* __restrict__ order) {
+  uint64_t p, q;
+  if (!q_slot(order, nq, p, q)) return;
+  uint64_t i = qi[p];
+  const uint64_t c = qc[p];
   if (i > w.n) { out_rank[q] = out_smaller[q] = WTG_NONE; return; }
   if (w.L < 64 && (1ull << w.L) <= c) { out_rank[q] = 0; out_smaller[q] = i; return; }
   uint64_t offset = 0, mask = 1ull << (w.L - 1), node_size = w.n, res = 0;
@@ -141,11 +308,12 @@ __global__ void k_wtint_lex_smaller(WtQ w, const uint64_t* __restrict__ qi, cons
 // vlb is clamped to 2^L - 1 the same way.
 __global__ void k_wtint_range_count(WtQ w, const uint64_t* __restrict__ qlb, const uint64_t* __restrict__ qrb,
                                     const uint64_t* __restrict__ qvlb, const uint64_t* __restrict__ qvrb,
-                                    uint64_t nq, uint64_t* __restrict__ out) {
-  const uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nq) return;
-  const uint64_t lb = qlb[q], rb = qrb[q];
-  uint64_t vlb = qvlb[q], vrb = qvrb[q];
+                                    uint64_t nq, uint64_t* __restrict__ out,
+                                    const uint32_t* __restrict__ order) {
+  uint64_t p, q;
+  if (!q_slot(order, nq, p, q)) return;
+  const uint64_t lb = qlb[p], rb = qrb[p];
+  uint64_t vlb = qvlb[p], vrb = qvrb[p];
   if (rb >= w.n) { out[q] = WTG_NONE; return; }
   const uint64_t top = w.L < 64 ? (1ull << w.L) : ~0ull;
   if (vrb > top) vrb = top;
@@ -167,11 +335,42 @@ __global__ void k_wtint_range_count(WtQ w, const uint64_t* __restrict__ qlb, con
   out[q] = hi.smaller - lo.smaller;
 }
 
+// The same in two walks for an ordered batch (each ordered by its own bound):
+// the lower one leaves its count or a mark, the upper one takes it from there.
+constexpr uint64_t WT_RANGE_EMPTY = WTG_NONE - 1;
+template <bool UPPER>
+__global__ void k_wtint_range_half(WtQ w, const uint64_t* __restrict__ qlb, const uint64_t* __restrict__ qrb,
+                                   const uint64_t* __restrict__ qv, const uint64_t* __restrict__ qvrb, uint64_t nq,
+                                   uint64_t* __restrict__ out, const uint32_t* __restrict__ order) {
+  uint64_t p, q;
+  if (!q_slot(order, nq, p, q)) return;
+  const uint64_t lb = qlb[p], rb = qrb[p];
+  const uint64_t top = w.L < 64 ? (1ull << w.L) : ~0ull;
+  uint64_t v = qv[p], rk, below, gr;
+  if (UPPER) {
+    const uint64_t low = out[q];
+    if (low == WTG_NONE) return;
+    if (low == WT_RANGE_EMPTY) { out[q] = 0; return; }
+    if (v >= top - (w.L < 64 ? 1 : 0)) below = rb + 1 - lb;  // every value is <= v
+    else wtint_lex(w, lb, rb + 1, v + 1, rk, below, gr);
+    out[q] = below - low;
+  } else {
+    uint64_t vrb = qvrb[p];
+    if (rb >= w.n) { out[q] = WTG_NONE; return; }
+    if (vrb > top) vrb = top;
+    if (v > vrb || lb > rb) { out[q] = WT_RANGE_EMPTY; return; }
+    if (w.L < 64 && v > top - 1) v = top - 1;
+    wtint_lex(w, lb, rb + 1, v, rk, below, gr);
+    out[q] = below;
+  }
+}
+
 __global__ void k_wtint_access(WtQ w, const uint64_t* __restrict__ qi, uint64_t nq,
-                               uint64_t* __restrict__ out_sym, uint64_t* __restrict__ out_rank) {
-  const uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nq) return;
-  uint64_t i = qi[q];
+                               uint64_t* __restrict__ out_sym, uint64_t* __restrict__ out_rank,
+                               const uint32_t* __restrict__ order) {
+  uint64_t p, q;
+  if (!q_slot(order, nq, p, q)) return;
+  uint64_t i = qi[p];
   if (i >= w.n) {
     out_sym[q] = WTG_NONE;
     if (out_rank) out_rank[q] = WTG_NONE;
@@ -192,11 +391,12 @@ __global__ void k_wtint_access(WtQ w, const uint64_t* __restrict__ qi, uint64_t 
 
 template <uint32_t MAXL>  // the tree's levels are at most MAXL
 __global__ void k_wtint_select(WtQ w, const uint64_t* __restrict__ qi, const uint64_t* __restrict__ qc,
-                               uint64_t nq, uint64_t* __restrict__ out) {
-  const uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nq) return;
-  uint64_t i = qi[q];
-  const uint64_t c = qc[q];
+                               uint64_t nq, uint64_t* __restrict__ out,
+                               const uint32_t* __restrict__ order) {
+  uint64_t p, q;
+  if (!q_slot(order, nq, p, q)) return;
+  uint64_t i = qi[p];
+  const uint64_t c = qc[p];
   uint64_t path_off[MAXL + 1], path_rank[MAXL + 1];
   uint64_t offset = 0, mask = 1ull << (w.L - 1), node_size = w.n;
   path_off[0] = path_rank[0] = 0;
@@ -360,37 +560,90 @@ static int q_check(wtg_ctx* ctx, const wtg_wtint* wt, uint64_t nq, const void* a
   return WTG_OK;
 }
 
+// Whether ordering a batch pays: level bits too many for an XCD's L2 beside the
+// directory, and queries enough for the three passes before the walk (~25 us).
+// us as it came -> ordered, rank / access / select / lex_count / range_count:
+//   2^23 bits, 2^20 queries:  81 -> 103,  81 -> 81,  164 -> 159, 126 -> 144,  222 -> 281
+//   2^24 bits, 2^18 queries:  63 -> 58,   62 -> 72,  104 -> 103,  78 -> 72,   129 -> 133
+//              2^20 queries: 220 -> 123, 217 -> 187, 366 -> 244, 284 -> 171,  502 -> 334
+//   2^27 bits, 2^17 queries:  53 -> 52,   52 -> 59,   89 -> 92,   71 -> 65,   112 -> 129
+//              2^18 queries:  94 -> 71,   94 -> 86,  154 -> 117, 130 -> 95,   211 -> 183
+//   2^28.3 bits, 2^20:       569 -> 275, 580 -> 323, 928 -> 521, 885 -> 503, 1487 -> 940
+static bool order_pays(const wtg_wtint* wt, uint64_t nq) {
+  return wt->nbits >= 1ull << 24 && nq >= (wt->nbits >= 1ull << 26 ? 1ull << 18 : 1ull << 19);
+}
+
+// A batch in chunks: walk(columns, queries, where they stood or null, answers' offset)
+// launches the kernels that answer one chunk.
+template <uint32_t NC, class F>
+static int q_ordered(wtg_ctx* ctx, char* scratch, const QCols& in, uint32_t key, uint64_t nq, F&& walk) {
+  QOrder o{};
+  for (uint32_t c = 0; c < QO_COLS; c++) o.col[c] = (uint64_t*)scratch + c * QO_CHUNK;
+  o.split = (uint64_t*)scratch + QO_COLS * QO_CHUNK;
+  o.tot = (uint32_t*)(o.split + QO_BINS);
+  o.cur = o.tot + QO_BINS;
+  o.q = o.cur + QO_BINS;
+  const uint64_t step = wtg_ceil_div(nq, wtg_ceil_div(nq, QO_CHUNK));  // chunks of one size
+  for (uint64_t at = 0; at < nq; at += step) {
+    const uint64_t m = nq - at < step ? nq - at : step;
+    QCols part{};
+    for (uint32_t c = 0; c < NC; c++) part.c[c] = in.c[c] + at;
+    const dim3 g((unsigned)wtg_ceil_div(m, QO_TILE)), b(QO_THREADS);
+    WTG_LAUNCH(ctx, "order_split", k_order_split, dim3(QO_SAMPLE / 16), dim3(256), 0, part.c[key], m, o);
+    WTG_LAUNCH(ctx, "order_count", k_order_count, g, b, 0, part.c[key], m, o);
+    WTG_LAUNCH(ctx, "order_put", k_order_put<NC>, g, b, 0, part, key, m, o);
+    QCols cols{};
+    for (uint32_t c = 0; c < NC; c++) cols.c[c] = o.col[c];
+    walk(cols, m, (const uint32_t*)o.q, at, dim3((unsigned)(wtg_ceil_div(m, 256 * QO_XCDS) * QO_XCDS)));
+  }
+  WTG_LAUNCH_CHECK();
+  return WTG_OK;
+}
+
+// The batch as it came, or ordered by column `key` where that pays.
+template <uint32_t NC, class F>
+static int q_batch(wtg_ctx* ctx, const wtg_wtint* wt, const QCols& in, uint32_t key, uint64_t nq, F&& walk) {
+  WTG_TRY(wtg_set_device(ctx));
+  char* scratch = order_pays(wt, nq) ? (char*)wtg_query_scratch(ctx, QO_BYTES) : nullptr;
+  if (scratch) {
+    WTG_TRY(q_ordered<NC>(ctx, scratch, in, key, nq, walk));
+  } else {
+    walk(in, nq, (const uint32_t*)nullptr, (uint64_t)0, dim3((unsigned)wtg_ceil_div(nq, 256)));
+    WTG_LAUNCH_CHECK();
+  }
+  return wtg_finish(ctx);
+}
+
 extern "C" int wtg_wtint_rank_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_i,
                                     const uint64_t* d_c, uint64_t nq, uint64_t* d_out) {
   WTG_TRY(q_check(ctx, wt, nq, d_i, d_out));
   WTG_REQUIRE(nq == 0 || d_c, "null d_c");
   if (!nq) return WTG_OK;
-  WTG_TRY(wtg_set_device(ctx));
-  WTG_LAUNCH(ctx, "wtint_rank", k_wtint_rank, dim3((unsigned)wtg_ceil_div(nq, 256)), dim3(256), 0,
-             make_q(wt), d_i, d_c, nq, d_out);
-  WTG_LAUNCH_CHECK();
-  return wtg_finish(ctx);
+  return q_batch<2>(ctx, wt, QCols{{d_i, d_c}}, 1, nq,
+                    [&](const QCols& c, uint64_t m, const uint32_t* order, uint64_t at, dim3 grid) {
+    WTG_LAUNCH(ctx, "wtint_rank", k_wtint_rank, grid, dim3(256), 0, make_q(wt), c.c[0], c.c[1], m, d_out + at, order);
+  });
+}
+static int access_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_i, uint64_t nq, uint64_t* d_sym,
+                        uint64_t* d_rank) {
+  return q_batch<1>(ctx, wt, QCols{{d_i}}, 0, nq,
+                    [&](const QCols& c, uint64_t m, const uint32_t* order, uint64_t at, dim3 grid) {
+    WTG_LAUNCH(ctx, "wtint_access", k_wtint_access, grid, dim3(256), 0, make_q(wt), c.c[0], m, d_sym + at,
+               d_rank ? d_rank + at : nullptr, order);
+  });
 }
 extern "C" int wtg_wtint_access_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_i,
                                       uint64_t nq, uint64_t* d_out) {
   WTG_TRY(q_check(ctx, wt, nq, d_i, d_out));
   if (!nq) return WTG_OK;
-  WTG_TRY(wtg_set_device(ctx));
-  WTG_LAUNCH(ctx, "wtint_access", k_wtint_access, dim3((unsigned)wtg_ceil_div(nq, 256)), dim3(256), 0,
-             make_q(wt), d_i, nq, d_out, (uint64_t*)nullptr);
-  WTG_LAUNCH_CHECK();
-  return wtg_finish(ctx);
+  return access_batch(ctx, wt, d_i, nq, d_out, nullptr);
 }
 extern "C" int wtg_wtint_inverse_select_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_i,
                                               uint64_t nq, uint64_t* d_rank, uint64_t* d_sym) {
   WTG_TRY(q_check(ctx, wt, nq, d_i, d_sym));
   WTG_REQUIRE(nq == 0 || d_rank, "null d_rank");
   if (!nq) return WTG_OK;
-  WTG_TRY(wtg_set_device(ctx));
-  WTG_LAUNCH(ctx, "wtint_access", k_wtint_access, dim3((unsigned)wtg_ceil_div(nq, 256)), dim3(256), 0,
-             make_q(wt), d_i, nq, d_sym, d_rank);
-  WTG_LAUNCH_CHECK();
-  return wtg_finish(ctx);
+  return access_batch(ctx, wt, d_i, nq, d_sym, d_rank);
 }
 extern "C" int wtg_wtint_lex_count_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_i,
                                          const uint64_t* d_j, const uint64_t* d_c, uint64_t nq, uint64_t* d_rank,
@@ -398,11 +651,11 @@ extern "C" int wtg_wtint_lex_count_batch(wtg_ctx* ctx, const wtg_wtint* wt, cons
   WTG_TRY(q_check(ctx, wt, nq, d_i, d_rank));
   WTG_REQUIRE(nq == 0 || (d_j && d_c && d_smaller && d_greater), "null argument");
   if (!nq) return WTG_OK;
-  WTG_TRY(wtg_set_device(ctx));
-  WTG_LAUNCH(ctx, "wtint_lex_count", k_wtint_lex_count, dim3((unsigned)wtg_ceil_div(nq, 256)), dim3(256), 0,
-             make_q(wt), d_i, d_j, d_c, nq, d_rank, d_smaller, d_greater);
-  WTG_LAUNCH_CHECK();
-  return wtg_finish(ctx);
+  return q_batch<3>(ctx, wt, QCols{{d_i, d_j, d_c}}, 2, nq,
+                    [&](const QCols& c, uint64_t m, const uint32_t* order, uint64_t at, dim3 grid) {
+    WTG_LAUNCH(ctx, "wtint_lex_count", k_wtint_lex_count, grid, dim3(256), 0, make_q(wt), c.c[0], c.c[1], c.c[2], m,
+               d_rank + at, d_smaller + at, d_greater + at, order);
+  });
 }
 extern "C" int wtg_wtint_lex_smaller_count_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_i,
                                                  const uint64_t* d_c, uint64_t nq, uint64_t* d_rank,
@@ -410,11 +663,11 @@ extern "C" int wtg_wtint_lex_smaller_count_batch(wtg_ctx* ctx, const wtg_wtint* 
   WTG_TRY(q_check(ctx, wt, nq, d_i, d_rank));
   WTG_REQUIRE(nq == 0 || (d_c && d_smaller), "null argument");
   if (!nq) return WTG_OK;
-  WTG_TRY(wtg_set_device(ctx));
-  WTG_LAUNCH(ctx, "wtint_lex_smaller", k_wtint_lex_smaller, dim3((unsigned)wtg_ceil_div(nq, 256)), dim3(256), 0,
-             make_q(wt), d_i, d_c, nq, d_rank, d_smaller);
-  WTG_LAUNCH_CHECK();
-  return wtg_finish(ctx);
+  return q_batch<2>(ctx, wt, QCols{{d_i, d_c}}, 1, nq,
+                    [&](const QCols& c, uint64_t m, const uint32_t* order, uint64_t at, dim3 grid) {
+    WTG_LAUNCH(ctx, "wtint_lex_smaller", k_wtint_lex_smaller, grid, dim3(256), 0, make_q(wt), c.c[0], c.c[1], m,
+               d_rank + at, d_smaller + at, order);
+  });
 }
 extern "C" int wtg_wtint_range_count_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_lb,
                                            const uint64_t* d_rb, const uint64_t* d_vlb, const uint64_t* d_vrb,
@@ -423,9 +676,26 @@ extern "C" int wtg_wtint_range_count_batch(wtg_ctx* ctx, const wtg_wtint* wt, co
   WTG_REQUIRE(nq == 0 || (d_rb && d_vlb && d_vrb), "null argument");
   if (!nq) return WTG_OK;
   WTG_TRY(wtg_set_device(ctx));
-  WTG_LAUNCH(ctx, "wtint_range_count", k_wtint_range_count, dim3((unsigned)wtg_ceil_div(nq, 256)), dim3(256), 0,
-             make_q(wt), d_lb, d_rb, d_vlb, d_vrb, nq, d_out);
-  WTG_LAUNCH_CHECK();
+  // the second walk reads the batch after the first has written: not over its own answers
+  bool apart = true;
+  for (const uint64_t* x : {d_lb, d_rb, d_vlb, d_vrb}) apart = apart && (x + nq <= d_out || d_out + nq <= x);
+  char* scratch = apart && order_pays(wt, nq) ? (char*)wtg_query_scratch(ctx, QO_BYTES) : nullptr;
+  if (scratch) {
+    WTG_TRY(q_ordered<4>(ctx, scratch, QCols{{d_lb, d_rb, d_vlb, d_vrb}}, 2, nq,
+                         [&](const QCols& c, uint64_t m, const uint32_t* order, uint64_t at, dim3 grid) {
+      WTG_LAUNCH(ctx, "wtint_range_lower", k_wtint_range_half<false>, grid, dim3(256), 0, make_q(wt), c.c[0], c.c[1],
+                 c.c[2], c.c[3], m, d_out + at, order);
+    }));
+    WTG_TRY(q_ordered<3>(ctx, scratch, QCols{{d_lb, d_rb, d_vrb}}, 2, nq,
+                         [&](const QCols& c, uint64_t m, const uint32_t* order, uint64_t at, dim3 grid) {
+      WTG_LAUNCH(ctx, "wtint_range_upper", k_wtint_range_half<true>, grid, dim3(256), 0, make_q(wt), c.c[0], c.c[1],
+                 c.c[2], (const uint64_t*)nullptr, m, d_out + at, order);
+    }));
+  } else {
+    WTG_LAUNCH(ctx, "wtint_range_count", k_wtint_range_count, dim3((unsigned)wtg_ceil_div(nq, 256)), dim3(256), 0,
+               make_q(wt), d_lb, d_rb, d_vlb, d_vrb, nq, d_out, (const uint32_t*)nullptr);
+    WTG_LAUNCH_CHECK();
+  }
   return wtg_finish(ctx);
 }
 extern "C" int wtg_wtint_select_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_i,
@@ -433,14 +703,13 @@ extern "C" int wtg_wtint_select_batch(wtg_ctx* ctx, const wtg_wtint* wt, const u
   WTG_TRY(q_check(ctx, wt, nq, d_i, d_out));
   WTG_REQUIRE(nq == 0 || d_c, "null d_c");
   if (!nq) return WTG_OK;
-  WTG_TRY(wtg_set_device(ctx));
-  if (wt->L <= 24) {
-    WTG_LAUNCH(ctx, "wtint_select", k_wtint_select<24>, dim3((unsigned)wtg_ceil_div(nq, 256)), dim3(256), 0,
-               make_q(wt), d_i, d_c, nq, d_out);
-  } else {
-    WTG_LAUNCH(ctx, "wtint_select", k_wtint_select<64>, dim3((unsigned)wtg_ceil_div(nq, 256)), dim3(256), 0,
-               make_q(wt), d_i, d_c, nq, d_out);
-  }
-  WTG_LAUNCH_CHECK();
-  return wtg_finish(ctx);
+  return q_batch<2>(ctx, wt, QCols{{d_i, d_c}}, 1, nq,
+                    [&](const QCols& c, uint64_t m, const uint32_t* order, uint64_t at, dim3 grid) {
+    if (wt->L <= 24)
+      WTG_LAUNCH(ctx, "wtint_select", k_wtint_select<24>, grid, dim3(256), 0, make_q(wt), c.c[0], c.c[1], m,
+                 d_out + at, order);
+    else
+      WTG_LAUNCH(ctx, "wtint_select", k_wtint_select<64>, grid, dim3(256), 0, make_q(wt), c.c[0], c.c[1], m,
+                 d_out + at, order);
+  });
 }
