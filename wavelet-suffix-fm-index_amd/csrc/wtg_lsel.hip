@@ -599,6 +599,167 @@ __global__ __launch_bounds__(256) void k_lsel_adam(const TrainVec* __restrict__ 
   tb.K[g].y -= lr * (m / bc1) / (sqrtf(s / bc2) + 1e-6f);
 }
 
+// Several training steps in one launch.  A step moves a knot by the samples of
+// the two intervals beside it alone, so a block that holds `knots` neighbours in
+// LDS carries all but the outer LSEL_STEPS on either side through LSEL_STEPS
+// steps by itself; it writes those, and the others are its neighbours' to write
+// (state in and state out are different arrays).  A thread keeps one item in
+// registers for all the steps: its targets and both weights of every sample, with
+// weights and target of 0 for the places of its aligned 16 that are not the
+// interval's, which add 0 to both sums.  Sums run in the item order of
+// k_lsel_items_sum, with the multiply-adds that k_lsel_items and k_lsel_adam are
+// compiled to: the same knots to the last bit.  With these two for each step, 50 steps of
+// 264448 knots and 4 M samples took 1027 us, now 349 (474 with 4 steps a launch, 404
+// with 6, 371 with 8: each launch spends about 19 us before its first step and 4 to 5
+// on a step, and the outer knots are 20 of the 52 that a dense model has in a block).
+constexpr uint32_t LSEL_STEPS = 10;
+struct TrainState {
+  const Knot* K;
+  const float *m1, *m2;
+  Knot* Ko;
+  float *m1o, *m2o;
+};
+struct TrainSteps {
+  float lr, b1, b2;
+  float bc1[LSEL_STEPS], bc2[LSEL_STEPS];
+  uint32_t n;
+};
+struct ItemAt {  // an item's samples u0..ue of its aligned block (targets from xb), its knots' arguments
+  const float* tgt;
+  uint64_t xb, u0, ue, T;
+  uint32_t ja, jb;
+};
+__device__ __forceinline__ ItemAt item_at(const TrainVec* __restrict__ tv, const Knot* __restrict__ K,
+                                          const TrainItems& it, uint32_t g, uint64_t i) {
+  const TrainVec& v = tv[it.model_of[g]];
+  const Knot a = K[g], b = K[(uint64_t)g + 1];
+  uint64_t t1, t2;
+  interval_samples(v, a, b, g - v.kfirst, t1, t2);
+  ItemAt r;
+  r.xb = ((t1 - 1) / LSEL_ITEM + (i - it.item_start[g])) * LSEL_ITEM;
+  r.u0 = r.xb + 1 > t1 ? r.xb + 1 : t1;
+  r.ue = r.xb + LSEL_ITEM < t2 ? r.xb + LSEL_ITEM : t2;
+  r.T = 1ull << v.tlog;
+  r.tgt = v.tgt + r.xb;
+  r.ja = a.j;
+  r.jb = b.j;
+  return r;
+}
+// A model's blocks: from block `first` of the launch on, `knots` neighbours each.
+struct TrainBlocks {
+  uint64_t first;
+  uint32_t knots;
+};
+constexpr uint32_t LSEL_TT = 1024, LSEL_TKNOTS = 512, LSEL_TITEMS = 7936;  // threads; most knots, items of a block
+__global__ __launch_bounds__(LSEL_TT) void k_lsel_train(const TrainVec* __restrict__ tv,
+                                                        const TrainBlocks* __restrict__ blocks, uint32_t nv,
+                                                        TrainItems it, TrainState ts, TrainSteps st) {
+  __shared__ float s_y[LSEL_TKNOTS], s_pa[LSEL_TITEMS], s_pc[LSEL_TITEMS];
+  __shared__ uint32_t s_at[LSEL_TKNOTS];  // first item of each interval
+  const uint32_t t = threadIdx.x;
+  uint32_t mo = 0;
+  while (mo + 1 < nv && blocks[mo + 1].first <= blockIdx.x) mo++;
+  const uint64_t k0 = tv[mo].kfirst, k1 = k0 + tv[mo].nknots, ns = tv[mo].ns;
+  const uint32_t own = blocks[mo].knots - 2 * LSEL_STEPS;
+  const uint64_t o0 = k0 + (blockIdx.x - blocks[mo].first) * own, o1 = o0 + own < k1 ? o0 + own : k1;
+  const uint64_t gl = o0 - k0 > LSEL_STEPS ? o0 - LSEL_STEPS : k0;
+  const uint64_t gr = o1 + LSEL_STEPS < k1 ? o1 + LSEL_STEPS : k1;
+  const uint32_t nl = (uint32_t)(gr - gl);
+  const float scale = 2.0f / (float)(ns ? ns : 1);
+  const uint64_t i0 = it.item_start[gl];
+  float m = 0.f, s2 = 0.f;
+  uint32_t kj = 0;
+  if (t < nl) {
+    const uint64_t g = gl + t;
+    const Knot k = ts.K[g];
+    s_y[t] = k.y;
+    kj = k.j;
+    s_at[t] = (uint32_t)(it.item_start[g] - i0);
+    m = ts.m1[g];
+    s2 = ts.m2[g];
+  }
+  __syncthreads();
+  const uint32_t ni = min(s_at[nl - 1], LSEL_TITEMS);  // of the intervals between the block's knots
+  float w[LSEL_ITEM], f[LSEL_ITEM], tg[LSEL_ITEM];  // weight of a, of b, target
+  uint32_t at = 0;
+#pragma unroll
+  for (uint32_t q = 0; q < LSEL_ITEM; q++) w[q] = f[q] = tg[q] = 0.f;
+  if (t < ni) {
+    const uint32_t g = it.item_g[i0 + t];
+    const ItemAt a = item_at(tv, ts.K, it, g, i0 + t);
+    at = (uint32_t)(g - gl);
+    const float span = (float)(a.jb - a.ja);
+    const float4* t4 = reinterpret_cast<const float4*>(a.tgt);
+#pragma unroll
+    for (uint32_t r = 0; r < LSEL_ITEM / 4; r++) {
+      const float4 x = t4[r];
+      tg[4 * r] = x.x;
+      tg[4 * r + 1] = x.y;
+      tg[4 * r + 2] = x.z;
+      tg[4 * r + 3] = x.w;
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < LSEL_ITEM; q++) {
+      const uint64_t u = a.xb + 1 + q;
+      const bool in = u >= a.u0 && u <= a.ue;
+      const float x = (float)(u * a.T - a.ja) / span;
+      f[q] = in ? x : 0.f;
+      w[q] = in ? 1.0f - x : 0.f;
+      tg[q] = in ? tg[q] : 0.f;
+    }
+  }
+  for (uint32_t step = 0; step < st.n; step++) {
+    if (t < ni) {
+      const float ya = s_y[at], yb = s_y[at + 1];
+      float sa = 0.f, sc = 0.f;
+#pragma unroll
+      for (uint32_t q = 0; q < LSEL_ITEM; q++) {
+        const float e = __builtin_fmaf(f[q], yb, w[q] * ya) - tg[q];
+        sa = __builtin_fmaf(e, w[q], sa);
+        sc = __builtin_fmaf(e, f[q], sc);
+      }
+      s_pa[t] = sa;
+      s_pc[t] = sc;
+    }
+    for (uint32_t i = t + LSEL_TT; i < ni; i += LSEL_TT) {  // items past one a thread: read again
+      const uint32_t g = it.item_g[i0 + i];
+      const ItemAt a = item_at(tv, ts.K, it, g, i0 + i);
+      const float ya = s_y[g - gl], yb = s_y[g - gl + 1], span = (float)(a.jb - a.ja);
+      float sa = 0.f, sc = 0.f;
+      for (uint64_t u = a.u0; u <= a.ue; u++) {
+        const float x = (float)(u * a.T - a.ja) / span;
+        const float e = __builtin_fmaf(x, yb, (1.0f - x) * ya) - a.tgt[u - 1 - a.xb];
+        sa = __builtin_fmaf(e, 1.0f - x, sa);
+        sc = __builtin_fmaf(e, x, sc);
+      }
+      s_pa[i] = sa;
+      s_pc[i] = sc;
+    }
+    __syncthreads();
+    if (t < nl) {
+      float sa = 0.f, sc = 0.f;
+      if (t + 1 < nl)
+        for (uint32_t q = s_at[t], q1 = min(s_at[t + 1], ni); q < q1; q++) sa += s_pa[q];
+      if (t >= 1)
+        for (uint32_t q = s_at[t - 1], q1 = min(s_at[t], ni); q < q1; q++) sc += s_pc[q];
+      float sg = 0.f;
+      sg += sa;
+      sg += sc;
+      const float grad = sg * scale;
+      m = __builtin_fmaf(st.b1, m, (1.f - st.b1) * grad);
+      s2 = __builtin_fmaf(st.b2, s2, (1.f - st.b2) * grad * grad);
+      s_y[t] -= st.lr * (m / st.bc1[step]) / (sqrtf(s2 / st.bc2[step]) + 1e-6f);
+    }
+    __syncthreads();
+  }
+  const uint64_t g = gl + t;
+  if (t < nl && g >= o0 && g < o1) {
+    ts.Ko[g] = Knot{kj, s_y[t]};
+    ts.m1o[g] = m;
+    ts.m2o[g] = s2;
+  }
+}
+
 // the gradient alone (for checks), one model
 __global__ void k_lsel_grad(const TrainVec* __restrict__ tv, TrainBufs tb, float* __restrict__ grad) {
   const uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -902,6 +1063,23 @@ static int train_grad(wtg_ctx* ctx, const TrainVec* d_tv, const TrainBufs& tb, u
   return WTG_OK;
 }
 
+// Each model's blocks of k_lsel_train: as many knots as have, on average, 900 items
+// between them (a thread each, and some to spare), and not more than LDS holds the
+// most items of (no interval is longer than max_gap).  None (a launch for each half
+// of a step) where that leaves a block fewer than 16 knots of its own (the split of a step costs 20 us of latency).
+static uint64_t train_blocks(const wtg_lsel_params& P, const std::vector<TrainVec>& tv, std::vector<TrainBlocks>& out) {
+  const uint64_t most = P.max_gap / P.train_stride / LSEL_ITEM + 3;
+  uint64_t n = 0;
+  for (const TrainVec& v : tv) {
+    const uint64_t items = v.nknots + v.ns / LSEL_ITEM;
+    const uint64_t knots = std::min<uint64_t>({LSEL_TKNOTS, 900ull * v.nknots / items, LSEL_TITEMS / most});
+    if (knots < 2 * LSEL_STEPS + 16) return 0;
+    out.push_back(TrainBlocks{n, (uint32_t)knots});
+    n += wtg_ceil_div(v.nknots, knots - 2 * LSEL_STEPS);
+  }
+  return n;
+}
+
 // knot placement, lookup tables, training and the eps check for the vectors
 // in `act` (all memory goes to ls->blocks, released by the caller on failure)
 static int lsel_models(wtg_ctx* ctx, wtg_lsel* ls, const wtg_lsel_params& P, const uint64_t* nbits,
@@ -1069,7 +1247,36 @@ static int lsel_models(wtg_ctx* ctx, wtg_lsel* ls, const wtg_lsel_params& P, con
   // 5. Adam on every knot of every model
   const float b1 = 0.9f, b2 = 0.999f;
   float p1 = 1.f, p2 = 1.f;
-  for (uint32_t e = 0; e < P.epochs; e++) {
+  std::vector<TrainBlocks> blocks;
+  const uint64_t nblocks = P.epochs ? train_blocks(P, tv, blocks) : 0;
+  if (nblocks) {
+    Knot* d_K2 = nullptr;
+    TrainBlocks* d_blocks = nullptr;
+    WTG_TRY(alloc_block(ctx, ls, nk_total * sizeof(Knot) + 256, (void**)&d_K2));
+    WTG_TRY(alloc_block(ctx, ls, na * sizeof(TrainBlocks), (void**)&d_blocks));
+    WTG_CHECK_HIP(hipMemcpyAsync(d_blocks, blocks.data(), na * sizeof(TrainBlocks), hipMemcpyHostToDevice, ctx->stream));
+    const uint32_t nl = (uint32_t)wtg_ceil_div(P.epochs, LSEL_STEPS);
+    // from the placed knots, the last launch into d_K; gl and gr, of no use between the losses, as second moments
+    const Knot* from = d_K0;
+    float *fm[2] = {m1, m2}, *om[2] = {gl, gr};
+    for (uint32_t l = 0; l < nl; l++) {
+      TrainSteps st{P.lr, b1, b2, {}, {}, 0};
+      for (uint32_t e = l * LSEL_STEPS; e < P.epochs && st.n < LSEL_STEPS; e++, st.n++) {
+        p1 *= b1;
+        p2 *= b2;
+        st.bc1[st.n] = 1.f - p1;
+        st.bc2[st.n] = 1.f - p2;
+      }
+      Knot* to = (nl - l) & 1 ? d_K : d_K2;
+      WTG_LAUNCH(ctx, "lsel_train", k_lsel_train, dim3((unsigned)nblocks), dim3(LSEL_TT), 0, d_tv, d_blocks, na, items,
+                 TrainState{from, fm[0], fm[1], to, om[0], om[1]}, st);
+      WTG_LAUNCH_CHECK();
+      from = to;
+      std::swap(fm[0], om[0]);
+      std::swap(fm[1], om[1]);
+    }
+  }
+  for (uint32_t e = 0; e < (nblocks ? 0 : P.epochs); e++) {
     WTG_LAUNCH(ctx, "lsel_fwd_bwd", k_lsel_items, dim3((unsigned)wtg_ceil_div(items.cap, 256)), dim3(256), 0, d_tv,
                tb, nk_total, items);
     WTG_LAUNCH_CHECK();
