@@ -268,10 +268,12 @@ __device__ __forceinline__ U wave_incl_scan(U v) {
 }
 // running max of a and min of b over the lanes (no NaNs, no -0: max and min
 // are exact and equal the sequential walk's); a lane with no source in a step
-// reads its own value
+// reads its own value (the instructions themselves: __builtin_fmax quiets its
+// operands first)
 __device__ __forceinline__ void wave_incl_maxmin_f64_dpp(double& a, double& b) {
 #define WTG_STEP(C, R) { const double ta = dpp_f64<C, R>(a, a), tb = dpp_f64<C, R>(b, b); \
-    a = __builtin_fmax(ta, a); b = __builtin_fmin(tb, b); }
+    asm("v_max_f64 %0, %1, %2" : "=v"(a) : "v"(ta), "v"(a)); \
+    asm("v_min_f64 %0, %1, %2" : "=v"(b) : "v"(tb), "v"(b)); }
   WTG_DPP_SCAN_STEPS(WTG_STEP)
 #undef WTG_STEP
 }

@@ -250,11 +250,6 @@ __device__ __forceinline__ double readlane_f64(double v, int l) {
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
   return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
-__device__ __forceinline__ uint64_t shfl_u64(uint64_t v, int l) {
-  const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)v, l);
-  const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(v >> 32), l);
-  return ((uint64_t)hi << 32) | lo;
-}
 
 // Greedy knot placement over one chunk of arguments [j0, j1], one wave per
 // chunk.  The sequential walk it reproduces: from the last knot (x0, y0) keep
@@ -271,15 +266,22 @@ __device__ __forceinline__ uint64_t shfl_u64(uint64_t v, int l) {
 // and the lanes from that one on are redone from the new knot.  Same double
 // arithmetic as the walk (no contraction), so the same knots.  The scans are
 // DPP moves (no LDS round trips).
+// Bound by vector instructions (four fifths of its time): 62 M ones of 16
+// run-structured vectors take 539 us (615 with a 64-bit select, 64-bit conversions and
+// quieting maxima).
 // Count pass (off == nullptr): cnt[flat] = the chunk's knots, and the first
-// LSEL_CAP of them to scratch[flat * LSEL_CAP ..].  Emit pass: a chunk with at
-// most LSEL_CAP knots copies them from scratch; a larger one walks again and
-// writes knots[off[flat] ..] (a different count sets *err).
-constexpr uint32_t LSEL_CAP = 64;
+// `keep` of them to scratch[flat * keep ..].  Emit pass: a chunk with at most
+// `keep` knots copies them from scratch; a larger one walks again and writes
+// knots[off[flat] ..] (a different count sets *err).  The host keeps 512, in
+// the context's workspace (64 where that is over 256 MiB: an allocation of that size
+// for each build costs more than the second walk): with 64 the emit pass of the same vectors took
+// 299 us for the few chunks that have more, with 512 7.
+constexpr uint32_t LSEL_KEEP = 512, LSEL_KEEP_MIN = 64;
+constexpr uint64_t LSEL_KEEP_BYTES = 256ull << 20;
 __global__ __launch_bounds__(256) void k_lsel_place(const PlaceVec* __restrict__ pv, const uint64_t* __restrict__ cbase,
                                                     uint32_t nv, uint64_t nflat, uint32_t gap_log, double tol,
                                                     uint32_t* __restrict__ cnt, const uint32_t* __restrict__ off,
-                                                    Knot* __restrict__ knots, Knot* __restrict__ scratch,
+                                                    Knot* __restrict__ knots, Knot* __restrict__ scratch, uint32_t keep,
                                                     uint32_t* __restrict__ err) {
 #pragma clang fp contract(off)
   const uint32_t lane = (uint32_t)lane_id();
@@ -293,12 +295,12 @@ __global__ __launch_bounds__(256) void k_lsel_place(const PlaceVec* __restrict__
   const uint64_t j0 = (c << gap_log) + 1;
   const uint64_t j1 = ((c + 1) << gap_log) < v.ones ? ((c + 1) << gap_log) : v.ones;
   const uint32_t lim = off ? off[flat + 1] - off[flat] : 0u;
-  if (off && lim <= LSEL_CAP) {  // the count pass kept them
-    for (uint32_t i = lane; i < lim; i += 64) knots[off[flat] + i] = scratch[flat * LSEL_CAP + i];
+  if (off && lim <= keep) {  // the count pass kept them
+    for (uint32_t i = lane; i < lim; i += 64) knots[off[flat] + i] = scratch[flat * keep + i];
     return;
   }
-  Knot* out = off ? knots + off[flat] : scratch + flat * LSEL_CAP;
-  const uint32_t cap = off ? lim : LSEL_CAP;
+  Knot* out = off ? knots + off[flat] : scratch + flat * keep;
+  const uint32_t cap = off ? lim : keep;
   uint32_t n = 0;  // wave-uniform
   auto put = [&](uint64_t jj, double val) {
     if (n < cap && lane == 0) out[n] = Knot{(uint32_t)jj, (float)(val - lsel_line(v.alpha, v.beta, (double)jj))};
@@ -342,11 +344,13 @@ __global__ __launch_bounds__(256) void k_lsel_place(const PlaceVec* __restrict__
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       const int32_t kw = wave_incl_max_dpp(first[lane]);
       const uint32_t ks = kw < 0 ? 0u : (uint32_t)kw;
-      const uint32_t ex_k = (uint32_t)__shfl((int)incl, (int)ks) - (uint32_t)__shfl((int)pc, (int)ks);
-      const uint64_t wk = shfl_u64(wd, (int)ks);
-      const uint32_t bit = lane < m ? select_in_word(wk, lane - ex_k) : 0u;
-      const double P = (double)(((w + ks) << 6) + bit);
-      const double jj = (double)(jn + lane);
+      const uint32_t ex_k = (uint32_t)__shfl((int)(incl - pc), (int)ks);
+      const uint32_t wk0 = (uint32_t)__shfl((int)(uint32_t)wd, (int)ks);
+      const uint32_t wk1 = (uint32_t)__shfl((int)(uint32_t)(wd >> 32), (int)ks);
+      const uint32_t bit = lane < m ? select_halves(wk0, wk1, lane - ex_k) : 0u;
+      // (whole numbers below 2^53: the sums are exact)
+      const double P = (double)(w << 6) + (double)((ks << 6) + bit);
+      const double jj = (double)jn + (double)lane;
       // the cone over lanes [start, m)
       uint32_t start = 0;
       for (uint32_t it = 0;; it++) {
@@ -391,7 +395,8 @@ __global__ __launch_bounds__(256) void k_lsel_place(const PlaceVec* __restrict__
       // consume the window's first m ones
       const uint32_t kl = (uint32_t)__builtin_amdgcn_readlane((int)ks, (int)(m - 1));
       const uint32_t bl = (uint32_t)__builtin_amdgcn_readlane((int)bit, (int)(m - 1));
-      const uint64_t wlast = shfl_u64(wd, (int)kl);
+      const uint64_t wlast = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(wd >> 32), (int)kl) << 32 |
+                             (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)wd, (int)kl);
       w += kl;
       x = wlast & ~((2ull << bl) - 1);
       jn += m;
@@ -1108,11 +1113,18 @@ static int lsel_models(wtg_ctx* ctx, wtg_lsel* ls, const wtg_lsel_params& P, con
   WTG_CHECK_HIP(hipMemcpyAsync(d_pv, pv.data(), na * sizeof(PlaceVec), hipMemcpyHostToDevice, ctx->stream));
   WTG_CHECK_HIP(hipMemcpyAsync(d_cbase, cbase.data(), (na + 1) * 8, hipMemcpyHostToDevice, ctx->stream));
   WTG_TRY(wtg_fill_u64(ctx, d_err, 1, 0));
-  Knot* d_scr = nullptr;  // the count pass keeps each chunk's first LSEL_CAP knots
-  WTG_TRY(wtg_malloc(ctx, (void**)&d_scr, nflat * LSEL_CAP * sizeof(Knot) + 256));
+  Knot* d_scr = nullptr;  // the count pass keeps each chunk's first knots
+  const bool in_ws = nflat * LSEL_KEEP * sizeof(Knot) <= LSEL_KEEP_BYTES;  // (the plain build is done with it)
+  const uint32_t keep = in_ws ? LSEL_KEEP : LSEL_KEEP_MIN;
+  if (in_ws) {
+    WTG_TRY(wtg_ws_reserve(ctx, nflat * keep * sizeof(Knot)));
+    d_scr = (Knot*)ctx->ws;
+  } else {
+    WTG_TRY(wtg_malloc(ctx, (void**)&d_scr, nflat * keep * sizeof(Knot) + 256));
+  }
   const unsigned gp = (unsigned)wtg_ceil_div(nflat, 4);  // a wave per chunk
   WTG_LAUNCH(ctx, "lsel_place", k_lsel_place, dim3(gp), dim3(256), 0, d_pv, d_cbase, na, nflat, gap_log,
-             (double)P.tol, d_cnt, (const uint32_t*)nullptr, (Knot*)nullptr, d_scr, d_err);
+             (double)P.tol, d_cnt, (const uint32_t*)nullptr, (Knot*)nullptr, d_scr, keep, d_err);
   WTG_LAUNCH_CHECK();
   std::vector<uint32_t> off(nflat + 1, 0);
   WTG_TRY(sync_copy(ctx, off.data(), d_cnt, nflat * 4, hipMemcpyDeviceToHost));
@@ -1138,11 +1150,11 @@ static int lsel_models(wtg_ctx* ctx, wtg_lsel* ls, const wtg_lsel_params& P, con
   WTG_TRY(alloc_block(ctx, ls, (na + 1) * 8, (void**)&d_kfirst));
   WTG_CHECK_HIP(hipMemcpyAsync(d_cnt, off.data(), (nflat + 1) * 4, hipMemcpyHostToDevice, ctx->stream));
   WTG_LAUNCH(ctx, "lsel_place", k_lsel_place, dim3(gp), dim3(256), 0, d_pv, d_cbase, na, nflat, gap_log,
-             (double)P.tol, (uint32_t*)nullptr, (const uint32_t*)d_cnt, d_K, d_scr, d_err);
+             (double)P.tol, (uint32_t*)nullptr, (const uint32_t*)d_cnt, d_K, d_scr, keep, d_err);
   WTG_LAUNCH_CHECK();
   uint32_t perr = 0;
   const int prc = sync_copy(ctx, &perr, d_err, 4, hipMemcpyDeviceToHost);
-  wtg_free(ctx, d_scr);
+  if (!in_ws) wtg_free(ctx, d_scr);
   WTG_TRY(prc);
   WTG_REQUIRE(perr == 0, "wtg_lsel_build: knot placement passes disagree");
   WTG_CHECK_HIP(hipMemcpyAsync(d_K0, d_K, nk_total * sizeof(Knot), hipMemcpyDeviceToDevice, ctx->stream));
