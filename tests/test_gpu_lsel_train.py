@@ -79,3 +79,36 @@ def test_steps_in_one_launch(wsfm, orc, ctx, epochs):
             ls.free()
         for d in dv:
             d.free()
+
+
+@pytest.mark.parametrize("sizes", [[100, 40000], [1 << 18, 1 << 16, (1 << 17) + 1, 33000] * 6, [1 << 21, 300], [5000]])
+def test_plain_structures_of_many_vectors(wsfm, ctx, sizes):
+    """Directories and select structures built together (or, of unlike sizes, one by
+    one): no ones, all ones, long superblocks, every query against the bits."""
+    rng = np.random.default_rng(len(sizes))
+    vecs = []
+    for b, nb in enumerate(sizes):
+        v = rng.random(nb) < (0.5, 0.002, 1.0, 0.0, 0.05, 0.9)[b % 6]
+        if b % 6 == 4:
+            v[nb // 4:3 * nb // 4] = False
+        vecs.append(v)
+    dv = []
+    for v in vecs:
+        w = np.zeros((v.size + 63) // 64 * 8 + 8, np.uint8)
+        p = np.packbits(v, bitorder="little")
+        w[:p.size] = p
+        dv.append(ctx.to_device(w.view(np.uint64)))
+    ls = wsfm.LearnedSelect(ctx, dv, sizes)
+    try:
+        for b, v in enumerate(vecs):
+            at = np.flatnonzero(v).astype(np.uint64)
+            assert ls.info(b)["ones"] == at.size
+            if at.size:
+                j = np.unique(np.concatenate([[1, at.size], rng.integers(1, at.size + 1, 3000)])).astype(np.uint64)
+                vv = np.full(j.size, b, np.uint32)
+                for learned in (False, True):
+                    assert np.array_equal(ls.select(vv, j, learned=learned), at[j.astype(np.int64) - 1]), (b, learned)
+    finally:
+        ls.free()
+        for d in dv:
+            d.free()

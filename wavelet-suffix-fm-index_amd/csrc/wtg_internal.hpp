@@ -158,6 +158,24 @@ int wtg_rank_select_begin(wtg_ctx* ctx, const uint64_t* d_words, uint64_t nbits,
                           char* ws_ext = nullptr, wtg_arena* ar = nullptr);
 int wtg_rank_select_count(wtg_ctx* ctx, wtg_rs_pending* pend, uint64_t ones);
 int wtg_rank_select_end(wtg_ctx* ctx, const wtg_rs_pending* pend, const uint32_t nl[2]);
+// The three halves for select1 of many vectors whose sizes are alike
+// (wtg_rank_select_many_fits), each kernel launched once for all of them; the
+// counts are where begin leaves them.  dev: 3 * nvec * WTG_RS_MANY_BYTES of device
+// memory for the argument tables, the object alive until the stream has been waited
+// for after end.
+constexpr size_t WTG_RS_MANY_BYTES = 256;
+struct wtg_rs_many {
+  std::vector<char> host[3];
+  char* dev = nullptr;
+};
+bool wtg_rank_select_many_fits(uint32_t nvec, const uint64_t* nbits);
+int wtg_rank_select_begin_many(wtg_ctx* ctx, uint32_t nvec, const uint64_t* const* d_words, const uint64_t* nbits,
+                               uint64_t* const* dirs, wtg_select* sel1, wtg_rs_pending* pend, char* ws, size_t stride,
+                               wtg_arena* ar, wtg_rs_many* many);
+int wtg_rank_select_count_many(wtg_ctx* ctx, uint32_t nvec, wtg_rs_pending* pend, const uint64_t* ones,
+                               wtg_rs_many* many);
+int wtg_rank_select_end_many(wtg_ctx* ctx, uint32_t nvec, const wtg_rs_pending* pend, const uint64_t* nl, wtg_arena* ar,
+                             wtg_rs_many* many);
 size_t wtg_rank_select_ws_bytes(uint64_t nbits);
 // arena bytes of one select structure: before the count (by nbits), after it
 // (by the number of ones), and its long pool (by the long count)

@@ -1324,7 +1324,7 @@ static int lsel_models(wtg_ctx* ctx, wtg_lsel* ls, const wtg_lsel_params& P, con
 // for the long-superblock counts (after_ones runs between the first two, its
 // device work queued ahead of the select counts)
 static int lsel_plain_build(wtg_ctx* ctx, wtg_lsel* ls, const uint64_t* const* d_words, const uint64_t* nbits,
-                            const std::function<int(const std::vector<uint64_t>&)>& after_ones) {
+                            wtg_rs_many* many, const std::function<int(const std::vector<uint64_t>&)>& after_ones) {
   const uint32_t nvec = ls->nvec;
   uint64_t dw = 0;
   size_t stride = 0, worst = 0;
@@ -1340,14 +1340,20 @@ static int lsel_plain_build(wtg_ctx* ctx, wtg_lsel* ls, const uint64_t* const* d
     dirs += wtg_align256(wtg_rank9_words(nbits[b]) * 8) / 8;
   }
   // per-vector workspaces, then the gathered counts
-  WTG_TRY(wtg_ws_reserve(ctx, stride * nvec + (size_t)nvec * 8 + 256));
+  const size_t o_many = stride * nvec + wtg_align256((size_t)nvec * 8);
+  WTG_TRY(wtg_ws_reserve(ctx, o_many + 3 * nvec * WTG_RS_MANY_BYTES));
   char* ws = (char*)ctx->ws;
   uint64_t* d_cnt = (uint64_t*)(ws + stride * nvec);
+  many->dev = ws + o_many;
+  const bool merged = wtg_rank_select_many_fits(nvec, nbits);
   wtg_arena ar[3]{};
   WTG_TRY(alloc_block(ctx, ls, worst, (void**)&ar[0].base));
   ar[0].size = worst;
   std::vector<wtg_rs_pending> pend(nvec);
-  for (uint32_t b = 0; b < nvec; b++)
+  if (merged)
+    WTG_TRY(wtg_rank_select_begin_many(ctx, nvec, d_words, nbits, ls->dirs.data(), ls->sel.data(), pend.data(), ws,
+                                       stride, &ar[0], many));
+  for (uint32_t b = 0; b < (merged ? 0 : nvec); b++)
     WTG_TRY(wtg_rank_select_begin(ctx, d_words[b], nbits[b], ls->dirs[b], true, &ls->sel[b], nullptr,
                                   WTG_ONES_DEFER, &pend[b], ws + stride * b, &ar[0]));
   std::vector<uint64_t> cnt(nvec);
@@ -1365,8 +1371,9 @@ static int lsel_plain_build(wtg_ctx* ctx, wtg_lsel* ls, const uint64_t* const* d
   ar[1].size = after;
   for (uint32_t b = 0; b < nvec; b++) {
     pend[b].ar = &ar[1];
-    WTG_TRY(wtg_rank_select_count(ctx, &pend[b], cnt[b]));
+    if (!merged) WTG_TRY(wtg_rank_select_count(ctx, &pend[b], cnt[b]));
   }
+  if (merged) WTG_TRY(wtg_rank_select_count_many(ctx, nvec, pend.data(), cnt.data(), many));
   WTG_TRY(gather(WTG_RS_NL_OFF + 4, 4));  // the select1 structure's long count
   size_t pool = 0;
   for (uint32_t b = 0; b < nvec; b++) pool += wtg_select_arena_pool((uint32_t)cnt[b]);
@@ -1374,6 +1381,7 @@ static int lsel_plain_build(wtg_ctx* ctx, wtg_lsel* ls, const uint64_t* const* d
     WTG_TRY(alloc_block(ctx, ls, pool, (void**)&ar[2].base));
     ar[2].size = pool;
   }
+  if (merged) return wtg_rank_select_end_many(ctx, nvec, pend.data(), cnt.data(), &ar[2], many);
   for (uint32_t b = 0; b < nvec; b++) {
     pend[b].ar = &ar[2];
     const uint32_t nl[2] = {0, (uint32_t)cnt[b]};
@@ -1411,6 +1419,7 @@ extern "C" int wtg_lsel_build(wtg_ctx* ctx, uint32_t nvec, const uint64_t* const
   //    of every vector, one launch; after 1, one host read of the first and
   //    last samples gives the baseline lines
   uint64_t* d_ends = nullptr;
+  wtg_rs_many many;             // (its tables, too, are upload sources)
   std::vector<LselDesc> desc0;  // the first upload's source (alive past the plain build's next host read)
   auto start_samples = [&](const std::vector<uint64_t>& ones) -> int {
     for (uint32_t b = 0; b < nvec; b++) {
@@ -1454,7 +1463,7 @@ extern "C" int wtg_lsel_build(wtg_ctx* ctx, uint32_t nvec, const uint64_t* const
   //    own workspace, so one host read brings the ones counts of all vectors
   //    and one the long counts; directories and select content sit in blocks.
   for (uint32_t b = 0; b < nvec; b++) std::memset(&ls->sel[b], 0, sizeof(wtg_select));
-  if ((rc = lsel_plain_build(ctx, ls, d_words, nbits, start_samples)) != WTG_OK) goto fail;
+  if ((rc = lsel_plain_build(ctx, ls, d_words, nbits, &many, start_samples)) != WTG_OK) goto fail;
   for (uint32_t b = 0; b < nvec; b++) {
     LselDesc& d = ls->desc[b];
     const wtg_select& s = ls->sel[b];

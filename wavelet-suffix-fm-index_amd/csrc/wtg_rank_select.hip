@@ -52,8 +52,8 @@ struct RankSelArgs {
 // ones per tile of 512 words (64 directory entries), one wave per tile,
 // lane-consecutive loads
 constexpr int RS_TILE_WORDS = 512;
-__global__ __launch_bounds__(256) void k_rank_tile_sums(const uint64_t* __restrict__ words, uint64_t W,
-                                                        uint64_t ntiles, uint32_t* __restrict__ tsum, bool aligned) {
+__device__ __forceinline__ void rank_tile_sums(const uint64_t* __restrict__ words, uint64_t W, uint64_t ntiles,
+                                               uint32_t* __restrict__ tsum, bool aligned) {
   const uint64_t waves = (uint64_t)gridDim.x * 4;
   for (uint64_t t = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6); t < ntiles; t += waves) {
     const uint64_t q0 = t * (RS_TILE_WORDS / 2) + lane_id();  // 16-byte pairs of words
@@ -71,6 +71,10 @@ __global__ __launch_bounds__(256) void k_rank_tile_sums(const uint64_t* __restri
     c = wave_sum(c);
     if (lane_id() == 0) tsum[t] = c;
   }
+}
+__global__ __launch_bounds__(256) void k_rank_tile_sums(const uint64_t* __restrict__ words, uint64_t W,
+                                                        uint64_t ntiles, uint32_t* __restrict__ tsum, bool aligned) {
+  rank_tile_sums(words, W, ntiles, tsum, aligned);
 }
 
 __device__ __forceinline__ void rs_wave_sync() {
@@ -123,7 +127,7 @@ __device__ __forceinline__ uint32_t rs_at(uint32_t widx) {  // a word's place in
   return widx ^ ((widx >> 5) & 7);
 }
 
-__global__ __launch_bounds__(256) void k_rank_entries(RankSelArgs a, uint64_t ntiles, bool write_dir, bool aligned) {
+__device__ __forceinline__ void rank_entries(const RankSelArgs& a, uint64_t ntiles, bool write_dir, bool aligned) {
   __shared__ uint64_t s_x[4][RS_TILE_WORDS];
   __shared__ uint16_t s_f[4][RS_TILE_WORDS];          // ones of the tile before each word
   __shared__ uint16_t s_slot[4][2][RS_SLOTS + 1], s_end[4][2][RS_ENDS + 1];
@@ -239,6 +243,9 @@ __global__ __launch_bounds__(256) void k_rank_entries(RankSelArgs a, uint64_t nt
     }
   }
 }
+__global__ __launch_bounds__(256) void k_rank_entries(RankSelArgs a, uint64_t ntiles, bool write_dir, bool aligned) {
+  rank_entries(a, ntiles, write_dir, aligned);
+}
 
 // ----------------------------------------------------- select assembly
 struct AsmArgs {
@@ -259,7 +266,7 @@ __device__ __forceinline__ uint32_t hi_dev(uint64_t x) { return x ? 63 - __clzll
 // thread per 4 mini slots (one 16-byte load and store): rebase the samples of
 // mini superblocks to their start, clear those of long superblocks; the first
 // thread of a superblock writes its widths and long flag
-__global__ __launch_bounds__(256) void k_select_assemble(AsmArgs a) {
+__device__ __forceinline__ void select_assemble(const AsmArgs& a) {
   const uint64_t idx4 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx4 >= a.sb * 16) return;
   const uint64_t k = idx4 >> 4;  // superblock (64 slots = 16 threads)
@@ -281,12 +288,13 @@ __global__ __launch_bounds__(256) void k_select_assemble(AsmArgs a) {
     a.long_flag[k] = lng ? 1u : 0u;
   }
 }
+__global__ __launch_bounds__(256) void k_select_assemble(AsmArgs a) { select_assemble(a); }
 
 // also lists the long superblocks (list[ex[k]] = k) and copies their count
 // ex[sb] to *nl_out
-__global__ void k_long_index(const uint32_t* __restrict__ flag, const uint32_t* __restrict__ ex,
-                             int64_t* __restrict__ li, uint64_t sb, uint32_t* __restrict__ list,
-                             uint32_t* __restrict__ nl_out) {
+__device__ __forceinline__ void long_index(const uint32_t* __restrict__ flag, const uint32_t* __restrict__ ex,
+                                           int64_t* __restrict__ li, uint64_t sb, uint32_t* __restrict__ list,
+                                           uint32_t* __restrict__ nl_out) {
   const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k < sb) {
     li[k] = flag[k] ? (int64_t)ex[k] : -1;
@@ -294,17 +302,20 @@ __global__ void k_long_index(const uint32_t* __restrict__ flag, const uint32_t* 
   }
   if (k == 0) *nl_out = ex[sb];
 }
+__global__ void k_long_index(const uint32_t* __restrict__ flag, const uint32_t* __restrict__ ex,
+                             int64_t* __restrict__ li, uint64_t sb, uint32_t* __restrict__ list,
+                             uint32_t* __restrict__ nl_out) {
+  long_index(flag, ex, li, sb, list, nl_out);
+}
 
 // one block of LF_THREADS per long superblock (list[blockIdx.x]): enumerate the
 // arguments in [a, e], one word per thread per round (a long superblock can
 // hold dense stretches, and each thread walks its word's set bits serially)
 constexpr int LF_THREADS = 1024;
-__global__ __launch_bounds__(LF_THREADS) void k_long_fill(const uint64_t* __restrict__ words, uint64_t nbits,
-                                                          int bit, const uint64_t* __restrict__ sbstart,
-                                                          const uint64_t* __restrict__ sbend,
-                                                          const unsigned long long* last,
-                                                          const uint32_t* __restrict__ list, uint64_t sb,
-                                                          uint64_t* __restrict__ pool) {
+__device__ __forceinline__ void long_fill(const uint64_t* __restrict__ words, uint64_t nbits, int bit,
+                                          const uint64_t* __restrict__ sbstart, const uint64_t* __restrict__ sbend,
+                                          const unsigned long long* last, const uint32_t* __restrict__ list,
+                                          uint64_t sb, uint64_t* __restrict__ pool) {
   constexpr int NWV = LF_THREADS / 64;
   __shared__ uint32_t s_wave[NWV];
   const uint64_t k = list[blockIdx.x];
@@ -340,6 +351,95 @@ __global__ __launch_bounds__(LF_THREADS) void k_long_fill(const uint64_t* __rest
     }
     run += tt;
   }
+}
+__global__ __launch_bounds__(LF_THREADS) void k_long_fill(const uint64_t* __restrict__ words, uint64_t nbits,
+                                                          int bit, const uint64_t* __restrict__ sbstart,
+                                                          const uint64_t* __restrict__ sbend,
+                                                          const unsigned long long* last,
+                                                          const uint32_t* __restrict__ list, uint64_t sb,
+                                                          uint64_t* __restrict__ pool) {
+  long_fill(words, nbits, bit, sbstart, sbend, last, list, sb, pool);
+}
+
+// ------------------------------------------- the same for many vectors
+// Vector blockIdx.y of each launch; its arguments are in a table.  16 vectors of
+// 2^25 bits, directory and select1: 16 x 9 launches of 2 to 7 us each made building
+// and asking them 3.25 ms, these seven 2.54 (sums 14 us, scan 5, entries 22,
+// assembly, its scan and the index 5 each).
+struct RsVec {
+  RankSelArgs a;
+  uint64_t wtiles;
+  uint32_t* tsum;
+  uint64_t* tpre;
+  uint64_t* ctr;  // the counter block (32 words)
+  bool aligned;
+};
+struct RsFin {
+  AsmArgs a;
+  uint32_t *ex, *list, *nl;
+  int64_t* li;
+};
+struct RsLong {
+  const uint64_t* words;
+  uint64_t nbits;
+  const uint64_t *sbstart, *sbend;
+  const unsigned long long* last;
+  const uint32_t* list;
+  uint64_t sb;
+  uint64_t* pool;
+  uint32_t nl;
+  int bit;
+};
+__global__ __launch_bounds__(256) void k_rank_tile_sums_many(const RsVec* __restrict__ v) {
+  const RsVec r = v[blockIdx.y];
+  if (blockIdx.x == 0 && threadIdx.x < 32) r.ctr[threadIdx.x] = 0;
+  rank_tile_sums(r.a.words, r.a.W, r.wtiles, r.tsum, r.aligned);
+}
+// exclusive prefix of in[0, n) with the sum at out[n]: one block, 4096 at a time
+template <typename OUT>
+__device__ __forceinline__ void scan_by_block(const uint32_t* __restrict__ in, OUT* __restrict__ out, uint64_t n) {
+  __shared__ uint32_t s_wave[4];
+  OUT run = 0;
+  for (uint64_t at = 0; at < n; at += 4096) {
+    const uint64_t b = at + (uint64_t)threadIdx.x * 16;
+    uint32_t x[16], c = 0, total;
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+      x[k] = b + k < n ? in[b + k] : 0u;
+      c += x[k];
+    }
+    OUT o = run + block_excl_scan_u32<true>(c, s_wave, total);
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+      if (b + k < n) out[b + k] = o;
+      o += x[k];
+    }
+    run += total;
+  }
+  if (threadIdx.x == 0) out[n] = run;
+}
+__global__ __launch_bounds__(256) void k_rank_scan_many(const RsVec* __restrict__ v) {
+  scan_by_block(v[blockIdx.y].tsum, v[blockIdx.y].tpre, v[blockIdx.y].wtiles);
+}
+__global__ __launch_bounds__(256) void k_rank_entries_many(const RsVec* __restrict__ v) {
+  const RsVec r = v[blockIdx.y];
+  rank_entries(r.a, r.wtiles, true, r.aligned);
+}
+__global__ __launch_bounds__(256) void k_select_assemble_many(const RsFin* __restrict__ f) {
+  const AsmArgs a = f[blockIdx.y].a;
+  select_assemble(a);
+}
+__global__ __launch_bounds__(256) void k_select_scan_many(const RsFin* __restrict__ f) {
+  scan_by_block(f[blockIdx.y].a.long_flag, f[blockIdx.y].ex, f[blockIdx.y].a.sb);
+}
+__global__ __launch_bounds__(256) void k_long_index_many(const RsFin* __restrict__ f) {
+  const RsFin r = f[blockIdx.y];
+  long_index(r.a.long_flag, r.ex, r.li, r.a.sb, r.list, r.nl);
+}
+__global__ __launch_bounds__(LF_THREADS) void k_long_fill_many(const RsLong* __restrict__ v) {
+  const RsLong r = v[blockIdx.y];
+  if (blockIdx.x >= r.nl) return;
+  long_fill(r.words, r.nbits, r.bit, r.sbstart, r.sbend, r.last, r.list, r.sb, r.pool);
 }
 
 // ------------------------------------------------------------- queries
@@ -423,8 +523,10 @@ FinScratch fin_scratch(char* scratch, uint64_t sb) {
 // counts: sel_count stages the widths, the long flags and their scan, and
 // writes the number of long superblocks to *d_nl; sel_fill allocates and
 // fills the long pool once that number is on the host
+// (many: its arguments go there instead of to launches)
 int sel_count(wtg_ctx* ctx, uint64_t nbits, wtg_select* s, uint64_t m, const uint64_t* sbend,
-              const unsigned long long* last, char* scratch, uint32_t* d_nl, wtg_arena* ar) {
+              const unsigned long long* last, char* scratch, uint32_t* d_nl, wtg_arena* ar,
+              std::vector<RsFin>* many = nullptr) {
   const uint64_t cap = (nbits + 63) / 64 * 64;
   s->arg_cnt = m;
   s->logn = (uint32_t)wtg_hi_host(cap) + 1;
@@ -435,17 +537,21 @@ int sel_count(wtg_ctx* ctx, uint64_t nbits, wtg_select* s, uint64_t m, const uin
   WTG_TRY(sel_take(ctx, ar, (void**)&s->mini_width, sb ? sb : 1));
   WTG_TRY(sel_take(ctx, ar, (void**)&s->long_width, sb ? sb : 1));
   WTG_TRY(sel_take(ctx, ar, (void**)&s->long_index, (sb ? sb : 1) * 8));
-  if (sb == 0) return wtg_fill_bytes_zero(ctx, d_nl, 4);
+  if (sb == 0) return many ? WTG_OK : wtg_fill_bytes_zero(ctx, d_nl, 4);  // (many: cleared with the counters)
   const FinScratch f = fin_scratch(scratch, sb);
   uint32_t* flag = f.flag;
   uint32_t* ex = f.ex;
   uint64_t* st = f.st;
   uint32_t* ctr = f.ctr;
-  WTG_TRY(wtg_fill_bytes_zero(ctx, st, (char*)ctr + 256 - (char*)st));
+  if (!many) WTG_TRY(wtg_fill_bytes_zero(ctx, st, (char*)ctr + 256 - (char*)st));
   AsmArgs aa{};
   aa.mini = s->mini; aa.mini_width = s->mini_width; aa.long_width = s->long_width;
   aa.long_flag = flag; aa.sbstart = s->superblock; aa.sbend = sbend; aa.last = last;
   aa.m = m; aa.sb = sb; aa.logn4 = s->logn4;
+  if (many) {
+    many->push_back(RsFin{aa, ex, f.list, d_nl, s->long_index});
+    return WTG_OK;
+  }
   WTG_LAUNCH(ctx, "select_assemble", k_select_assemble, dim3((unsigned)wtg_ceil_div(sb * 16, 256)),
              dim3(256), 0, aa);
   WTG_LAUNCH_CHECK();
@@ -459,12 +565,17 @@ int sel_count(wtg_ctx* ctx, uint64_t nbits, wtg_select* s, uint64_t m, const uin
 }
 
 int sel_fill(wtg_ctx* ctx, const uint64_t* d_words, uint64_t nbits, wtg_select* s, uint32_t nl,
-             const uint64_t* sbend, const unsigned long long* last, const char* scratch, wtg_arena* ar) {
+             const uint64_t* sbend, const unsigned long long* last, const char* scratch, wtg_arena* ar,
+             std::vector<RsLong>* many = nullptr) {
   const uint64_t sb = s->sb;
   s->n_long = nl;
   if (sb == 0 || nl == 0) return WTG_OK;
   const FinScratch f = fin_scratch(const_cast<char*>(scratch), sb);
   WTG_TRY(sel_take(ctx, ar, (void**)&s->long_pool, (uint64_t)nl * 4096 * 8));
+  if (many) {
+    many->push_back(RsLong{d_words, nbits, s->superblock, sbend, last, f.list, sb, s->long_pool, nl, s->bit});
+    return WTG_OK;
+  }
   WTG_TRY(wtg_fill_u64(ctx, s->long_pool, (uint64_t)nl * 4096, 0));
   WTG_LAUNCH(ctx, "select_longfill", k_long_fill, dim3(nl), dim3(LF_THREADS), 0, d_words, nbits, s->bit,
              s->superblock, sbend, last, f.list, sb, s->long_pool);
@@ -631,6 +742,115 @@ int wtg_rank_select_end(wtg_ctx* ctx, const wtg_rs_pending* pend, const uint32_t
     if (pend->outs[t])
       WTG_TRY(sel_fill(ctx, pend->d_words, pend->nbits, pend->outs[t], nl[t], pend->sbend[t], pend->last[t],
                        pend->fin[t], pend->ar));
+  return WTG_OK;
+}
+
+// a host table to its place in device memory (kept in `host` until the caller's
+// next wait)
+template <typename T>
+static int many_upload(wtg_ctx* ctx, const std::vector<T>& v, std::vector<char>& host, char* dev) {
+  static_assert(sizeof(T) <= WTG_RS_MANY_BYTES, "table entries");
+  host.assign((const char*)v.data(), (const char*)(v.data() + v.size()));
+  WTG_CHECK_HIP(hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, ctx->stream));
+  return WTG_OK;
+}
+
+// Many vectors in one launch of each kernel pay where none is much larger than
+// the others (the grid is as wide as the largest for each) and one block scans a
+// vector's tiles; nbits >= 1 each.
+bool wtg_rank_select_many_fits(uint32_t nvec, const uint64_t* nbits) {
+  uint64_t sum = 0, most = 0;
+  for (uint32_t b = 0; b < nvec; b++) {
+    const uint64_t t = rs_layout(nbits[b]).wtiles;
+    sum += t;
+    most = std::max(most, t);
+  }
+  return nvec >= 2 && most <= 65536 && most * nvec <= 8 * sum;
+}
+
+int wtg_rank_select_begin_many(wtg_ctx* ctx, uint32_t nvec, const uint64_t* const* d_words, const uint64_t* nbits,
+                               uint64_t* const* dirs, wtg_select* sel1, wtg_rs_pending* pend, char* ws, size_t stride,
+                               wtg_arena* ar, wtg_rs_many* many) {
+  std::vector<RsVec> t(nvec);
+  uint64_t most = 1;
+  for (uint32_t b = 0; b < nvec; b++) {
+    const RsLayout L = rs_layout(nbits[b]);
+    char* w = ws + stride * b;
+    unsigned long long* last = (unsigned long long*)(w + L.o_ctr + 128);
+    WTG_TRY(sel_alloc_worst(ctx, nbits[b], 1, &sel1[b], ar));
+    RsVec& r = t[b];
+    r = RsVec{};
+    r.a.words = d_words[b]; r.a.nbits = nbits[b]; r.a.W = L.W; r.a.S = L.S; r.a.D = dirs[b];
+    r.a.err = ctx->d_flag;
+    r.a.tpre = (const uint64_t*)(w + L.o_tpre);
+    r.a.ones_total = (unsigned long long*)(w + L.o_ctr + WTG_RS_ONES_OFF);
+    r.a.want[1] = 1;
+    r.a.sel[1] = SelOut{sel1[b].mini, sel1[b].superblock, (uint64_t*)(w + L.o_end1), last + 1};
+    r.wtiles = L.wtiles;
+    r.tsum = (uint32_t*)(w + L.o_tsum);
+    r.tpre = (uint64_t*)(w + L.o_tpre);
+    r.ctr = (uint64_t*)(w + L.o_ctr);
+    r.aligned = ((uintptr_t)d_words[b] & 15) == 0;
+    most = std::max(most, L.wtiles);
+    wtg_rs_pending& p = pend[b];
+    p = wtg_rs_pending{};
+    p.active = true;
+    p.d_words = d_words[b];
+    p.nbits = nbits[b];
+    p.d_nl = (const uint32_t*)(w + L.o_ctr + WTG_RS_NL_OFF);
+    p.ar = ar;
+    p.want[1] = true;
+    p.outs[1] = &sel1[b];
+    p.sbend[1] = r.a.sel[1].sbend;
+    p.last[1] = last + 1;
+    p.fin[1] = w + L.o_fin + L.fin_bytes;
+  }
+  WTG_TRY(many_upload(ctx, t, many->host[0], many->dev));
+  const RsVec* d = (const RsVec*)many->dev;
+  const dim3 g((unsigned)wtg_ceil_div(most, 4), nvec);
+  WTG_LAUNCH(ctx, "rank_sums", k_rank_tile_sums_many, g, dim3(256), 0, d);
+  WTG_LAUNCH(ctx, "rank_scan", k_rank_scan_many, dim3(1, nvec), dim3(256), 0, d);
+  WTG_LAUNCH(ctx, "rank_select", k_rank_entries_many, g, dim3(256), 0, d);
+  WTG_LAUNCH_CHECK();
+  return WTG_OK;
+}
+
+int wtg_rank_select_count_many(wtg_ctx* ctx, uint32_t nvec, wtg_rs_pending* pend, const uint64_t* ones,
+                               wtg_rs_many* many) {
+  std::vector<RsFin> t;
+  for (uint32_t b = 0; b < nvec; b++)
+    WTG_TRY(sel_count(ctx, pend[b].nbits, pend[b].outs[1], ones[b], pend[b].sbend[1], pend[b].last[1],
+                      const_cast<char*>(pend[b].fin[1]), const_cast<uint32_t*>(pend[b].d_nl) + 1, pend[b].ar, &t));
+  if (t.empty()) return WTG_OK;
+  uint64_t sb = 1;
+  for (const RsFin& f : t) sb = std::max(sb, f.a.sb);
+  char* dev = many->dev + nvec * WTG_RS_MANY_BYTES;
+  WTG_TRY(many_upload(ctx, t, many->host[1], dev));
+  const RsFin* d = (const RsFin*)dev;
+  const unsigned nv = (unsigned)t.size();
+  WTG_LAUNCH(ctx, "select_assemble", k_select_assemble_many, dim3((unsigned)wtg_ceil_div(sb * 16, 256), nv), dim3(256),
+             0, d);
+  WTG_LAUNCH(ctx, "select_scan", k_select_scan_many, dim3(1, nv), dim3(256), 0, d);
+  WTG_LAUNCH(ctx, "select_longidx", k_long_index_many, dim3((unsigned)wtg_ceil_div(sb, 256), nv), dim3(256), 0, d);
+  WTG_LAUNCH_CHECK();
+  return WTG_OK;
+}
+
+int wtg_rank_select_end_many(wtg_ctx* ctx, uint32_t nvec, const wtg_rs_pending* pend, const uint64_t* nl, wtg_arena* ar,
+                             wtg_rs_many* many) {
+  std::vector<RsLong> t;
+  for (uint32_t b = 0; b < nvec; b++)
+    WTG_TRY(sel_fill(ctx, pend[b].d_words, pend[b].nbits, pend[b].outs[1], (uint32_t)nl[b], pend[b].sbend[1],
+                     pend[b].last[1], pend[b].fin[1], ar, &t));
+  if (t.empty()) return WTG_OK;
+  uint32_t most = 1;
+  for (const RsLong& r : t) most = std::max(most, r.nl);
+  WTG_TRY(wtg_fill_u64(ctx, ar->base, ar->used / 8, 0));
+  char* dev = many->dev + 2 * nvec * WTG_RS_MANY_BYTES;
+  WTG_TRY(many_upload(ctx, t, many->host[2], dev));
+  WTG_LAUNCH(ctx, "select_longfill", k_long_fill_many, dim3(most, (unsigned)t.size()), dim3(LF_THREADS), 0,
+             (const RsLong*)dev);
+  WTG_LAUNCH_CHECK();
   return WTG_OK;
 }
 
