@@ -150,14 +150,18 @@ __device__ __forceinline__ uint32_t word_leaf(const mld_u4& q, uint32_t e, uint3
 // leaf counts of the tiles, one wave per MLD_WT keys of a tile (the waves of a
 // tile share its counters).  A wave's keys are read as the aligned 16-byte
 // words that cover them, all loads in flight at once; counting needs no key
-// order, so every element of every word is counted (LDS atomics; a slot whose
-// 64 elements share one leaf adds once) and the elements of the two edge words
-// that lie outside the wave's range are taken back afterwards.  The aligned
-// words never leave the pages of the range's own bytes.
-// Trees of at most SG leaves per tile (SG > 0) count by ballots instead: per
-// slot and leaf one ballot of the lanes holding it, the counts in scalar
-// registers (a few leaves would otherwise put every lane's atomic on one of a
-// few LDS words).
+// order, so every element of every word is counted (LDS atomics; 64 words of one
+// leaf add once) and the elements of the two edge words that lie outside the
+// wave's range are taken back afterwards.  The aligned words never leave the
+// pages of the range's own bytes.  Groups of at most 64 leaves have four copies
+// of each counter, a lane's by its number, in neighbouring banks.
+// Trees of at most SG leaves per tile (SG > 0) count in registers instead, a byte
+// to a leaf, and add the lanes up at the end (a few leaves would otherwise put
+// every lane's atomic on one of a few LDS words).
+// Bound by vector instructions before (a test of every element of the words for one
+// leaf, a ballot for each leaf): bytes, 2 levels, 171 M keys 154 us, now 86; 5
+// levels, 148 M keys 112, now 80; 8 levels, 127 M keys 107, now 78 (the chain of
+// tile, segment and key loads of each wave).
 __device__ __forceinline__ void wave_sync_lds_mld() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -231,15 +235,18 @@ __global__ __launch_bounds__(256) void k_mld_count(MldArgs a) {
       cm_lo = cm_hi = hm * (B == 8 ? 0x01010101u : B == 16 ? 0x00010001u : 1u);
     }
   }
+  const uint32_t rl = a.g <= 6 ? 2 : 0;  // log2 of the copies of each counter
   if (sub == 0)
-    for (uint32_t i = lane; i < G; i += 64) s_cnt[i] = 0;
+    for (uint32_t i = lane; i < G << rl; i += 64) s_cnt[i] = 0;
   if (wl) __syncthreads();
   else wave_sync_lds_mld();
   uint32_t acc_lo = 0, acc_hi = 0;  // OR of the interior words (edge words are tested per key below)
   bool bad = false;
-  uint32_t sc[SG > 0 ? SG : 1];  // SG > 0: the counts per leaf (wave-uniform)
-#pragma unroll
-  for (uint32_t d = 0; d < (SG > 0 ? SG : 1); d++) sc[d] = 0;
+  std::conditional_t<SG == 8, uint64_t, uint32_t> sc = 0;  // SG > 0: this lane's counts, a byte to a leaf
+  static_assert(NW * E < 256, "a lane's keys in a byte");
+  char* const my_cnt = reinterpret_cast<char*>(s_cnt + (lane & ((1u << rl) - 1)));
+  const uint32_t fm = KW == 8 ? 0u : ((1u << gw) - 1u) << (tsh & 31) & (gw ? ~0u : 0u);
+  const uint32_t fmr = B == 8 ? fm * 0x01010101u : B == 16 ? fm * 0x00010001u : fm;  // the leaf field of a dword's keys
 #pragma unroll
   for (uint32_t m = 0; m < NW; m++) {
     if (m * 64 >= nw) break;  // wave-uniform
@@ -250,26 +257,45 @@ __global__ __launch_bounds__(256) void k_mld_count(MldArgs a) {
       acc_lo |= v[m].x | v[m].z;
       acc_hi |= v[m].y | v[m].w;
     }
+    if constexpr (SG > 0) {
+      if (act) {
 #pragma unroll
-    for (uint32_t e = 0; e < E; e++) {
-      const uint32_t d = word_leaf<K>(v[m], e, tsh, gw, gmask);
-      if constexpr (SG > 0) {
-#pragma unroll
-        for (uint32_t q = 0; q < SG; q++) sc[q] += popc64(wave_ballot(act && d == q));
+        for (uint32_t e = 0; e < E; e++)
+          sc += (decltype(sc))1 << (8 * word_leaf<K>(v[m], e, tsh, gw, gmask));
+      }
+    } else {
+      bool same;  // the leaf of every key of every lane's word is d0
+      const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)word_leaf<K>(v[m], 0, tsh, gw, gmask));
+      if constexpr (KW == 8) {
+        same = wave_ballot(act && (word_leaf<K>(v[m], 0, tsh, gw, gmask) != d0 ||
+                                   word_leaf<K>(v[m], 1, tsh, gw, gmask) != d0)) == 0;
       } else {
-        const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);  // lane 0 is active
-        if (wave_ballot(act && d != d0) == 0) {
-          if (lane == 0) atomicAdd(&s_cnt[d0], nact);
-        } else if (act) {
-          atomicAdd(&s_cnt[d], 1u);
-        }
+        const uint32_t x0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)v[m].x);  // lane 0 is active
+        const uint32_t df = ((v[m].x ^ x0) | (v[m].y ^ x0) | (v[m].z ^ x0) | (v[m].w ^ x0)) & fmr;
+        const uint32_t turned = (x0 >> (B & 31)) | (x0 << ((32 - B) & 31));
+        same = ((x0 ^ turned) & fmr) == 0 && wave_ballot(act && df != 0) == 0;
+      }
+      if (same) {
+        if (lane == 0) atomicAdd(&s_cnt[d0 << rl], nact * E);
+      } else if (act) {
+#pragma unroll
+        for (uint32_t e = 0; e < E; e++)
+          atomicAdd(reinterpret_cast<uint32_t*>(my_cnt + (word_leaf<K>(v[m], e, tsh, gw, gmask) << (rl + 2))), 1u);
       }
     }
   }
   if constexpr (SG > 0) {
 #pragma unroll
-    for (uint32_t q = 0; q < SG; q++)
-      if (lane == q && q < G && nw) atomicAdd(&s_cnt[q], sc[q]);
+    for (uint32_t h = 0; h < SG / 4; h++) {
+      const uint32_t x = (uint32_t)(sc >> (16 * h) >> (16 * h));
+      const uint32_t even = wave_incl_sum_dpp(x & 0xFF00FFu), odd = wave_incl_sum_dpp((x >> 8) & 0xFF00FFu);
+      if (lane == 63 && nw) {
+        const uint32_t c[4] = {even & 0xFFFFu, odd & 0xFFFFu, even >> 16, odd >> 16};
+#pragma unroll
+        for (uint32_t q = 0; q < 4; q++)
+          if (4 * h + q < G) atomicAdd(&s_cnt[(4 * h + q) << rl], c[q]);
+      }
+    }
   }
   // edge words: elements outside [b0, b1) were counted above; the others
   // get the per-key bad-key test
@@ -280,7 +306,7 @@ __global__ __launch_bounds__(256) void k_mld_count(MldArgs a) {
     for (uint32_t e = 0; e < E; e++) {
       const uintptr_t ea = w0 + 16 * (uintptr_t)k + e * KW;
       if (ea < b0 || ea >= b1) {
-        atomicSub(&s_cnt[word_leaf<K>(q, e, tsh, gw, gmask)], 1u);
+        atomicSub(&s_cnt[word_leaf<K>(q, e, tsh, gw, gmask) << rl], 1u);
       } else if (a.check && (word_elem<K>(q, e) >> a.chk_shift) != 0) {
         bad = true;
       }
@@ -290,7 +316,11 @@ __global__ __launch_bounds__(256) void k_mld_count(MldArgs a) {
   if (wl) __syncthreads();
   else wave_sync_lds_mld();
   if (ok)  // the waves of a tile write its counts in turns of 64 leaves
-    for (uint32_t i = lane + 64 * sub; i < G; i += 64u << wl) a.tcnt_w[(uint64_t)t * G + i] = s_cnt[i];
+    for (uint32_t i = lane + 64 * sub; i < G; i += 64u << wl) {
+      uint32_t c = 0;
+      for (uint32_t r = 0; r < 1u << rl; r++) c += s_cnt[(i << rl) + r];
+      a.tcnt_w[(uint64_t)t * G + i] = c;
+    }
 }
 
 // buf[a + b] = x in LDS.  The element index is one add-and-shift (left to
