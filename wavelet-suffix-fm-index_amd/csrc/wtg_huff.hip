@@ -52,6 +52,8 @@ struct HuffTab {
   uint8_t lvl_first[64];     // first inner node id at depth l (ids are BFS, so a level is a range)
   uint8_t lvl_bits[64];      // bits for an id offset within level l plus one "none" value
   uint8_t depth[256];        // per inner node
+  uint8_t leaf[256];         // the symbols in the order of the leaves
+  uint8_t lo[256], hi[256];  // per inner node: its first and last leaf in that order
   uint32_t n_inner, max_depth, sigma, single;  // single: the symbol when sigma == 1
 };
 }  // namespace
@@ -90,6 +92,14 @@ __device__ __forceinline__ void wave_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// 16 bytes' LDS atomics, nothing but the byte's place between them (the histogram
+// of 67 MB of 256 symbols: 78 us through the masks of bytes still to count, 40 so)
+__device__ __forceinline__ void count16(uint32_t* h, const uint4& v) {
+  const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int b = 0; b < 16; b++) atomicAdd(&h[(x[b >> 2] >> (8 * (b & 3))) & 0xFFu], 1u);
 }
 
 // byte histogram: LDS atomics into HF_HIST_REPS replicas per wave (replica =
@@ -148,6 +158,11 @@ __global__ __launch_bounds__(HF_THREADS) void k_huff_hist(const uint8_t* __restr
   if (left) setv[0] = 0x100u, setv[1] = 0x100u, setv[2] = 0x100u, setv[3] = 0x100u, setv[4] = 0x100u,
             setv[5] = 0x100u, setv[6] = 0x100u, setv[7] = 0x100u;
   static_assert(HF_HIST_SET == 8, "setv reset above lists 8 entries");
+  if (left && base0 + chunk <= n) {  // whole pieces, and no values in registers
+#pragma unroll
+    for (int pc = 0; pc < HF_HIST_PIECES; pc++) count16(h, v[pc]);
+    continue;
+  }
   uint32_t cnt[HF_HIST_SET];
 #pragma unroll
   for (int q = 0; q < HF_HIST_SET; q++) cnt[q] = 0;
@@ -323,32 +338,39 @@ __global__ __launch_bounds__(HF_THREADS) void k_huff_count_swar(SegArgs a) {
 }
 
 // pass 2 for larger trees: a byte histogram of the segment (LDS atomics into 4
-// padded replicas), then each present symbol adds its count to every inner node
-// on its path.
+// padded replicas) and its prefix in the order of the leaves, of which every inner
+// node covers a range.  67 MB of text: 47 us (83 with each symbol adding its count
+// along its path, the nodes of a path one LDS read after the other, and a test of
+// every byte for the end of the text).
 __global__ __launch_bounds__(HF_THREADS) void k_huff_count_hist(SegArgs a) {
   __shared__ uint32_t s_h[HF_THREADS / 64][4 * HF_HIST_ROW];
-  __shared__ uint32_t s_cnt[HF_THREADS / 64][256];
-  __shared__ uint64_t s_code[256];
-  __shared__ uint16_t s_child[256][2];
-  __shared__ uint8_t s_len[256];
-  for (int k = threadIdx.x; k < 256; k += HF_THREADS) {
-    s_code[k] = a.tab->code[k];
-    s_len[k] = a.tab->len[k];
-    s_child[k][0] = a.tab->child[k][0];
-    s_child[k][1] = a.tab->child[k][1];
-  }
-  __syncthreads();
+  __shared__ uint32_t s_pre[HF_THREADS / 64][257];  // the segment's bytes before each leaf
   const int lane = lane_id(), w = threadIdx.x >> 6;
+  const uint32_t sigma = a.tab->sigma;
+  uint32_t leaf[4], lo[4], hi[4];  // of leaves 4 lane + q, and of nodes 64 q + lane
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    leaf[q] = a.tab->leaf[4 * lane + q];
+    lo[q] = a.tab->lo[64 * q + lane];
+    hi[q] = a.tab->hi[64 * q + lane] + 1;
+  }
   uint32_t* hw = s_h[w];
   uint32_t* h = hw + (lane & 3) * HF_HIST_ROW;
-  uint32_t* cnt = s_cnt[w];
+  uint32_t* pre = s_pre[w];
   const uint64_t waves = (uint64_t)gridDim.x * (HF_THREADS / 64);
   for (uint64_t s = (uint64_t)blockIdx.x * (HF_THREADS / 64) + w; s < a.nseg; s += waves) {
     for (int k = lane; k < 4 * HF_HIST_ROW; k += 64) hw[k] = 0;
-#pragma unroll
-    for (int q = 0; q < 4; q++) cnt[64 * q + lane] = 0;
     wave_sync_lds();
-    for (uint32_t off = 0; off < a.S; off += HF_PIECE) {
+    uint32_t off = 0;
+    // four whole pieces at a time, their loads in flight together
+    for (; off + 4 * HF_PIECE <= a.S && s * a.S + off + 4 * HF_PIECE <= a.n; off += 4 * HF_PIECE) {
+      uint4 v[4];
+#pragma unroll
+      for (int p = 0; p < 4; p++) v[p] = load16(a.text, a.n, s * a.S + off + p * HF_PIECE + (uint64_t)lane * 16, a.aligned);
+#pragma unroll
+      for (int p = 0; p < 4; p++) count16(h, v[p]);
+    }
+    for (; off < a.S; off += HF_PIECE) {
       const uint64_t base = s * a.S + off + (uint64_t)lane * 16;
       if (base - (uint64_t)lane * 16 >= a.n) break;
       const uint4 wv = load16(a.text, a.n, base, a.aligned);
@@ -360,23 +382,26 @@ __global__ __launch_bounds__(HF_THREADS) void k_huff_count_hist(SegArgs a) {
       }
     }
     wave_sync_lds();
+    uint32_t t[4];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-      const uint32_t c = (uint32_t)(64 * q + lane);
-      const uint32_t t = hw[c] + hw[HF_HIST_ROW + c] + hw[2 * HF_HIST_ROW + c] + hw[3 * HF_HIST_ROW + c];
-      const uint32_t len = t ? (uint32_t)s_len[c] : 0u;
-      const uint64_t code = s_code[c];
-      uint32_t node = 0;
-      for (uint32_t l = 0; l < len; l++) {
-        atomicAdd(&cnt[node], t);
-        node = s_child[node][(code >> l) & 1];
-      }
+      const uint32_t c = leaf[q];
+      t[q] = (uint32_t)(4 * lane + q) < sigma
+                 ? hw[c] + hw[HF_HIST_ROW + c] + hw[2 * HF_HIST_ROW + c] + hw[3 * HF_HIST_ROW + c] : 0u;
     }
+    const uint32_t sum = t[0] + t[1] + t[2] + t[3], incl = wave_incl_sum_dpp(sum);
+    uint32_t run = incl - sum;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      pre[4 * lane + q] = run;
+      run += t[q];
+    }
+    if (lane == 63) pre[256] = run;
     wave_sync_lds();
 #pragma unroll
     for (int q = 0; q < 4; q++) {
       const uint32_t v = (uint32_t)(64 * q + lane);
-      if (v < a.n_inner) a.cnt[(uint64_t)v * a.nseg + s] = cnt[v];
+      if (v < a.n_inner) a.cnt[(uint64_t)v * a.nseg + s] = pre[hi[q]] - pre[lo[q]];
     }
     wave_sync_lds();
   }
@@ -1205,6 +1230,22 @@ void build_shape(const uint64_t* cnt, uint64_t n, wtg_huff_shape& S, HuffTab& T)
       while ((1u << kb) - 1 < cnt) kb++;
       T.lvl_first[l] = bfs ? (uint8_t)first : 0;
       T.lvl_bits[l] = bfs ? (uint8_t)kb : (uint8_t)full;
+    }
+  }
+  // the leaves below each node, from the last node up, then their places from the root down
+  {
+    std::vector<int> below(order.size(), 1), at(order.size(), 0);
+    for (size_t k = order.size(); k-- > 0;)
+      if (inner_of[k] >= 0) below[k] = below[S.child[k][0]] + below[S.child[k][1]];
+    for (size_t k = 0; k < order.size(); k++) {
+      if (inner_of[k] < 0) {
+        T.leaf[at[k]] = (uint8_t)S.sym[k];
+        continue;
+      }
+      at[S.child[k][0]] = at[k];
+      at[S.child[k][1]] = at[k] + below[S.child[k][0]];
+      T.lo[inner_of[k]] = (uint8_t)at[k];
+      T.hi[inner_of[k]] = (uint8_t)(at[k] + below[k] - 1);
     }
   }
   uint32_t maxd = 0;
