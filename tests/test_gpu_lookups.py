@@ -103,3 +103,23 @@ def test_ordered_answers_over_their_queries(ctx, large):
     assert np.array_equal(d[1].get(), ranks)
     for x in d:
         x.free()
+
+
+@pytest.mark.parametrize("m", [12, 13, 32])
+def test_ordered_patterns(ctx, m):
+    """A batch of patterns in order gives the counts of the same patterns in small
+    batches, as they came (2^26 code bits, 16 symbols, some patterns of absent ones)."""
+    rng = np.random.default_rng(m)
+    n = (1 << 24) + 1
+    wt = ctx.huff_build(ctx.to_device((rng.integers(0, 16, n) * 3).astype(np.uint8)))
+    try:
+        for nq in (1 << 19, (1 << 20) + 5):
+            pats = (rng.integers(0, 16, (nq, m)) * 3).astype(np.uint8)
+            pats[:, :m - 5] = pats[rng.integers(0, 50, nq), :m - 5]  # some counts stay above 0
+            pats[::7, -1] = 1
+            pats[5::7, 0] = 255
+            got = wt.fm_count(pats)
+            step = 1 << 18
+            assert np.array_equal(got, np.concatenate([wt.fm_count(pats[at:at + step]) for at in range(0, nq, step)]))
+    finally:
+        wt.free()

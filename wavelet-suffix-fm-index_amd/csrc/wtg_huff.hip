@@ -31,6 +31,7 @@
 //                    words OR-ed).
 // Then rank9 + select1 + select0 over the bits, and the per-node rank bases.
 #include "wtg_internal.hpp"
+#include "wtg_order.hpp"
 #include <cstring>
 #include <queue>
 #include <vector>
@@ -1058,14 +1059,18 @@ __global__ __launch_bounds__(256) void k_huff_select(HQ h, const uint64_t* __res
 // (NP t .. NP t + NP-1) interleave their searches step by step.
 template <int NP>
 __global__ __launch_bounds__(256) void k_fm_count(HQ h, const uint8_t* __restrict__ pats, uint32_t m,
-                                                  uint64_t npat, uint64_t* __restrict__ out) {
+                                                  uint64_t npat, uint64_t* __restrict__ out,
+                                                  const uint32_t* __restrict__ order) {
   __shared__ QLds Q;
   __shared__ uint64_t s_C[257];
   load_q(Q, h.tab);
   for (int k = threadIdx.x; k < 257; k += blockDim.x) s_C[k] = h.tab->C[k];
   __syncthreads();
   const uint64_t ngroup = (npat + NP - 1) / NP;
-  for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < ngroup;
+  // (an ordered batch: consecutive blocks are on different XCDs, each takes an eighth)
+  const uint32_t blk = order && gridDim.x % QO_XCDS == 0
+                           ? blockIdx.x % QO_XCDS * (gridDim.x / QO_XCDS) + blockIdx.x / QO_XCDS : blockIdx.x;
+  for (uint64_t t = (uint64_t)blk * blockDim.x + threadIdx.x; t < ngroup;
        t += (uint64_t)gridDim.x * blockDim.x) {
     const uint8_t* P[NP];
     uint64_t sp[NP], ep[NP];
@@ -1130,13 +1135,46 @@ __global__ __launch_bounds__(256) void k_fm_count(HQ h, const uint8_t* __restric
     }
 #pragma unroll
     for (int p = 0; p < NP; p++)
-      if (NP * t + p < npat) out[NP * t + p] = ep[p] > sp[p] ? ep[p] - sp[p] : 0;
+      if (NP * t + p < npat) out[order ? order[NP * t + p] : NP * t + p] = ep[p] > sp[p] ? ep[p] - sp[p] : 0;
   }
 }
 // patterns per lane: with the loads of a level issued before their use, one
 // pattern per lane (full occupancy) measured fastest on 10^6 length-20 DNA
 // patterns: 0.66 ms, against 0.75 ms for two and 0.78 ms for four
 #define FM_NP 1
+
+// A large batch in the order of the patterns' last eight bytes, the last one first:
+// those are the first steps, and patterns that share them walk the same part of
+// the bits, which the later steps spread out again.
+__global__ __launch_bounds__(256) void k_fm_keys(const uint8_t* __restrict__ pats, uint32_t m, uint64_t npat,
+                                                 uint64_t* __restrict__ key) {
+  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= npat) return;
+  const uint8_t* p = pats + t * m + m - 8;  // m >= 8
+  uint64_t k = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < 8; i++) k |= (uint64_t)p[i] << (8 * i);
+  key[t] = k;
+}
+// the rows in order, four bytes a thread
+__global__ __launch_bounds__(256) void k_fm_rows(const uint8_t* __restrict__ pats, uint32_t m, uint32_t bytes,
+                                                 const uint32_t* __restrict__ order, uint8_t* __restrict__ rows) {
+  const uint32_t f = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  if (f >= bytes) return;
+  uint32_t r = f / m, c = f - r * m, x = 0;
+  uint64_t at = (uint64_t)order[r] * m;
+#pragma unroll
+  for (uint32_t i = 0; i < 4; i++) {
+    if (f + i < bytes) x |= (uint32_t)pats[at + c] << (8 * i);
+    if (++c == m && f + i + 1 < bytes) {
+      c = 0;
+      at = (uint64_t)order[++r] * m;
+    }
+  }
+  if (f + 4 <= bytes) *reinterpret_cast<uint32_t*>(rows + f) = x;
+  else
+    for (uint32_t i = 0; f + i < bytes; i++) rows[f + i] = (uint8_t)(x >> (8 * i));
+}
 
 // --------------------------------------------------------------- host side
 // Huffman shape (wt_huff/wt_huff_par.hpp:92-117) and the BFS layout of the
@@ -1577,14 +1615,49 @@ extern "C" int wtg_huff_select_batch(wtg_ctx* ctx, const wtg_huff* wt, const uin
   WTG_LAUNCH_CHECK();
   return wtg_finish(ctx);
 }
+// Whether ordering a batch of patterns pays: index bits too many for an XCD's L2,
+// patterns enough for the five passes before the search (~70 us with the rows), and
+// not so long that the steps past the ordered bytes outweigh the first.  DNA, 20-byte
+// patterns, us as they came -> ordered:
+//   2^25 symbols (2^26.2 bits): 2^18 167 -> 172, 2^19 302 -> 280, 2^20 558 -> 494
+//   (of which the search 431; all eight bytes sorted, not 256 parts of them: 357);
+//   12 bytes, 2^20: 336 -> 299; 32 bytes: 907 -> 893; 8 bytes: 203 -> 203
+//   2^24 symbols, 2^20: 520 -> 481 (32 bytes 858 -> 857); 2^22 symbols, 2^20: 431 -> 446
+static bool fm_order_pays(const wtg_huff* wt, uint32_t m, uint64_t npat) {
+  return wt->shape.bv_size >= 1ull << 26 && npat >= 1ull << 19 && m >= 12 && m <= 32;
+}
+
 extern "C" int wtg_fm_count_batch(wtg_ctx* ctx, const wtg_huff* wt, const uint8_t* d_pats, uint32_t m,
                                   uint64_t npat, uint64_t* d_out) {
   WTG_TRY(hq_check(ctx, wt, npat, d_pats, d_out));
   WTG_REQUIRE(m >= 1, "pattern length 0");
   if (!npat) return WTG_OK;
   WTG_TRY(wtg_set_device(ctx));
-  WTG_LAUNCH(ctx, "fm_count", k_fm_count<FM_NP>, dim3(query_grid((npat + FM_NP - 1) / FM_NP)), dim3(256), 0,
-             make_hq(wt), d_pats, m, npat, d_out);
+  char* scratch = fm_order_pays(wt, m, npat) ? (char*)wtg_query_scratch(ctx, QO_BYTES) : nullptr;
+  if (scratch) {
+    // keys | tables | places | rows, chunks of one size
+    const uint64_t cap = std::min<uint64_t>(QO_CHUNK, (QO_BYTES - QO_BINS * 16 - 256) / (8 + 4 + m));
+    const QOrder o = order_layout(scratch, cap, 1);
+    uint8_t* rows = (uint8_t*)(((uintptr_t)(o.q + cap) + 255) & ~(uintptr_t)255);
+    const uint64_t step = wtg_ceil_div(npat, wtg_ceil_div(npat, cap));
+    for (uint64_t at = 0; at < npat; at += step) {
+      const uint64_t n = std::min(step, npat - at);
+      const uint8_t* part = d_pats + at * m;
+      const uint32_t bytes = (uint32_t)(n * m);
+      WTG_LAUNCH(ctx, "fm_keys", k_fm_keys, dim3((unsigned)wtg_ceil_div(n, 256)), dim3(256), 0, part, m, n, o.col[0]);
+      QCols in{};
+      in.c[0] = o.col[0];
+      order_chunk<0>(ctx, in, 0, n, o);
+      WTG_LAUNCH(ctx, "fm_rows", k_fm_rows, dim3((unsigned)wtg_ceil_div(bytes, 1024)), dim3(256), 0, part, m, bytes,
+                 (const uint32_t*)o.q, rows);
+      WTG_LAUNCH(ctx, "fm_count", k_fm_count<FM_NP>, dim3(wtg_ceil_div(query_grid((n + FM_NP - 1) / FM_NP), QO_XCDS) * QO_XCDS),
+                 dim3(256), 0,
+                 make_hq(wt), (const uint8_t*)rows, m, n, d_out + at, (const uint32_t*)o.q);
+    }
+  } else {
+    WTG_LAUNCH(ctx, "fm_count", k_fm_count<FM_NP>, dim3(query_grid((npat + FM_NP - 1) / FM_NP)), dim3(256), 0,
+               make_hq(wt), d_pats, m, npat, d_out, (const uint32_t*)nullptr);
+  }
   WTG_LAUNCH_CHECK();
   return wtg_finish(ctx);
 }
