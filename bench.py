@@ -265,12 +265,13 @@ def bench_wt_int(pkg, args, full):
     ctx.close()
 
     step_ms = ms / args.steps
-    # the multi-level direct passes: groups of up to 8 levels; per group the
+    # the multi-level direct passes: groups of up to 8 levels, of near-equal widths; per group the
     # count kernel reads the keys, the emit kernel reads them, writes the group's
     # level bits and (all but the last group) the keys in the next order (uint32)
     groups, s_ = [], 0
     while s_ < L:
-        g_ = min(8, L - s_)
+        left = (L - 1) // 8 + 1 - len(groups)
+        g_ = (L - s_ + left - 1) // left
         groups.append(g_)
         s_ += g_
     kw = [w] + [4] * (len(groups) - 1)

@@ -29,7 +29,7 @@
 // entries give the block and, by their 9-bit word counts, the word; one word
 // read and an in-word select finish.  The answer is exact whatever the model
 // predicts: outside that window the plain select answers.  The plain sampled
-// select stays available (wtg_lsel_plain_batch) as the judge.
+// select stays available (wtg_lsel_plain_batch) to compare with.
 #include "wtg_internal.hpp"
 #include <functional>
 #include <algorithm>

@@ -19,8 +19,8 @@
 // Tiles are segment-aligned (each covers <= 2^tl keys of one level-s node),
 // so every key of a tile shares the top s bits and a tile's ranks are those of
 // its own local subtree over the next g levels.  Per group:
-//   k_mld_count   per tile, the key count of each leaf d (wave ballots find
-//                 the lanes with equal d, the group leader adds its size);
+//   k_mld_count   per tile, the key count of each leaf d (few leaves in
+//                 registers, more by LDS atomics);
 //   k_mld_scan1/2 column-wise exclusive prefix of those counts over the tiles
 //                 (carry(t, d) = P[t][d] - P[first tile of t's segment][d]);
 //   k_mld_hist    the histogram of the top s+g bits from that prefix, then
