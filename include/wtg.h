@@ -202,6 +202,10 @@ int wtg_wtint_info(const wtg_wtint* wt, uint64_t* n, uint32_t* levels, uint64_t*
                    const uint64_t** d_words, const uint64_t** d_dir);
 const wtg_select* wtg_wtint_select1(const wtg_wtint* wt);
 const wtg_select* wtg_wtint_select0(const wtg_wtint* wt);
+/* The batches of queries below answer every query in its place; large ones on a
+ * large tree are put in order first, in one 38 MB block that the context allocates
+ * at the first such batch and frees with itself (without memory for it, or while
+ * the stream is being captured, they are answered as they come). */
 /* rank(i,c) = #c in [0,i)  (wt_int_par.hpp:553-577) */
 int wtg_wtint_rank_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_i,
                          const uint64_t* d_c, uint64_t nq, uint64_t* d_out);
@@ -304,7 +308,8 @@ int wtg_bwt_from_sa(const uint8_t* text, const int64_t* sa, uint64_t n, uint8_t*
 /* Backward-search count of npat patterns of m bytes each (d_pats, pattern q at
  * q*m) over the wt_huff of a BWT (the index fm-index/par/WT.C:33-45 builds; the
  * reference stops after construction).  out[q] = occurrences of pattern q in
- * the text, exact when the text ends with a unique smallest byte. */
+ * the text, exact when the text ends with a unique smallest byte.  Large batches
+ * are put in order as the wt_int ones are, in the same block. */
 int wtg_fm_count_batch(wtg_ctx* ctx, const wtg_huff* bwt_wt, const uint8_t* d_pats,
                        uint32_t m, uint64_t npat, uint64_t* d_out);
 
