@@ -1536,11 +1536,15 @@ int mld_sparse_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint64_t*
   q.m = 1u << S;
   mld_local_launch<KO>(ctx, (unsigned)wtg_ceil_div(n, LOC_W), q);
   WTG_LAUNCH_CHECK();
-  // how many large nodes are left: read back where that is allowed (not while
-  // the stream is being captured), so that no empty round is launched
+  // how many large nodes are left: read back where the call waits in any case (in
+  // a blocking context, or for the distinct count, and not while the stream is
+  // being captured), so that no empty round is launched.  Otherwise the call only
+  // enqueues: every round, for the longest list there can be (6000011 keys, 40
+  // levels: 530 us on the stream against 410 read back with no large node, 565
+  // against 580 with half of the keys in three values).
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   WTG_CHECK_HIP(hipStreamIsCapturing(ctx->stream, &cs));
-  const bool ask = cs == hipStreamCaptureStatusNone;
+  const bool ask = (ctx->blocking || d_distinct) && cs == hipStreamCaptureStatusNone;
   uint32_t cur = 0;
   for (uint32_t s = S; s < L;) {
     uint32_t hb = cap;
