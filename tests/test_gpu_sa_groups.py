@@ -41,3 +41,16 @@ def test_mixed_sizes(wsfm, ctx):
     pick = rng.choice(60, 9000, p=(w := 1.0 / np.arange(1, 61) ** 1.3) / w.sum())
     parts = [np.concatenate([blocks[k], rng.integers(65, 91, 3).astype(np.uint8)]) for k in pick]
     check(wsfm, ctx, np.concatenate(parts))
+
+
+@pytest.mark.parametrize("copies", [63, 65, 66, 130, 257, 500, 1000])
+@pytest.mark.parametrize("repeats", [1, 3])
+def test_groups_sorted_in_a_block(wsfm, ctx, copies, repeats):
+    """Groups on either side of the size from which a block is sorted: `copies` of one
+    block of letters with few differences among them, so that the ranks h bytes on are
+    equal for many suffixes over several rounds; next to small groups."""
+    rng = np.random.default_rng(copies + repeats)
+    t = np.tile(rng.integers(65, 69, 90).astype(np.uint8), copies)
+    at = rng.choice(t.size, copies * repeats // 2 + 1, replace=False)
+    t[at] = rng.integers(65, 69, at.size)
+    check(wsfm, ctx, np.concatenate([t, rng.integers(65, 69, 3000).astype(np.uint8), np.zeros(1, np.uint8), t[:700]]))

@@ -247,6 +247,67 @@ __global__ __launch_bounds__(256) void k_sa_gather(const uint32_t* __restrict__ 
   key2[k] = i < n ? rank[i] + 1 : 0u;
 }
 
+constexpr uint32_t SA_CAP = 2048, SA_W = 1536;
+// Groups longer than this are sorted, not counted.  Copies of one text with 0.01% of
+// the bytes changed: 1000 copies of 32 KB 68.0 -> 24.3 ms (39.4 with a radix sort of the
+// list each round), 300 of 32 KB 9.6 -> 4.8 (15.5), 100 of 320 KB 17.9 -> 16.0 (39.5).
+// From 24 to 96 it makes no difference; with 160 the last one takes 19.9 ms.
+constexpr uint32_t SA_COUNT = 64;
+
+// Bitonic sort of a block's SA_CAP distinct keys, thread t's being 8 t .. 8 t + 7
+// before and after: partners less than 8 apart are in the thread's registers, less than
+// 512 apart in the wave, the three other steps go through s_x[SA_CAP].
+__device__ __forceinline__ void sa_block_sort(uint64_t (&x)[8], uint64_t* s_x) {
+  const uint32_t t = threadIdx.x;
+  const auto inside = [&](uint32_t s, bool up) {  // partners s < 8 apart
+#pragma unroll
+    for (uint32_t r = 0; r < 8; r++)
+      if ((r & s) == 0) {
+        const uint64_t a = x[r], b = x[r | s];
+        const bool keep = (a < b) == up;
+        x[r] = keep ? a : b;
+        x[r | s] = keep ? b : a;
+      }
+  };
+  const auto take = [&](uint32_t r, uint64_t y, bool lower) { x[r] = (y < x[r]) == lower ? y : x[r]; };
+#pragma unroll
+  for (uint32_t r = 0; r < 8; r += 2) {  // runs of 2, up and down in turn
+    const uint64_t a = x[r], b = x[r + 1];
+    const bool keep = (a < b) == ((r & 2) == 0);
+    x[r] = keep ? a : b;
+    x[r + 1] = keep ? b : a;
+  }
+#pragma unroll
+  for (uint32_t s = 2; s > 0; s >>= 1)  // runs of 4
+#pragma unroll
+    for (uint32_t r = 0; r < 8; r++)
+      if ((r & s) == 0) {
+        const uint64_t a = x[r], b = x[r | s];
+        const bool keep = (a < b) == ((r & 4) == 0);
+        x[r] = keep ? a : b;
+        x[r | s] = keep ? b : a;
+      }
+  for (uint32_t k = 1; k <= SA_CAP / 8; k <<= 1) {  // runs of 8 k
+    const bool up = (t & k) == 0;
+    for (uint32_t s = k >> 1; s >= 64; s >>= 1) {  // threads of another wave
+      __syncthreads();
+#pragma unroll
+      for (uint32_t r = 0; r < 8; r++) s_x[r * 256 + t] = x[r];
+      __syncthreads();
+#pragma unroll
+      for (uint32_t r = 0; r < 8; r++) take(r, s_x[r * 256 + (t ^ s)], ((t & s) == 0) == up);
+    }
+    for (uint32_t s = k >> 1 < 32 ? k >> 1 : 32; s > 0; s >>= 1) {
+#pragma unroll
+      for (uint32_t r = 0; r < 8; r++)
+        take(r, (uint64_t)__shfl_xor((unsigned long long)x[r], (int)s), ((t & s) == 0) == up);
+    }
+    inside(4, up);
+    inside(2, up);
+    inside(1, up);
+  }
+}
+
 // One round over the list: a block takes the groups that start in its window of
 // SA_W list positions and end within SA_CAP of the window's start (as long as a
 // group has at most SA_CAP - SA_W suffixes it does).  For each suffix it counts
@@ -255,20 +316,26 @@ __global__ __launch_bounds__(256) void k_sa_gather(const uint32_t* __restrict__ 
 // larger groups go to (bkey, bval) for a sort.  The blocks' outputs follow one
 // another in any order: groups stay whole, and nothing else is read from the
 // order of the list.
+// Counting reads a group's ranks once for each of its suffixes.  A block with a
+// group of more than SA_COUNT sorts its suffixes by (group, rank h bytes on) instead.
+// Six waves a SIMD: the sort's registers would leave four (20 copies of 1.6 MB 13.1
+// against 12.7 ms).
 // Groups are mostly small, and one pass over a round's list takes the place of a
 // radix sort's seven passes plus run marking, scan and compaction: 2^25 DNA bytes
 // with copied segments, all rounds after the first
 // 7.2 -> 1.0 ms.
-constexpr uint32_t SA_CAP = 2048, SA_W = 1536;
-__global__ __launch_bounds__(256) void k_sa_refine(const uint32_t* __restrict__ idx, const uint32_t* __restrict__ grp,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_sa_refine(const uint32_t* __restrict__ idx, const uint32_t* __restrict__ grp,
                                                    const uint32_t* __restrict__ key2, uint64_t m, uint64_t n,
                                                    uint32_t sh, uint32_t* __restrict__ rank, int64_t* __restrict__ sa,
                                                    uint32_t* __restrict__ idx2, uint32_t* __restrict__ grp2,
                                                    uint32_t* __restrict__ counts, uint64_t* __restrict__ bkey,
                                                    uint32_t* __restrict__ bval, uint32_t* __restrict__ err) {
   constexpr uint32_t M = SA_CAP / 256, NONE = 0xFFFFFFFFu;
-  __shared__ uint32_t s_g[SA_CAP], s_k[SA_CAP], s_i[SA_CAP];
+  __shared__ uint64_t s_x[SA_CAP];  // the list's groups and ranks, or the keys of a sort
+  __shared__ uint32_t s_i[SA_CAP];
   __shared__ uint64_t s_h[SA_CAP / 64], s_kp[SA_CAP / 64];
+  uint32_t* const s_g = reinterpret_cast<uint32_t*>(s_x);
+  uint32_t* const s_k = s_g + SA_CAP;
   __shared__ uint32_t s_base, s_bbase;
   const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (uint32_t)lane_id();
   const uint64_t lo = (uint64_t)blockIdx.x * SA_W;
@@ -321,18 +388,19 @@ __global__ __launch_bounds__(256) void k_sa_refine(const uint32_t* __restrict__ 
     pre = end > SA_CAP - SA_W || (lo > SA_W && grp[lo - SA_W - 1] == s_g[0]);
   }
   uint32_t np[M], ng[M];  // new place and rank (NONE: leaves the list, or not this block's)
-  uint32_t nbig = 0;
+  uint32_t span[M];       // its group's start | end << 16 (0: not this block's)
+  uint32_t nbig = 0, most = 0;
   uint64_t bigm[M];
   const uint64_t upto = ~0ull >> (63 - lane);
 #pragma unroll
   for (uint32_t j = 0; j < M; j++) {
     const uint32_t c = w + 4 * j, p = c * 64 + lane;
-    const bool mine = p >= f && p < e;
     const bool big = p < width && ((p < f && pre) || (f < SA_CAP && p >= f && p >= e));
     bigm[j] = wave_ballot(big);
     nbig += popc64(bigm[j]);
     np[j] = ng[j] = NONE;
-    if (mine) {
+    span[j] = 0;
+    if (p >= f && p < e) {
       uint32_t q = c;
       uint64_t h = s_h[q] & upto;
       while (h == 0) h = s_h[--q];  // (f starts a group at or before p)
@@ -342,24 +410,80 @@ __global__ __launch_bounds__(256) void k_sa_refine(const uint32_t* __restrict__ 
       h = s_h[q] & ~upto;
       while (h == 0 && ++q < SA_CAP / 64) h = s_h[q];
       if (h) E = q * 64 + (uint32_t)__builtin_ctzll(h);
-      uint32_t less = 0, eq = 0, eqb = 0;
-      for (uint32_t t = S; t < E; t++) {
-        const uint32_t kt = s_k[t];
-        less += kt < kk[j];
-        const uint32_t same = kt == kk[j];
-        eq += same;
-        eqb += t < p ? same : 0u;
-      }
-      const uint32_t r = g[j] + less;
-      if (less) rank[ii[j]] = r;
-      if (eq == 1) {
-        if (r < n) sa[r] = (int64_t)ii[j];
-        else wtg_raise(err, WTG_FLAG_SA_RANKS);  // ranks inconsistent: not expected
-      } else {
-        ng[j] = r;
-      }
-      np[j] = S + less + eqb;
+      span[j] = S | E << 16;
+      most = max(most, E - S);
     }
+  }
+  // the suffix of place j is the less-th of its group, before it eqb of eq like it
+  const auto placed = [&](uint32_t j, uint32_t less, bool alone, uint32_t place) {
+    const uint32_t r = g[j] + less;
+    if (less) rank[ii[j]] = r;
+    if (alone) {
+      if (r < n) sa[r] = (int64_t)ii[j];
+      else wtg_raise(err, WTG_FLAG_SA_RANKS);  // ranks inconsistent: not expected
+    } else {
+      ng[j] = r;
+    }
+    np[j] = place;
+  };
+  if (__syncthreads_or(most > SA_COUNT)) {
+    // sorted by group (its start), rank h bytes on, place: what lies before the
+    // block's groups and behind them stays there
+#pragma unroll
+    for (uint32_t j = 0; j < M; j++) {
+      const uint32_t p = (w + 4 * j) * 64 + lane;
+      const uint64_t S = span[j] ? span[j] & 0xFFFFu : p < f ? 0u : SA_CAP - 1;  // (no group of two starts there)
+      s_x[p] = S << 43 | (uint64_t)(span[j] ? kk[j] : p < f ? 0u : ~0u) << 11 | p;
+    }
+    __syncthreads();
+    uint64_t x[8];
+#pragma unroll
+    for (uint32_t r = 0; r < 8; r++) x[r] = s_x[threadIdx.x * 8 + r];
+    sa_block_sort(x, s_x);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < 8; r++) s_x[threadIdx.x * 8 + r] = x[r];
+    __syncthreads();
+    // starts of equal keys, and from them what each suffix's own thread has to know
+#pragma unroll
+    for (uint32_t j = 0; j < M; j++) {
+      const uint32_t c = w + 4 * j, p = c * 64 + lane;
+      const uint64_t hm = wave_ballot(p == 0 || s_x[p] >> 11 != s_x[p ? p - 1 : 0] >> 11);
+      if (lane == 0) s_kp[c] = hm;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < M; j++) {
+      const uint32_t c = w + 4 * j, p = c * 64 + lane;
+      uint32_t q = c;
+      uint64_t h = s_kp[q] & upto;
+      while (h == 0) h = s_kp[--q];  // (place 0 is a start)
+      const uint32_t head = q * 64 + 63u - (uint32_t)__builtin_clzll(h);
+      const bool ends = p + 1 >= e || (s_kp[(p + 1) >> 6] >> ((p + 1) & 63) & 1u);
+      s_i[(uint32_t)s_x[p] & (SA_CAP - 1)] = p | head << 11 | (uint32_t)(head == p && ends) << 22;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < M; j++)
+      if (span[j]) {
+        const uint32_t v = s_i[(w + 4 * j) * 64 + lane];
+        placed(j, (v >> 11 & (SA_CAP - 1)) - (span[j] & 0xFFFFu), v >> 22, v & (SA_CAP - 1));
+      }
+  } else {
+#pragma unroll
+    for (uint32_t j = 0; j < M; j++)
+      if (span[j]) {
+        const uint32_t p = (w + 4 * j) * 64 + lane, S = span[j] & 0xFFFFu, E = span[j] >> 16;
+        uint32_t less = 0, eq = 0, eqb = 0;
+        for (uint32_t t = S; t < E; t++) {
+          const uint32_t kt = s_k[t];
+          less += kt < kk[j];
+          const uint32_t same = kt == kk[j];
+          eq += same;
+          eqb += t < p ? same : 0u;
+        }
+        placed(j, less, eq == 1, S + less + eqb);
+      }
   }
   __syncthreads();
 #pragma unroll
