@@ -42,6 +42,11 @@ int wtg_device_count(int* out);
  * Contexts are independent; a context is used by one host thread at a time. */
 int wtg_ctx_create(int device, wtg_ctx** out);
 int wtg_ctx_destroy(wtg_ctx* ctx);
+/* Waits for the stream and gives back the scratch that the context keeps from call
+ * to call besides its workspace: that of wtg_suffix_array_gpu (about 50 bytes per
+ * text byte, at most 8 GiB; larger ones are not kept), of wtg_lsel_build (at most
+ * 256 MiB) and of ordered query batches (38 MB).  Later calls allocate it again. */
+int wtg_ctx_trim(wtg_ctx* ctx);
 /* Wait for all work queued on the context's stream; reports device-side errors. */
 int wtg_ctx_sync(wtg_ctx* ctx);
 /* 1 (default): every entry point returns after its work finished.

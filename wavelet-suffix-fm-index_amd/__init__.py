@@ -74,6 +74,7 @@ SIGNATURES = {
     "wtg_device_count": (i32, [C.POINTER(i32)]),
     "wtg_ctx_create": (i32, [i32, C.POINTER(vp)]),
     "wtg_ctx_destroy": (i32, [vp]),
+    "wtg_ctx_trim": (i32, [vp]),
     "wtg_ctx_sync": (i32, [vp]),
     "wtg_ctx_set_blocking": (i32, [vp, i32]),
     "wtg_ctx_set_level_method": (i32, [vp, i32]),
@@ -400,6 +401,10 @@ class Context:
 
     def sync(self):
         _check(lib().wtg_ctx_sync(self.h))
+
+    def trim(self):
+        """Give back the scratch that the context keeps besides its workspace."""
+        _check(lib().wtg_ctx_trim(self.h))
 
     def set_blocking(self, b):
         _check(lib().wtg_ctx_set_blocking(self.h, 1 if b else 0))

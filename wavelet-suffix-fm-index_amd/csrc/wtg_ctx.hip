@@ -77,6 +77,7 @@ extern "C" int wtg_ctx_destroy(wtg_ctx* ctx) {
   if (ctx->ws) (void)hipFree(ctx->ws);
   if (ctx->d_small) (void)hipFree(ctx->d_small);
   if (ctx->qscratch) (void)hipFree(ctx->qscratch);
+  if (ctx->scratch) (void)hipFree(ctx->scratch);
   if (ctx->t0) (void)hipEventDestroy(ctx->t0);
   if (ctx->t1) (void)hipEventDestroy(ctx->t1);
   if (ctx->h2d_ev) (void)hipEventDestroy(ctx->h2d_ev);
@@ -187,6 +188,32 @@ int wtg_ws_reserve(wtg_ctx* ctx, size_t bytes) {
   return WTG_OK;
 }
 
+int wtg_scratch_reserve(wtg_ctx* ctx, size_t bytes) {
+  if (bytes <= ctx->scratch_bytes) return WTG_OK;
+  WTG_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+  if (ctx->scratch) { WTG_CHECK_HIP(hipFree(ctx->scratch)); ctx->scratch = nullptr; ctx->scratch_bytes = 0; }
+  if (hipMalloc(&ctx->scratch, bytes) != hipSuccess) {
+    ctx->scratch = nullptr;
+    (void)hipGetLastError();
+    wtg_set_error("scratch allocation failed");
+    return WTG_ERR_NOMEM;
+  }
+  ctx->scratch_bytes = bytes;
+  return WTG_OK;
+}
+
+extern "C" int wtg_ctx_trim(wtg_ctx* ctx) {
+  WTG_REQUIRE(ctx, "null ctx");
+  WTG_TRY(wtg_set_device(ctx));
+  WTG_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+  if (ctx->scratch) WTG_CHECK_HIP(hipFree(ctx->scratch));
+  ctx->scratch = nullptr;
+  ctx->scratch_bytes = 0;
+  if (ctx->qscratch) WTG_CHECK_HIP(hipFree(ctx->qscratch));
+  ctx->qscratch = nullptr;
+  return WTG_OK;
+}
+
 void* wtg_query_scratch(wtg_ctx* ctx, size_t bytes) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
@@ -209,7 +236,17 @@ void* wtg_query_scratch(wtg_ctx* ctx, size_t bytes) {
 extern "C" int wtg_malloc(wtg_ctx* ctx, void** dptr, uint64_t bytes) {
   WTG_REQUIRE(ctx && dptr, "wtg_malloc: null argument");
   WTG_TRY(wtg_set_device(ctx));
-  hipError_t e = ctx->pooled ? hipMallocAsync(dptr, bytes ? bytes : 1, ctx->stream) : hipMalloc(dptr, bytes ? bytes : 1);
+  const auto take = [&] {
+    return ctx->pooled ? hipMallocAsync(dptr, bytes ? bytes : 1, ctx->stream) : hipMalloc(dptr, bytes ? bytes : 1);
+  };
+  hipError_t e = take();
+  if (e != hipSuccess && (ctx->scratch || ctx->qscratch)) {  // what is kept for later calls may make room
+    (void)hipGetLastError();
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone &&
+        wtg_ctx_trim(ctx) == WTG_OK)
+      e = take();
+  }
   if (e != hipSuccess) {
     (void)hipGetLastError();
     *dptr = nullptr;

@@ -273,7 +273,7 @@ __device__ __forceinline__ double readlane_f64(double v, int l) {
 // `keep` of them to scratch[flat * keep ..].  Emit pass: a chunk with at most
 // `keep` knots copies them from scratch; a larger one walks again and writes
 // knots[off[flat] ..] (a different count sets *err).  The host keeps 512, in
-// the context's workspace (64 where that is over 256 MiB: an allocation of that size
+// the context's scratch (64 where that is over 256 MiB: an allocation of that size
 // for each build costs more than the second walk): with 64 the emit pass of the same vectors took
 // 299 us for the few chunks that have more, with 512 7.
 constexpr uint32_t LSEL_KEEP = 512, LSEL_KEEP_MIN = 64;
@@ -1114,14 +1114,11 @@ static int lsel_models(wtg_ctx* ctx, wtg_lsel* ls, const wtg_lsel_params& P, con
   WTG_CHECK_HIP(hipMemcpyAsync(d_cbase, cbase.data(), (na + 1) * 8, hipMemcpyHostToDevice, ctx->stream));
   WTG_TRY(wtg_fill_u64(ctx, d_err, 1, 0));
   Knot* d_scr = nullptr;  // the count pass keeps each chunk's first knots
-  const bool in_ws = nflat * LSEL_KEEP * sizeof(Knot) <= LSEL_KEEP_BYTES;  // (the plain build is done with it)
-  const uint32_t keep = in_ws ? LSEL_KEEP : LSEL_KEEP_MIN;
-  if (in_ws) {
-    WTG_TRY(wtg_ws_reserve(ctx, nflat * keep * sizeof(Knot)));
-    d_scr = (Knot*)ctx->ws;
-  } else {
-    WTG_TRY(wtg_malloc(ctx, (void**)&d_scr, nflat * keep * sizeof(Knot) + 256));
-  }
+  const bool kept = nflat * LSEL_KEEP * sizeof(Knot) <= LSEL_KEEP_BYTES &&
+                    wtg_scratch_reserve(ctx, nflat * LSEL_KEEP * sizeof(Knot)) == WTG_OK;
+  const uint32_t keep = kept ? LSEL_KEEP : LSEL_KEEP_MIN;
+  if (kept) d_scr = (Knot*)ctx->scratch;
+  else WTG_TRY(wtg_malloc(ctx, (void**)&d_scr, nflat * keep * sizeof(Knot) + 256));
   const unsigned gp = (unsigned)wtg_ceil_div(nflat, 4);  // a wave per chunk
   WTG_LAUNCH(ctx, "lsel_place", k_lsel_place, dim3(gp), dim3(256), 0, d_pv, d_cbase, na, nflat, gap_log,
              (double)P.tol, d_cnt, (const uint32_t*)nullptr, (Knot*)nullptr, d_scr, keep, d_err);
@@ -1154,7 +1151,7 @@ static int lsel_models(wtg_ctx* ctx, wtg_lsel* ls, const wtg_lsel_params& P, con
   WTG_LAUNCH_CHECK();
   uint32_t perr = 0;
   const int prc = sync_copy(ctx, &perr, d_err, 4, hipMemcpyDeviceToHost);
-  if (!in_ws) wtg_free(ctx, d_scr);
+  if (!kept) wtg_free(ctx, d_scr);
   WTG_TRY(prc);
   WTG_REQUIRE(perr == 0, "wtg_lsel_build: knot placement passes disagree");
   WTG_CHECK_HIP(hipMemcpyAsync(d_K0, d_K, nk_total * sizeof(Knot), hipMemcpyDeviceToDevice, ctx->stream));

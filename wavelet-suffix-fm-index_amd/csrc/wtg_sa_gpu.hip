@@ -587,24 +587,22 @@ extern "C" int wtg_suffix_array_gpu(wtg_ctx* ctx, const uint8_t* d_text, uint64_
     }
     tmp_bytes = b > tmp_bytes ? b : tmp_bytes;
   }
-  // All buffers in one block: the context's workspace, or for a large text (its
-  // workspace would stay that large) an allocation of this call.  Thirteen
-  // allocations of 4 to 8 n bytes from the pool cost 2.5 to 50 ms a call
+  // All buffers in one block: the context's scratch, or for a large text (it would
+  // stay that large), and where there is no memory for it outside the pool, an
+  // allocation of this call.  From the pool, thirteen allocations of 4 to 8 n bytes
+  // cost 2.5 to 50 ms a call and one for all of them 50 ms between calls that allocate too
   // (n = 2^25: the pool unmaps and maps what does not fit its free blocks).
   size_t o = 0;
   const auto take = [&](size_t bytes) { const size_t at = o; o = wtg_align256(o + bytes); return at; };
   const size_t o_k0 = take(n * 8), o_k1 = take(n * 8), o_v0 = take(n * 4), o_v1 = take(n * 4), o_rank = take(n * 4);
   const size_t o_i0 = take(n * 4), o_i1 = take(n * 4), o_g0 = take(n * 4), o_g1 = take(n * 4), o_key2 = take(n * 4);
   const size_t o_tab = take((3 * tiles + 4) * 4), o_pres = take(256 * 4 + 256 * 2), o_tmp = take(tmp_bytes);
-  constexpr size_t SA_WS_MAX = 8ull << 30;
+  constexpr size_t SA_KEEP_MAX = 8ull << 30;
   char* mem = nullptr;
   int rc = WTG_OK;
-  if (o <= SA_WS_MAX) {
-    WTG_TRY(wtg_ws_reserve(ctx, o));
-    mem = (char*)ctx->ws;
-  } else {
-    WTG_TRY(wtg_malloc(ctx, (void**)&mem, o));
-  }
+  const bool kept = o <= SA_KEEP_MAX && wtg_scratch_reserve(ctx, o) == WTG_OK;
+  if (kept) mem = (char*)ctx->scratch;
+  else WTG_TRY(wtg_malloc(ctx, (void**)&mem, o));
   k0 = (uint64_t*)(mem + o_k0);
   k1 = (uint64_t*)(mem + o_k1);
   v0 = (uint32_t*)(mem + o_v0);
@@ -686,7 +684,7 @@ extern "C" int wtg_suffix_array_gpu(wtg_ctx* ctx, const uint8_t* d_text, uint64_
   rc = wtg_finish(ctx);
 out:
   if (rc != WTG_OK) wtg_abandon(ctx);
-  if (o > SA_WS_MAX) wtg_free(ctx, mem);
+  if (!kept) wtg_free(ctx, mem);
   return rc;
 }
 #undef SA_LAUNCH_CHECK
