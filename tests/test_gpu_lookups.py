@@ -123,3 +123,85 @@ def test_ordered_patterns(ctx, m):
             assert np.array_equal(got, np.concatenate([wt.fm_count(pats[at:at + step]) for at in range(0, nq, step)]))
     finally:
         wt.free()
+
+
+def in_runs(rng, x, runs, down):
+    """x rearranged as `runs` sorted stretches of one length, up or down."""
+    x = np.array_split(rng.permutation(x), runs)
+    return np.concatenate([np.sort(p)[::-1] if down else np.sort(p) for p in x])
+
+
+@pytest.mark.parametrize("nq", [1 << 18, (1 << 20) + 5])
+@pytest.mark.parametrize("runs,down", [(1, False), (1, True), (15, False), (16, True), (17, False), (40, True)])
+def test_batch_in_order(ctx, large, nq, runs, down):
+    """Batches that come in order, up or down, in few runs or in more than count as order,
+    give what the same queries give in small batches, as they came."""
+    wt, rng = large, np.random.default_rng(nq + runs)
+    n, top = wt.n, 1 << wt.L
+    i, j = (in_runs(rng, rng.integers(0, n, nq).astype(np.uint64), runs, down) for _ in range(2))
+    lo, hi = (in_runs(rng, rng.integers(0, top, nq).astype(np.uint64), runs, down) for _ in range(2))
+    k = rng.integers(1, 3000, nq).astype(np.uint64)
+    calls = [(wt.rank, (i, lo)), (wt.access, (i,)), (wt.inverse_select, (i,)), (wt.lex_count, (np.minimum(i, j), np.maximum(i, j), lo)),
+             (wt.lex_smaller_count, (i, lo)), (wt.range_count, (np.minimum(i, j), np.maximum(i, j), lo, rng.permutation(hi))),
+             (wt.select, (k, lo))]
+    step = 100000
+    for f, a in calls:
+        got = f(*a)
+        parts = [f(*(x[at:at + step] for x in a)) for at in range(0, nq, step)]
+        if isinstance(got, list):
+            want = [np.concatenate([p[c] for p in parts]) for c in range(len(got))]
+            assert all(np.array_equal(g, w) for g, w in zip(got, want)), f.__name__
+        else:
+            assert np.array_equal(got, np.concatenate(parts)), f.__name__
+
+
+@pytest.mark.parametrize("m", [12, 19, 32])
+def test_patterns_in_order(ctx, m):
+    """Patterns in the order of their last eight bytes (last byte first), up and down, and
+    one pattern over and over: counts as in small batches."""
+    rng = np.random.default_rng(m)
+    n = (1 << 24) + 1
+    wt = ctx.huff_build(ctx.to_device((rng.integers(0, 16, n) * 3).astype(np.uint8)))
+    try:
+        nq = (1 << 20) + 5
+        pats = (rng.integers(0, 16, (nq, m)) * 3).astype(np.uint8)
+        pats[:, :m - 5] = pats[rng.integers(0, 50, nq), :m - 5]
+        key = np.ascontiguousarray(pats[:, m - 8:]).view("<u8").reshape(-1)
+        up = pats[np.argsort(key, kind="stable")]
+        for p in (up, up[::-1], np.repeat(pats[:1], nq, 0), np.concatenate([up[::7]] * 7)[:nq]):
+            got, step = wt.fm_count(p), 1 << 18
+            assert np.array_equal(got, np.concatenate([wt.fm_count(p[at:at + step]) for at in range(0, p.shape[0], step)]))
+    finally:
+        wt.free()
+
+
+def test_captured_batches(wsfm, ctx, large):
+    """Large batches recorded as a graph (answered as they come, with no block shared with
+    other work), replayed over other queries in the same place."""
+    import ctypes as C
+    hip, wt, nq = wsfm.lib(), large, 1 << 18
+    stream = C.c_void_p(hip.wtg_ctx_stream(ctx.h))
+    rng = np.random.default_rng(9)
+    i, c, out, inv = (ctx.empty(nq) for _ in range(4))
+    i.zero()
+    c.zero()
+    graph, run = C.c_void_p(), C.c_void_p()
+    ctx.set_blocking(False)
+    try:
+        assert hip.hipStreamBeginCapture(stream, 1) == 0  # thread-local mode
+        wsfm._check(hip.wtg_wtint_rank_batch(ctx.h, wt.h, i.ptr, c.ptr, nq, out.ptr))
+        wsfm._check(hip.wtg_wtint_access_batch(ctx.h, wt.h, i.ptr, nq, inv.ptr))
+        assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    finally:
+        ctx.set_blocking(True)
+    assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+    for _ in range(3):
+        qi, qc = rng.integers(0, wt.n, nq).astype(np.uint64), rng.integers(0, 1 << wt.L, nq).astype(np.uint64)
+        for d, q in ((i, qi), (c, qc)):
+            wsfm._check(hip.wtg_memcpy_h2d(ctx.h, d.ptr, C.c_void_p(q.ctypes.data), q.nbytes))
+        assert hip.hipGraphLaunch(run, stream) == 0
+        ctx.sync()
+        assert np.array_equal(out.get(), wt.rank(qi, qc)) and np.array_equal(inv.get(), wt.access(qi))
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+    for x in (i, c, out, inv):
+        x.free()

@@ -1057,12 +1057,18 @@ __global__ __launch_bounds__(256) void k_huff_select(HQ h, const uint64_t* __res
 // last pattern byte; rank_c of both ends walks the same nodes, and both rank
 // blocks of a level are loaded before either is used.  NP patterns per lane
 // (NP t .. NP t + NP-1) interleave their searches step by step.
+struct FmBatch {  // patterns as they came and, where they were to be put in order, in order (as QBatch)
+  const uint8_t *came, *put;
+  const uint32_t *place, *asis;
+};
 template <int NP>
-__global__ __launch_bounds__(256) void k_fm_count(HQ h, const uint8_t* __restrict__ pats, uint32_t m,
-                                                  uint64_t npat, uint64_t* __restrict__ out,
-                                                  const uint32_t* __restrict__ order) {
+__global__ __launch_bounds__(256) void k_fm_count(HQ h, FmBatch b, uint32_t m, uint64_t npat,
+                                                  uint64_t* __restrict__ out) {
   __shared__ QLds Q;
   __shared__ uint64_t s_C[257];
+  const bool put = b.place && *b.asis == 0;
+  const uint8_t* __restrict__ pats = put ? b.put : b.came;
+  const uint32_t* __restrict__ order = put ? b.place : nullptr;
   load_q(Q, h.tab);
   for (int k = threadIdx.x; k < 257; k += blockDim.x) s_C[k] = h.tab->C[k];
   __syncthreads();
@@ -1146,21 +1152,20 @@ __global__ __launch_bounds__(256) void k_fm_count(HQ h, const uint8_t* __restric
 // A large batch in the order of the patterns' last eight bytes, the last one first:
 // those are the first steps, and patterns that share them walk the same part of
 // the bits, which the later steps spread out again.
-__global__ __launch_bounds__(256) void k_fm_keys(const uint8_t* __restrict__ pats, uint32_t m, uint64_t npat,
-                                                 uint64_t* __restrict__ key) {
-  const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= npat) return;
-  const uint8_t* p = pats + t * m + m - 8;  // m >= 8
-  uint64_t k = 0;
-#pragma unroll
-  for (uint32_t i = 0; i < 8; i++) k |= (uint64_t)p[i] << (8 * i);
-  key[t] = k;
-}
+struct KeyTail {
+  const uint8_t* pats;
+  uint32_t m;  // >= 8
+  __device__ __forceinline__ uint64_t operator()(uint64_t i) const {
+    typedef uint64_t u64_a1 __attribute__((aligned(1)));
+    return *reinterpret_cast<const u64_a1*>(pats + i * m + m - 8);
+  }
+};
 // the rows in order, four bytes a thread
 __global__ __launch_bounds__(256) void k_fm_rows(const uint8_t* __restrict__ pats, uint32_t m, uint32_t bytes,
-                                                 const uint32_t* __restrict__ order, uint8_t* __restrict__ rows) {
+                                                 const uint32_t* __restrict__ order, const uint32_t* __restrict__ asis,
+                                                 uint8_t* __restrict__ rows) {
   const uint32_t f = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (f >= bytes) return;
+  if (f >= bytes || *asis) return;
   uint32_t r = f / m, c = f - r * m, x = 0;
   uint64_t at = (uint64_t)order[r] * m;
 #pragma unroll
@@ -1635,28 +1640,25 @@ extern "C" int wtg_fm_count_batch(wtg_ctx* ctx, const wtg_huff* wt, const uint8_
   WTG_TRY(wtg_set_device(ctx));
   char* scratch = fm_order_pays(wt, m, npat) ? (char*)wtg_query_scratch(ctx, QO_BYTES) : nullptr;
   if (scratch) {
-    // keys | tables | places | rows, chunks of one size
-    const uint64_t cap = std::min<uint64_t>(QO_CHUNK, (QO_BYTES - QO_BINS * 16 - 256) / (8 + 4 + m));
-    const QOrder o = order_layout(scratch, cap, 1);
-    uint8_t* rows = (uint8_t*)(((uintptr_t)(o.q + cap) + 255) & ~(uintptr_t)255);
+    // tables | places | rows, chunks of one size
+    const uint64_t cap = std::min<uint64_t>(QO_CHUNK, (QO_BYTES - QO_BINS * 16) / (4 + m));
+    const QOrder o = order_layout(scratch, cap, 0);
+    uint8_t* rows = (uint8_t*)(o.q + cap);
     const uint64_t step = wtg_ceil_div(npat, wtg_ceil_div(npat, cap));
     for (uint64_t at = 0; at < npat; at += step) {
       const uint64_t n = std::min(step, npat - at);
       const uint8_t* part = d_pats + at * m;
       const uint32_t bytes = (uint32_t)(n * m);
-      WTG_LAUNCH(ctx, "fm_keys", k_fm_keys, dim3((unsigned)wtg_ceil_div(n, 256)), dim3(256), 0, part, m, n, o.col[0]);
-      QCols in{};
-      in.c[0] = o.col[0];
-      order_chunk<0>(ctx, in, 0, n, o);
+      order_chunk<0>(ctx, QCols{}, KeyTail{part, m}, n, o);
       WTG_LAUNCH(ctx, "fm_rows", k_fm_rows, dim3((unsigned)wtg_ceil_div(bytes, 1024)), dim3(256), 0, part, m, bytes,
-                 (const uint32_t*)o.q, rows);
+                 (const uint32_t*)o.q, (const uint32_t*)o.asis, rows);
       WTG_LAUNCH(ctx, "fm_count", k_fm_count<FM_NP>, dim3(wtg_ceil_div(query_grid((n + FM_NP - 1) / FM_NP), QO_XCDS) * QO_XCDS),
                  dim3(256), 0,
-                 make_hq(wt), (const uint8_t*)rows, m, n, d_out + at, (const uint32_t*)o.q);
+                 make_hq(wt), FmBatch{part, rows, o.q, o.asis}, m, n, d_out + at);
     }
   } else {
     WTG_LAUNCH(ctx, "fm_count", k_fm_count<FM_NP>, dim3(query_grid((npat + FM_NP - 1) / FM_NP)), dim3(256), 0,
-               make_hq(wt), d_pats, m, npat, d_out, (const uint32_t*)nullptr);
+               make_hq(wt), FmBatch{d_pats, nullptr, nullptr, nullptr}, m, npat, d_out);
   }
   WTG_LAUNCH_CHECK();
   return wtg_finish(ctx);

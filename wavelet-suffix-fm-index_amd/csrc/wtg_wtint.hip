@@ -33,23 +33,37 @@ struct WtQ {
 // every one of them.  Ordered batches below.
 __device__ __forceinline__ RankAt wt_fetch(const WtQ& w, uint64_t i) { return rank9_fetch(w.D, w.words, w.W, i); }
 
-// the query of this thread: where its columns are (p) and its answer goes (q);
-// false past the end.  An ordered batch's grid is a multiple of the XCDs.
-__device__ __forceinline__ bool q_slot(const uint32_t* __restrict__ order, uint64_t nq, uint64_t& p, uint64_t& q) {
-  const uint32_t b = order ? (blockIdx.x % QO_XCDS) * (gridDim.x / QO_XCDS) + blockIdx.x / QO_XCDS : blockIdx.x;
-  p = (uint64_t)b * blockDim.x + threadIdx.x;
-  if (p >= nq) return false;
-  q = order ? order[p] : p;
-  return true;
+// A batch's columns as they came and, where it was to be put in order, in order,
+// with the places the queries had; asis: it was in order, the others were not written.
+struct QBatch {
+  QCols came, put;
+  const uint32_t *place, *asis;
+};
+// the query of this thread: where its columns are (p) and its answer goes (q); not
+// in the batch past its end.  The grid of a batch to be put in order is a multiple of the XCDs.
+struct QSlot {
+  uint64_t p, q;
+  bool put, in;
+};
+__device__ __forceinline__ QSlot q_slot(const QBatch& b, uint64_t nq) {
+  QSlot s;
+  s.put = b.place && *b.asis == 0;
+  const uint32_t blk = s.put ? (blockIdx.x % QO_XCDS) * (gridDim.x / QO_XCDS) + blockIdx.x / QO_XCDS : blockIdx.x;
+  s.p = (uint64_t)blk * blockDim.x + threadIdx.x;
+  s.in = s.p < nq;
+  s.q = s.in && s.put ? b.place[s.p] : s.p;
+  return s;
+}
+__device__ __forceinline__ uint64_t q_col(const QBatch& b, const QSlot& s, uint32_t c) {
+  return (s.put ? b.put.c[c] : b.came.c[c])[s.p];
 }
 
-__global__ void k_wtint_rank(WtQ w, const uint64_t* __restrict__ qi, const uint64_t* __restrict__ qc,
-                             uint64_t nq, uint64_t* __restrict__ out,
-                             const uint32_t* __restrict__ order) {
-  uint64_t p, q;
-  if (!q_slot(order, nq, p, q)) return;
-  uint64_t i = qi[p];
-  const uint64_t c = qc[p];
+__global__ void k_wtint_rank(WtQ w, QBatch b, uint64_t nq, uint64_t* __restrict__ out) {
+  const QSlot slot = q_slot(b, nq);
+  if (!slot.in) return;
+  const uint64_t q = slot.q;
+  uint64_t i = q_col(b, slot, 0);
+  const uint64_t c = q_col(b, slot, 1);
   if (i > w.n) { out[q] = WTG_NONE; return; }
   if (w.L < 64 && (1ull << w.L) <= c) { out[q] = 0; return; }
   uint64_t offset = 0, mask = 1ull << (w.L - 1), node_size = w.n;
@@ -110,15 +124,13 @@ __device__ __forceinline__ void wtint_lex(const WtQ& w, uint64_t i, uint64_t j, 
   gr = x.greater;
 }
 
-__global__ void k_wtint_lex_count(WtQ w, const uint64_t* __restrict__ qi, const uint64_t* __restrict__ qj,
-                                  const uint64_t* __restrict__ qc, uint64_t nq, uint64_t* __restrict__ out_rank,
-                                  uint64_t* __restrict__ out_smaller, uint64_t* __restrict__ out_greater,
-                                  const uint32_t* __restrict__ order) {
-  uint64_t p, q;
-  if (!q_slot(order, nq, p, q)) return;
-  const uint64_t i = qi[p], j = qj[p];
+__global__ void k_wtint_lex_count(WtQ w, QBatch b, uint64_t nq, uint64_t* __restrict__ out_rank,
+                                  uint64_t* __restrict__ out_smaller, uint64_t* __restrict__ out_greater) {
+  const QSlot slot = q_slot(b, nq);
+  if (!slot.in) return;
+  const uint64_t q = slot.q, i = q_col(b, slot, 0), j = q_col(b, slot, 1), c = q_col(b, slot, 2);
   uint64_t rk = WTG_NONE, sm = WTG_NONE, gr = WTG_NONE;
-  if (i <= j && j <= w.n) wtint_lex(w, i, j, qc[p], rk, sm, gr);
+  if (i <= j && j <= w.n) wtint_lex(w, i, j, c, rk, sm, gr);
   out_rank[q] = rk;
   out_smaller[q] = sm;
   out_greater[q] = gr;
@@ -126,13 +138,13 @@ __global__ void k_wtint_lex_count(WtQ w, const uint64_t* __restrict__ qi, const 
 
 // lex_smaller_count (wt_int/wt_int_par.hpp:753-780): rank(i,c) and the number of
 // values below c in [0, i)
-__global__ void k_wtint_lex_smaller(WtQ w, const uint64_t* __restrict__ qi, const uint64_t* __restrict__ qc,
-                                    uint64_t nq, uint64_t* __restrict__ out_rank, uint64_t* __restrict__ out_smaller,
-                                    const uint32_t* __restrict__ order) {
-  uint64_t p, q;
-  if (!q_slot(order, nq, p, q)) return;
-  uint64_t i = qi[p];
-  const uint64_t c = qc[p];
+__global__ void k_wtint_lex_smaller(WtQ w, QBatch b, uint64_t nq, uint64_t* __restrict__ out_rank,
+                                    uint64_t* __restrict__ out_smaller) {
+  const QSlot slot = q_slot(b, nq);
+  if (!slot.in) return;
+  const uint64_t q = slot.q;
+  uint64_t i = q_col(b, slot, 0);
+  const uint64_t c = q_col(b, slot, 1);
   if (i > w.n) { out_rank[q] = out_smaller[q] = WTG_NONE; return; }
   if (w.L < 64 && (1ull << w.L) <= c) { out_rank[q] = 0; out_smaller[q] = i; return; }
   uint64_t offset = 0, mask = 1ull << (w.L - 1), node_size = w.n, res = 0;
@@ -153,14 +165,11 @@ __global__ void k_wtint_lex_smaller(WtQ w, const uint64_t* __restrict__ qi, cons
 // lex_count "smaller" counts over [lb, rb + 1).  The reference clamps vrb to 2^L
 // and its leaf test does not compare vlb, so vlb = 2^L counts the value 2^L - 1:
 // vlb is clamped to 2^L - 1 the same way.
-__global__ void k_wtint_range_count(WtQ w, const uint64_t* __restrict__ qlb, const uint64_t* __restrict__ qrb,
-                                    const uint64_t* __restrict__ qvlb, const uint64_t* __restrict__ qvrb,
-                                    uint64_t nq, uint64_t* __restrict__ out,
-                                    const uint32_t* __restrict__ order) {
-  uint64_t p, q;
-  if (!q_slot(order, nq, p, q)) return;
-  const uint64_t lb = qlb[p], rb = qrb[p];
-  uint64_t vlb = qvlb[p], vrb = qvrb[p];
+__global__ void k_wtint_range_count(WtQ w, QBatch b, uint64_t nq, uint64_t* __restrict__ out) {
+  const uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= nq) return;
+  const uint64_t lb = b.came.c[0][q], rb = b.came.c[1][q];
+  uint64_t vlb = b.came.c[2][q], vrb = b.came.c[3][q];
   if (rb >= w.n) { out[q] = WTG_NONE; return; }
   const uint64_t top = w.L < 64 ? (1ull << w.L) : ~0ull;
   if (vrb > top) vrb = top;
@@ -186,14 +195,12 @@ __global__ void k_wtint_range_count(WtQ w, const uint64_t* __restrict__ qlb, con
 // the lower one leaves its count or a mark, the upper one takes it from there.
 constexpr uint64_t WT_RANGE_EMPTY = WTG_NONE - 1;
 template <bool UPPER>
-__global__ void k_wtint_range_half(WtQ w, const uint64_t* __restrict__ qlb, const uint64_t* __restrict__ qrb,
-                                   const uint64_t* __restrict__ qv, const uint64_t* __restrict__ qvrb, uint64_t nq,
-                                   uint64_t* __restrict__ out, const uint32_t* __restrict__ order) {
-  uint64_t p, q;
-  if (!q_slot(order, nq, p, q)) return;
-  const uint64_t lb = qlb[p], rb = qrb[p];
+__global__ void k_wtint_range_half(WtQ w, QBatch b, uint64_t nq, uint64_t* __restrict__ out) {
+  const QSlot slot = q_slot(b, nq);
+  if (!slot.in) return;
+  const uint64_t q = slot.q, lb = q_col(b, slot, 0), rb = q_col(b, slot, 1);
   const uint64_t top = w.L < 64 ? (1ull << w.L) : ~0ull;
-  uint64_t v = qv[p], rk, below, gr;
+  uint64_t v = q_col(b, slot, 2), rk, below, gr;
   if (UPPER) {
     const uint64_t low = out[q];
     if (low == WTG_NONE) return;
@@ -202,7 +209,7 @@ __global__ void k_wtint_range_half(WtQ w, const uint64_t* __restrict__ qlb, cons
     else wtint_lex(w, lb, rb + 1, v + 1, rk, below, gr);
     out[q] = below - low;
   } else {
-    uint64_t vrb = qvrb[p];
+    uint64_t vrb = q_col(b, slot, 3);
     if (rb >= w.n) { out[q] = WTG_NONE; return; }
     if (vrb > top) vrb = top;
     if (v > vrb || lb > rb) { out[q] = WT_RANGE_EMPTY; return; }
@@ -212,12 +219,12 @@ __global__ void k_wtint_range_half(WtQ w, const uint64_t* __restrict__ qlb, cons
   }
 }
 
-__global__ void k_wtint_access(WtQ w, const uint64_t* __restrict__ qi, uint64_t nq,
-                               uint64_t* __restrict__ out_sym, uint64_t* __restrict__ out_rank,
-                               const uint32_t* __restrict__ order) {
-  uint64_t p, q;
-  if (!q_slot(order, nq, p, q)) return;
-  uint64_t i = qi[p];
+__global__ void k_wtint_access(WtQ w, QBatch b, uint64_t nq, uint64_t* __restrict__ out_sym,
+                               uint64_t* __restrict__ out_rank) {
+  const QSlot slot = q_slot(b, nq);
+  if (!slot.in) return;
+  const uint64_t q = slot.q;
+  uint64_t i = q_col(b, slot, 0);
   if (i >= w.n) {
     out_sym[q] = WTG_NONE;
     if (out_rank) out_rank[q] = WTG_NONE;
@@ -237,13 +244,12 @@ __global__ void k_wtint_access(WtQ w, const uint64_t* __restrict__ qi, uint64_t 
 }
 
 template <uint32_t MAXL>  // the tree's levels are at most MAXL
-__global__ void k_wtint_select(WtQ w, const uint64_t* __restrict__ qi, const uint64_t* __restrict__ qc,
-                               uint64_t nq, uint64_t* __restrict__ out,
-                               const uint32_t* __restrict__ order) {
-  uint64_t p, q;
-  if (!q_slot(order, nq, p, q)) return;
-  uint64_t i = qi[p];
-  const uint64_t c = qc[p];
+__global__ void k_wtint_select(WtQ w, QBatch b, uint64_t nq, uint64_t* __restrict__ out) {
+  const QSlot slot = q_slot(b, nq);
+  if (!slot.in) return;
+  const uint64_t q = slot.q;
+  uint64_t i = q_col(b, slot, 0);
+  const uint64_t c = q_col(b, slot, 1);
   uint64_t path_off[MAXL + 1], path_rank[MAXL + 1];
   uint64_t offset = 0, mask = 1ull << (w.L - 1), node_size = w.n;
   path_off[0] = path_rank[0] = 0;
@@ -420,8 +426,8 @@ static bool order_pays(const wtg_wtint* wt, uint64_t nq) {
   return wt->nbits >= 1ull << 24 && nq >= (wt->nbits >= 1ull << 26 ? 1ull << 18 : 1ull << 19);
 }
 
-// A batch in chunks: walk(columns, queries, where they stood or null, answers' offset)
-// launches the kernels that answer one chunk.
+// A batch in chunks: walk(batch, queries, answers' offset, grid) launches the kernel
+// that answers one chunk.
 template <uint32_t NC, class F>
 static int q_ordered(wtg_ctx* ctx, char* scratch, const QCols& in, uint32_t key, uint64_t nq, F&& walk) {
   const QOrder o = order_layout(scratch, QO_CHUNK, QO_COLS);
@@ -430,10 +436,10 @@ static int q_ordered(wtg_ctx* ctx, char* scratch, const QCols& in, uint32_t key,
     const uint64_t m = nq - at < step ? nq - at : step;
     QCols part{};
     for (uint32_t c = 0; c < NC; c++) part.c[c] = in.c[c] + at;
-    order_chunk<NC>(ctx, part, key, m, o);
-    QCols cols{};
-    for (uint32_t c = 0; c < NC; c++) cols.c[c] = o.col[c];
-    walk(cols, m, (const uint32_t*)o.q, at, dim3((unsigned)(wtg_ceil_div(m, 256 * QO_XCDS) * QO_XCDS)));
+    order_chunk<NC>(ctx, part, KeyCol{part.c[key]}, m, o);
+    QBatch b{part, {}, o.q, o.asis};
+    for (uint32_t c = 0; c < NC; c++) b.put.c[c] = o.col[c];
+    walk(b, m, at, dim3((unsigned)(wtg_ceil_div(m, 256 * QO_XCDS) * QO_XCDS)));
   }
   WTG_LAUNCH_CHECK();
   return WTG_OK;
@@ -447,7 +453,7 @@ static int q_batch(wtg_ctx* ctx, const wtg_wtint* wt, const QCols& in, uint32_t 
   if (scratch) {
     WTG_TRY(q_ordered<NC>(ctx, scratch, in, key, nq, walk));
   } else {
-    walk(in, nq, (const uint32_t*)nullptr, (uint64_t)0, dim3((unsigned)wtg_ceil_div(nq, 256)));
+    walk(QBatch{in, {}, nullptr, nullptr}, nq, (uint64_t)0, dim3((unsigned)wtg_ceil_div(nq, 256)));
     WTG_LAUNCH_CHECK();
   }
   return wtg_finish(ctx);
@@ -459,16 +465,16 @@ extern "C" int wtg_wtint_rank_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uin
   WTG_REQUIRE(nq == 0 || d_c, "null d_c");
   if (!nq) return WTG_OK;
   return q_batch<2>(ctx, wt, QCols{{d_i, d_c}}, 1, nq,
-                    [&](const QCols& c, uint64_t m, const uint32_t* order, uint64_t at, dim3 grid) {
-    WTG_LAUNCH(ctx, "wtint_rank", k_wtint_rank, grid, dim3(256), 0, make_q(wt), c.c[0], c.c[1], m, d_out + at, order);
+                    [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
+    WTG_LAUNCH(ctx, "wtint_rank", k_wtint_rank, grid, dim3(256), 0, make_q(wt), b, m, d_out + at);
   });
 }
 static int access_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_i, uint64_t nq, uint64_t* d_sym,
                         uint64_t* d_rank) {
   return q_batch<1>(ctx, wt, QCols{{d_i}}, 0, nq,
-                    [&](const QCols& c, uint64_t m, const uint32_t* order, uint64_t at, dim3 grid) {
-    WTG_LAUNCH(ctx, "wtint_access", k_wtint_access, grid, dim3(256), 0, make_q(wt), c.c[0], m, d_sym + at,
-               d_rank ? d_rank + at : nullptr, order);
+                    [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
+    WTG_LAUNCH(ctx, "wtint_access", k_wtint_access, grid, dim3(256), 0, make_q(wt), b, m, d_sym + at,
+               d_rank ? d_rank + at : nullptr);
   });
 }
 extern "C" int wtg_wtint_access_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_i,
@@ -491,9 +497,9 @@ extern "C" int wtg_wtint_lex_count_batch(wtg_ctx* ctx, const wtg_wtint* wt, cons
   WTG_REQUIRE(nq == 0 || (d_j && d_c && d_smaller && d_greater), "null argument");
   if (!nq) return WTG_OK;
   return q_batch<3>(ctx, wt, QCols{{d_i, d_j, d_c}}, 2, nq,
-                    [&](const QCols& c, uint64_t m, const uint32_t* order, uint64_t at, dim3 grid) {
-    WTG_LAUNCH(ctx, "wtint_lex_count", k_wtint_lex_count, grid, dim3(256), 0, make_q(wt), c.c[0], c.c[1], c.c[2], m,
-               d_rank + at, d_smaller + at, d_greater + at, order);
+                    [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
+    WTG_LAUNCH(ctx, "wtint_lex_count", k_wtint_lex_count, grid, dim3(256), 0, make_q(wt), b, m, d_rank + at,
+               d_smaller + at, d_greater + at);
   });
 }
 extern "C" int wtg_wtint_lex_smaller_count_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_i,
@@ -503,9 +509,9 @@ extern "C" int wtg_wtint_lex_smaller_count_batch(wtg_ctx* ctx, const wtg_wtint* 
   WTG_REQUIRE(nq == 0 || (d_c && d_smaller), "null argument");
   if (!nq) return WTG_OK;
   return q_batch<2>(ctx, wt, QCols{{d_i, d_c}}, 1, nq,
-                    [&](const QCols& c, uint64_t m, const uint32_t* order, uint64_t at, dim3 grid) {
-    WTG_LAUNCH(ctx, "wtint_lex_smaller", k_wtint_lex_smaller, grid, dim3(256), 0, make_q(wt), c.c[0], c.c[1], m,
-               d_rank + at, d_smaller + at, order);
+                    [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
+    WTG_LAUNCH(ctx, "wtint_lex_smaller", k_wtint_lex_smaller, grid, dim3(256), 0, make_q(wt), b, m, d_rank + at,
+               d_smaller + at);
   });
 }
 extern "C" int wtg_wtint_range_count_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_lb,
@@ -521,18 +527,18 @@ extern "C" int wtg_wtint_range_count_batch(wtg_ctx* ctx, const wtg_wtint* wt, co
   char* scratch = apart && order_pays(wt, nq) ? (char*)wtg_query_scratch(ctx, QO_BYTES) : nullptr;
   if (scratch) {
     WTG_TRY(q_ordered<4>(ctx, scratch, QCols{{d_lb, d_rb, d_vlb, d_vrb}}, 2, nq,
-                         [&](const QCols& c, uint64_t m, const uint32_t* order, uint64_t at, dim3 grid) {
-      WTG_LAUNCH(ctx, "wtint_range_lower", k_wtint_range_half<false>, grid, dim3(256), 0, make_q(wt), c.c[0], c.c[1],
-                 c.c[2], c.c[3], m, d_out + at, order);
+                         [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
+      WTG_LAUNCH(ctx, "wtint_range_lower", k_wtint_range_half<false>, grid, dim3(256), 0, make_q(wt), b, m,
+                 d_out + at);
     }));
     WTG_TRY(q_ordered<3>(ctx, scratch, QCols{{d_lb, d_rb, d_vrb}}, 2, nq,
-                         [&](const QCols& c, uint64_t m, const uint32_t* order, uint64_t at, dim3 grid) {
-      WTG_LAUNCH(ctx, "wtint_range_upper", k_wtint_range_half<true>, grid, dim3(256), 0, make_q(wt), c.c[0], c.c[1],
-                 c.c[2], (const uint64_t*)nullptr, m, d_out + at, order);
+                         [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
+      WTG_LAUNCH(ctx, "wtint_range_upper", k_wtint_range_half<true>, grid, dim3(256), 0, make_q(wt), b, m,
+                 d_out + at);
     }));
   } else {
     WTG_LAUNCH(ctx, "wtint_range_count", k_wtint_range_count, dim3((unsigned)wtg_ceil_div(nq, 256)), dim3(256), 0,
-               make_q(wt), d_lb, d_rb, d_vlb, d_vrb, nq, d_out, (const uint32_t*)nullptr);
+               make_q(wt), QBatch{{{d_lb, d_rb, d_vlb, d_vrb}}, {}, nullptr, nullptr}, nq, d_out);
     WTG_LAUNCH_CHECK();
   }
   return wtg_finish(ctx);
@@ -543,12 +549,10 @@ extern "C" int wtg_wtint_select_batch(wtg_ctx* ctx, const wtg_wtint* wt, const u
   WTG_REQUIRE(nq == 0 || d_c, "null d_c");
   if (!nq) return WTG_OK;
   return q_batch<2>(ctx, wt, QCols{{d_i, d_c}}, 1, nq,
-                    [&](const QCols& c, uint64_t m, const uint32_t* order, uint64_t at, dim3 grid) {
+                    [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
     if (wt->L <= 24)
-      WTG_LAUNCH(ctx, "wtint_select", k_wtint_select<24>, grid, dim3(256), 0, make_q(wt), c.c[0], c.c[1], m,
-                 d_out + at, order);
+      WTG_LAUNCH(ctx, "wtint_select", k_wtint_select<24>, grid, dim3(256), 0, make_q(wt), b, m, d_out + at);
     else
-      WTG_LAUNCH(ctx, "wtint_select", k_wtint_select<64>, grid, dim3(256), 0, make_q(wt), c.c[0], c.c[1], m,
-                 d_out + at, order);
+      WTG_LAUNCH(ctx, "wtint_select", k_wtint_select<64>, grid, dim3(256), 0, make_q(wt), b, m, d_out + at);
   });
 }
