@@ -205,3 +205,25 @@ def test_captured_batches(wsfm, ctx, large):
     assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
     for x in (i, c, out, inv):
         x.free()
+
+
+@pytest.mark.parametrize("levels", [2, 4, 8, 11])
+def test_large_batch_on_few_levels(ctx, levels):
+    """2^26 level bits in few levels, batches on either side of 2^18 queries: large ones
+    walk a lookup at a time; answers against the small batches'."""
+    rng = np.random.default_rng(levels)
+    n, top = (1 << 26) // levels + 3, 1 << levels
+    wt = ctx.wtint_build(ctx.to_device(np.minimum(rng.geometric(0.2, n) - 1, top - 1).astype(np.uint16)), n, levels)
+    try:
+        for nq in ((1 << 18) - 1, 1 << 18, (1 << 20) + 1):
+            i, j = np.sort(rng.integers(0, n, (2, nq)), axis=0).astype(np.uint64)
+            lo, hi = np.sort(rng.integers(0, top + 1, (2, nq)), axis=0).astype(np.uint64)
+            step = 100000
+            for f, a in ((wt.rank, (i, lo)), (wt.access, (i,)), (wt.lex_count, (i, j, lo)), (wt.lex_smaller_count, (i, lo)),
+                         (wt.range_count, (i, j, lo, hi)), (wt.select, (np.uint64(1) + i % np.uint64(5000), lo))):
+                got = f(*a)
+                parts = [f(*(x[at:at + step] for x in a)) for at in range(0, nq, step)]
+                got, parts = ([got], [[p] for p in parts]) if not isinstance(got, list) else (got, parts)
+                assert all(np.array_equal(g, np.concatenate([p[c] for p in parts])) for c, g in enumerate(got)), f.__name__
+    finally:
+        wt.free()

@@ -478,11 +478,22 @@ typedef uint32_t wtg_u4_a8 __attribute__((ext_vector_type(4), aligned(8)));
 struct RankAt {
   uint64_t i, base, sub, word;
 };
+__device__ __forceinline__ void rank9_entry(RankAt& a, const uint64_t* __restrict__ D, uint64_t i) {
+  const wtg_u4_a8 d = *reinterpret_cast<const wtg_u4_a8*>(D + 2 * (i >> 9));
+  a.i = i;
+  a.base = (uint64_t)d.x | (uint64_t)d.y << 32;
+  a.sub = (uint64_t)d.z | (uint64_t)d.w << 32;
+}
+__device__ __forceinline__ void rank9_word(RankAt& a, const uint64_t* __restrict__ words, uint64_t W) {
+  const uint64_t k = a.i >> 6;
+  a.word = words[k < W ? k : W - 1];
+}
 __device__ __forceinline__ RankAt rank9_fetch(const uint64_t* __restrict__ D, const uint64_t* __restrict__ words,
                                               uint64_t W, uint64_t i) {
-  const wtg_u4_a8 d = *reinterpret_cast<const wtg_u4_a8*>(D + 2 * (i >> 9));
-  const uint64_t k = i >> 6;
-  return {i, (uint64_t)d.x | (uint64_t)d.y << 32, (uint64_t)d.z | (uint64_t)d.w << 32, words[k < W ? k : W - 1]};
+  RankAt a;
+  rank9_entry(a, D, i);
+  rank9_word(a, words, W);
+  return a;
 }
 __device__ __forceinline__ uint64_t rank9_of(const RankAt& a) {
   const uint32_t lo = (uint32_t)a.i;

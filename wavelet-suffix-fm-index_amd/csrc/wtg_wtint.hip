@@ -7,6 +7,7 @@
 #include "wtg_internal.hpp"
 #include "wtg_order.hpp"
 #include <cstring>
+#include <type_traits>
 
 struct wtg_wtint {
   uint64_t n = 0, sigma = 0, nbits = 0;
@@ -22,6 +23,7 @@ struct WtQ {
   SelQ s1, s0;
   uint64_t n, W;
   uint32_t L;
+  uint32_t apart;  // q_apart
 };
 
 // Every level of a walk looks up two to four positions whose loads do not
@@ -31,7 +33,25 @@ struct WtQ {
 // 540 us, access 850 -> 554, select 953 -> 897, lex_count 1030 -> 843,
 // range_count 2157 -> 1540: 128-byte lines from behind the L2 at 7.4 TB/s, the same in
 // every one of them.  Ordered batches below.
-__device__ __forceinline__ RankAt wt_fetch(const WtQ& w, uint64_t i) { return rank9_fetch(w.D, w.words, w.W, i); }
+// The directory's entries first, then the words (73 -> 64 us of 2^17 lex_counts in 20
+// levels with the two in turn).  APART (q_apart): a lookup's word once its entry is
+// there, and only then the next lookup.
+template <bool APART, uint32_t N>
+__device__ __forceinline__ void wt_fetch(const WtQ& w, const uint64_t (&at)[N], RankAt (&f)[N]) {
+  if constexpr (APART) {
+#pragma unroll
+    for (uint32_t k = 0; k < N; k++) {
+      rank9_entry(f[k], w.D, at[k]);
+      asm volatile("" : "+v"(f[k].base));  // waits for the entry
+      rank9_word(f[k], w.words, w.W);
+    }
+  } else {
+#pragma unroll
+    for (uint32_t k = 0; k < N; k++) rank9_entry(f[k], w.D, at[k]);
+#pragma unroll
+    for (uint32_t k = 0; k < N; k++) rank9_word(f[k], w.words, w.W);
+  }
+}
 
 // A batch's columns as they came and, where it was to be put in order, in order,
 // with the places the queries had; asis: it was in order, the others were not written.
@@ -58,6 +78,23 @@ __device__ __forceinline__ uint64_t q_col(const QBatch& b, const QSlot& s, uint3
   return (s.put ? b.put.c[c] : b.came.c[c])[s.p];
 }
 
+// the walk of c from the root: i becomes rank(i, c), the result the number of values
+// below c in [0, i) (wt_int/wt_int_par.hpp:553-577, :753-780)
+template <bool APART>
+__device__ __forceinline__ uint64_t rank_walk(const WtQ& w, uint64_t& i, uint64_t c) {
+  uint64_t offset = 0, mask = 1ull << (w.L - 1), node_size = w.n, res = 0;
+  for (uint32_t k = 0; k < w.L && i; k++) {
+    RankAt f[3];
+    wt_fetch<APART>(w, {offset, offset + i, offset + node_size}, f);
+    const uint64_t o = rank9_of(f[0]), oi = rank9_of(f[1]) - o, oe = rank9_of(f[2]) - o;
+    if (c & mask) { offset += node_size - oe; node_size = oe; res += i - oi; i = oi; }
+    else { node_size -= oe; i -= oi; }
+    offset += w.n;
+    mask >>= 1;
+  }
+  return res;
+}
+
 __global__ void k_wtint_rank(WtQ w, QBatch b, uint64_t nq, uint64_t* __restrict__ out) {
   const QSlot slot = q_slot(b, nq);
   if (!slot.in) return;
@@ -66,15 +103,8 @@ __global__ void k_wtint_rank(WtQ w, QBatch b, uint64_t nq, uint64_t* __restrict_
   const uint64_t c = q_col(b, slot, 1);
   if (i > w.n) { out[q] = WTG_NONE; return; }
   if (w.L < 64 && (1ull << w.L) <= c) { out[q] = 0; return; }
-  uint64_t offset = 0, mask = 1ull << (w.L - 1), node_size = w.n;
-  for (uint32_t k = 0; k < w.L && i; k++) {
-    const RankAt fo = wt_fetch(w, offset), fi = wt_fetch(w, offset + i), fe = wt_fetch(w, offset + node_size);
-    const uint64_t o = rank9_of(fo), oi = rank9_of(fi) - o, oe = rank9_of(fe) - o;
-    if (c & mask) { offset += node_size - oe; node_size = oe; i = oi; }
-    else { node_size -= oe; i -= oi; }
-    offset += w.n;
-    mask >>= 1;
-  }
+  if (w.apart && !slot.put) rank_walk<true>(w, i, c);
+  else rank_walk<false>(w, i, c);
   out[q] = i;
 }
 
@@ -90,14 +120,14 @@ __device__ __forceinline__ LexWalk lex_begin(const WtQ& w, uint64_t i, uint64_t 
   return x;
 }
 struct LexAt {
-  RankAt o, i, j, e;
+  RankAt f[4];
 };
-__device__ __forceinline__ LexAt lex_fetch(const WtQ& w, const LexWalk& x) {
-  return {wt_fetch(w, x.offset), wt_fetch(w, x.offset + x.i), wt_fetch(w, x.offset + x.j),
-          wt_fetch(w, x.offset + x.size)};
+template <bool APART>
+__device__ __forceinline__ void lex_fetch(const WtQ& w, const LexWalk& x, LexAt& a) {
+  wt_fetch<APART>(w, {x.offset, x.offset + x.i, x.offset + x.j, x.offset + x.size}, a.f);
 }
 __device__ __forceinline__ void lex_step(const WtQ& w, LexWalk& x, const LexAt& a, uint64_t mask) {
-  const uint64_t o = rank9_of(a.o), oi = rank9_of(a.i) - o, oj = rank9_of(a.j) - o, oe = rank9_of(a.e) - o;
+  const uint64_t o = rank9_of(a.f[0]), oi = rank9_of(a.f[1]) - o, oj = rank9_of(a.f[2]) - o, oe = rank9_of(a.f[3]) - o;
   if (x.c & mask) {
     x.offset += x.size - oe;
     x.size = oe;
@@ -112,12 +142,21 @@ __device__ __forceinline__ void lex_step(const WtQ& w, LexWalk& x, const LexAt& 
   }
   x.offset += w.n;
 }
-__device__ __forceinline__ void wtint_lex(const WtQ& w, uint64_t i, uint64_t j, uint64_t c, uint64_t& rk,
+template <bool APART>
+__device__ __forceinline__ void lex_walk(const WtQ& w, LexWalk& x) {
+  uint64_t mask = 1ull << (w.L - 1);
+  for (uint32_t k = 0; k < w.L; k++, mask >>= 1) {
+    LexAt a;
+    lex_fetch<APART>(w, x, a);
+    lex_step(w, x, a, mask);
+  }
+}
+__device__ __forceinline__ void wtint_lex(const WtQ& w, bool apart, uint64_t i, uint64_t j, uint64_t c, uint64_t& rk,
                                           uint64_t& sm, uint64_t& gr) {
   LexWalk x = lex_begin(w, i, j, c);
   if (!x.out) {
-    uint64_t mask = 1ull << (w.L - 1);
-    for (uint32_t k = 0; k < w.L; k++, mask >>= 1) lex_step(w, x, lex_fetch(w, x), mask);
+    if (apart) lex_walk<true>(w, x);
+    else lex_walk<false>(w, x);
   }
   rk = x.i;
   sm = x.smaller;
@@ -130,7 +169,7 @@ __global__ void k_wtint_lex_count(WtQ w, QBatch b, uint64_t nq, uint64_t* __rest
   if (!slot.in) return;
   const uint64_t q = slot.q, i = q_col(b, slot, 0), j = q_col(b, slot, 1), c = q_col(b, slot, 2);
   uint64_t rk = WTG_NONE, sm = WTG_NONE, gr = WTG_NONE;
-  if (i <= j && j <= w.n) wtint_lex(w, i, j, c, rk, sm, gr);
+  if (i <= j && j <= w.n) wtint_lex(w, w.apart && !slot.put, i, j, c, rk, sm, gr);
   out_rank[q] = rk;
   out_smaller[q] = sm;
   out_greater[q] = gr;
@@ -147,15 +186,7 @@ __global__ void k_wtint_lex_smaller(WtQ w, QBatch b, uint64_t nq, uint64_t* __re
   const uint64_t c = q_col(b, slot, 1);
   if (i > w.n) { out_rank[q] = out_smaller[q] = WTG_NONE; return; }
   if (w.L < 64 && (1ull << w.L) <= c) { out_rank[q] = 0; out_smaller[q] = i; return; }
-  uint64_t offset = 0, mask = 1ull << (w.L - 1), node_size = w.n, res = 0;
-  for (uint32_t k = 0; k < w.L && i; k++) {
-    const RankAt fo = wt_fetch(w, offset), fi = wt_fetch(w, offset + i), fe = wt_fetch(w, offset + node_size);
-    const uint64_t o = rank9_of(fo), oi = rank9_of(fi) - o, oe = rank9_of(fe) - o;
-    if (c & mask) { offset += node_size - oe; node_size = oe; res += i - oi; i = oi; }
-    else { node_size -= oe; i -= oi; }
-    offset += w.n;
-    mask >>= 1;
-  }
+  const uint64_t res = w.apart && !slot.put ? rank_walk<true>(w, i, c) : rank_walk<false>(w, i, c);
   out_rank[q] = i;
   out_smaller[q] = res;
 }
@@ -180,14 +211,19 @@ __global__ void k_wtint_range_count(WtQ w, QBatch b, uint64_t nq, uint64_t* __re
   const bool all = w.L < 64 ? vrb >= top - 1 : vrb == ~0ull;
   if (all) hi.smaller = rb + 1 - lb;
   else hi.c = vrb + 1;
-  uint64_t mask = 1ull << (w.L - 1);
-  for (uint32_t k = 0; k < w.L; k++, mask >>= 1) {
-    const LexAt al = lex_fetch(w, lo);
-    LexAt ah{};
-    if (!all) ah = lex_fetch(w, hi);
-    lex_step(w, lo, al, mask);
-    if (!all) lex_step(w, hi, ah, mask);
-  }
+  const auto walk = [&](auto apart) __attribute__((always_inline)) {
+    constexpr bool APART = decltype(apart)::value;
+    uint64_t mask = 1ull << (w.L - 1);
+    for (uint32_t k = 0; k < w.L; k++, mask >>= 1) {
+      LexAt al, ah{};
+      lex_fetch<APART>(w, lo, al);
+      if (!all) lex_fetch<APART>(w, hi, ah);
+      lex_step(w, lo, al, mask);
+      if (!all) lex_step(w, hi, ah, mask);
+    }
+  };
+  if (w.apart) walk(std::true_type{});
+  else walk(std::false_type{});
   out[q] = hi.smaller - lo.smaller;
 }
 
@@ -201,12 +237,13 @@ __global__ void k_wtint_range_half(WtQ w, QBatch b, uint64_t nq, uint64_t* __res
   const uint64_t q = slot.q, lb = q_col(b, slot, 0), rb = q_col(b, slot, 1);
   const uint64_t top = w.L < 64 ? (1ull << w.L) : ~0ull;
   uint64_t v = q_col(b, slot, 2), rk, below, gr;
+  const bool apart = w.apart && !slot.put;
   if (UPPER) {
     const uint64_t low = out[q];
     if (low == WTG_NONE) return;
     if (low == WT_RANGE_EMPTY) { out[q] = 0; return; }
     if (v >= top - (w.L < 64 ? 1 : 0)) below = rb + 1 - lb;  // every value is <= v
-    else wtint_lex(w, lb, rb + 1, v + 1, rk, below, gr);
+    else wtint_lex(w, apart, lb, rb + 1, v + 1, rk, below, gr);
     out[q] = below - low;
   } else {
     uint64_t vrb = q_col(b, slot, 3);
@@ -214,7 +251,7 @@ __global__ void k_wtint_range_half(WtQ w, QBatch b, uint64_t nq, uint64_t* __res
     if (vrb > top) vrb = top;
     if (v > vrb || lb > rb) { out[q] = WT_RANGE_EMPTY; return; }
     if (w.L < 64 && v > top - 1) v = top - 1;
-    wtint_lex(w, lb, rb + 1, v, rk, below, gr);
+    wtint_lex(w, apart, lb, rb + 1, v, rk, below, gr);
     out[q] = below;
   }
 }
@@ -233,9 +270,10 @@ __global__ void k_wtint_access(WtQ w, QBatch b, uint64_t nq, uint64_t* __restric
   uint64_t offset = 0, res = 0, node_size = w.n;
   for (uint32_t k = 0; k < w.L; k++) {
     res <<= 1;
-    const RankAt fo = wt_fetch(w, offset), fi = wt_fetch(w, offset + i), fe = wt_fetch(w, offset + node_size);
-    const uint64_t o = rank9_of(fo), oi = rank9_of(fi) - o, oe = rank9_of(fe) - o;
-    if ((fi.word >> ((offset + i) & 63)) & 1ull) { offset += node_size - oe; node_size = oe; i = oi; res |= 1; }
+    RankAt f[3];
+    wt_fetch<false>(w, {offset, offset + i, offset + node_size}, f);
+    const uint64_t o = rank9_of(f[0]), oi = rank9_of(f[1]) - o, oe = rank9_of(f[2]) - o;
+    if ((f[1].word >> ((offset + i) & 63)) & 1ull) { offset += node_size - oe; node_size = oe; i = oi; res |= 1; }
     else { node_size -= oe; i -= oi; }
     offset += w.n;
   }
@@ -254,8 +292,9 @@ __global__ void k_wtint_select(WtQ w, QBatch b, uint64_t nq, uint64_t* __restric
   uint64_t offset = 0, mask = 1ull << (w.L - 1), node_size = w.n;
   path_off[0] = path_rank[0] = 0;
   for (uint32_t k = 0; k < w.L && node_size; k++) {
-    const RankAt fo = wt_fetch(w, offset), fe = wt_fetch(w, offset + node_size);
-    const uint64_t o = rank9_of(fo), oe = rank9_of(fe) - o;
+    RankAt f[2];
+    wt_fetch<false>(w, {offset, offset + node_size}, f);
+    const uint64_t o = rank9_of(f[0]), oe = rank9_of(f[1]) - o;
     path_rank[k] = o;
     if (c & mask) { offset += node_size - oe; node_size = oe; }
     else node_size -= oe;
@@ -278,7 +317,18 @@ __global__ void k_wtint_select(WtQ w, QBatch b, uint64_t nq, uint64_t* __restric
   out[q] = i - 1;
 }
 
-static WtQ make_q(const wtg_wtint* wt) {
+// Whether a batch of nq symbol queries that is walked as it came takes one lookup's
+// entry and word after the other.  With all of a level in flight at once a large batch on levels larger
+// than an L2 asks for lines again that are on their way: 2^18 lex_counts on 2^27 bits in
+// 4 levels take 2.6 M lines from behind the L2s, and 1.3 M so.
+// us at once -> apart, rank / lex_count:
+//   2^27 bits, 4 levels: 2^17 25 -> 27, 34 -> 32; 2^18 38 -> 31, 59 -> 40; 2^20 113 -> 104, 199 -> 187
+//              8 levels: 2^17 31 -> 34, 46 -> 42; 2^18 53 -> 40, 82 -> 58; 2^20 189 -> 176, 307 -> 313
+//   2^26 bits, 8 levels: 2^17 28 -> 31, 38 -> 38; 2^18 42 -> 37, 63 -> 53; 2^20 136 -> 129, 209 -> 214
+//   2^20 bits, 10 levels: 2^12 17 -> 20, 19 -> 21; 2^18 27 -> 27, 34 -> 34; 2^20 66 -> 71, 90 -> 101
+static bool q_apart(const wtg_wtint* wt, uint64_t nq) { return wt->nbits >= 1ull << 26 && nq >= 1ull << 18; }
+
+static WtQ make_q(const wtg_wtint* wt, uint64_t nq) {
   WtQ w{};
   w.words = wt->words;
   w.D = wt->dir;
@@ -288,6 +338,7 @@ static WtQ make_q(const wtg_wtint* wt) {
   w.n = wt->n;
   w.W = W;
   w.L = wt->L;
+  w.apart = q_apart(wt, nq);
   return w;
 }
 
@@ -466,14 +517,14 @@ extern "C" int wtg_wtint_rank_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uin
   if (!nq) return WTG_OK;
   return q_batch<2>(ctx, wt, QCols{{d_i, d_c}}, 1, nq,
                     [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
-    WTG_LAUNCH(ctx, "wtint_rank", k_wtint_rank, grid, dim3(256), 0, make_q(wt), b, m, d_out + at);
+    WTG_LAUNCH(ctx, "wtint_rank", k_wtint_rank, grid, dim3(256), 0, make_q(wt, nq), b, m, d_out + at);
   });
 }
 static int access_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_i, uint64_t nq, uint64_t* d_sym,
                         uint64_t* d_rank) {
   return q_batch<1>(ctx, wt, QCols{{d_i}}, 0, nq,
                     [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
-    WTG_LAUNCH(ctx, "wtint_access", k_wtint_access, grid, dim3(256), 0, make_q(wt), b, m, d_sym + at,
+    WTG_LAUNCH(ctx, "wtint_access", k_wtint_access, grid, dim3(256), 0, make_q(wt, nq), b, m, d_sym + at,
                d_rank ? d_rank + at : nullptr);
   });
 }
@@ -498,7 +549,7 @@ extern "C" int wtg_wtint_lex_count_batch(wtg_ctx* ctx, const wtg_wtint* wt, cons
   if (!nq) return WTG_OK;
   return q_batch<3>(ctx, wt, QCols{{d_i, d_j, d_c}}, 2, nq,
                     [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
-    WTG_LAUNCH(ctx, "wtint_lex_count", k_wtint_lex_count, grid, dim3(256), 0, make_q(wt), b, m, d_rank + at,
+    WTG_LAUNCH(ctx, "wtint_lex_count", k_wtint_lex_count, grid, dim3(256), 0, make_q(wt, nq), b, m, d_rank + at,
                d_smaller + at, d_greater + at);
   });
 }
@@ -510,7 +561,7 @@ extern "C" int wtg_wtint_lex_smaller_count_batch(wtg_ctx* ctx, const wtg_wtint* 
   if (!nq) return WTG_OK;
   return q_batch<2>(ctx, wt, QCols{{d_i, d_c}}, 1, nq,
                     [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
-    WTG_LAUNCH(ctx, "wtint_lex_smaller", k_wtint_lex_smaller, grid, dim3(256), 0, make_q(wt), b, m, d_rank + at,
+    WTG_LAUNCH(ctx, "wtint_lex_smaller", k_wtint_lex_smaller, grid, dim3(256), 0, make_q(wt, nq), b, m, d_rank + at,
                d_smaller + at);
   });
 }
@@ -528,17 +579,17 @@ extern "C" int wtg_wtint_range_count_batch(wtg_ctx* ctx, const wtg_wtint* wt, co
   if (scratch) {
     WTG_TRY(q_ordered<4>(ctx, scratch, QCols{{d_lb, d_rb, d_vlb, d_vrb}}, 2, nq,
                          [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
-      WTG_LAUNCH(ctx, "wtint_range_lower", k_wtint_range_half<false>, grid, dim3(256), 0, make_q(wt), b, m,
+      WTG_LAUNCH(ctx, "wtint_range_lower", k_wtint_range_half<false>, grid, dim3(256), 0, make_q(wt, nq), b, m,
                  d_out + at);
     }));
     WTG_TRY(q_ordered<3>(ctx, scratch, QCols{{d_lb, d_rb, d_vrb}}, 2, nq,
                          [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
-      WTG_LAUNCH(ctx, "wtint_range_upper", k_wtint_range_half<true>, grid, dim3(256), 0, make_q(wt), b, m,
+      WTG_LAUNCH(ctx, "wtint_range_upper", k_wtint_range_half<true>, grid, dim3(256), 0, make_q(wt, nq), b, m,
                  d_out + at);
     }));
   } else {
     WTG_LAUNCH(ctx, "wtint_range_count", k_wtint_range_count, dim3((unsigned)wtg_ceil_div(nq, 256)), dim3(256), 0,
-               make_q(wt), QBatch{{{d_lb, d_rb, d_vlb, d_vrb}}, {}, nullptr, nullptr}, nq, d_out);
+               make_q(wt, nq), QBatch{{{d_lb, d_rb, d_vlb, d_vrb}}, {}, nullptr, nullptr}, nq, d_out);
     WTG_LAUNCH_CHECK();
   }
   return wtg_finish(ctx);
@@ -551,8 +602,8 @@ extern "C" int wtg_wtint_select_batch(wtg_ctx* ctx, const wtg_wtint* wt, const u
   return q_batch<2>(ctx, wt, QCols{{d_i, d_c}}, 1, nq,
                     [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
     if (wt->L <= 24)
-      WTG_LAUNCH(ctx, "wtint_select", k_wtint_select<24>, grid, dim3(256), 0, make_q(wt), b, m, d_out + at);
+      WTG_LAUNCH(ctx, "wtint_select", k_wtint_select<24>, grid, dim3(256), 0, make_q(wt, nq), b, m, d_out + at);
     else
-      WTG_LAUNCH(ctx, "wtint_select", k_wtint_select<64>, grid, dim3(256), 0, make_q(wt), b, m, d_out + at);
+      WTG_LAUNCH(ctx, "wtint_select", k_wtint_select<64>, grid, dim3(256), 0, make_q(wt, nq), b, m, d_out + at);
   });
 }
