@@ -125,6 +125,17 @@ def test_ordered_patterns(ctx, m):
         wt.free()
 
 
+@pytest.fixture(scope="module")
+def wide(ctx):
+    """2^26 level bits in 16 levels: symbol batches of 2^18 queries are put in order."""
+    n = (1 << 22) + 5
+    s = np.random.default_rng(6).integers(0, 1 << 16, n)
+    s[::3] = 777
+    wt = ctx.wtint_build(ctx.to_device(s.astype(np.uint16)), n, 16)
+    yield wt
+    wt.free()
+
+
 def in_runs(rng, x, runs, down):
     """x rearranged as `runs` sorted stretches of one length, up or down."""
     x = np.array_split(rng.permutation(x), runs)
@@ -133,10 +144,10 @@ def in_runs(rng, x, runs, down):
 
 @pytest.mark.parametrize("nq", [1 << 18, (1 << 20) + 5])
 @pytest.mark.parametrize("runs,down", [(1, False), (1, True), (15, False), (16, True), (17, False), (40, True)])
-def test_batch_in_order(ctx, large, nq, runs, down):
+def test_batch_in_order(ctx, wide, nq, runs, down):
     """Batches that come in order, up or down, in few runs or in more than count as order,
     give what the same queries give in small batches, as they came."""
-    wt, rng = large, np.random.default_rng(nq + runs)
+    wt, rng = wide, np.random.default_rng(nq + runs)
     n, top = wt.n, 1 << wt.L
     i, j = (in_runs(rng, rng.integers(0, n, nq).astype(np.uint64), runs, down) for _ in range(2))
     lo, hi = (in_runs(rng, rng.integers(0, top, nq).astype(np.uint64), runs, down) for _ in range(2))
@@ -175,11 +186,11 @@ def test_patterns_in_order(ctx, m):
         wt.free()
 
 
-def test_captured_batches(wsfm, ctx, large):
+def test_captured_batches(wsfm, ctx, wide):
     """Large batches recorded as a graph (answered as they come, with no block shared with
     other work), replayed over other queries in the same place."""
     import ctypes as C
-    hip, wt, nq = wsfm.lib(), large, 1 << 18
+    hip, wt, nq = wsfm.lib(), wide, 1 << 18
     stream = C.c_void_p(hip.wtg_ctx_stream(ctx.h))
     rng = np.random.default_rng(9)
     i, c, out, inv = (ctx.empty(nq) for _ in range(4))
@@ -227,3 +238,13 @@ def test_large_batch_on_few_levels(ctx, levels):
                 assert all(np.array_equal(g, np.concatenate([p[c] for p in parts])) for c, g in enumerate(got)), f.__name__
     finally:
         wt.free()
+
+
+@pytest.mark.parametrize("nq", [1 << 18, (1 << 19) + 2049])
+@pytest.mark.parametrize("keys", ["any", "one", "few", "refused"])
+def test_ordered_batch_on_many_levels(ctx, wide, nq, keys):
+    test_ordered_batch(ctx, wide, nq, keys)
+
+
+def test_ordered_answers_over_their_queries_on_many_levels(ctx, wide):
+    test_ordered_answers_over_their_queries(ctx, wide)

@@ -8,7 +8,7 @@
 // an eighth of them, and an XCD's queries in flight share a small part of every
 // level.  Answers are written where the query stood.  A batch whose sample is in
 // order is walked as it came.  What it measured stands with the rules of its users
-// (order_pays, fm_order_pays).
+// (the order_pays functions).
 #pragma once
 #include "wtg_internal.hpp"
 

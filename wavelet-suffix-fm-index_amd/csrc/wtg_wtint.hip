@@ -7,7 +7,6 @@
 #include "wtg_internal.hpp"
 #include "wtg_order.hpp"
 #include <cstring>
-#include <type_traits>
 
 struct wtg_wtint {
   uint64_t n = 0, sigma = 0, nbits = 0;
@@ -33,23 +32,14 @@ struct WtQ {
 // 540 us, access 850 -> 554, select 953 -> 897, lex_count 1030 -> 843,
 // range_count 2157 -> 1540: 128-byte lines from behind the L2 at 7.4 TB/s, the same in
 // every one of them.  Ordered batches below.
-// The directory's entries first, then the words (73 -> 64 us of 2^17 lex_counts in 20
-// levels with the two in turn).  APART (q_apart): a lookup's word once its entry is
-// there, and only then the next lookup.
+// APART (q_apart): a lookup's word once its entry is there, and only then the next lookup.
 template <bool APART, uint32_t N>
 __device__ __forceinline__ void wt_fetch(const WtQ& w, const uint64_t (&at)[N], RankAt (&f)[N]) {
-  if constexpr (APART) {
 #pragma unroll
-    for (uint32_t k = 0; k < N; k++) {
-      rank9_entry(f[k], w.D, at[k]);
-      asm volatile("" : "+v"(f[k].base));  // waits for the entry
-      rank9_word(f[k], w.words, w.W);
-    }
-  } else {
-#pragma unroll
-    for (uint32_t k = 0; k < N; k++) rank9_entry(f[k], w.D, at[k]);
-#pragma unroll
-    for (uint32_t k = 0; k < N; k++) rank9_word(f[k], w.words, w.W);
+  for (uint32_t k = 0; k < N; k++) {
+    rank9_entry(f[k], w.D, at[k]);
+    if constexpr (APART) asm volatile("" : "+v"(f[k].base));  // waits for the entry
+    rank9_word(f[k], w.words, w.W);
   }
 }
 
@@ -196,6 +186,7 @@ __global__ void k_wtint_lex_smaller(WtQ w, QBatch b, uint64_t nq, uint64_t* __re
 // lex_count "smaller" counts over [lb, rb + 1).  The reference clamps vrb to 2^L
 // and its leaf test does not compare vlb, so vlb = 2^L counts the value 2^L - 1:
 // vlb is clamped to 2^L - 1 the same way.
+template <bool APART>
 __global__ void k_wtint_range_count(WtQ w, QBatch b, uint64_t nq, uint64_t* __restrict__ out) {
   const uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= nq) return;
@@ -211,19 +202,14 @@ __global__ void k_wtint_range_count(WtQ w, QBatch b, uint64_t nq, uint64_t* __re
   const bool all = w.L < 64 ? vrb >= top - 1 : vrb == ~0ull;
   if (all) hi.smaller = rb + 1 - lb;
   else hi.c = vrb + 1;
-  const auto walk = [&](auto apart) __attribute__((always_inline)) {
-    constexpr bool APART = decltype(apart)::value;
-    uint64_t mask = 1ull << (w.L - 1);
-    for (uint32_t k = 0; k < w.L; k++, mask >>= 1) {
-      LexAt al, ah{};
-      lex_fetch<APART>(w, lo, al);
-      if (!all) lex_fetch<APART>(w, hi, ah);
-      lex_step(w, lo, al, mask);
-      if (!all) lex_step(w, hi, ah, mask);
-    }
-  };
-  if (w.apart) walk(std::true_type{});
-  else walk(std::false_type{});
+  uint64_t mask = 1ull << (w.L - 1);
+  for (uint32_t k = 0; k < w.L; k++, mask >>= 1) {
+    LexAt al, ah{};
+    lex_fetch<APART>(w, lo, al);
+    if (!all) lex_fetch<APART>(w, hi, ah);
+    lex_step(w, lo, al, mask);
+    if (!all) lex_step(w, hi, ah, mask);
+  }
   out[q] = hi.smaller - lo.smaller;
 }
 
@@ -465,16 +451,36 @@ static int q_check(wtg_ctx* ctx, const wtg_wtint* wt, uint64_t nq, const void* a
 }
 
 // Whether ordering a batch pays: level bits too many for an XCD's L2 beside the
-// directory, and queries enough for the three passes before the walk (~25 us).
-// us as it came -> ordered, rank / access / select / lex_count / range_count:
-//   2^23 bits, 2^20 queries:  81 -> 103,  81 -> 81,  164 -> 159, 126 -> 144,  222 -> 281
-//   2^24 bits, 2^18 queries:  63 -> 58,   62 -> 72,  104 -> 103,  78 -> 72,   129 -> 133
-//              2^20 queries: 220 -> 123, 217 -> 187, 366 -> 244, 284 -> 171,  502 -> 334
-//   2^27 bits, 2^17 queries:  53 -> 52,   52 -> 59,   89 -> 92,   71 -> 65,   112 -> 129
-//              2^18 queries:  94 -> 71,   94 -> 86,  154 -> 117, 130 -> 95,   211 -> 183
-//   2^28.3 bits, 2^20:       569 -> 275, 580 -> 323, 928 -> 521, 885 -> 503, 1487 -> 940
-static bool order_pays(const wtg_wtint* wt, uint64_t nq) {
-  return wt->nbits >= 1ull << 24 && nq >= (wt->nbits >= 1ull << 26 ? 1ull << 18 : 1ull << 19);
+// directory, and queries enough for the three passes before the walk (17 to 30 us; 9 us
+// where the sample shows a batch in order).  By symbol it needs symbols enough, too: on
+// few levels the queries share the lines as they come.
+// us as it came -> ordered, uniform symbols / a few of them common:
+//   rank        2^24 bits, 16 levels, 2^18: 70 -> 58 / 64 -> 60;   2^19: 134 -> 80 / 119 -> 84
+//               2^26 bits, 12 levels, 2^18: 70 -> 58 / 61 -> 64;   2^19: 129 -> 80 / 110 -> 94
+//               2^27 bits, 10 levels, 2^18:  55 -> 60 / 48 -> 67;  2^19: 111 -> 83 / 97 -> 103
+//               2^27 bits,  8 levels, 2^19:  87 -> 81 / 83 -> 105; 2^20: 183 -> 126 / 176 -> 178
+//                           4 levels, 2^20: 103 -> 111 / 104 -> 133
+//               2^28.3 bits, 20 levels, 2^17: 78 -> 61 / 70 -> 62; 2^18: 147 -> 82 / 139 -> 92; 2^20: 592 -> 210 / 578 -> 274
+//   select      2^26 bits, 16 levels, 2^18: 128 -> 101 / 114 -> 112; 2^20: 452 -> 241 / 374 -> 256
+//               2^27 bits,  8 levels, 2^18:  53 -> 66 / 51 -> 70;  2^19: 86 -> 86 / 77 -> 92; 2^25: 2^19 85 -> 87 / 591 -> 414
+//   lex_count   2^26 bits, 12 levels, 2^18: 95 -> 75 / 87 -> 84;   2^27, 8, 2^20: 313 -> 202 / 313 -> 302
+//   range_count (two walks, each with its own order)
+//               2^26 bits, 12 levels, 2^18: 155 -> 138 / 140 -> 154; 16 levels: 197 -> 148 / 188 -> 161
+//   access (by position)
+//               2^24 bits, 16 levels, 2^19: 132 -> 139 / 118 -> 116; 2^20: 257 -> 246 / 226 -> 196
+//               2^26 bits, 20 levels, 2^18: 111 -> 117 / 96 -> 94;   2^19: 214 -> 204 / 187 -> 154
+//               2^27 bits,  4 levels, 2^18:  36 -> 44 / 37 -> 43;    2^19:  61 -> 55 / 61 -> 54
+//               2^27 bits,  8 levels, 2^18:  54 -> 53 / 52 -> 49;    2^20: 191 -> 114 / 188 -> 92
+static bool order_pays_position(const wtg_wtint* wt, uint64_t nq) {
+  return wt->nbits >= 1ull << 24 && nq >= (wt->nbits >= 1ull << 27 && wt->L >= 8 ? 1ull << 18 : 1ull << 19);
+}
+static bool order_pays_symbol(const wtg_wtint* wt, uint64_t nq, uint32_t walks = 1) {
+  if (wt->nbits < 1ull << 24 || wt->L < 8) return false;
+  if (wt->L < 10) return nq >= 15ull << 16;
+  return nq >= (wt->L >= 12 && wt->nbits >= 1ull << 26 && (walks == 1 || wt->L >= 16) ? 1ull << 18 : 1ull << 19);
+}
+static bool order_pays_select(const wtg_wtint* wt, uint64_t nq) {
+  return order_pays_symbol(wt, nq) || (wt->nbits >= 1ull << 24 && wt->L >= 8 && nq >= 1ull << 19);
 }
 
 // A batch in chunks: walk(batch, queries, answers' offset, grid) launches the kernel
@@ -498,9 +504,9 @@ static int q_ordered(wtg_ctx* ctx, char* scratch, const QCols& in, uint32_t key,
 
 // The batch as it came, or ordered by column `key` where that pays.
 template <uint32_t NC, class F>
-static int q_batch(wtg_ctx* ctx, const wtg_wtint* wt, const QCols& in, uint32_t key, uint64_t nq, F&& walk) {
+static int q_batch(wtg_ctx* ctx, const QCols& in, uint32_t key, bool pays, uint64_t nq, F&& walk) {
   WTG_TRY(wtg_set_device(ctx));
-  char* scratch = order_pays(wt, nq) ? (char*)wtg_query_scratch(ctx, QO_BYTES) : nullptr;
+  char* scratch = pays ? (char*)wtg_query_scratch(ctx, QO_BYTES) : nullptr;
   if (scratch) {
     WTG_TRY(q_ordered<NC>(ctx, scratch, in, key, nq, walk));
   } else {
@@ -515,14 +521,14 @@ extern "C" int wtg_wtint_rank_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uin
   WTG_TRY(q_check(ctx, wt, nq, d_i, d_out));
   WTG_REQUIRE(nq == 0 || d_c, "null d_c");
   if (!nq) return WTG_OK;
-  return q_batch<2>(ctx, wt, QCols{{d_i, d_c}}, 1, nq,
+  return q_batch<2>(ctx, QCols{{d_i, d_c}}, 1, order_pays_symbol(wt, nq), nq,
                     [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
     WTG_LAUNCH(ctx, "wtint_rank", k_wtint_rank, grid, dim3(256), 0, make_q(wt, nq), b, m, d_out + at);
   });
 }
 static int access_batch(wtg_ctx* ctx, const wtg_wtint* wt, const uint64_t* d_i, uint64_t nq, uint64_t* d_sym,
                         uint64_t* d_rank) {
-  return q_batch<1>(ctx, wt, QCols{{d_i}}, 0, nq,
+  return q_batch<1>(ctx, QCols{{d_i}}, 0, order_pays_position(wt, nq), nq,
                     [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
     WTG_LAUNCH(ctx, "wtint_access", k_wtint_access, grid, dim3(256), 0, make_q(wt, nq), b, m, d_sym + at,
                d_rank ? d_rank + at : nullptr);
@@ -547,7 +553,7 @@ extern "C" int wtg_wtint_lex_count_batch(wtg_ctx* ctx, const wtg_wtint* wt, cons
   WTG_TRY(q_check(ctx, wt, nq, d_i, d_rank));
   WTG_REQUIRE(nq == 0 || (d_j && d_c && d_smaller && d_greater), "null argument");
   if (!nq) return WTG_OK;
-  return q_batch<3>(ctx, wt, QCols{{d_i, d_j, d_c}}, 2, nq,
+  return q_batch<3>(ctx, QCols{{d_i, d_j, d_c}}, 2, order_pays_symbol(wt, nq), nq,
                     [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
     WTG_LAUNCH(ctx, "wtint_lex_count", k_wtint_lex_count, grid, dim3(256), 0, make_q(wt, nq), b, m, d_rank + at,
                d_smaller + at, d_greater + at);
@@ -559,7 +565,7 @@ extern "C" int wtg_wtint_lex_smaller_count_batch(wtg_ctx* ctx, const wtg_wtint* 
   WTG_TRY(q_check(ctx, wt, nq, d_i, d_rank));
   WTG_REQUIRE(nq == 0 || (d_c && d_smaller), "null argument");
   if (!nq) return WTG_OK;
-  return q_batch<2>(ctx, wt, QCols{{d_i, d_c}}, 1, nq,
+  return q_batch<2>(ctx, QCols{{d_i, d_c}}, 1, order_pays_symbol(wt, nq), nq,
                     [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
     WTG_LAUNCH(ctx, "wtint_lex_smaller", k_wtint_lex_smaller, grid, dim3(256), 0, make_q(wt, nq), b, m, d_rank + at,
                d_smaller + at);
@@ -575,7 +581,7 @@ extern "C" int wtg_wtint_range_count_batch(wtg_ctx* ctx, const wtg_wtint* wt, co
   // the second walk reads the batch after the first has written: not over its own answers
   bool apart = true;
   for (const uint64_t* x : {d_lb, d_rb, d_vlb, d_vrb}) apart = apart && (x + nq <= d_out || d_out + nq <= x);
-  char* scratch = apart && order_pays(wt, nq) ? (char*)wtg_query_scratch(ctx, QO_BYTES) : nullptr;
+  char* scratch = apart && order_pays_symbol(wt, nq, 2) ? (char*)wtg_query_scratch(ctx, QO_BYTES) : nullptr;
   if (scratch) {
     WTG_TRY(q_ordered<4>(ctx, scratch, QCols{{d_lb, d_rb, d_vlb, d_vrb}}, 2, nq,
                          [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
@@ -588,8 +594,12 @@ extern "C" int wtg_wtint_range_count_batch(wtg_ctx* ctx, const wtg_wtint* wt, co
                  d_out + at);
     }));
   } else {
-    WTG_LAUNCH(ctx, "wtint_range_count", k_wtint_range_count, dim3((unsigned)wtg_ceil_div(nq, 256)), dim3(256), 0,
-               make_q(wt, nq), QBatch{{{d_lb, d_rb, d_vlb, d_vrb}}, {}, nullptr, nullptr}, nq, d_out);
+    const dim3 grid((unsigned)wtg_ceil_div(nq, 256));
+    const QBatch b{{{d_lb, d_rb, d_vlb, d_vrb}}, {}, nullptr, nullptr};
+    if (q_apart(wt, nq))
+      WTG_LAUNCH(ctx, "wtint_range_count", k_wtint_range_count<true>, grid, dim3(256), 0, make_q(wt, nq), b, nq, d_out);
+    else
+      WTG_LAUNCH(ctx, "wtint_range_count", k_wtint_range_count<false>, grid, dim3(256), 0, make_q(wt, nq), b, nq, d_out);
     WTG_LAUNCH_CHECK();
   }
   return wtg_finish(ctx);
@@ -599,7 +609,7 @@ extern "C" int wtg_wtint_select_batch(wtg_ctx* ctx, const wtg_wtint* wt, const u
   WTG_TRY(q_check(ctx, wt, nq, d_i, d_out));
   WTG_REQUIRE(nq == 0 || d_c, "null d_c");
   if (!nq) return WTG_OK;
-  return q_batch<2>(ctx, wt, QCols{{d_i, d_c}}, 1, nq,
+  return q_batch<2>(ctx, QCols{{d_i, d_c}}, 1, order_pays_select(wt, nq), nq,
                     [&](const QBatch& b, uint64_t m, uint64_t at, dim3 grid) {
     if (wt->L <= 24)
       WTG_LAUNCH(ctx, "wtint_select", k_wtint_select<24>, grid, dim3(256), 0, make_q(wt, nq), b, m, d_out + at);
