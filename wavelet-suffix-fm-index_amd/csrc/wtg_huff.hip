@@ -1621,13 +1621,17 @@ extern "C" int wtg_huff_select_batch(wtg_ctx* ctx, const wtg_huff* wt, const uin
   return wtg_finish(ctx);
 }
 // Whether ordering a batch of patterns pays: index bits too many for an XCD's L2,
-// patterns enough for the five passes before the search (~70 us with the rows), and
-// not so long that the steps past the ordered bytes outweigh the first.  DNA, 20-byte
-// patterns, us as they came -> ordered:
-//   2^25 symbols (2^26.2 bits): 2^18 167 -> 172, 2^19 302 -> 280, 2^20 558 -> 494
-//   (of which the search 431; all eight bytes sorted, not 256 parts of them: 357);
-//   12 bytes, 2^20: 336 -> 299; 32 bytes: 907 -> 893; 8 bytes: 203 -> 203
-//   2^24 symbols, 2^20: 520 -> 481 (32 bytes 858 -> 857); 2^22 symbols, 2^20: 431 -> 446
+// patterns enough for the four passes before the search (~60 us with the rows; 10 us
+// where the sample shows a batch in order), and not so long that the steps past the
+// ordered bytes outweigh the first.  DNA, us as they came -> ordered, patterns as drawn / sorted
+// from their first byte on:
+//   2^25 symbols (2^26.2 bits), 20 bytes: 2^18 167 -> 170, 2^19 306 -> 290 / 279 -> 281,
+//   2^20 579 -> 522 / 509 -> 502 (of which the search 413; all eight bytes sorted, not 256
+//   parts of them: 357); 2^20 of 12 bytes 345 -> 313, of 32 bytes 953 -> 885
+//   2^24 symbols (2^25.2 bits), 20 bytes: 2^19 291 -> 279 / 263 -> 271, 2^20 552 -> 503 / 472 -> 509
+//   2^23 symbols: 2^20 482 -> 489 / 413 -> 464
+// The line is at 2^26 bits, above which sorted patterns lose nothing: at 2^25.2 they
+// lose as much as patterns in no order gain.
 static bool fm_order_pays(const wtg_huff* wt, uint32_t m, uint64_t npat) {
   return wt->shape.bv_size >= 1ull << 26 && npat >= 1ull << 19 && m >= 12 && m <= 32;
 }
