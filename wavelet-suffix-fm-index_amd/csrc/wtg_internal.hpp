@@ -499,9 +499,6 @@ __device__ __forceinline__ uint64_t rank9_of(const RankAt& a) {
   const uint32_t lo = (uint32_t)a.i;
   return a.base + ((a.sub >> (63 - 9 * ((lo >> 6) & 7))) & 0x1FF) + popc64(a.word & ((1ull << (lo & 63)) - 1));
 }
-__device__ __forceinline__ int bit_dev(const uint64_t* __restrict__ words, uint64_t i) {
-  return (int)((words[i >> 6] >> (i & 63)) & 1ull);
-}
 
 struct SelQ {
   const uint64_t* superblock;

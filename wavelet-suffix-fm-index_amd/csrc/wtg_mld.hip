@@ -543,7 +543,7 @@ __global__ __launch_bounds__(T / 8) __attribute__((amdgpu_waves_per_eu(8))) void
   __shared__ uint16_t s_tpre[(1u << MLD_GMAX) + 1];   // exclusive prefix over d of the tile's counts
   __shared__ __align__(8) uint32_t s_bits[MLD_GMAX][BW];  // level bits in the tile's level order
   static_assert(BW % 2 == 0, "64-bit rows");
-  __shared__ uint16_t s_xy[2u << MLD_GMAX];          // node tables of the levels (see below)
+  __shared__ __align__(4) uint16_t s_xy[2u << MLD_GMAX];  // node tables of the levels (see below)
   __shared__ uint32_t s_lvl0[MLD_GMAX];
   __shared__ uint32_t s_wave[4];
   __shared__ uint32_t s_wz[MLD_GMAX][8];              // per level and wave: zeros in the waves before it
