@@ -42,3 +42,26 @@ def test_split_schedule_itself(ctx):
     finally:
         ctx.set_level_method(0)
     assert np.array_equal(w, closed_form(s, L))
+
+
+@pytest.mark.parametrize("n,values", [(2000003, 1000), (3000017, 1500), (6000011, 4000)])
+@pytest.mark.parametrize("L,dt", [(24, np.uint32), (40, np.uint64)])
+def test_many_large_nodes(ctx, n, values, L, dt):
+    """Up to some thousands of values with 1500 to 2000 keys each: lists of large nodes on
+    either side of the size that one launch makes the tables of."""
+    rng = np.random.default_rng(n + L)
+    s = rng.integers(0, (1 << L) - 1, values, dtype=np.uint64, endpoint=True)[rng.integers(0, values, n)].astype(dt)
+    d, w, w1 = ctx.to_device(s), ctx.empty((n * L + 63) // 64), ctx.empty((n * L + 63) // 64)
+    try:
+        ctx.levels_build(d, n, L, w)
+        ctx.set_level_method(1)
+        ctx.levels_build(d, n, L, w1)
+        assert np.array_equal(w.get(), w1.get())
+        ctx.set_level_method(0)
+        wt = ctx.wtint_build(d, n, L)
+        assert wt.sigma == np.unique(s).size
+        wt.free()
+    finally:
+        ctx.set_level_method(0)
+        for x in (d, w, w1):
+            x.free()

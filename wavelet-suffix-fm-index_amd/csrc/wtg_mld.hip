@@ -77,10 +77,6 @@ struct MldArgs {
   uint32_t* err;
 };
 
-__device__ __forceinline__ uint32_t mld_ntiles(const MldArgs& a) {
-  return a.s == 0 ? a.ntiles0 : a.tstart[a.nseg];
-}
-
 // tile t -> (segment, first key in P_s, keys, first tile of the segment)
 __device__ __forceinline__ bool mld_tile(const MldArgs& a, uint32_t t, uint32_t& seg, uint64_t& base,
                                          uint32_t& len, uint32_t& first) {
@@ -494,20 +490,6 @@ __global__ __launch_bounds__(256) void k_mld_tseg(const uint32_t* __restrict__ t
     if (tstart[mid] <= t) lo = mid; else hi = mid;
   }
   tseg[t] = (uint32_t)lo;
-}
-
-// inclusive prefix sum over the 64 lanes with DPP moves (no LDS round trip):
-// row_shr 1, 2, 4, 8 scan each 16-lane row (lanes shifted in from outside the
-// row read 0), then row_bcast 15 adds row 0's total to row 1 and row 2's to
-// row 3, and row_bcast 31 adds the total of rows 0-1 to rows 2-3
-__device__ __forceinline__ uint32_t wave_incl_scan_dpp(uint32_t v) {
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);
-  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);
-  return v;
 }
 
 // 64 bits of an LDS bit array from bit position p (p + 64 < bits + 64 pad)
@@ -1216,6 +1198,8 @@ struct LocArgs {
   uint64_t* words;            // level l's bits at bit l * n
   unsigned long long* distinct;  // nullable: += the nodes that level L would have
   uint32_t* err;
+  const uint32_t* left;       // modes 1 and 2, nullable: the large nodes left,
+  uint32_t* tell;             // for the host here (pinned)
 };
 
 // the first i in [0, m] with st[i] >= v, where st[m] stands for a value >= v
@@ -1254,6 +1238,8 @@ __global__ __launch_bounds__(256) void k_mld_local(LocArgs a) {
   __shared__ uint32_t s_flag[2];
   const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t lane = (uint32_t)lane_id();
+  if (a.left && blockIdx.x == 0 && threadIdx.x == 0)
+    __hip_atomic_store(a.tell, *a.left, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   // the block's keys: [a0, a0 + len) of P_s
   uint32_t a0 = 0, len = 0;
   if (a.mode == 0) {
@@ -1435,6 +1421,37 @@ __global__ __launch_bounds__(256) void k_mld_list_tiles(const uint32_t* __restri
   nt[i] = i < *nb ? (uint32_t)(((uint64_t)bc[i] + (1u << tl) - 1) >> tl) : 0u;
 }
 
+// The tiles of a list of at most LIST_ONE segments in one launch: their count per
+// segment (none past the list), first tiles and the tile -> segment map, for which four
+// launches (k_mld_list_tiles, a fill, a scan, k_mld_tseg) take the other lists.
+constexpr uint32_t LIST_ONE = 1024;
+__global__ __launch_bounds__(LIST_ONE) void k_mld_list(const uint32_t* __restrict__ bc, const uint32_t* __restrict__ nb,
+                                                       uint32_t cap, uint32_t tl, uint32_t* __restrict__ tst,
+                                                       uint32_t* __restrict__ tseg, uint64_t maxtiles) {
+  __shared__ uint32_t s_st[LIST_ONE + 1], s_w[LIST_ONE / 64];
+  const uint32_t t = threadIdx.x, w = t >> 6;
+  const uint32_t n = t < cap && t < *nb ? (uint32_t)(((uint64_t)bc[t] + (1u << tl) - 1) >> tl) : 0u;
+  const uint32_t incl = wave_incl_sum_dpp(n);
+  if ((t & 63) == 63) s_w[w] = incl;
+  __syncthreads();
+  uint32_t st = incl - n;
+  for (uint32_t k = 0; k < w; k++) st += s_w[k];
+  s_st[t] = st;
+  if (t == LIST_ONE - 1) s_st[LIST_ONE] = st + n;
+  __syncthreads();
+  if (t < cap) tst[t] = st;
+  const uint32_t total = s_st[cap];
+  if (t == 0) tst[cap] = total;
+  for (uint32_t k = t; k < total && k < maxtiles; k += LIST_ONE) {
+    uint32_t lo = 0, hi = cap;  // s_st[lo] <= k < s_st[hi]
+    while (hi - lo > 1) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (s_st[mid] <= k) lo = mid; else hi = mid;
+    }
+    tseg[k] = lo;
+  }
+}
+
 // per listed segment (a block each): its leaves' starts, the large leaves as
 // the next list, or (last group) its distinct leaves
 __global__ __launch_bounds__(256) void k_mld_leaf(MldArgs a, uint32_t* __restrict__ lst, const uint32_t* __restrict__ nb,
@@ -1533,9 +1550,6 @@ int mld_sparse_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint64_t*
   q.s = S;
   q.mode = 1;
   q.st = cum;
-  q.m = 1u << S;
-  mld_local_launch<KO>(ctx, (unsigned)wtg_ceil_div(n, LOC_W), q);
-  WTG_LAUNCH_CHECK();
   // how many large nodes are left: read back where the call waits in any case (in
   // a blocking context, or for the distinct count, and not while the stream is
   // being captured), so that no empty round is launched.  Otherwise the call only
@@ -1545,11 +1559,18 @@ int mld_sparse_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint64_t*
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   WTG_CHECK_HIP(hipStreamIsCapturing(ctx->stream, &cs));
   const bool ask = (ctx->blocking || d_distinct) && cs == hipStreamCaptureStatusNone;
+  // (the small nodes' kernel stores it to pinned memory: a read is a wait, without a copy)
+  q.m = 1u << S;
+  q.left = ask ? nb : nullptr;
+  q.tell = (uint32_t*)((char*)ctx->d_flag + WTG_STAGE_AUX + 64);
+  mld_local_launch<KO>(ctx, (unsigned)wtg_ceil_div(n, LOC_W), q);
+  WTG_LAUNCH_CHECK();
   uint32_t cur = 0;
   for (uint32_t s = S; s < L;) {
     uint32_t hb = cap;
     if (ask) {
-      WTG_TRY(wtg_stage_d2h(ctx, &hb, nb + 2 * cur, 4));
+      WTG_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+      hb = *reinterpret_cast<volatile uint32_t*>(ctx->h_stage + WTG_STAGE_AUX + 64);
       if (hb > cap) hb = cap;  // (flagged on the device)
       if (hb == 0) break;
     }
@@ -1587,16 +1608,22 @@ int mld_sparse_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint64_t*
     a.words = d_words;
     a.kout = last ? nullptr : kbuf[kb ^ 1];
     a.err = ctx->d_flag;
-    WTG_LAUNCH(ctx, "mld_ntiles", k_mld_list_tiles, dim3(sgrid), dim3(256), 0, bc, nb + 2 * cur, hb,
-               (uint32_t*)(ws + o_nt), 11u);
-    WTG_LAUNCH_CHECK();
-    WTG_TRY(wtg_fill_bytes_zero(ctx, scst, (char*)ctr + 256 - (char*)scst));
-    WTG_LAUNCH(ctx, "mld_tiles", k_scan_u32<uint32_t>, dim3(stiles), dim3(256), 0, (uint32_t*)(ws + o_nt), tst,
-               (uint64_t)hb, scst, ctr, ctx->d_flag);
-    WTG_LAUNCH_CHECK();
-    WTG_LAUNCH(ctx, "mld_tseg", k_mld_tseg, dim3((unsigned)wtg_ceil_div(grid, 256)), dim3(256), 0, tst, (uint64_t)hb,
-               (uint32_t*)(ws + o_tseg), maxt);
-    WTG_LAUNCH_CHECK();
+    if (hb <= LIST_ONE) {
+      WTG_LAUNCH(ctx, "mld_tiles", k_mld_list, dim3(1), dim3(LIST_ONE), 0, bc, nb + 2 * cur, hb, 11u, tst,
+                 (uint32_t*)(ws + o_tseg), maxt);
+      WTG_LAUNCH_CHECK();
+    } else {
+      WTG_LAUNCH(ctx, "mld_ntiles", k_mld_list_tiles, dim3(sgrid), dim3(256), 0, bc, nb + 2 * cur, hb,
+                 (uint32_t*)(ws + o_nt), 11u);
+      WTG_LAUNCH_CHECK();
+      WTG_TRY(wtg_fill_bytes_zero(ctx, scst, (char*)ctr + 256 - (char*)scst));
+      WTG_LAUNCH(ctx, "mld_tiles", k_scan_u32<uint32_t>, dim3(stiles), dim3(256), 0, (uint32_t*)(ws + o_nt), tst,
+                 (uint64_t)hb, scst, ctr, ctx->d_flag);
+      WTG_LAUNCH_CHECK();
+      WTG_LAUNCH(ctx, "mld_tseg", k_mld_tseg, dim3((unsigned)wtg_ceil_div(grid, 256)), dim3(256), 0, tst, (uint64_t)hb,
+                 (uint32_t*)(ws + o_tseg), maxt);
+      WTG_LAUNCH_CHECK();
+    }
     mld_count_launch<KO>(ctx, (unsigned)grid, a);
     WTG_LAUNCH_CHECK();
     WTG_LAUNCH(ctx, "mld_scan", k_mld_scan1, dim3(nblocks), dim3(256), 0, tcnt, ploc, bsum,
@@ -1624,6 +1651,7 @@ int mld_sparse_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint64_t*
     q.tseg = a.tseg;
     q.seg_start = bs;
     q.seg_cnt = bc;
+    q.left = ask ? nb + 2 * cur : nullptr;
     mld_local_launch<KO>(ctx, (unsigned)(grid * LOC_TW), q);
     WTG_LAUNCH_CHECK();
   }
