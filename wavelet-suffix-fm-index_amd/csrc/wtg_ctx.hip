@@ -45,8 +45,12 @@ extern "C" int wtg_ctx_create(int device, wtg_ctx** out) {
   WTG_CHECK_HIP(hipEventCreateWithFlags(&c->h2d_ev, hipEventDisableTiming));
   WTG_CHECK_HIP(hipHostMalloc((void**)&c->h_stage, WTG_STAGE_BYTES, hipHostMallocDefault));
   std::memset(c->h_stage, 0, 256);
-  WTG_CHECK_HIP(hipMalloc(&c->d_small, 256));
-  WTG_CHECK_HIP(hipHostGetDevicePointer((void**)&c->d_flag, c->h_stage, 0));
+  WTG_CHECK_HIP(hipHostGetDevicePointer((void**)&c->d_stage, c->h_stage, 0));
+  WTG_CHECK_HIP(hipMalloc(&c->d_small, 512));
+  c->d_flag = (uint32_t*)((char*)c->d_small + 256);
+  uint32_t flags[64] = {};
+  std::memcpy(flags + WTG_FLAG_HOST, &c->d_stage, sizeof(c->d_stage));
+  WTG_CHECK_HIP(hipMemcpy(c->d_flag, flags, sizeof(flags), hipMemcpyHostToDevice));
   // library allocations come stream-ordered from the device's default pool,
   // which keeps freed memory for reuse (WTG_NO_POOL=1: plain hipMalloc)
   if (!std::getenv("WTG_NO_POOL")) {
@@ -96,6 +100,7 @@ static uint32_t flags_take(wtg_ctx* ctx) {
       f |= 1u << k;
       hf[k] = 0;
     }
+  if (f) (void)wtg_fill_u64(ctx, ctx->d_flag, WTG_FLAG_WORDS / 2, 0);  // (before what the stream runs next)
   return f;
 }
 

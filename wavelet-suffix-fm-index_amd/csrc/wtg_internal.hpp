@@ -39,9 +39,11 @@ struct wtg_ctx {
   size_t ws_bytes = 0;
   // error flags, one word per WTG_FLAG bit, in the pinned staging area: kernels
   // store to them (wtg_raise), so a call's last step is the stream's
-  // synchronization alone, with no copy queued for it
-  uint32_t* d_flag = nullptr;  // the area's first words, as the device sees them
-  void* d_small = nullptr;     // 256 device bytes for a call's counters
+  // synchronization alone, with no copy queued for it.  Each has a word in device
+  // memory before it, so that a kernel in which every wave finds an error stores once.
+  uint32_t* d_flag = nullptr;  // the words in device memory, then where the others are (in d_small)
+  void* d_small = nullptr;     // 512 device bytes: a call's counters, from 256 on d_flag
+  uint8_t* d_stage = nullptr;  // h_stage as the device sees it
   // pinned host staging for small transfers (async copies need no bounce
   // buffer): [0, 256) the error flags, [WTG_STAGE_D2H, +16 KiB) device-to-host
   // reads (each followed by a stream sync before use), [WTG_STAGE_H2D, +32 KiB)
@@ -85,6 +87,7 @@ int wtg_stage_d2h(wtg_ctx* ctx, void* dst, const void* d_src, size_t bytes);
 int wtg_stage_h2d(wtg_ctx* ctx, void* d_dst, const void* src, size_t bytes);
 // bits of the device error flags (word k of ctx->d_flag: bit k), decoded by wtg_ctx_sync
 constexpr uint32_t WTG_FLAG_WORDS = 4;
+constexpr uint32_t WTG_FLAG_HOST = 4;  // word of d_flag where the address of the pinned words begins
 constexpr uint32_t WTG_FLAG_WAIT = 1u;      // a bounded look-back wait expired
 constexpr uint32_t WTG_FLAG_BADSYM = 2u;    // input symbol >= 2^levels / tables inconsistent with the keys
 constexpr uint32_t WTG_FLAG_SA_RANKS = 4u;  // suffix ranks inconsistent
@@ -219,16 +222,24 @@ static inline int wtg_hi_host(uint64_t x) { int r = 0; if (!x) return 0; while (
 #define WTG_WAVE 64
 #define WTG_SPIN_LIMIT (1u << 26)   // bounded waits: iterations before giving up
 
-// raise an error flag (a plain store to pinned host memory: atomic read-modify-
-// write operations do not reach it; storing the same word twice is harmless)
-__device__ __forceinline__ void wtg_raise(uint32_t* err, uint32_t flag) {
-  __hip_atomic_store(err + __builtin_ctz(flag), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 __device__ __forceinline__ int lane_id() { return (int)__lane_id(); }
 __device__ __forceinline__ uint32_t mbcnt64(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                    __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+// raise an error flag: one lane of the wave, and of the waves the first, stores to
+// pinned host memory (a plain store: atomic read-modify-write operations do not reach
+// it).  The others mostly see the word that a wave before them left in their L2 (an older 0
+// costs one exchange more).
+__device__ __forceinline__ void wtg_raise(uint32_t* err, uint32_t flag) {
+  if (mbcnt64(__builtin_amdgcn_read_exec()) != 0) return;
+  const uint32_t k = (uint32_t)__builtin_ctz(flag);
+  if (__hip_atomic_load(err + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0) return;
+  const bool first = atomicExch(err + k, 1u) == 0;
+  __hip_atomic_store(err + k, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  if (!first) return;
+  uint32_t* const host = *reinterpret_cast<uint32_t* const*>(err + WTG_FLAG_HOST);
+  __hip_atomic_store(host + k, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 __device__ __forceinline__ uint64_t wave_ballot(bool p) { return __ballot(p); }
 __device__ __forceinline__ uint32_t popc64(uint64_t x) { return (uint32_t)__popcll(x); }

@@ -695,6 +695,7 @@ __global__ __launch_bounds__(T / 8) __attribute__((amdgpu_waves_per_eu(8))) void
   }
   if (threadIdx.x == 0) s_cpre[G] = ctot;
   __syncthreads();
+  bool off = false;  // tables inconsistent with the keys: what they put out of range is not written
   {
     const uint32_t r = threadIdx.x;
     uint32_t nw = 0;
@@ -704,11 +705,8 @@ __global__ __launch_bounds__(T / 8) __attribute__((amdgpu_waves_per_eu(8))) void
       const uint32_t cnt = s_tpre[hi] - s_tpre[lo];
       const uint64_t lb = (uint64_t)(a.s + j - a.lvl0) * n;  // the level's first bit
       const uint64_t gs = lb + s_cum[lo] + (s_cpre[hi] - s_cpre[lo]);
-      if (gs < lb || gs + cnt > lb + n) {
-        wtg_raise(a.err, WTG_FLAG_BADSYM);  // tables inconsistent with the keys: write nothing
-      } else if (cnt) {
-        nw = (uint32_t)(((gs + cnt - 1) >> 6) - (gs >> 6) + 1);
-      }
+      if (gs < lb || gs + cnt > lb + n) off = true;
+      else if (cnt) nw = (uint32_t)(((gs + cnt - 1) >> 6) - (gs >> 6) + 1);
       s_rgs[r] = gs;
       s_rls[r] = s_tpre[lo];
       s_rcnt[r] = cnt;
@@ -746,13 +744,14 @@ __global__ __launch_bounds__(T / 8) __attribute__((amdgpu_waves_per_eu(8))) void
       if (i < len) {
         const uint32_t x = s_k[i];
         const uint32_t dest = s_lb[(x >> sh) & (G - 1)] + i;
-        if (dest >= n) wtg_raise(a.err, WTG_FLAG_BADSYM);
+        if (dest >= n) off = true;
         else if constexpr (WIDE)
           reinterpret_cast<uint64_t*>(a.kout)[dest] = (uint64_t) reinterpret_cast<const K*>(a.keys)[src + (x & 0xFFFFu)];
         else reinterpret_cast<uint32_t*>(a.kout)[dest] = x;
       }
     }
   }
+  if (off) wtg_raise(a.err, WTG_FLAG_BADSYM);
 }
 
 // WTnode record v from the histogram prefix of all L bits (node (l, p) holds
@@ -1562,7 +1561,7 @@ int mld_sparse_t(wtg_ctx* ctx, const K* d_sym, uint64_t n, uint32_t L, uint64_t*
   // (the small nodes' kernel stores it to pinned memory: a read is a wait, without a copy)
   q.m = 1u << S;
   q.left = ask ? nb : nullptr;
-  q.tell = (uint32_t*)((char*)ctx->d_flag + WTG_STAGE_AUX + 64);
+  q.tell = (uint32_t*)(ctx->d_stage + WTG_STAGE_AUX + 64);
   mld_local_launch<KO>(ctx, (unsigned)wtg_ceil_div(n, LOC_W), q);
   WTG_LAUNCH_CHECK();
   uint32_t cur = 0;
