@@ -42,3 +42,29 @@ def test_both_paths_give_the_same_knots(wsfm, ctx, epochs):
         two.free()
         for d in dv:
             d.free()
+
+
+@pytest.mark.parametrize("ones", [1, 20, 31])
+def test_vectors_without_models(wsfm, ones):
+    """Vectors of too few ones for a model, in a context that only enqueues: their tables'
+    sources outlive the copies, and every query gets the plain answer."""
+    rng = np.random.default_rng(ones)
+    nb, nvec = 1 << 20, 200
+    with wsfm.Context(0) as ctx:
+        ctx.set_blocking(False)
+        at = [np.sort(rng.choice(nb, ones, replace=False)) for _ in range(nvec)]
+        dv = []
+        for a in at:
+            v = np.zeros(nb // 64 + 1, np.uint64)
+            np.bitwise_or.at(v, a >> 6, np.uint64(1) << (a & 63).astype(np.uint64))
+            dv.append(ctx.to_device(v))
+        ls = wsfm.LearnedSelect(ctx, dv, [nb] * nvec)
+        junk = [np.full(1 << 14, 0xFF, np.uint8) for _ in range(64)]  # (where freed sources lay)
+        vec, j = np.repeat(np.arange(nvec, dtype=np.uint32), ones), np.tile(np.arange(1, ones + 1, dtype=np.uint64), nvec)
+        for learned in (False, True):
+            assert np.array_equal(ls.select(vec, j, learned=learned), np.concatenate(at))
+        assert all(ls.info(b)["learned"] == 0 for b in range(nvec)) and len(junk) == 64
+        ctx.sync()
+        ls.free()
+        for d in dv:
+            d.free()

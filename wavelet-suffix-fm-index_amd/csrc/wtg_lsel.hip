@@ -1481,9 +1481,15 @@ extern "C" int wtg_lsel_build(wtg_ctx* ctx, uint32_t nvec, const uint64_t* const
   }
   if (!act.empty() && (rc = lsel_models(ctx, ls, P, nbits, pos, ns, act)) != WTG_OK) goto fail;
   if ((rc = wtg_finish(ctx)) != WTG_OK) goto fail;
+  if (!ctx->blocking && act.empty() && hipStreamSynchronize(ctx->stream) != hipSuccess) {  // (the models' last read waits)
+    wtg_set_error("wtg_lsel_build: sync failed");
+    rc = WTG_ERR_HIP;
+    goto fail;
+  }
   *out = ls;
   return WTG_OK;
 fail:
+  (void)hipStreamSynchronize(ctx->stream);  // the upload sources end with this call
   lsel_release(ctx, ls);
   return rc;
 }
