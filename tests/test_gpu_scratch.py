@@ -35,6 +35,31 @@ def test_trim_gives_back(wsfm):
         sa.free()
 
 
+def test_allocation_that_does_not_fit(wsfm):
+    """An allocation larger than the device gives the scratch back, fails, and leaves the
+    context usable; learned select, which allocates while it holds it, too."""
+    n = 1 << 23
+    t = wsfm.gen_dna(6, n)
+    with wsfm.Context(0) as ctx:
+        d, sa = ctx.to_device(t), ctx.empty(n, np.int64)
+        run = lambda: wsfm._check(wsfm.lib().wtg_suffix_array_gpu(ctx.h, d.ptr, n, sa.ptr))  # noqa: E731
+        run()
+        first, held = sa.get(), free_bytes(wsfm.lib())
+        with pytest.raises(wsfm.WtgError):
+            ctx.empty(1 << 42, np.uint8)
+        assert free_bytes(wsfm.lib()) - held >= 40 * n
+        run()
+        assert np.array_equal(sa.get(), first)
+        bits = ctx.to_device(np.append(np.random.default_rng(2).integers(0, 1 << 63, 1 << 14).astype(np.uint64), np.uint64(0)))
+        for _ in range(2):
+            ls = wsfm.LearnedSelect(ctx, [bits], [1 << 20])
+            assert ls.info(0)["nknots"] > 0
+            ls.free()
+            ctx.trim()
+        for x in (d, sa, bits):
+            x.free()
+
+
 def test_recorded_graph_outlives_larger_scratch(wsfm):
     """A recorded tree build reads the workspace; a suffix array and a learned select
     built after it, both with more scratch, leave it where it is."""

@@ -193,22 +193,26 @@ int wtg_ws_reserve(wtg_ctx* ctx, size_t bytes) {
   return WTG_OK;
 }
 
-int wtg_scratch_reserve(wtg_ctx* ctx, size_t bytes) {
-  if (bytes <= ctx->scratch_bytes) return WTG_OK;
-  WTG_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-  if (ctx->scratch) { WTG_CHECK_HIP(hipFree(ctx->scratch)); ctx->scratch = nullptr; ctx->scratch_bytes = 0; }
-  if (hipMalloc(&ctx->scratch, bytes) != hipSuccess) {
+wtg_scratch_use::wtg_scratch_use(wtg_ctx* c, size_t bytes) : ctx(c) {
+  if (bytes == 0 || ctx->scratch_used) return;
+  if (bytes > ctx->scratch_bytes) {
+    if (hipStreamSynchronize(ctx->stream) != hipSuccess) return;
+    if (ctx->scratch) (void)hipFree(ctx->scratch);
     ctx->scratch = nullptr;
-    (void)hipGetLastError();
-    wtg_set_error("scratch allocation failed");
-    return WTG_ERR_NOMEM;
+    ctx->scratch_bytes = 0;
+    if (hipMalloc(&ctx->scratch, bytes) != hipSuccess) {
+      ctx->scratch = nullptr;
+      (void)hipGetLastError();
+      return;
+    }
+    ctx->scratch_bytes = bytes;
   }
-  ctx->scratch_bytes = bytes;
-  return WTG_OK;
+  mem = (char*)ctx->scratch;
+  ctx->scratch_used = true;
 }
 
 extern "C" int wtg_ctx_trim(wtg_ctx* ctx) {
-  WTG_REQUIRE(ctx, "null ctx");
+  WTG_REQUIRE(ctx && !ctx->scratch_used, "wtg_ctx_trim: null ctx");
   WTG_TRY(wtg_set_device(ctx));
   WTG_CHECK_HIP(hipStreamSynchronize(ctx->stream));
   if (ctx->scratch) WTG_CHECK_HIP(hipFree(ctx->scratch));
@@ -245,7 +249,7 @@ extern "C" int wtg_malloc(wtg_ctx* ctx, void** dptr, uint64_t bytes) {
     return ctx->pooled ? hipMallocAsync(dptr, bytes ? bytes : 1, ctx->stream) : hipMalloc(dptr, bytes ? bytes : 1);
   };
   hipError_t e = take();
-  if (e != hipSuccess && (ctx->scratch || ctx->qscratch)) {  // what is kept for later calls may make room
+  if (e != hipSuccess && !ctx->scratch_used && (ctx->scratch || ctx->qscratch)) {  // what is kept for later calls may make room
     (void)hipGetLastError();
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone &&

@@ -52,9 +52,10 @@ struct wtg_ctx {
   hipEvent_t h2d_ev = nullptr;
   // where large query batches are put in order (wtg_query_scratch)
   void* qscratch = nullptr;
-  // scratch of calls that wait for their own work (wtg_scratch_reserve)
+  // scratch of calls that wait for their own work (wtg_scratch_use)
   void* scratch = nullptr;
   size_t scratch_bytes = 0;
+  bool scratch_used = false;  // by the call that is running: not to be given back
   // stream timer
   hipEvent_t t0 = nullptr, t1 = nullptr;
   // per-kernel timing
@@ -68,9 +69,17 @@ struct wtg_ctx {
 
 // workspace of at least `bytes`, 256-byte aligned regions carved by the caller
 int wtg_ws_reserve(wtg_ctx* ctx, size_t bytes);
-// ctx->scratch of at least `bytes`, for calls that cannot be captured: growing it,
-// or giving it back (wtg_ctx_trim), moves nothing that a recorded graph reads.
-int wtg_scratch_reserve(wtg_ctx* ctx, size_t bytes);
+// ctx->scratch of at least `bytes` while this lives (null: 0, or no memory for it), for calls
+// that cannot be captured: growing it, or giving it back (wtg_ctx_trim, or an
+// allocation that finds no memory), moves nothing that a recorded graph reads.
+struct wtg_scratch_use {
+  wtg_ctx* const ctx;
+  char* mem = nullptr;
+  wtg_scratch_use(wtg_ctx* c, size_t bytes);
+  ~wtg_scratch_use() { if (mem) ctx->scratch_used = false; }
+  wtg_scratch_use(const wtg_scratch_use&) = delete;
+  wtg_scratch_use& operator=(const wtg_scratch_use&) = delete;
+};
 // A block of `bytes` (the same in every call) for a batch of queries, allocated at
 // the first use, never moved, and freed with the context.  Null while the stream
 // is being captured (a graph may be replayed beside the context's other work) or

@@ -1114,10 +1114,10 @@ static int lsel_models(wtg_ctx* ctx, wtg_lsel* ls, const wtg_lsel_params& P, con
   WTG_CHECK_HIP(hipMemcpyAsync(d_cbase, cbase.data(), (na + 1) * 8, hipMemcpyHostToDevice, ctx->stream));
   WTG_TRY(wtg_fill_u64(ctx, d_err, 1, 0));
   Knot* d_scr = nullptr;  // the count pass keeps each chunk's first knots
-  const bool kept = nflat * LSEL_KEEP * sizeof(Knot) <= LSEL_KEEP_BYTES &&
-                    wtg_scratch_reserve(ctx, nflat * LSEL_KEEP * sizeof(Knot)) == WTG_OK;
-  const uint32_t keep = kept ? LSEL_KEEP : LSEL_KEEP_MIN;
-  if (kept) d_scr = (Knot*)ctx->scratch;
+  const uint64_t keep_bytes = nflat * LSEL_KEEP * sizeof(Knot);
+  const wtg_scratch_use kept(ctx, keep_bytes <= LSEL_KEEP_BYTES ? keep_bytes : 0);
+  const uint32_t keep = kept.mem ? LSEL_KEEP : LSEL_KEEP_MIN;
+  if (kept.mem) d_scr = (Knot*)kept.mem;
   else WTG_TRY(wtg_malloc(ctx, (void**)&d_scr, nflat * keep * sizeof(Knot) + 256));
   const unsigned gp = (unsigned)wtg_ceil_div(nflat, 4);  // a wave per chunk
   WTG_LAUNCH(ctx, "lsel_place", k_lsel_place, dim3(gp), dim3(256), 0, d_pv, d_cbase, na, nflat, gap_log,
@@ -1151,7 +1151,7 @@ static int lsel_models(wtg_ctx* ctx, wtg_lsel* ls, const wtg_lsel_params& P, con
   WTG_LAUNCH_CHECK();
   uint32_t perr = 0;
   const int prc = sync_copy(ctx, &perr, d_err, 4, hipMemcpyDeviceToHost);
-  if (!kept) wtg_free(ctx, d_scr);
+  if (!kept.mem) wtg_free(ctx, d_scr);
   WTG_TRY(prc);
   WTG_REQUIRE(perr == 0, "wtg_lsel_build: knot placement passes disagree");
   WTG_CHECK_HIP(hipMemcpyAsync(d_K0, d_K, nk_total * sizeof(Knot), hipMemcpyDeviceToDevice, ctx->stream));

@@ -600,8 +600,8 @@ extern "C" int wtg_suffix_array_gpu(wtg_ctx* ctx, const uint8_t* d_text, uint64_
   constexpr size_t SA_KEEP_MAX = 8ull << 30;
   char* mem = nullptr;
   int rc = WTG_OK;
-  const bool kept = o <= SA_KEEP_MAX && wtg_scratch_reserve(ctx, o) == WTG_OK;
-  if (kept) mem = (char*)ctx->scratch;
+  const wtg_scratch_use kept(ctx, o <= SA_KEEP_MAX ? o : 0);
+  if (kept.mem) mem = kept.mem;
   else WTG_TRY(wtg_malloc(ctx, (void**)&mem, o));
   k0 = (uint64_t*)(mem + o_k0);
   k1 = (uint64_t*)(mem + o_k1);
@@ -684,7 +684,7 @@ extern "C" int wtg_suffix_array_gpu(wtg_ctx* ctx, const uint8_t* d_text, uint64_
   rc = wtg_finish(ctx);
 out:
   if (rc != WTG_OK) wtg_abandon(ctx);
-  if (!kept) wtg_free(ctx, mem);
+  if (mem != kept.mem) wtg_free(ctx, mem);
   return rc;
 }
 #undef SA_LAUNCH_CHECK
