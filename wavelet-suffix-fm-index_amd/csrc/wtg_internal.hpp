@@ -81,9 +81,10 @@ struct wtg_scratch_use {
   wtg_scratch_use& operator=(const wtg_scratch_use&) = delete;
 };
 // A block of `bytes` (the same in every call) for a batch of queries, allocated at
-// the first use, never moved, and freed with the context.  Null while the stream
-// is being captured (a graph may be replayed beside the context's other work) or
-// when there is no memory: the caller then answers the batch as it came.
+// the first use, and given back by wtg_ctx_trim, by an allocation that finds no memory, or
+// with the context.  Null while the stream is being captured (a graph may be replayed
+// beside the context's other work) or when there is no memory: the caller then answers
+// the batch as it came.
 void* wtg_query_scratch(wtg_ctx* ctx, size_t bytes);
 constexpr size_t WTG_STAGE_AUX = 256;  // [256, 4096): reads collected by a later sync of the call
 constexpr size_t WTG_STAGE_D2H = 4096, WTG_STAGE_D2H_MAX = 16384;

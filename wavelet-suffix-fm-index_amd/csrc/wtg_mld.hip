@@ -501,10 +501,10 @@ __device__ __forceinline__ uint64_t lds_bits64(const uint32_t* row, uint32_t p) 
 }
 
 // T keys per tile (mld_tile_log), T / 8 threads (8 chunks of 64 keys per wave).
-// Bound by VALU issue (80% of the SIMDs' time; 11 instructions per 64 keys and
-// level, ~500 per wave for tables, runs and scatter), not by memory: the 7-level
-// pass over 2^28 uint32 keys 1.34 ms, 714 M instructions before the zero
-// prefixes moved to the scalar unit, 612 M since.
+// Bound by VALU issue (70% of the SIMDs' time in the 7-level pass over 2^28 uint32
+// keys, 1.33 ms under the profiler, and 77% in the 6-level one), not by memory: 714 M
+// instructions a 7-level pass while every wave kept the zero prefixes of its chunks
+// in vector registers, 570 M with them on the scalar unit and in one LDS word a wave.
 // WIDE (trees of more than 32 levels): the level loop moves the leaf d above
 // the key's place in the tile instead of the key, and the scatter reads the
 // 64-bit key again by that place

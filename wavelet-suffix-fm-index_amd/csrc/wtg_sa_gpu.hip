@@ -8,9 +8,9 @@
 // order (32 bits).  The suffixes still in groups of two or more form a list in
 // that order, (suffix, group rank) each.  A later round h = q, 2q, 4q, ... reads
 // every listed suffix's rank h bytes on (+ 1; 0 past the end) and orders each
-// group by it: groups that fit a block in LDS by counting the smaller and equal
-// ranks (k_sa_refine), larger ones by a radix sort of (group rank, rank h bytes
-// on).  New rank = group rank + the smaller ones.  A suffix alone in its new
+// group by it (k_sa_refine): groups that fit a block in LDS by counting the smaller and
+// equal ranks, or by a sort where a group is larger than SA_COUNT, and groups larger
+// than a block's by a radix sort of (group rank, rank h bytes on) over all of them.  New rank = group rank + the smaller ones.  A suffix alone in its new
 // group keeps its final rank (the ranks stay consistent, as in Larsson-Sadakane
 // doubling), its sa entry is written and it leaves the list; the end is an empty
 // list.
